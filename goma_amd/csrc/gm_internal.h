@@ -34,6 +34,23 @@ struct ElemLayout {
   long long off_mp, off_cv, off_cp, total;
 };
 
+// One triangular sweep of ILU(0) as per-wave streams of chunks (see
+// k_ilu_sweep): a patch's waves walk their streams in step, level by level.
+struct IluStream {
+  int *d_sp = nullptr;     // [npatch * waves + 1] chunk range of each wave
+  int *d_pre = nullptr;    // [npatch * waves] levels before the wave's first node
+  int4 *d_ctl = nullptr;   // [chunks] (first row in the patch | flags, rows, barriers, -)
+  int *d_idx = nullptr;    // [chunks * 64 * CE] column: row in the patch, halo slot or ~row
+  int *d_src = nullptr;    // [chunks * 64 * CE] position in the factors, -1: padding
+  int2 *d_node = nullptr;  // [nodes] (first row, last chunk) of each node
+  int *d_hptr = nullptr, *d_halo = nullptr;  // [npatch + 1], rows outside the patch it reads
+  void *d_val[2] = {nullptr, nullptr};       // per precision: the entries, in stream order
+  void *d_inv[2] = {nullptr, nullptr};       // per precision: [chunks][8][8] inverse triangles, at last chunks
+  long long chunks = 0, entries = 0;
+  int nodes = 0, lds_rows = 0;
+  bool halo_lds = true;    // every patch's rows and halo fit in LDS
+};
+
 struct IluPlan {
   int bins = -1;
   int ncol = 0, npatch = 0;
@@ -54,10 +71,10 @@ struct IluPlan {
   int *d_node_first = nullptr, *d_node_last = nullptr;  // [N] node row range of each row
   int levels = 0;             // total forward levels over all patches
   std::vector<long long> col_rows, col_nnzL, col_nnzU;  // per patch colour
-  // per-patch level schedules, [0] forward / factorisation, [1] backward
-  int *d_lv_ptr[2] = {nullptr, nullptr}, *d_lv_nstart[2] = {nullptr, nullptr};
-  int *d_lv_node[2] = {nullptr, nullptr}, *d_lv_rstart[2] = {nullptr, nullptr};
-  int *d_lv_row[2] = {nullptr, nullptr};
+  // per-patch level schedule of the factorisation
+  int *d_lv_ptr = nullptr, *d_lv_nstart = nullptr, *d_lv_node = nullptr, *d_lv_rstart = nullptr;
+  int *d_lv_row = nullptr;
+  IluStream sweep[2];         // forward, backward
 };
 
 struct KrylovWork {

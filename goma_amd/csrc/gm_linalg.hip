@@ -372,115 +372,223 @@ int gm_dot(gm_ctx *c, const double *a, const double *b, double *out) {
 // patch.  Inside a patch the rows keep their sequential (IKJ) order of
 // dependence; the host groups the patch's nodes into levels (a node depends
 // on every earlier node of the patch its rows reference in L, or later node in
-// U), and the workgroup walks the levels: all rows of a level first take the
-// contributions from outside their own node in parallel, then one thread per
-// node resolves the node's small diagonal block.  The arithmetic per entry is
-// the sequential algorithm's; only the summation order inside a row differs.
+// U), and the workgroup walks the levels.  The arithmetic per entry is the
+// sequential algorithm's; only the summation order inside a row differs.
 
 static constexpr int ILU_MAXPATCH = 8192;  // rows of one patch held in LDS by the sweeps
-static constexpr int ILU_NT = 256;         // threads per patch workgroup (sweeps)
+static constexpr int ILU_NW = 8;           // waves per patch workgroup (sweeps)
+static constexpr int ILU_D = 4;            // chunks a wave loads ahead
 static constexpr int ILU_FT = 512;         // threads per patch workgroup (factorisation)
+static constexpr int ILU_LDS = 160 * 1024; // LDS of a CU
+static constexpr int ILU_FIRST = 1 << 16, ILU_LAST = 1 << 17, ILU_R8 = 1 << 18;  // chunk flags
 
 struct IluLv {
   const int *rowptr, *col, *diag, *node_first, *node_last, *patch_row;
   const int *lv_ptr, *lv_nstart, *lv_node, *lv_rstart, *lv_row;
 };
 
-template <int G, typename T>
-__device__ inline T group_sum(T v) {
-#pragma unroll
-  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
+struct IluSw {
+  const int *patch_row, *sp, *pre, *idx, *hptr, *halo;
+  const int4 *ctl;
+};
+
+// v from the lane that the DPP control picks in the same row of 16 lanes
+template <int CTRL>
+__device__ inline float dpp_mov(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ inline double dpp_mov(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
+  const unsigned hi =
+      (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// sum over 8 consecutive lanes, on all of them: quad swaps, then the half-row mirror
+template <typename T>
+__device__ inline T sum8(T v) {
+  v += dpp_mov<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_mov<0x141>(v);  // row_half_mirror
   return v;
 }
 
-// forward sweep  y = L^-1 (P b),  L unit lower; y in permuted numbering
-template <typename VT, typename BT, typename WT, int G>
-__global__ __launch_bounds__(ILU_NT) void k_ilu_lower(IluLv S, const VT *__restrict__ lu,
-                                                      int patch0, const int *__restrict__ perm,
-                                                      const BT *__restrict__ b, WT *y) {
-  __shared__ WT s_y[ILU_MAXPATCH];
-  constexpr int NG = ILU_NT / G;
+// One triangular sweep over the patches of one colour: y = L^-1 (P b) (UPPER
+// false, L unit lower) or y = U^-1 y with the unpermuted copy in out (UPPER).
+//
+// The sweep is a chain of levels (about 65 for an 8 x 8 QUAD9 patch, 105 for
+// a 4 x 4 x 4 HEX27 one) with only a few nodes each, so it is bound by the
+// latency of one level, not by bandwidth.  Nothing but the solution itself
+// may therefore sit on that chain: the entries come from streams laid out in
+// the order they are used, one per wave, and are loaded ILU_D chunks ahead
+// into registers; the patch's rows and the rows of other patches it reads (its
+// halo) are in LDS; and a node's small triangle T is applied as its inverse,
+// already multiplied into the node's entries, T^-1 (b - B y) = T^-1 b -
+// (T^-1 B) y, where T^-1 b needs nothing of the level before.  A level is then
+// LDS reads of y, a few FMAs, one row reduction, an LDS write and a barrier.
+// A chunk is CE entries per lane of one node: four rows of 16 lanes, or eight
+// rows of 8 lanes (nodes of more than four unknowns).  LDSH: every patch's
+// halo is in LDS; otherwise a load of y may stand in the chain, and the wait
+// for it takes the loads in flight along.  A wave without a node in a level
+// only takes its barrier (ctl.z).
+// Measured on the 32 x 32 QUAD9 cavity (four patches a colour, 62 levels): 29
+// us a launch, 0.46 us a level; with the entries read through the CSR factors
+// level by level, two barriers a level and the triangle solved row after row
+// it took 226 (upper) and 190 us (lower).
+template <typename VT, typename BT, typename OT, int CE, bool UPPER, bool LDSH>
+__global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__restrict__ val,
+                                                           const VT *__restrict__ inv, int patch0,
+                                                           const int *__restrict__ perm,
+                                                           const BT *__restrict__ b, VT *y,
+                                                           OT *__restrict__ out) {
+  extern __shared__ __align__(16) unsigned char s_raw[];
+  VT *s_y = (VT *)s_raw;
   const int P = patch0 + blockIdx.x;
-  const int r0 = S.patch_row[P], r1 = S.patch_row[P + 1];
-  const int tid = threadIdx.x, lane = tid % G, grp = tid / G;
-  for (int l = S.lv_ptr[P]; l < S.lv_ptr[P + 1]; l++) {
-    const int ra = S.lv_rstart[l], rb = S.lv_rstart[l + 1];
-    for (int k = ra + grp; k < rb; k += NG) {
-      const int r = S.lv_row[k];
-      const int nf = S.node_first[r];
-      WT s = 0;
-      const int e = S.diag[r];
-      for (int t = S.rowptr[r] + lane; t < e; t += G) {
-        const int cc = S.col[t];
-        if (cc < nf) s += (WT)lu[t] * (cc >= r0 ? s_y[cc - r0] : y[cc]);
-      }
-      s = group_sum<G>(s);
-      if (lane == 0) s_y[r - r0] = (WT)b[perm[r]] - s;
+  const int r0 = S.patch_row[P], nr = S.patch_row[P + 1] - r0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c0 = S.sp[P * ILU_NW + w], c1 = S.sp[P * ILU_NW + w + 1];
+  const int npre = S.pre[P * ILU_NW + w];
+
+  VT rv[ILU_D][CE], ri[ILU_D];
+  int rx[ILU_D][CE];
+  int4 rc[ILU_D];
+  // The control words go through vector registers (vz is 0, but not known to
+  // be): a scalar load in flight would have to be waited for at every LDS wait.
+  const int vz = (tid >> 6) - w;
+  auto fetch = [&](int d, int c) {
+    rc[d] = S.ctl[c + vz];
+    const size_t at = (size_t)c * (64 * CE) + lane;
+#pragma unroll
+    for (int e = 0; e < CE; e++) {
+      rv[d][e] = val[at + 64 * e];
+      rx[d][e] = S.idx[at + 64 * e];
     }
-    __syncthreads();
-    for (int k = S.lv_nstart[l] + tid; k < S.lv_nstart[l + 1]; k += ILU_NT) {
-      const int nf = S.lv_node[k];
-      const int nl = S.node_last[nf];
-      for (int r = nf + 1; r <= nl; r++) {
-        WT s = s_y[r - r0];
-        for (int t = S.diag[r] - 1; t >= S.rowptr[r]; t--) {
-          const int cc = S.col[t];
-          if (cc < nf) break;
-          s -= (WT)lu[t] * s_y[cc - r0];
-        }
-        s_y[r - r0] = s;
+    ri[d] = inv[(size_t)c * 64 + lane];
+  };
+#pragma unroll
+  for (int d = 0; d < ILU_D; d++) fetch(d, c0 + d);  // the streams end in ILU_D spare chunks
+
+  for (int i = tid; i < nr; i += ILU_NW * 64) s_y[i] = UPPER ? y[r0 + i] : (VT)b[perm[r0 + i]];
+  const int h0 = S.hptr[P], nh = S.hptr[P + 1] - h0;
+  for (int i = tid; i < nh; i += ILU_NW * 64) s_y[nr + i] = y[S.halo[h0 + i]];
+  auto level_end = [&]() {  // the solution in LDS, nothing of the loads in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  level_end();
+  for (int k = 0; k < npre; k++) level_end();
+
+  VT acc = 0;
+  for (int c = c0; c < c1; c += ILU_D) {
+#pragma unroll
+    for (int d = 0; d < ILU_D; d++) {
+      const int flags = __builtin_amdgcn_readfirstlane(rc[d].x), n = __builtin_amdgcn_readfirstlane(rc[d].y);
+      const int bars = __builtin_amdgcn_readfirstlane(rc[d].z);
+      const int lsh = (flags & ILU_R8) ? 3 : 4;  // log2 of the lanes of a row
+      const int row = flags & (ILU_FIRST - 1), k = lane & ((1 << lsh) - 1);
+      VT s = acc;
+      if (flags & ILU_FIRST) s = k < n ? ri[d] * s_y[row + k] : (VT)0;
+#pragma unroll
+      for (int e = 0; e < CE; e++) {
+        const int j = rx[d][e];
+        s -= rv[d][e] * (LDSH || j >= 0 ? s_y[j] : y[~j]);
       }
+      acc = s;
+      fetch(d, c + d + ILU_D);
+      if (flags & ILU_LAST) {
+        s = sum8(s);
+        if (lsh == 4) s += dpp_mov<0x140>(s);  // row_mirror: the other half of the 16 lanes
+        const int i = lane >> lsh;
+        if (k == 0 && i < n) s_y[row + i] = s;
+      }
+      for (int q = 0; q < bars; q++) level_end();
     }
-    __syncthreads();
   }
-  for (int r = r0 + tid; r < r1; r += ILU_NT) y[r] = s_y[r - r0];
+  level_end();
+  for (int i = tid; i < nr; i += ILU_NW * 64) {
+    const VT v = s_y[i];
+    y[r0 + i] = v;
+    if (UPPER) out[perm[r0 + i]] = (OT)v;
+  }
 }
 
-// backward sweep x = U^-1 y in place on y (permuted), plus the unpermuted copy
-template <typename VT, typename WT, typename OT, int G>
-__global__ __launch_bounds__(ILU_NT) void k_ilu_upper(IluLv S, const VT *__restrict__ lu,
-                                                      int patch0, const int *__restrict__ perm,
-                                                      WT *y, OT *__restrict__ out) {
-  __shared__ WT s_x[ILU_MAXPATCH];
-  constexpr int NG = ILU_NT / G;
-  const int P = patch0 + blockIdx.x;
-  const int r0 = S.patch_row[P], r1 = S.patch_row[P + 1];
-  const int tid = threadIdx.x, lane = tid % G, grp = tid / G;
-  for (int l = S.lv_ptr[P]; l < S.lv_ptr[P + 1]; l++) {
-    const int ra = S.lv_rstart[l], rb = S.lv_rstart[l + 1];
-    for (int k = ra + grp; k < rb; k += NG) {
-      const int r = S.lv_row[k];
-      const int nl = S.node_last[S.node_first[r]];
-      WT s = 0;
-      const int e = S.rowptr[r + 1];
-      for (int t = S.diag[r] + 1 + lane; t < e; t += G) {
-        const int cc = S.col[t];
-        if (cc > nl) s += (WT)lu[t] * (cc < r1 ? s_x[cc - r0] : y[cc]);
-      }
-      s = group_sum<G>(s);
-      if (lane == 0) s_x[r - r0] = y[r] - s;
-    }
-    __syncthreads();
-    for (int k = S.lv_nstart[l] + tid; k < S.lv_nstart[l + 1]; k += ILU_NT) {
-      const int nf = S.lv_node[k];
-      const int nl = S.node_last[nf];
-      for (int r = nl; r >= nf; r--) {
-        WT s = s_x[r - r0];
-        const int d = S.diag[r];
-        for (int t = d + 1; t < S.rowptr[r + 1]; t++) {
-          const int cc = S.col[t];
-          if (cc > nl) break;
-          s -= (WT)lu[t] * s_x[cc - r0];
-        }
-        s_x[r - r0] = s / (WT)lu[d];
+// Inverse of each node's triangle of the factors (at most 8 x 8): entry (i, k)
+// at lane k of the lanes that row i has in the node's chunks, zero outside the
+// node's rows; at its first chunk's place.  A wave per node, in FP64.
+template <typename VT, bool UPPER>
+__global__ __launch_bounds__(256) void k_ilu_node_inv(int nodes, const int2 *__restrict__ node,
+                                                      const int *__restrict__ node_last,
+                                                      const int *__restrict__ rowptr,
+                                                      const int *__restrict__ col,
+                                                      const int *__restrict__ diag,
+                                                      const VT *__restrict__ lu, VT *__restrict__ inv) {
+  __shared__ double sm[4][8][9], sx[4][8][9];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + w, i = lane >> 3, k = lane & 7;
+  int n = 0;
+  if (t < nodes) {
+    const int nf = node[t].x;
+    n = node_last[nf] - nf + 1;
+    double v = 0.0;
+    if (i < n && k < n) {
+      const int r = nf + i, cc = nf + k, d = diag[r];
+      if (!UPPER) {
+        for (int p = d - 1; p >= rowptr[r] && col[p] >= cc; p--)
+          if (col[p] == cc) v = (double)lu[p];
+        if (i == k) v = 1.0;
+      } else {
+        for (int p = d; p < rowptr[r + 1] && col[p] <= cc; p++)
+          if (col[p] == cc) v = (double)lu[p];
       }
     }
-    __syncthreads();
+    sm[w][i][k] = v;
+    sx[w][i][k] = 0.0;
   }
-  for (int r = r0 + tid; r < r1; r += ILU_NT) {
-    const WT v = s_x[r - r0];
-    y[r] = v;
-    out[perm[r]] = (OT)v;
+  __syncthreads();
+  if (t < nodes && lane < n) {
+    const int c = lane;  // column c of the inverse
+    for (int a = 0; a < n; a++) {
+      const int r = UPPER ? n - 1 - a : a;
+      double s = r == c ? 1.0 : 0.0;
+      if (UPPER)
+        for (int j = r + 1; j < n; j++) s -= sm[w][r][j] * sx[w][j][c];
+      else
+        for (int j = 0; j < r; j++) s -= sm[w][r][j] * sx[w][j][c];
+      sx[w][r][c] = s / sm[w][r][r];
+    }
+  }
+  __syncthreads();
+  if (t < nodes) {
+    const int lsh = n > 4 ? 3 : 4, row = lane >> lsh, q = lane & ((1 << lsh) - 1);
+    inv[(size_t)node[t].y * 64 + lane] = (VT)(row < 8 && q < 8 ? sx[w][row][q] : 0.0);
+  }
+}
+
+// The factors' off-node entries in stream order, each node's rows multiplied by
+// the inverse of its triangle (zero where a chunk is padded); a wave per chunk.
+template <typename VT, int CE>
+__global__ __launch_bounds__(256) void k_ilu_pack(int chunks, const int4 *__restrict__ ctl,
+                                                  const int *__restrict__ src,
+                                                  const VT *__restrict__ lu,
+                                                  const VT *__restrict__ inv, VT *__restrict__ val) {
+  const int lane = threadIdx.x & 63;
+  for (int c = blockIdx.x * 4 + (threadIdx.x >> 6); c < chunks; c += gridDim.x * 4) {
+    const int4 ct = ctl[c];
+    const size_t at = (size_t)c * (64 * CE) + lane;
+    const int lsh = (ct.x & ILU_R8) ? 3 : 4, row = lane >> lsh, l = lane & ((1 << lsh) - 1);
+    const double iv = ct.y ? (double)inv[(size_t)ct.w * 64 + lane] : 0.0;
+#pragma unroll
+    for (int e = 0; e < CE; e++) {
+      const int k = src[at + 64 * e];
+      const double v = k >= 0 ? (double)lu[k] : 0.0;
+      double s = 0.0;
+      for (int q = 0; q < ct.y; q++) s += __shfl(iv, (row << lsh) + q) * __shfl(v, (q << lsh) + l);
+      val[at + 64 * e] = (VT)s;
+    }
   }
 }
 
@@ -563,7 +671,7 @@ __global__ void k_gather(long long n, const int *__restrict__ src, const VT *__r
     lu[i] = (DT)a[src[i]];
 }
 
-static IluLv lv_args(const IluPlan &P, bool upper) {
+static IluLv lv_args(const IluPlan &P) {
   IluLv S;
   S.rowptr = P.d_rowptr;
   S.col = P.d_col;
@@ -571,22 +679,23 @@ static IluLv lv_args(const IluPlan &P, bool upper) {
   S.node_first = P.d_node_first;
   S.node_last = P.d_node_last;
   S.patch_row = P.d_patch_row;
-  const int u = upper ? 1 : 0;
-  S.lv_ptr = P.d_lv_ptr[u];
-  S.lv_nstart = P.d_lv_nstart[u];
-  S.lv_node = P.d_lv_node[u];
-  S.lv_rstart = P.d_lv_rstart[u];
-  S.lv_row = P.d_lv_row[u];
+  S.lv_ptr = P.d_lv_ptr;
+  S.lv_nstart = P.d_lv_nstart;
+  S.lv_node = P.d_lv_node;
+  S.lv_rstart = P.d_lv_rstart;
+  S.lv_row = P.d_lv_row;
   return S;
 }
 
 static void free_plan(IluPlan &P) {
   void *ptrs[] = {P.d_perm, P.d_rowptr, P.d_col, P.d_diag, P.d_src, P.d_patch_row, P.d_lu,
-                  P.d_lu32, P.d_y, P.d_y32, P.d_node_first, P.d_node_last};
+                  P.d_lu32, P.d_y, P.d_y32, P.d_node_first, P.d_node_last,
+                  P.d_lv_ptr, P.d_lv_nstart, P.d_lv_node, P.d_lv_rstart, P.d_lv_row};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
-  for (int u = 0; u < 2; u++) {
-    void *q[] = {P.d_lv_ptr[u], P.d_lv_nstart[u], P.d_lv_node[u], P.d_lv_rstart[u], P.d_lv_row[u]};
+  for (const IluStream &T : P.sweep) {
+    void *q[] = {T.d_sp, T.d_pre, T.d_ctl, T.d_idx, T.d_src, T.d_node, T.d_hptr, T.d_halo,
+                 T.d_val[0], T.d_val[1], T.d_inv[0], T.d_inv[1]};
     for (void *p : q)
       if (p) (void)hipFree(p);
   }
@@ -597,6 +706,151 @@ template <typename T>
 static int up(T **d, const std::vector<T> &h) {
   GM_HIP(hipMalloc(d, std::max<size_t>(h.size(), 1) * sizeof(T)));
   if (!h.empty()) GM_HIP(hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+  return GM_OK;
+}
+
+struct IluHost {
+  const std::vector<int> &rowptr, &col, &diag, &node_first, &node_last;
+};
+
+// The per-wave chunk streams of one sweep (k_ilu_sweep): each level's nodes
+// dealt to the waves in turn, a node's couplings to the patch's other nodes
+// (or to rows outside the patch) cut into chunks of CE entries per lane.
+static int build_stream(IluPlan &P, const IluHost &H, bool upper, int CE,
+                        const std::vector<int> &lv_ptr, const std::vector<int> &lv_nstart,
+                        const std::vector<int> &lv_node) {
+  IluStream &T = P.sweep[upper ? 1 : 0];
+  const int np = P.npatch;
+  // off-node entries of row r: [first, last) of its CSR range
+  auto range = [&](int r, int *a, int *e) {
+    const int nf = H.node_first[r], nl = H.node_last[nf];
+    if (!upper) {
+      *a = H.rowptr[r];
+      *e = H.diag[r];
+      while (*e > *a && H.col[*e - 1] >= nf) (*e)--;
+    } else {
+      *a = H.diag[r] + 1;
+      *e = H.rowptr[r + 1];
+      while (*a < *e && H.col[*a] <= nl) (*a)++;
+    }
+  };
+  // the off-node columns of a node's rows, ascending
+  auto columns = [&](int nf, std::vector<int> &u) {
+    u.clear();
+    for (int r = nf; r <= H.node_last[nf]; r++) {
+      int a, e;
+      range(r, &a, &e);
+      u.insert(u.end(), H.col.begin() + a, H.col.begin() + e);
+    }
+    std::sort(u.begin(), u.end());
+    u.erase(std::unique(u.begin(), u.end()), u.end());
+  };
+  // chunks of each node, in level order
+  std::vector<int> nchunk(lv_node.size());
+#pragma omp parallel
+  {
+    std::vector<int> u;
+#pragma omp for schedule(static)
+    for (size_t k = 0; k < lv_node.size(); k++) {
+      const int nf = lv_node[k], per = (H.node_last[nf] - nf + 1 > 4 ? 8 : 16) * CE;
+      columns(nf, u);
+      nchunk[k] = std::max(1, ((int)u.size() + per - 1) / per);
+    }
+  }
+  // stream lengths, rounded up to whole groups of ILU_D chunks
+  std::vector<int> sp((size_t)np * ILU_NW + 1, 0), pre((size_t)np * ILU_NW, 0);
+  for (int p = 0; p < np; p++)
+    for (int l = lv_ptr[p]; l < lv_ptr[p + 1]; l++)
+      for (int k = lv_nstart[l]; k < lv_nstart[l + 1]; k++)
+        sp[(size_t)p * ILU_NW + (k - lv_nstart[l]) % ILU_NW + 1] += nchunk[k];
+  for (size_t i = 1; i < sp.size(); i++) {
+    const long long len = (sp[i] + ILU_D - 1) / ILU_D * ILU_D + (long long)sp[i - 1];
+    if (len + ILU_D >= (1LL << 31)) {
+      gm_set_error("ILU sweep streams too long");
+      return GM_ERR_ARG;
+    }
+    sp[i] = (int)len;
+  }
+  T.chunks = (long long)sp.back() + ILU_D;
+  T.entries = T.chunks * 64 * CE;
+  T.nodes = (int)lv_node.size();
+  std::vector<int4> ctl(T.chunks, make_int4(0, 0, 0, 0));
+  std::vector<int> idx(T.entries, 0), src(T.entries, -1);
+  std::vector<int2> node(lv_node.size());
+  std::vector<std::vector<int>> halo(np);
+  T.lds_rows = 1;
+#pragma omp parallel for schedule(dynamic, 1)
+  for (int p = 0; p < np; p++) {
+    const int r0 = P.patch_row[p], r1 = P.patch_row[p + 1];
+    // rows outside the patch that it reads: in LDS behind its own when they fit
+    std::vector<int> &h = halo[p], u;
+    for (int k = lv_nstart[lv_ptr[p]]; k < lv_nstart[lv_ptr[p + 1]]; k++)
+      for (int r = lv_node[k]; r <= H.node_last[lv_node[k]]; r++) {
+        int a, e;
+        range(r, &a, &e);
+        for (int t = a; t < e; t++)
+          if (H.col[t] < r0 || H.col[t] >= r1) h.push_back(H.col[t]);
+      }
+    std::sort(h.begin(), h.end());
+    h.erase(std::unique(h.begin(), h.end()), h.end());
+    const bool fits = (size_t)(r1 - r0 + h.size()) * sizeof(double) <= (size_t)ILU_LDS;
+    if (!fits) h.clear();
+    int at[ILU_NW];
+    int last[ILU_NW];
+    for (int w = 0; w < ILU_NW; w++) {
+      at[w] = sp[(size_t)p * ILU_NW + w];
+      last[w] = -1;
+    }
+    for (int l = lv_ptr[p]; l < lv_ptr[p + 1]; l++) {
+      for (int k = lv_nstart[l]; k < lv_nstart[l + 1]; k++) {
+        const int w = (k - lv_nstart[l]) % ILU_NW;
+        const int nf = lv_node[k], n = H.node_last[nf] - nf + 1, lanes = n > 4 ? 8 : 16;
+        columns(nf, u);
+        for (int i = 0; i < n; i++) {
+          int t, e;
+          range(nf + i, &t, &e);
+          for (int q = 0; q < (int)u.size(); q++) {
+            const int ch = at[w] + q / (lanes * CE), rem = q % (lanes * CE), cc = u[q];
+            const size_t pos = (size_t)ch * 64 * CE + (size_t)(rem / lanes) * 64 + i * lanes + rem % lanes;
+            if (t < e && H.col[t] == cc) src[pos] = t++;
+            if (cc >= r0 && cc < r1) idx[pos] = cc - r0;
+            else if (fits)
+              idx[pos] = r1 - r0 + (int)(std::lower_bound(h.begin(), h.end(), cc) - h.begin());
+            else idx[pos] = ~cc;
+          }
+        }
+        for (int ch = 0; ch < nchunk[k]; ch++) {
+          int4 &ct = ctl[at[w] + ch];
+          ct.x = (nf - r0) | (ch == 0 ? ILU_FIRST : 0) | (ch == nchunk[k] - 1 ? ILU_LAST : 0) |
+                 (n > 4 ? ILU_R8 : 0);
+          ct.y = n;
+          ct.w = at[w];
+        }
+        at[w] += nchunk[k];
+        last[w] = at[w] - 1;
+        node[k] = make_int2(nf, last[w] + 1 - nchunk[k]);
+      }
+      for (int w = 0; w < ILU_NW; w++) {
+        if (last[w] < 0) pre[(size_t)p * ILU_NW + w]++;
+        else ctl[last[w]].z++;
+      }
+    }
+#pragma omp critical
+    {
+      T.lds_rows = std::max(T.lds_rows, r1 - r0 + (int)h.size());
+      T.halo_lds = T.halo_lds && fits;
+    }
+  }
+  std::vector<int> hptr(np + 1, 0), hall;
+  for (int p = 0; p < np; p++) {
+    hall.insert(hall.end(), halo[p].begin(), halo[p].end());
+    hptr[p + 1] = (int)hall.size();
+  }
+  int rc;
+  if ((rc = up(&T.d_sp, sp)) || (rc = up(&T.d_pre, pre)) || (rc = up(&T.d_ctl, ctl)) ||
+      (rc = up(&T.d_idx, idx)) || (rc = up(&T.d_src, src)) || (rc = up(&T.d_node, node)) ||
+      (rc = up(&T.d_hptr, hptr)) || (rc = up(&T.d_halo, hall)))
+    return rc;
   return GM_OK;
 }
 
@@ -738,15 +992,33 @@ int gm_ilu_plan(gm_ctx *c, int bins) {
       (rc = up(&P.d_diag, diag)) || (rc = up(&P.d_src, src)) || (rc = up(&P.d_patch_row, P.patch_row)) ||
       (rc = up(&P.d_node_first, node_first)) || (rc = up(&P.d_node_last, node_last)))
     return rc;
+  if ((rc = up(&P.d_lv_ptr, lv_ptr[0])) || (rc = up(&P.d_lv_nstart, lv_nstart[0])) ||
+      (rc = up(&P.d_lv_node, lv_node[0])) || (rc = up(&P.d_lv_rstart, lv_rstart[0])) ||
+      (rc = up(&P.d_lv_row, lv_row[0])))
+    return rc;
+  const IluHost H{rowptr, col, diag, node_first, node_last};
   for (int u = 0; u < 2; u++)
-    if ((rc = up(&P.d_lv_ptr[u], lv_ptr[u])) || (rc = up(&P.d_lv_nstart[u], lv_nstart[u])) ||
-        (rc = up(&P.d_lv_node[u], lv_node[u])) || (rc = up(&P.d_lv_rstart[u], lv_rstart[u])) ||
-        (rc = up(&P.d_lv_row[u], lv_row[u])))
+    if ((rc = build_stream(P, H, u == 1, c->dim == 2 ? 3 : 4, lv_ptr[u], lv_nstart[u], lv_node[u])))
       return rc;
   GM_HIP(hipMalloc(&P.d_lu, nnz * sizeof(double)));
   GM_HIP(hipMalloc(&P.d_y, N * sizeof(double)));
   P.bins = bins;
   return GM_OK;
+}
+
+// the sweeps' streams from the factors: entries and inverse triangles
+template <typename VT>
+static void ilu_streams(gm_ctx *c, const VT *lu, int pi) {
+  IluPlan &P = c->ilu;
+  for (int u = 0; u < 2; u++) {
+    IluStream &T = P.sweep[u];
+    auto kern = u ? k_ilu_node_inv<VT, true> : k_ilu_node_inv<VT, false>;
+    kern<<<(T.nodes + 3) / 4, 256, 0, c->stream>>>(T.nodes, T.d_node, P.d_node_last, P.d_rowptr,
+                                                   P.d_col, P.d_diag, lu, (VT *)T.d_inv[pi]);
+    auto pack = c->dim == 2 ? k_ilu_pack<VT, 3> : k_ilu_pack<VT, 4>;
+    pack<<<(int)std::min<long long>((T.chunks + 3) / 4, 16384), 256, 0, c->stream>>>(
+        (int)T.chunks, T.d_ctl, T.d_src, lu, (const VT *)T.d_inv[pi], (VT *)T.d_val[pi]);
+  }
 }
 
 // factorise the (scaled) Jacobian; prec 0: FP64 values, 1: FP32 values
@@ -756,6 +1028,13 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
     GM_HIP(hipMalloc(&P.d_lu32, P.nnz * sizeof(float)));
     GM_HIP(hipMalloc(&P.d_y32, c->N * sizeof(float)));
   }
+  const int pi = prec == GM_PREC_MIXED ? 1 : 0;
+  const size_t es = pi ? sizeof(float) : sizeof(double);
+  for (IluStream &T : P.sweep)
+    if (!T.d_val[pi]) {
+      GM_HIP(hipMalloc(&T.d_inv[pi], (size_t)T.chunks * 64 * es));
+      GM_HIP(hipMalloc(&T.d_val[pi], (size_t)T.entries * es));
+    }
   GM_HIP(hipMemsetAsync(c->d_flag + 2, 0, sizeof(int), c->stream));
   if (prec == GM_PREC_MIXED) {
     if (val32) k_gather<float, float><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val32, P.d_lu32);
@@ -763,7 +1042,7 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
   } else {
     k_gather<double, double><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val, P.d_lu);
   }
-  const IluLv S = lv_args(P, false);
+  const IluLv S = lv_args(P);
   for (int col = 0; col < P.ncol; col++) {
     const int p0 = P.colour_ptr[col], cnt = P.colour_ptr[col + 1] - p0;
     if (!cnt) continue;
@@ -774,6 +1053,8 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
       gm_launch(c, GM_K_ILU_FACT, 0.0, k_ilu_factor<double>, dim3(cnt), dim3(ILU_FT), 0, c->stream,
                 S, P.d_lu, p0, c->d_flag);
   }
+  if (prec == GM_PREC_MIXED) ilu_streams<float>(c, P.d_lu32, 1);
+  else ilu_streams<double>(c, P.d_lu, 0);
   GM_HIP(hipGetLastError());
   int flag = 0;
   GM_HIP(hipMemcpyAsync(&flag, c->d_flag + 2, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -786,36 +1067,39 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
 }
 
 // z = M^-1 r  (r, z unpermuted)
-template <typename VT, typename RT, typename ZT>
-static void ilu_apply(gm_ctx *c, const VT *lu, VT *ywork, const RT *r, ZT *z) {
+template <typename VT, typename RT, typename ZT, int CE>
+static int ilu_apply_ce(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
   IluPlan &P = c->ilu;
-  const IluLv SL = lv_args(P, false), SU = lv_args(P, true);
-  for (int col = 0; col < P.ncol; col++) {
-    const int p0 = P.colour_ptr[col], cnt = P.colour_ptr[col + 1] - p0;
-    if (!cnt) continue;
-    // L values + column ids, row pointers, diagonals, node ranges, level lists,
-    // permutation, input (gathered) and output vectors
-    const double bytes = (double)P.col_nnzL[col] * (sizeof(VT) + 4) +
-                         (double)P.col_rows[col] * (6 * 4 + sizeof(RT) + sizeof(VT));
-    if (c->dim == 2)
-      gm_launch(c, GM_K_ILU_LOWER, bytes, k_ilu_lower<VT, RT, VT, 16>, dim3(cnt), dim3(ILU_NT), 0,
-                c->stream, SL, lu, p0, P.d_perm, r, ywork);
-    else
-      gm_launch(c, GM_K_ILU_LOWER, bytes, k_ilu_lower<VT, RT, VT, 64>, dim3(cnt), dim3(ILU_NT), 0,
-                c->stream, SL, lu, p0, P.d_perm, r, ywork);
+  constexpr int pi = sizeof(VT) == 8 ? 0 : 1;
+  for (int u = 0; u < 2; u++) {
+    const IluStream &T = P.sweep[u];
+    auto kern = T.halo_lds ? (u ? k_ilu_sweep<VT, RT, ZT, CE, true, true> : k_ilu_sweep<VT, RT, ZT, CE, false, true>)
+                           : (u ? k_ilu_sweep<VT, RT, ZT, CE, true, false> : k_ilu_sweep<VT, RT, ZT, CE, false, false>);
+    const size_t lds = (size_t)T.lds_rows * sizeof(VT);
+    if (lds > 64 * 1024)
+      GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, ILU_LDS));
+    const IluSw S{P.d_patch_row, T.d_sp, T.d_pre, T.d_idx, T.d_hptr, T.d_halo, T.d_ctl};
+    for (int k = 0; k < P.ncol; k++) {
+      const int col = u ? P.ncol - 1 - k : k;
+      const int p0 = P.colour_ptr[col], cnt = P.colour_ptr[col + 1] - p0;
+      if (!cnt) continue;
+      // values + columns of the triangle, the permutation, the input (gathered)
+      // and output vectors
+      const double bytes = (double)(u ? P.col_nnzU[col] : P.col_nnzL[col]) * (sizeof(VT) + 4) +
+                           (double)P.col_rows[col] * (4 + (u ? 2 * sizeof(VT) + sizeof(ZT)
+                                                             : sizeof(RT) + sizeof(VT)));
+      gm_launch(c, u ? GM_K_ILU_UPPER : GM_K_ILU_LOWER, bytes, kern, dim3(cnt), dim3(ILU_NW * 64), lds,
+                c->stream, S, (const VT *)T.d_val[pi], (const VT *)T.d_inv[pi], p0,
+                (const int *)P.d_perm, r, ywork, z);
+    }
   }
-  for (int col = P.ncol - 1; col >= 0; col--) {
-    const int p0 = P.colour_ptr[col], cnt = P.colour_ptr[col + 1] - p0;
-    if (!cnt) continue;
-    const double bytes = (double)P.col_nnzU[col] * (sizeof(VT) + 4) +
-                         (double)P.col_rows[col] * (6 * 4 + 2 * sizeof(VT) + sizeof(ZT));
-    if (c->dim == 2)
-      gm_launch(c, GM_K_ILU_UPPER, bytes, k_ilu_upper<VT, VT, ZT, 16>, dim3(cnt), dim3(ILU_NT), 0,
-                c->stream, SU, lu, p0, P.d_perm, ywork, z);
-    else
-      gm_launch(c, GM_K_ILU_UPPER, bytes, k_ilu_upper<VT, VT, ZT, 64>, dim3(cnt), dim3(ILU_NT), 0,
-                c->stream, SU, lu, p0, P.d_perm, ywork, z);
-  }
+  return GM_OK;
+}
+
+template <typename VT, typename RT, typename ZT>
+static int ilu_apply(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
+  return c->dim == 2 ? ilu_apply_ce<VT, RT, ZT, 3>(c, ywork, r, z)
+                     : ilu_apply_ce<VT, RT, ZT, 4>(c, ywork, r, z);
 }
 
 // ---------------------------------------------------------------- Krylov kernels
@@ -951,7 +1235,7 @@ static int ensure_krylov(gm_ctx *c, int m, int prec) {
 // convergence ||b - A x|| / ||b - A x0|| < tol (Goma's AztecOO defaults
 // AZ_gmres / AZ_classic / AZ_r0, src/sl_util.c:392-960).
 template <typename BT, typename VT>
-static int gmres_t(gm_ctx *c, const VT *a, const VT *lu, VT *ywork, const double *b, double *x,
+static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x,
                    const gm_solver_opts *o, int *its_out, double *relres) {
   const int N = c->N, m = o->kspace;
   KrylovWork &K = c->kry;
@@ -972,7 +1256,7 @@ static int gmres_t(gm_ctx *c, const VT *a, const VT *lu, VT *ywork, const double
     } else if (o->precond == GM_PC_BAND) {
       gm_band_apply(c, (const double *)in, (double *)out);
     } else if (pc) {
-      ilu_apply<VT, BT, BT>(c, lu, ywork, in, out);
+      (void)ilu_apply<VT, BT, BT>(c, ywork, in, out);
     } else {
       k_scale_into<BT><<<grid, 256, 0, c->stream>>>(N, in, 1.0, out);
     }
@@ -1103,9 +1387,9 @@ int gm_gmres_run_nofactor(gm_ctx *c, const double *val, const float *val32, cons
     }
     // FP32 Jacobian values and preconditioner; Krylov basis, dot products
     // and the update in FP64
-    return gmres_t<double, float>(c, val32, c->ilu.d_lu32, c->ilu.d_y32, b, x, o, its, relres);
+    return gmres_t<double, float>(c, val32, c->ilu.d_y32, b, x, o, its, relres);
   }
-  return gmres_t<double, double>(c, val, c->ilu.d_lu, c->ilu.d_y, b, x, o, its, relres);
+  return gmres_t<double, double>(c, val, c->ilu.d_y, b, x, o, its, relres);
 }
 
 void gm_free_linalg(gm_ctx *c) {

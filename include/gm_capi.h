@@ -377,8 +377,8 @@ int gm_mg_copy_coarse_inverse(const gm_ctx *ctx, double *out);
  * each array counted once per launch) of those launches. */
 #define GM_K_FILL 0       /* k_fill: assembly + scatter of one element colour */
 #define GM_K_SPMV 1       /* k_spmv_msr: MSR matvec */
-#define GM_K_ILU_LOWER 2  /* k_ilu_lower: forward sweep of one patch colour */
-#define GM_K_ILU_UPPER 3  /* k_ilu_upper: backward sweep of one patch colour */
+#define GM_K_ILU_LOWER 2  /* k_ilu_sweep: forward sweep of one patch colour */
+#define GM_K_ILU_UPPER 3  /* k_ilu_sweep: backward sweep of one patch colour */
 #define GM_K_ILU_FACT 4   /* k_ilu_factor: ILU(0) of one patch colour */
 #define GM_K_MDOT 5       /* k_mdot: Gram-Schmidt projections */
 #define GM_K_ORTH 6       /* k_orth_update: Gram-Schmidt update */

@@ -1077,7 +1077,7 @@ static int ilu_apply_ce(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
                            : (u ? k_ilu_sweep<VT, RT, ZT, CE, true, false> : k_ilu_sweep<VT, RT, ZT, CE, false, false>);
     const size_t lds = (size_t)T.lds_rows * sizeof(VT);
     if (lds > 64 * 1024)
-      GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, ILU_LDS));
+      GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const IluSw S{P.d_patch_row, T.d_sp, T.d_pre, T.d_idx, T.d_hptr, T.d_halo, T.d_ctl};
     for (int k = 0; k < P.ncol; k++) {
       const int col = u ? P.ncol - 1 - k : k;

@@ -317,6 +317,402 @@ __global__ void k_mlp_copy_out(int M, int n_out, const float *__restrict__ y, fl
   out[i] = y[(size_t)p * OUT_PAD + o];
 }
 
+// ------------------------------------------------ whole-network kernels
+// Networks of width 64 .. NET_W run through one kernel per batch: a workgroup
+// takes a tile of points through every layer with the activations in LDS.
+// Each product has the weights as the row operand and the points as the
+// columns, so a lane of the result holds four consecutive features of one
+// point: one 8-byte LDS write, and the next layer's operand is read back
+// along the features.  The four waves split a layer's features, so each reads
+// its own rows of the weights (from L2) and nothing is staged.  Sums run over
+// the same 32-feature steps as the layer-by-layer kernels: the same bits.
+static constexpr int NET_W = 256, NET_L = 16;
+static constexpr int NET_LDS = 160 * 1024;
+
+struct NetArgs {
+  int L, n_in, n_out, M, Mpad;
+  const bf16_t *W[NET_L], *WT[NET_L];
+  const float *b[NET_L];
+  InNorm nrm;
+  const float *in;
+  const int *idx;
+  float *out;  // prediction [M][n_out]
+  // training: targets and masks, 2 / (points x outputs) and the loss partials,
+  // and the layer inputs and pre-activation gradients as MFMA operands of a
+  // product over points: [features / 16][Mpad / 32][lane][8 points]
+  const float *t, *m;
+  float norm;
+  double *lpart;
+  bf16_t *actT[NET_L], *dzT[NET_L];
+};
+
+__device__ inline unsigned pack2(float a, float b) {
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, b2{(__bf16)a, (__bf16)b});
+}
+
+// The weights of a whole product, and the product with them: small tiles load
+// a layer's weights before the previous layer's tanh.
+template <int TN, int KS>
+__device__ inline void net_load(const bf16_t *__restrict__ W, int ldw, int row0, bf8 (&w)[KS][TN]) {
+  const int lane = threadIdx.x & 63;
+  const bf16_t *pw = W + (size_t)(row0 + (lane & 15)) * ldw + (lane >> 4) * 8;
+#pragma unroll
+  for (int k = 0; k < KS; k++)
+#pragma unroll
+    for (int i = 0; i < TN; i++) w[k][i] = load8(pw + (size_t)16 * i * ldw + 32 * k);
+}
+template <int TN, int TM, int KS>
+__device__ inline void net_mul(const bf8 (&w)[KS][TN], const bf16_t *s, int lds, f4 (&acc)[TN][TM]) {
+  const int lane = threadIdx.x & 63;
+  const bf16_t *ps = s + (size_t)(lane & 15) * lds + (lane >> 4) * 8;
+#pragma unroll
+  for (int k = 0; k < KS; k++) {
+    bf8 x[TM];
+#pragma unroll
+    for (int j = 0; j < TM; j++) x[j] = load8(ps + (size_t)16 * j * lds + 32 * k);
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+      for (int j = 0; j < TM; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k][i], x[j], acc[i][j], 0, 0, 0);
+  }
+}
+
+// acc[i][j] += W rows (row0 + 16 i ..) times the points 16 j .. of s over
+// 32 KS features; the weights of the next PD - 1 steps are in flight.
+template <int TN, int TM, int KS>
+__device__ inline void net_product(const bf16_t *__restrict__ W, int ldw, int row0,
+                                   const bf16_t *s, int lds, f4 (&acc)[TN][TM]) {
+  constexpr int PD = TM <= 2 ? KS : (KS < 2 ? KS : 2);
+  const int lane = threadIdx.x & 63, r = lane & 15, kg = (lane >> 4) * 8;
+  const bf16_t *pw = W + (size_t)(row0 + r) * ldw + kg;
+  const bf16_t *ps = s + (size_t)r * lds + kg;
+  bf8 w[PD][TN];
+#pragma unroll
+  for (int d = 0; d < PD; d++)
+#pragma unroll
+    for (int i = 0; i < TN; i++) w[d][i] = load8(pw + (size_t)16 * i * ldw + 32 * d);
+#pragma unroll
+  for (int k = 0; k < KS; k++) {
+    bf8 x[TM];
+#pragma unroll
+    for (int j = 0; j < TM; j++) x[j] = load8(ps + (size_t)16 * j * lds + 32 * k);
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+      for (int j = 0; j < TM; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k % PD][i], x[j], acc[i][j], 0, 0, 0);
+    if (k + PD < KS) {
+#pragma unroll
+      for (int i = 0; i < TN; i++) w[k % PD][i] = load8(pw + (size_t)16 * i * ldw + 32 * (k + PD));
+    }
+  }
+}
+
+// One tile of 16 TM points through a network of width 16 TN NW (NW waves).
+// Prediction (TRAIN false) keeps one layer's activations; training keeps
+// every layer's, forms the loss and the output deltas and walks back: the
+// gradient of a layer's pre-activations replaces the activations that its tanh
+// made.  Large batches are bound by tanhf (about 45 VALU instructions per
+// value against 16 MFMA cycles per 16 x 16 x 32): 128-point tiles, two
+// workgroups a CU, one's products beside the other's tanh.  Small batches are
+// bound by the latency of a layer (weights from L2, then the tanh): 32-point
+// tiles, so that a batch of 8192 still has a workgroup per CU, with the
+// features split over more waves.  Measured, 4-256x4-5 network: prediction of
+// 1,000,000 points 2.83 -> 0.87 ms (459 TFLOP/s); a training step of 8192
+// points 305 us in 29 launches -> 72 us in three (41 of them here).
+template <int NW, int TN, int TM, bool TRAIN>
+__global__ __launch_bounds__(64 * NW, NW == 4 && !TRAIN ? 2 : (NW + 3) / 4) void k_mlp_net(NetArgs A) {
+  constexpr int W = 16 * TN * NW, PTS = 16 * TM, LDW = W + 8, LD0 = 40, KS = W / 32, NT = 64 * NW;
+  extern __shared__ __align__(16) bf16_t s_net[];
+  bf16_t *s0 = s_net, *sa = s_net + PTS * LD0;  // inputs (then output deltas); activations
+  auto slot = [&](int l) { return TRAIN ? sa + (size_t)(l - 1) * PTS * LDW : sa; };  // input of layer l >= 1
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int r = lane & 15, g4 = (lane >> 4) * 4;
+  const int m0 = blockIdx.x * PTS, n0 = wave * 16 * TN;
+  for (int i = tid; i < PTS * 32; i += NT) {
+    const int p = m0 + (i >> 5), c = i & 31;
+    const long long src = p < A.M ? (A.idx ? A.idx[p] : p) : -1;
+    float v = 0.f;
+    if (src >= 0 && c < A.n_in) v = (A.in[src * A.n_in + c] - A.nrm.sh[c]) * A.nrm.sc[c];
+    s0[(i >> 5) * LD0 + c] = f2bf(v);
+  }
+  __syncthreads();
+  // training: a finished array of the tile (nf features in LDS) to global memory
+  auto export_tile = [&](const bf16_t *s, int ld, int nf, bf16_t *out) {
+    static_assert(!TRAIN || PTS == 32, "one operand step a tile");
+    for (int f = wave; f < nf / 16; f += NW) {
+      const bf16_t *at = s + (lane >> 4) * 8 * ld + 16 * f + r;
+      u4v v;
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] = (unsigned)at[2 * e * ld] | ((unsigned)at[(2 * e + 1) * ld] << 16);
+      *(u4v *)(out + ((size_t)f * (A.Mpad / 32) + blockIdx.x) * 512 + lane * 8) = v;
+    }
+  };
+  if (TRAIN) export_tile(s0, LD0, 16, A.actT[0]);
+  f4 acc[TN][TM];
+  const f4 z = f4{0.f, 0.f, 0.f, 0.f};
+  constexpr bool AHEAD = TM <= 2;  // a layer's weights in registers before its turn
+  bf8 wn[AHEAD ? KS : 1][TN];
+  for (int l = 0; l < A.L - 1; l++) {
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+      for (int j = 0; j < TM; j++) acc[i][j] = z;
+    if (l == 0) net_product<TN, TM, 1>(A.W[0], IN_PAD, n0, s0, LD0, acc);
+    else if constexpr (AHEAD) net_mul<TN, TM, KS>(wn, slot(l), LDW, acc);
+    else net_product<TN, TM, KS>(A.W[l], W, n0, slot(l), LDW, acc);
+    if constexpr (AHEAD)
+      if (l + 1 < A.L - 1) net_load<TN, KS>(A.W[l + 1], W, n0, wn);
+    const float *bias = A.b[l];
+    if (!TRAIN) __syncthreads();  // the layer's input has been read
+    bf16_t *dst = slot(l + 1);
+#pragma unroll
+    for (int i = 0; i < TN; i++) {
+      const int n = n0 + 16 * i + g4;
+      const f4 bv = *(const f4 *)(bias + n);
+#pragma unroll
+      for (int j = 0; j < TM; j++) {
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = tanhf(acc[i][j][q] + bv[q]);
+        const uint2 h = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+        *(uint2 *)(dst + (16 * j + r) * LDW + n) = h;
+      }
+    }
+    if (TRAIN && l == 0) {  // every wave is past the inputs once the next product starts
+      __syncthreads();
+      for (int i = tid; i < PTS * LD0; i += NT) s0[i] = 0;
+    }
+    __syncthreads();
+    if (TRAIN) export_tile(dst, LDW, W, A.actT[l + 1]);
+  }
+  // output layer: at most 8 outputs, 16 points a wave
+  double ls = 0.0;
+  for (int j = wave; j < TM; j += NW) {
+    f4 y[1][1] = {{z}};
+    net_product<1, 1, KS>(A.W[A.L - 1], W, 0, slot(A.L - 1) + (size_t)16 * j * LDW, LDW, y);
+    const int p = m0 + 16 * j + r;
+    const long long src = TRAIN && p < A.M ? (A.idx ? A.idx[p] : p) : -1;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int o = g4 + q;
+      if (!TRAIN) {
+        if (o < A.n_out && p < A.M) A.out[(long long)p * A.n_out + o] = y[0][0][q] + A.b[A.L - 1][o];
+        continue;
+      }
+      float d = 0.f;
+      if (src >= 0 && o < A.n_out) {
+        const float e = y[0][0][q] + A.b[A.L - 1][o] - A.t[src * A.n_out + o];
+        const float mk = A.m[src * A.n_out + o];
+        ls += (double)mk * (double)e * (double)e;
+        d = 2.f * mk * e * A.norm;
+      }
+      s0[(16 * j + r) * LD0 + o] = f2bf(d);
+    }
+  }
+  if constexpr (TRAIN) {
+  __shared__ double sh[NW];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) ls += __shfl_xor(ls, o, 64);
+  if (lane == 0) sh[wave] = ls;
+  __syncthreads();
+  if (tid == 0) {
+    double t = 0.0;
+    for (int w = 0; w < NW; w++) t += sh[w];
+    A.lpart[blockIdx.x] = t;
+  }
+  export_tile(s0, LD0, 16, A.dzT[A.L - 1]);
+  for (int l = A.L - 1; l >= 1; l--) {
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+      for (int j = 0; j < TM; j++) acc[i][j] = z;
+    if (l == A.L - 1) net_product<TN, TM, 1>(A.WT[l], OUT_PAD, n0, s0, LD0, acc);
+    else net_mul<TN, TM, KS>(wn, slot(l + 1), LDW, acc);
+    if (l > 1) net_load<TN, KS>(A.WT[l - 1], W, n0, wn);
+    bf16_t *dst = slot(l);
+#pragma unroll
+    for (int i = 0; i < TN; i++) {
+      const int n = n0 + 16 * i + g4;
+#pragma unroll
+      for (int j = 0; j < TM; j++) {
+        uint2 *at = (uint2 *)(dst + (16 * j + r) * LDW + n);
+        const uint2 a = *at;
+        const float a0 = bf2f((bf16_t)a.x), a1 = bf2f((bf16_t)(a.x >> 16)), a2 = bf2f((bf16_t)a.y),
+                    a3 = bf2f((bf16_t)(a.y >> 16));
+        const uint2 h = make_uint2(pack2(acc[i][j][0] * (1.f - a0 * a0), acc[i][j][1] * (1.f - a1 * a1)),
+                                   pack2(acc[i][j][2] * (1.f - a2 * a2), acc[i][j][3] * (1.f - a3 * a3)));
+        *at = h;
+      }
+    }
+    __syncthreads();
+    export_tile(dst, LDW, W, A.dzT[l - 1]);
+  }
+  }  // TRAIN
+}
+
+// Weight and bias gradients of every layer in one launch, from the deltas and
+// layer inputs in operand order (a wave's operand is 1 KB in a row): part[l][s][n][k] over the chunk s of SPLIT points, in
+// 32-point steps as k_mlp_wgrad.  A workgroup takes a 64 x 64 tile of one
+// layer and chunk; past the tiles, workgroups sum the biases of one layer and
+// chunk, points in order.  Rows of padded inputs and outputs are skipped from
+// 16 on.  The tiles of one chunk share their operands, so each XCD takes a
+// contiguous range of tiles.  Measured at 8192 points, width 256: 21 us for all layers
+// (33 with operands strided by the batch, 83 in five launches staged through LDS).
+struct WgradArgs {
+  int L, M, nsplit;
+  const bf16_t *D[NET_L], *X[NET_L];
+  int N[NET_L], K[NET_L], nlim[NET_L], klim[NET_L];
+  int tile0[NET_L + 1];
+  float *part[NET_L], *partb[NET_L];
+};
+__global__ __launch_bounds__(256) void k_mlp_wgrad_all(WgradArgs A) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int blk = xcd_block();
+  if (blk >= A.tile0[A.L]) {
+    blk -= A.tile0[A.L];
+    const int l = blk / A.nsplit, s = blk - l * A.nsplit;
+    const int mbeg = s * SPLIT, mend = min(A.M, mbeg + SPLIT);
+    for (int n = tid; n < A.nlim[l]; n += 256) {
+      const bf16_t *d = A.D[l] + ((size_t)(n >> 4) * (A.M / 32)) * 512 + (n & 15) * 8;
+      float sum = 0.f;
+      for (int mb = mbeg; mb < mend; mb += 128) {
+        u4v v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = *(const u4v *)(d + (mb / 32 + u / 4) * 512 + (u & 3) * 128);
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            sum += bf2f((bf16_t)(v[u][e] & 0xffffu));
+            sum += bf2f((bf16_t)(v[u][e] >> 16));
+          }
+      }
+      A.partb[l][(size_t)s * A.N[l] + n] = sum;
+    }
+    return;
+  }
+  int l = 0;
+  while (blk >= A.tile0[l + 1]) l++;
+  blk -= A.tile0[l];
+  const int tk = (A.klim[l] + 63) / 64, tn = (A.nlim[l] + 63) / 64;
+  const int s = blk / (tk * tn), rem = blk - s * tk * tn;
+  const int n0 = (rem / tk) * 64 + (wave >> 1) * 32, k0 = (rem % tk) * 64 + (wave & 1) * 32;
+  if (n0 >= A.nlim[l] || k0 >= A.klim[l]) return;
+  const bool n2 = n0 + 16 < A.nlim[l], k2 = k0 + 16 < A.klim[l];
+  const int mbeg = s * SPLIT, mend = min(A.M, mbeg + SPLIT);
+  const int r = lane & 15;
+  const size_t step = (size_t)(A.M / 32) * 512;  // 16 features
+  const bf16_t *pd = A.D[l] + (n0 / 16) * step + lane * 8, *px = A.X[l] + (k0 / 16) * step + lane * 8;
+  const size_t d1 = n2 ? step : 0, x1 = k2 ? step : 0;  // skipped rows repeat the first
+  f4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+  static_assert(PT % 128 == 0 && SPLIT % 128 == 0, "four 32-point steps at a time");
+  for (int mb = mbeg; mb < mend; mb += 128) {
+    bf8 a[4][2], b[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      a[u][0] = load8(pd + (mb / 32 + u) * 512);
+      a[u][1] = load8(pd + d1 + (mb / 32 + u) * 512);
+      b[u][0] = load8(px + (mb / 32 + u) * 512);
+      b[u][1] = load8(px + x1 + (mb / 32 + u) * 512);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][i], b[u][j], acc[i][j], 0, 0, 0);
+  }
+  float *out = A.part[l] + (size_t)s * A.N[l] * A.K[l];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      if ((i && !n2) || (j && !k2)) continue;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int n = n0 + 16 * i + 4 * (lane >> 4) + q, k = k0 + 16 * j + r;
+        out[(size_t)n * A.K[l] + k] = acc[i][j][q];
+      }
+    }
+}
+
+// Sums of the chunk partials in their order, then (adam set) the update of
+// every weight and bias and the weights' BF16 copies, or (adam not set) the
+// gradients themselves; block 0 also sums the loss partials.
+struct UpdateArgs {
+  int L, nsplit, nloss;
+  int blk0[NET_L + 1];  // first block of each layer
+  int N[NET_L], K[NET_L], Nr[NET_L], Kr[NET_L];
+  const float *part[NET_L], *partb[NET_L];
+  float *W[NET_L], *mW[NET_L], *vW[NET_L], *b[NET_L], *mb[NET_L], *vb[NET_L], *gW[NET_L], *gb[NET_L];
+  bf16_t *Wb[NET_L], *WbT[NET_L];
+  const double *lpart;
+  double lnorm, *loss;
+  int adam;
+  AdamArgs a;
+};
+__global__ __launch_bounds__(256) void k_mlp_update(UpdateArgs U) {
+  if (blockIdx.x == 0) {
+    __shared__ double sh[4];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < U.nloss; i += 256) s += U.lpart[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) *U.loss = (sh[0] + sh[1] + sh[2] + sh[3]) * U.lnorm;
+  }
+  int l = 0;
+  while ((int)blockIdx.x >= U.blk0[l + 1]) l++;
+  const int N = U.N[l], K = U.K[l], i = (blockIdx.x - U.blk0[l]) * 256 + threadIdx.x;
+  const AdamArgs a = U.a;
+  auto step = [&](float g, float *w, float *m, float *v) {
+    const float mi = a.b1 * *m + (1.f - a.b1) * g;
+    const float vi = a.b2 * *v + (1.f - a.b2) * g * g;
+    *m = mi;
+    *v = vi;
+    const float wn = *w - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+    *w = wn;
+    return wn;
+  };
+  const int n = i / K, k = i - n * K;
+  if (n < U.Nr[l] && k < U.Kr[l]) {
+    float g = 0.f;
+    const float *part = U.part[l] + i;
+    const size_t NK = (size_t)N * K;
+    int s = 0;
+    for (; s + 8 <= U.nsplit; s += 8) {
+      float p[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) p[u] = part[(s + u) * NK];
+#pragma unroll
+      for (int u = 0; u < 8; u++) g += p[u];
+    }
+    for (; s < U.nsplit; s++) g += part[s * NK];
+    if (U.adam) {
+      const bf16_t h = f2bf(step(g, U.W[l] + i, U.mW[l] + i, U.vW[l] + i));
+      U.Wb[l][i] = h;
+      U.WbT[l][(size_t)k * N + n] = h;
+    } else {
+      U.gW[l][i] = g;
+    }
+  }
+  if (i < U.Nr[l]) {
+    float g = 0.f;
+    for (int s = 0; s < U.nsplit; s++) g += U.partb[l][(size_t)s * N + i];
+    if (U.adam) step(g, U.b[l] + i, U.mb[l] + i, U.vb[l] + i);
+    else U.gb[l][i] = g;
+  }
+}
+
 // Network outputs at the nodes and element sample points -> unknowns.
 struct GuessMap {
   int num_nodes, num_elems, dim, energy, n_out, spe;  // spe: sample points per element
@@ -475,6 +871,11 @@ struct gm_mlp {
   float *din = nullptr, *dt = nullptr, *dm = nullptr;
   int *dperm = nullptr;
   long long adam_t = 0;
+  // whole-network training (k_mlp_net): transposed layer inputs and deltas
+  std::vector<bf16_t *> actT, dzT;
+  std::vector<float *> partL, partbL;
+  double *lpartN = nullptr;
+  long long ncap = 0;
   // inference / guess scratch
   float *gin = nullptr, *gout = nullptr;
   long long gcap = 0;
@@ -553,6 +954,158 @@ static InNorm in_norm(const gm_mlp *m) {
   return n;
 }
 
+// LDS of k_mlp_net: the padded inputs, and one layer's activations or (training)
+// every layer's
+static size_t net_lds(int width, int hidden, int pts, bool train) {
+  return ((size_t)pts * 40 + (size_t)(train ? hidden : 1) * pts * (width + 8)) * sizeof(bf16_t);
+}
+// the whole-network kernels take this network (others go layer by layer)
+static bool net_fits(const gm_mlp *m, bool train) {
+  return m->s.width <= NET_W && m->L <= NET_L &&
+         (!train || net_lds(m->s.width, m->s.hidden, 32, true) <= (size_t)NET_LDS - 1024);
+}
+
+template <bool LARGE, bool TRAIN>
+static int net_launch(gm_mlp *m, const NetArgs &A, long long points) {
+  constexpr int TM = LARGE ? 8 : 2;
+  const int w = m->s.width;
+  const size_t lds = net_lds(w, m->s.hidden, 16 * TM, TRAIN);
+  void (*kern)(NetArgs);
+  int nw = 4;
+  if constexpr (LARGE) {
+    kern = w == 64 ? k_mlp_net<4, 1, TM, TRAIN> : w == 128 ? k_mlp_net<4, 2, TM, TRAIN>
+         : w == 192 ? k_mlp_net<4, 3, TM, TRAIN> : k_mlp_net<4, 4, TM, TRAIN>;
+  } else {
+    kern = w == 64 ? k_mlp_net<4, 1, TM, TRAIN> : w == 128 ? k_mlp_net<8, 1, TM, TRAIN>
+         : w == 192 ? k_mlp_net<12, 1, TM, TRAIN> : k_mlp_net<8, 2, TM, TRAIN>;
+    nw = w == 64 ? 4 : w == 192 ? 12 : 8;
+  }
+  if (lds > 64 * 1024)
+    GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  kern<<<(unsigned)((points + 16 * TM - 1) / (16 * TM)), 64 * nw, lds, m->stream>>>(A);
+  return GM_OK;
+}
+
+static NetArgs net_args(const gm_mlp *m, const float *in, long long M) {
+  NetArgs A{};
+  A.L = m->L;
+  A.n_in = m->s.n_in;
+  A.n_out = m->s.n_out;
+  A.M = (int)M;
+  A.nrm.sh[0] = 0.f;
+  for (int i = 0; i < m->s.n_in; i++) {
+    A.nrm.sh[i] = (float)m->s.in_shift[i];
+    A.nrm.sc[i] = (float)m->s.in_scale[i];
+  }
+  A.in = in;
+  for (int l = 0; l < m->L; l++) {
+    A.W[l] = m->Wb[l];
+    A.WT[l] = m->WbT[l];
+    A.b[l] = m->b[l];
+  }
+  return A;
+}
+
+// y = network(in) on the device, one launch per 2^30 points
+static int net_predict(gm_mlp *m, long long npts, const float *in, float *out) {
+  int rc;
+  for (long long off = 0; off < npts; off += 1LL << 30) {
+    const long long M = std::min<long long>(1LL << 30, npts - off);
+    NetArgs A = net_args(m, in + off * m->s.n_in, M);
+    A.out = out + off * m->s.n_out;
+    // 128-point tiles from two workgroups a CU on
+    if (M >= 128 * 512) rc = net_launch<true, false>(m, A, M);
+    else rc = net_launch<false, false>(m, A, M);
+    if (rc) return rc;
+  }
+  return GM_OK;
+}
+
+static int ensure_net(gm_mlp *m, long long M) {
+  if (M <= m->ncap) return GM_OK;
+  const long long cap = std::max<long long>((M + PT - 1) / PT * PT, 4096);
+  const int nsplit = (int)((cap + SPLIT - 1) / SPLIT);
+  for (auto *v : {&m->actT, &m->dzT}) {
+    for (bf16_t *p : *v) dfree(p);
+    v->assign(m->L, nullptr);
+  }
+  for (auto *v : {&m->partL, &m->partbL}) {
+    for (float *p : *v) dfree(p);
+    v->assign(m->L, nullptr);
+  }
+  dfree(m->lpartN);
+  m->lpartN = nullptr;
+  m->ncap = 0;
+  int rc;
+  for (int l = 0; l < m->L; l++) {
+    // rows beyond the first 16 of a padded input or output are never touched
+    const size_t k = l == 0 ? 16 : m->K[l], n = l == m->L - 1 ? 16 : m->N[l];
+    if ((rc = dalloc(&m->actT[l], k * cap)) || (rc = dalloc(&m->dzT[l], n * cap)) ||
+        (rc = dalloc(&m->partL[l], (size_t)nsplit * m->N[l] * m->K[l])) ||
+        (rc = dalloc(&m->partbL[l], (size_t)nsplit * m->N[l])))
+      return rc;
+  }
+  if ((rc = dalloc(&m->lpartN, (size_t)cap / 32))) return rc;
+  m->ncap = cap;
+  return GM_OK;
+}
+
+// Loss and gradients of one batch (rows idx of the inputs, targets and masks,
+// or the first M); then Adam with `a`, or the gradients into gW / gb.
+static int net_step(gm_mlp *m, int M, const int *idx, const float *in, const float *t, const float *mk,
+                    long long slot, const AdamArgs *a) {
+  const int Mpad = (M + PT - 1) / PT * PT, L = m->L, nsplit = (Mpad + SPLIT - 1) / SPLIT;
+  const double norm = 1.0 / ((double)M * m->s.n_out);
+  NetArgs A = net_args(m, in, M);
+  WgradArgs G{};
+  UpdateArgs U{};
+  A.Mpad = G.M = Mpad;
+  A.idx = idx;
+  A.t = t;
+  A.m = mk;
+  A.norm = (float)norm;
+  A.lpart = m->lpartN;
+  U.lpart = m->lpartN;
+  U.nloss = Mpad / 32;
+  U.lnorm = norm;
+  U.loss = m->lossbuf + slot;
+  G.L = U.L = L;
+  G.nsplit = U.nsplit = nsplit;
+  for (int l = 0; l < L; l++) {
+    G.X[l] = A.actT[l] = m->actT[l];
+    G.D[l] = A.dzT[l] = m->dzT[l];
+    G.N[l] = U.N[l] = m->N[l];
+    G.K[l] = U.K[l] = m->K[l];
+    G.nlim[l] = l == L - 1 ? 16 : m->N[l];
+    G.klim[l] = l == 0 ? 16 : m->K[l];
+    G.tile0[l + 1] = G.tile0[l] + nsplit * ((G.nlim[l] + 63) / 64) * ((G.klim[l] + 63) / 64);
+    G.part[l] = m->partL[l];
+    G.partb[l] = m->partbL[l];
+    U.part[l] = m->partL[l];
+    U.partb[l] = m->partbL[l];
+    U.blk0[l + 1] = U.blk0[l] + m->Nr[l] * m->K[l] / 256 + 1;
+    U.Nr[l] = m->Nr[l];
+    U.Kr[l] = m->Kr[l];
+    U.W[l] = m->W[l];
+    U.mW[l] = m->mW[l];
+    U.vW[l] = m->vW[l];
+    U.b[l] = m->b[l];
+    U.mb[l] = m->mb[l];
+    U.vb[l] = m->vb[l];
+    U.gW[l] = m->gW[l];
+    U.gb[l] = m->gb[l];
+    U.Wb[l] = m->Wb[l];
+    U.WbT[l] = m->WbT[l];
+  }
+  U.adam = a != nullptr;
+  if (a) U.a = *a;
+  int rc = net_launch<false, true>(m, A, Mpad);
+  if (rc) return rc;
+  k_mlp_wgrad_all<<<G.tile0[L] + L * nsplit, 256, 0, m->stream>>>(G);
+  k_mlp_update<<<U.blk0[L], 256, 0, m->stream>>>(U);
+  return GM_OK;
+}
+
 static void gather(gm_mlp *m, int M, int Mpad, const int *idx, const float *in, const float *t,
                    const float *mk) {
   const long long total = (long long)Mpad * IN_PAD;
@@ -598,7 +1151,7 @@ static void backward(gm_mlp *m, int Mpad) {
   }
 }
 
-static void adam(gm_mlp *m, double lr, const gm_mlp_train_opts *o) {
+static AdamArgs adam_args(gm_mlp *m, double lr, const gm_mlp_train_opts *o) {
   m->adam_t++;
   AdamArgs a;
   a.lr = (float)lr;
@@ -607,6 +1160,10 @@ static void adam(gm_mlp *m, double lr, const gm_mlp_train_opts *o) {
   a.eps = (float)o->eps;
   a.c1 = (float)(1.0 - std::pow(o->beta1, (double)m->adam_t));
   a.c2 = (float)(1.0 - std::pow(o->beta2, (double)m->adam_t));
+  return a;
+}
+
+static void adam(gm_mlp *m, const AdamArgs &a) {
   for (int l = 0; l < m->L; l++) {
     const int NK = m->N[l] * m->K[l];
     k_mlp_adam_w<<<(NK + 255) / 256, 256, 0, m->stream>>>(m->N[l], m->K[l], m->Nr[l], m->Kr[l],
@@ -647,6 +1204,11 @@ static void free_mlp(gm_mlp *m) {
   for (bf16_t *p : m->Wb) ps.push_back(p);
   for (bf16_t *p : m->WbT) ps.push_back(p);
   for (bf16_t *p : m->act) ps.push_back(p);
+  for (auto *v : {&m->actT, &m->dzT})
+    for (bf16_t *p : *v) ps.push_back(p);
+  for (auto *v : {&m->partL, &m->partbL})
+    for (float *p : *v) ps.push_back(p);
+  ps.push_back(m->lpartN);
   void *more[] = {m->y,   m->dz[0], m->dz[1], m->part, m->partb, m->bt,  m->bm,  m->lpart,
                   m->lossbuf, m->din, m->dt,  m->dm,   m->dperm, m->gin, m->gout, m->gx, m->d_gpts,
                   m->Q,   m->wgt,  m->qpart, m->qc,  m->qv};
@@ -813,7 +1375,8 @@ extern "C" int gm_mlp_train(gm_mlp *m, const gm_mlp_train_opts *o, double *loss_
     return GM_ERR_ARG;
   }
   int rc;
-  if ((rc = ensure_cap(m, o->batch))) return rc;
+  const bool net = net_fits(m, true);
+  if ((rc = net ? ensure_net(m, o->batch) : ensure_cap(m, o->batch))) return rc;
   const long long steps = (m->npts + o->batch - 1) / o->batch;
   if ((rc = ensure_lossbuf(m, steps))) return rc;
   const long long total = steps * o->epochs;
@@ -834,11 +1397,16 @@ extern "C" int gm_mlp_train(gm_mlp *m, const gm_mlp_train_opts *o, double *loss_
       const int Mpad = (M + PT - 1) / PT * PT;
       const double frac = total > 1 ? (double)step / (double)(total - 1) : 1.0;
       const double lr = o->lr_final + 0.5 * (o->lr - o->lr_final) * (1.0 + std::cos(M_PI * frac));
+      const AdamArgs a = adam_args(m, lr, o);
+      if (net) {
+        if ((rc = net_step(m, M, m->dperm + b * o->batch, m->din, m->dt, m->dm, b, &a))) return rc;
+        continue;
+      }
       gather(m, M, Mpad, m->dperm + b * o->batch, m->din, m->dt, m->dm);
       forward(m, Mpad);
       loss(m, M, Mpad, b);
       backward(m, Mpad);
-      adam(m, lr, o);
+      adam(m, a);
     }
     GM_HIP(hipGetLastError());
     GM_HIP(hipMemcpyAsync(hl.data(), m->lossbuf, steps * sizeof(double), hipMemcpyDeviceToHost,
@@ -864,7 +1432,8 @@ extern "C" int gm_mlp_loss_grad(gm_mlp *m, int npts, const float *in, const floa
     return GM_ERR_ARG;
   const int Mpad = (npts + PT - 1) / PT * PT;
   int rc;
-  if ((rc = ensure_cap(m, Mpad)) || (rc = ensure_lossbuf(m, 1))) return rc;
+  const bool net = net_fits(m, true);
+  if ((rc = net ? ensure_net(m, Mpad) : ensure_cap(m, Mpad)) || (rc = ensure_lossbuf(m, 1))) return rc;
   float *din, *dt, *dm;
   if ((rc = dalloc(&din, (size_t)npts * m->s.n_in))) return rc;
   if ((rc = dalloc(&dt, (size_t)npts * m->s.n_out))) {
@@ -888,10 +1457,14 @@ extern "C" int gm_mlp_loss_grad(gm_mlp *m, int npts, const float *in, const floa
     gm_set_error("gm_mlp_loss_grad: upload failed");
     return done(GM_ERR_HIP);
   }
-  gather(m, npts, Mpad, nullptr, din, dt, dm);
-  forward(m, Mpad);
-  loss(m, npts, Mpad, 0);
-  backward(m, Mpad);
+  if (net) {
+    if ((rc = net_step(m, npts, nullptr, din, dt, dm, 0, nullptr))) return done(rc);
+  } else {
+    gather(m, npts, Mpad, nullptr, din, dt, dm);
+    forward(m, Mpad);
+    loss(m, npts, Mpad, 0);
+    backward(m, Mpad);
+  }
   if (hipStreamSynchronize(m->stream) != hipSuccess) {
     gm_set_error("gm_mlp_loss_grad: %s", hipGetErrorString(hipGetLastError()));
     return done(GM_ERR_HIP);
@@ -912,6 +1485,12 @@ extern "C" int gm_mlp_loss_grad(gm_mlp *m, int npts, const float *in, const floa
 extern "C" int gm_mlp_predict_dev(gm_mlp *m, long long npts, const float *in_dev, float *out_dev) {
   if (!m || npts < 0 || (npts && (!in_dev || !out_dev))) return GM_ERR_ARG;
   int rc;
+  if (net_fits(m, false)) {
+    if ((rc = net_predict(m, npts, in_dev, out_dev))) return rc;
+    GM_HIP(hipGetLastError());
+    GM_HIP(hipStreamSynchronize(m->stream));
+    return GM_OK;
+  }
   if ((rc = ensure_cap(m, std::min<long long>(std::max<long long>(npts, 1), 65536)))) return rc;
   for (long long off = 0; off < npts; off += m->cap) {
     const int M = (int)std::min<long long>(m->cap, npts - off);
@@ -933,6 +1512,13 @@ extern "C" int gm_mlp_predict_noalloc_dev(gm_mlp *m, long long npts, const float
     gm_set_error("gm_mlp_predict_noalloc_dev: layer width %d exceeds the scratch's %d features",
                  maxdim(m), NA_W);
     return GM_ERR_ARG;
+  }
+  if (net_fits(m, false)) {  // its activations stay in LDS
+    const int rc = net_predict(m, npts, in_dev, out_dev);
+    if (rc) return rc;
+    GM_HIP(hipGetLastError());
+    GM_HIP(hipStreamSynchronize(m->stream));
+    return GM_OK;
   }
   void *base = (m->dev >= 0 && m->dev < NA_MAX_DEV) ? g_scratch_ptr[m->dev] : nullptr;
   if (!base) {

@@ -13,17 +13,23 @@
 // entries outside the band start at zero and stay exactly zero (each of their
 // updates has a zero factor).  Without pivoting no fill leaves the band.
 //
-// Factorisation, right-looking in panels of NB = 64 columns:
-//   k_band_a11     A11 = L11 U11 (one workgroup, in LDS), for the first
-//                  panel; later ones are factored at the end of the previous
-//                  update, by the workgroup whose tile holds them;
-//   k_band_panel   L21 = A21 U11^-1 (a thread per row) and
-//                  U12 = L11^-1 A12 (a thread per column);
-//   k_band_update  A22 -= L21 U12 (64 x 64 tiles, 4 x 4 per thread).
-// A launch never writes what another of its workgroups reads.
-// Solve: forward and backward substitution, one launch per NB block: a wave
-// solves the block's triangle, the workgroup updates the rows the block
-// couples to.  Zero pivots are reported (GM_ERR_PIVOT), never divided by.
+// Factorisation, right-looking in panels of NB = 64 columns, with the inverse
+// triangles of each diagonal block, so that everything but that block is a
+// matrix product (FP64 matrix cores):
+//   k_band_diag    A11 = L11 U11, as L11^-1 and U11^-1, of the first panel;
+//                  later ones come at the end of the previous update, from the
+//                  workgroup whose tile holds them;
+//   k_band_panel   L21 = A21 U11^-1 and U12 = L11^-1 A12, a 64 x 64 tile each;
+//   k_band_update  A22 -= L21 U12 by 64 x 64 tiles.
+// The chain of panels bounds it for bandwidths of a few thousand, and in it
+// the diagonal block.  (The inverse of the whole block in place of its
+// triangles saves the panel launch, but costs a digit and a half: relative
+// residual 5.9e-10 against 7e-11 on a shear-thinning 8 x 8 case, 1.7e-11 with
+// scalar triangular solves.)
+// Solve: forward and backward by pairs of panels (SB = 128 unknowns), whose
+// operators k_band_ops forms for all pairs at once after the factorisation;
+// one launch per pair and direction.  Zero pivots are reported
+// (GM_ERR_PIVOT), never divided by.
 #include <algorithm>
 #include <cmath>
 
@@ -50,271 +56,355 @@ __global__ __launch_bounds__(256) void k_band_load(int N, const VT *__restrict__
   for (int k = bindx[i]; k < bindx[i + 1]; k++) ab[off + i + (size_t)bindx[k] * lda] = (T)val[k];
 }
 
-// In-place LU (no pivoting) of the kb x kb block in LDS by all 256 threads of
-// the workgroup (every thread must call it): on return s holds L (strictly
-// lower, unit diagonal implied) and U.
-template <typename T>
-__device__ inline void block_lu(T (*s)[NB + 1], int kb, int *flag) {
-  // thread (i = tid / 4, q = tid % 4) owns row i, columns q, q + 4, ..., q + 60
-  const int tid = threadIdx.x, i = tid >> 2, q = tid & 3;
-  for (int k = 0; k < kb; k++) {
-    __syncthreads();
-    T piv = s[k][k];
-    if (piv == T(0)) {
-      if (tid == 0) atomicOr(flag, 1);
-      piv = T(1);
-    }
-    const bool act = i > k && i < kb;
-    T l = T(0);
-    if (act) l = s[i][k] / piv;
-    __syncthreads();  // every thread has read s[i][k] and row k before they change
-    if (act) {
-      if (q == 0) s[i][k] = l;
+constexpr int SB = 2 * NB;  // unknowns a solve step takes
+constexpr int LDT = NB + 2; // LDS row of a 64 x 64 block
+constexpr int OPS = SB * SB * 2;  // operators of one pair of panels
+constexpr int TRI = 2 * NB * NB;   // inverse triangles of one panel
+
+typedef double d4v __attribute__((ext_vector_type(4)));
+
+// D[m][n] = sum_k fa(k, m) fb(k, n) over k < 64 on one wave's 32 x 32 quadrant
+// (m0, n0) of a 64 x 64 block; the lane holds rows m0 + 16 u + l / 16 + 4 r and
+// column n0 + 16 v + l % 16 (v_mfma_f64_16x16x4f64).
+template <typename FA, typename FB>
+__device__ __forceinline__ void product64(int m0, int n0, FA fa, FB fb, d4v (&acc)[2][2]) {
+  const int lane = threadIdx.x & 63, r16 = lane & 15, kk = lane >> 4;
 #pragma unroll
-      for (int c = 0; c < NB / 4; c++) {
-        const int j = q + 4 * c;
-        if (j > k && j < kb) s[i][j] -= l * s[k][j];
+  for (int k0 = 0; k0 < NB; k0 += 16) {
+    double a[4][2], b[4][2];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        a[q][u] = fa(k0 + 4 * q + kk, m0 + 16 * u + r16);
+        b[q][u] = fb(k0 + 4 * q + kk, n0 + 16 * u + r16);
+      }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int v = 0; v < 2; v++)
+          acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q][u], b[q][v], acc[u][v], 0, 0, 0);
+  }
+}
+__device__ inline void clear(d4v (&acc)[2][2]) {
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++) acc[u][v] = d4v{0.0, 0.0, 0.0, 0.0};
+}
+// f(row, column, value) over the quadrant's entries that this lane holds
+template <typename F>
+__device__ inline void each(int m0, int n0, const d4v (&acc)[2][2], F f) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) f(m0 + 16 * u + (lane >> 4) + 4 * r, n0 + 16 * v + (lane & 15), acc[u][v][r]);
+}
+
+// LU (no pivoting) of the 64 x 64 block s (LDS) by all 256 threads, as the
+// inverse triangles L^-1 (column-major, tri) and U^-1 (row-major, tri + 64 x
+// 64), each as its panel product reads it.  The
+// block is in registers (thread (tr, tc) of a 16 x 16 grid: rows tr + 16 a,
+// columns tc + 16 b) and both inverses grow in place: step k subtracts the
+// pivot row's multiples from the rows below it (their columns left of k hold
+// L^-1) and, right of k, from the rows above it (U^-1).  One barrier a step:
+// the pivot row and column pass through LDS, buffers alternating.
+__device__ __forceinline__ void block_triangles(const double (*s)[LDT], double *__restrict__ tri, int *flag) {
+  __shared__ double s_c[2][NB], s_r[2][NB];
+  const int tid = threadIdx.x, tr = tid & 15, tc = tid >> 4;
+  double A[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; a++)
+#pragma unroll
+    for (int b = 0; b < 4; b++) A[a][b] = s[tr + 16 * a][tc + 16 * b];
+  bool zero = false;
+#pragma unroll
+  for (int K = 0; K < 4; K++) {
+#pragma unroll 1
+    for (int r = 0; r < 16; r++) {
+      const int q = r & 1;
+      if (tc == r) {
+#pragma unroll
+        for (int a = 0; a < 4; a++) s_c[q][tr + 16 * a] = A[a][K];
+      }
+      if (tr == r) {
+#pragma unroll
+        for (int b = 0; b < 4; b++) s_r[q][tc + 16 * b] = A[K][b];
+      }
+      __syncthreads();
+      double piv = s_r[q][16 * K + r];
+      if (piv == 0.0) {
+        zero = true;
+        piv = 1.0;
+      }
+      const double d = 1.0 / piv;
+      double c[4], rb[4];
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        c[a] = s_c[q][tr + 16 * a];
+        rb[a] = s_r[q][tc + 16 * a] * d;
+      }
+      const double row = rb[K];  // the pivot row's scaled entry in column block K
+      const double lo = tc == r ? d : row, hi = tc < r ? 0.0 : lo;
+      const double own = A[K][K];
+      if (tc == r) {
+#pragma unroll
+        for (int a = 0; a < 4; a++) A[a][K] = 0.0;
+      }
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        if (a < K) {
+          A[a][K] -= c[a] * hi;
+#pragma unroll
+          for (int b = K + 1; b < 4; b++) A[a][b] -= c[a] * rb[b];
+        } else if (a > K) {
+#pragma unroll
+          for (int b = 0; b < 4; b++) A[a][b] -= c[a] * (b == K ? lo : rb[b]);
+        } else {
+          const double cl = tr > r ? c[a] : 0.0, ch = tr == r ? 0.0 : c[a];
+#pragma unroll
+          for (int b = 0; b < K; b++) A[a][b] -= cl * rb[b];
+          A[a][K] -= (tc < r ? cl : ch) * lo;
+#pragma unroll
+          for (int b = K + 1; b < 4; b++) A[a][b] -= ch * rb[b];
+        }
+      }
+      if (tr == r) {
+#pragma unroll
+        for (int b = K + 1; b < 4; b++) A[K][b] = rb[b];
+        A[K][K] = tc < r ? own : lo;
       }
     }
   }
-  __syncthreads();
-}
-
-// A11 = L11 U11 in place (the first panel, or a panel whose predecessor
-// launched no update).
-template <typename T>
-__global__ __launch_bounds__(256) void k_band_a11(int j0, int kb, T *__restrict__ ab, long long off,
-                                                  long long lda, int *flag) {
-  __shared__ T sA[NB][NB + 1];
-  T *__restrict__ base = ab + off;
-  const int tid = threadIdx.x;
-  for (int t = tid; t < NB * NB; t += 256) {
-    const int j = t >> 6, i = t & 63;
-    sA[i][j] = (i < kb && j < kb) ? base[(j0 + i) + (size_t)(j0 + j) * lda] : T(0);
-  }
-  block_lu<T>(sA, kb, flag);
-  for (int t = tid; t < NB * NB; t += 256) {
-    const int j = t >> 6, i = t & 63;
-    if (i < kb && j < kb) base[(j0 + i) + (size_t)(j0 + j) * lda] = sA[i][j];
-  }
-}
-
-// With A11 factored: workgroups [0, nrb) compute 256 rows of L21 each,
-// [nrb, gridDim.x) 256 columns of U12.  A11 is only read.
-template <typename T>
-__global__ __launch_bounds__(256) void k_band_panel(int j0, int kb, int R, int C, int nrb,
-                                                    T *__restrict__ ab, long long off, long long lda) {
-  __shared__ T sA[NB][NB + 1];
-  __shared__ T sR[NB];  // 1 / U11 diagonal
-  const int tid = threadIdx.x;
-  T *__restrict__ base = ab + off;
-  for (int t = tid; t < NB * NB; t += 256) {
-    const int j = t >> 6, i = t & 63;
-    sA[i][j] = (i < kb && j < kb) ? base[(j0 + i) + (size_t)(j0 + j) * lda] : T(0);
-  }
-  if (tid < NB) {
-    const T d = tid < kb ? base[(j0 + tid) + (size_t)(j0 + tid) * lda] : T(1);
-    sR[tid] = T(1) / (d == T(0) ? T(1) : d);
-  }
-  __syncthreads();
-  const int b = blockIdx.x;
-  if (b < nrb) {
-    // L21 row: l U11 = a
-    const int rr = b * 256 + tid;
-    if (rr >= R) return;
-    const size_t i = (size_t)j0 + kb + rr;
-    T a[NB];
+  if (zero && tid == 0) atomicOr(flag, 1);
 #pragma unroll
-    for (int k = 0; k < NB; k++) a[k] = k < kb ? base[i + (size_t)(j0 + k) * lda] : T(0);
+  for (int a = 0; a < 4; a++)
 #pragma unroll
-    for (int k = 0; k < NB; k++) {
-      if (k < kb) {
-        a[k] *= sR[k];
-#pragma unroll
-        for (int j = k + 1; j < NB; j++) a[j] -= a[k] * sA[k][j];
-      }
+    for (int b = 0; b < 4; b++) {
+      const int i = tr + 16 * a, j = tc + 16 * b;
+      tri[j * NB + i] = i > j ? A[a][b] : (i == j ? 1.0 : 0.0);
+      tri[NB * NB + i * NB + j] = i <= j ? A[a][b] : 0.0;
     }
-#pragma unroll
-    for (int k = 0; k < NB; k++)
-      if (k < kb) base[i + (size_t)(j0 + k) * lda] = a[k];
+}
+
+// Inverse triangles of the panel at j0 (kb columns, padded with the identity).
+template <typename T>
+__global__ __launch_bounds__(256) void k_band_diag(int j0, int kb, const T *__restrict__ ab, long long off,
+                                                   long long lda, double *__restrict__ tri, int *flag) {
+  __shared__ double s[NB][LDT];
+  const T *__restrict__ base = ab + off;
+  for (int t = threadIdx.x; t < NB * NB; t += 256) {
+    const int j = t >> 6, i = t & 63;
+    s[i][j] = (i < kb && j < kb) ? (double)base[(j0 + i) + (size_t)(j0 + j) * lda] : (i == j ? 1.0 : 0.0);
+  }
+  __syncthreads();
+  block_triangles(s, tri, flag);
+}
+
+// Workgroups [0, rt): 64 rows of L21 = A21 U11^-1; [rt, gridDim.x): 64 columns
+// of U12 = L11^-1 A12; in place, the window's rows [j0 + 64, re) and columns
+// [j0 + 64, ce).  The products are formed so that a column's entries of the
+// band lie along the lanes.
+template <typename T>
+__global__ __launch_bounds__(256) void k_band_panel(int j0, int re, int ce, int rt, T *__restrict__ ab,
+                                                    long long off, long long lda,
+                                                    const double *__restrict__ tri) {
+  __shared__ double s_u[NB][LDT];  // A12 [k][column]
+  T *__restrict__ base = ab + off;
+  const int tid = threadIdx.x, wave = tid >> 6, m0 = (wave >> 1) * 32, n0 = (wave & 1) * 32;
+  d4v acc[2][2];
+  clear(acc);
+  if ((int)blockIdx.x < rt) {
+    const int r0 = j0 + NB + blockIdx.x * NB;
+    const double *U = tri + NB * NB;
+    product64(m0, n0, [&](int k, int m) { return U[k * NB + m]; },
+              [&](int k, int i) {
+                return r0 + i < re ? (double)base[(size_t)(r0 + i) + (size_t)(j0 + k) * lda] : 0.0;
+              },
+              acc);
+    __syncthreads();  // every wave has read its rows
+    each(m0, n0, acc, [&](int m, int i, double v) {
+      if (r0 + i < re) base[(size_t)(r0 + i) + (size_t)(j0 + m) * lda] = (T)v;
+    });
   } else {
-    // U12 column: L11 u = a (unit lower)
-    const int cc = (b - nrb) * 256 + tid;
-    if (cc >= C) return;
-    const size_t j = (size_t)j0 + kb + cc;
-    T a[NB];
-#pragma unroll
-    for (int k = 0; k < NB; k++) a[k] = k < kb ? base[(j0 + k) + j * lda] : T(0);
-#pragma unroll
-    for (int k = 0; k < NB; k++) {
-      if (k < kb) {
-#pragma unroll
-        for (int i = k + 1; i < NB; i++) a[i] -= sA[i][k] * a[k];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NB; k++)
-      if (k < kb) base[(j0 + k) + j * lda] = a[k];
-  }
-}
-
-// A[rs..re) x [cs..ce) -= L(rows, k0..k0+K) U(k0..k0+K, cols), K taken in
-// chunks of NB; 64 x 64 tiles, 4 x 4 per thread (measured faster than 128 x 128
-// tiles with 8 x 8 per thread, whose LDS allows one workgroup per CU).  With
-// fuse > 0, workgroup (0, 0) -- whose tile then holds the next panel's
-// diagonal block, now final -- also factors that block's fuse x fuse corner in
-// place (from its own tile in LDS).
-template <typename T>
-__global__ __launch_bounds__(256) void k_band_update(int k0, int K, int rs, int re, int cs, int ce,
-                                                     int fuse, T *__restrict__ ab, long long off,
-                                                     long long lda, int *flag) {
-  __shared__ T sL[NB][NB + 1];  // [k][row]; then the updated tile of workgroup (0, 0), [row][col]
-  __shared__ T sU[NB][NB + 1];  // [k][column]
-  T *__restrict__ base = ab + off;
-  const int tid = threadIdx.x;
-  const int r0 = rs + blockIdx.x * NB, c0 = cs + blockIdx.y * NB;
-  const int tr = tid & 15, tc = tid >> 4;
-  T acc[4][4];
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) acc[u][v] = T(0);
-  for (int kc = 0; kc < K; kc += NB) {
-    const int kn = min(NB, K - kc);
-    if (kc) __syncthreads();
-    for (int t = tid; t < NB * NB; t += 256) {
-      const int k = t >> 6, i = t & 63;
-      sL[k][i] = (k < kn && r0 + i < re) ? base[(size_t)(r0 + i) + (size_t)(k0 + kc + k) * lda] : T(0);
-    }
+    const int c0 = j0 + NB + ((int)blockIdx.x - rt) * NB;
     for (int t = tid; t < NB * NB; t += 256) {
       const int j = t >> 6, k = t & 63;
-      sU[k][j] = (k < kn && c0 + j < ce) ? base[(size_t)(k0 + kc + k) + (size_t)(c0 + j) * lda] : T(0);
+      s_u[k][j] = c0 + j < ce ? (double)base[(size_t)(j0 + k) + (size_t)(c0 + j) * lda] : 0.0;
     }
     __syncthreads();
-    for (int k = 0; k < kn; k++) {
-      T a[4], bv[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        a[u] = sL[k][tr + 16 * u];
-        bv[u] = sU[k][tc + 16 * u];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[u][v] += a[u] * bv[v];
-    }
-  }
-  const bool fz = fuse > 0 && blockIdx.x == 0 && blockIdx.y == 0;
-  if (fz) __syncthreads();  // uniform per workgroup: sL is reused below
-#pragma unroll
-  for (int v = 0; v < 4; v++) {
-    const int cj = c0 + tc + 16 * v;
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int ri = r0 + tr + 16 * u;
-      if (ri < re && cj < ce) {
-        T *p = base + (size_t)ri + (size_t)cj * lda;
-        const T nv = *p - acc[u][v];
-        *p = nv;
-        if (fz) sL[tr + 16 * u][tc + 16 * v] = nv;
-      }
-    }
-  }
-  if (!fz) return;
-  block_lu<T>(sL, fuse, flag);
-  for (int t = tid; t < NB * NB; t += 256) {
-    const int j = t >> 6, i = t & 63;
-    if (i < fuse && j < fuse) base[(size_t)(r0 + i) + (size_t)(c0 + j) * lda] = sL[i][j];
+    product64(m0, n0, [&](int k, int j) { return s_u[k][j]; }, [&](int k, int i) { return tri[k * NB + i]; }, acc);
+    each(m0, n0, acc, [&](int j, int i, double v) {
+      if (c0 + j < ce) base[(size_t)(j0 + i) + (size_t)(c0 + j) * lda] = (T)v;
+    });
   }
 }
 
-// Forward substitution of one block: y[blk] = L11^-1 w[blk] (w holds b minus
-// the earlier blocks' contributions), then w[j0+kb .. j0+kb+R) -= L21 y[blk].
-// w[blk] is only read in this launch, so every workgroup solves the block
-// itself (from L11 staged in LDS); workgroup 0 writes it to y.
+// One 64 x 64 tile of A22 -= L21 U12 for the panel at j0, formed transposed so
+// that the band's columns are read and written along their rows.  With next >
+// 0, workgroup (0, 0), whose tile holds the next panel's diagonal block, now
+// final, takes the inverse triangles of its next x next corner into
+// tri_next.  Measured at bandwidth 620 (FP64): 44 us a panel (this
+// launch and k_band_panel) against 118 with an LU in LDS, two barriers a
+// column, and a thread's triangular solve per row and column.
 template <typename T>
-__global__ __launch_bounds__(256) void k_band_fwd(int j0, int kb, int R, const T *__restrict__ ab,
-                                                  long long off, long long lda, double *__restrict__ w,
-                                                  double *__restrict__ y) {
-  __shared__ T sT[NB][NB + 1];
-  __shared__ double sy[NB];
-  const T *__restrict__ base = ab + off;
-  const int tid = threadIdx.x, lane = tid & 63;
+__global__ __launch_bounds__(256) void k_band_update(int j0, int re, int ce, int next, T *__restrict__ ab,
+                                                     long long off, long long lda,
+                                                     double *__restrict__ tri_next, int *flag) {
+  __shared__ double s_u[NB][LDT];  // U12 [k][column]; then the updated tile of workgroup (0, 0)
+  T *__restrict__ base = ab + off;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m0 = (wave >> 1) * 32, n0 = (wave & 1) * 32;
+  const int r0 = j0 + NB + blockIdx.x * NB, c0 = j0 + NB + blockIdx.y * NB;
   for (int t = tid; t < NB * NB; t += 256) {
-    const int j = t >> 6, i = t & 63;
-    sT[i][j] = (i < kb && j < kb && i > j) ? base[(j0 + i) + (size_t)(j0 + j) * lda] : T(0);
+    const int j = t >> 6, k = t & 63;
+    s_u[k][j] = c0 + j < ce ? (double)base[(size_t)(j0 + k) + (size_t)(c0 + j) * lda] : 0.0;
   }
-  if (tid < NB) sy[tid] = tid < kb ? w[j0 + tid] : 0.0;
+  double cv[2][2][4];  // the tile itself, loaded ahead of the product
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int j = m0 + 16 * u + (lane >> 4) + 4 * r, i = n0 + 16 * v + (lane & 15);
+        cv[u][v][r] = (r0 + i < re && c0 + j < ce) ? (double)base[(size_t)(r0 + i) + (size_t)(c0 + j) * lda] : 0.0;
+      }
   __syncthreads();
-  if (tid < 64) {
-    double v = sy[lane];
-    for (int k = 0; k < kb; k++) {
-      const double vk = __shfl(v, k);
-      v -= (double)sT[lane][k] * vk;  // zero for lane <= k
-    }
-    sy[lane] = v;
-    if (blockIdx.x == 0 && lane < kb) y[j0 + lane] = v;
-  }
+  d4v acc[2][2];
+  clear(acc);
+  product64(m0, n0, [&](int k, int j) { return s_u[k][j]; },
+            [&](int k, int i) {
+              return r0 + i < re ? (double)base[(size_t)(r0 + i) + (size_t)(j0 + k) * lda] : 0.0;
+            },
+            acc);
+  const bool fuse = next > 0 && blockIdx.x == 0 && blockIdx.y == 0;
+  if (fuse) __syncthreads();  // uniform per workgroup: s_u is reused below
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int j = m0 + 16 * u + (lane >> 4) + 4 * r, i = n0 + 16 * v + (lane & 15);
+        const double c = cv[u][v][r] - acc[u][v][r];
+        if (r0 + i < re && c0 + j < ce) base[(size_t)(r0 + i) + (size_t)(c0 + j) * lda] = (T)c;
+        if (fuse) s_u[i][j] = (i < next && j < next) ? (double)(T)c : (i == j ? 1.0 : 0.0);
+      }
+  if (!fuse) return;
   __syncthreads();
-  const int rr = blockIdx.x * 256 + tid;
-  if (rr >= R) return;
-  const size_t i = (size_t)j0 + kb + rr;
-  const T *__restrict__ col = base + i + (size_t)j0 * lda;
-  double s0 = 0.0, s1 = 0.0;
-  int k = 0;
-#pragma unroll 8
-  for (; k + 1 < kb; k += 2) {
-    s0 += (double)col[(size_t)k * lda] * sy[k];
-    s1 += (double)col[(size_t)(k + 1) * lda] * sy[k + 1];
-  }
-  if (k < kb) s0 += (double)col[(size_t)k * lda] * sy[k];
-  w[i] -= s0 + s1;
+  block_triangles(s_u, tri_next, flag);
 }
 
-// Backward substitution of one block: x[blk] = U11^-1 w[blk], then
-// w[j0-R .. j0) -= U(.., blk) x[blk].
+// Operators of one pair of panels (0, 1) from their inverse triangles and the
+// couplings L10, U01: column-major 128 x 128
+//   F = [L0^-1 0; -L1^-1 L10 L0^-1  L1^-1]   (forward:  y = F w)
+//   G = [U0^-1 -U0^-1 U01 U1^-1; 0 U1^-1]    (backward: x = G w)
+// A missing second panel has the identity and no couplings.
 template <typename T>
-__global__ __launch_bounds__(256) void k_band_bwd(int j0, int kb, int R, const T *__restrict__ ab,
-                                                  long long off, long long lda, double *__restrict__ w,
-                                                  double *__restrict__ x) {
-  __shared__ T sT[NB][NB + 1];
-  __shared__ double sx[NB], sr[NB];
+__global__ __launch_bounds__(256) void k_band_ops(int N, const T *__restrict__ ab, long long off, long long lda,
+                                                  int kl, int ku, int npanel,
+                                                  const double *__restrict__ tri, double *__restrict__ ops) {
+  __shared__ double s_t[NB][LDT];
   const T *__restrict__ base = ab + off;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x, wave = tid >> 6, m0 = (wave >> 1) * 32, n0 = (wave & 1) * 32;
+  const int j0 = blockIdx.x * SB, j1 = j0 + NB;
+  const bool two = 2 * (int)blockIdx.x + 1 < npanel;
+  const double *L0 = tri + (size_t)2 * blockIdx.x * TRI, *U0 = L0 + NB * NB, *L1 = L0 + TRI, *U1 = L1 + NB * NB;
+  double *F = ops + (size_t)blockIdx.x * OPS, *G = F + SB * SB;
+  auto l1 = [&](int i, int k) { return two ? L1[k * NB + i] : (i == k ? 1.0 : 0.0); };
+  auto u1 = [&](int i, int k) { return two ? U1[i * NB + k] : (i == k ? 1.0 : 0.0); };
+  auto l10 = [&](int i, int k) {
+    return two && j1 + i < N && NB + i - k <= kl ? (double)base[(size_t)(j1 + i) + (size_t)(j0 + k) * lda] : 0.0;
+  };
+  auto u01 = [&](int k, int j) {
+    return two && j1 + j < N && NB + j - k <= ku ? (double)base[(size_t)(j0 + k) + (size_t)(j1 + j) * lda] : 0.0;
+  };
   for (int t = tid; t < NB * NB; t += 256) {
     const int j = t >> 6, i = t & 63;
-    sT[i][j] = (i < kb && j < kb && i <= j) ? base[(j0 + i) + (size_t)(j0 + j) * lda] : T(0);
+    F[(size_t)j * SB + i] = L0[j * NB + i];
+    F[(size_t)(NB + j) * SB + NB + i] = l1(i, j);
+    F[(size_t)(NB + j) * SB + i] = 0.0;
+    G[(size_t)j * SB + i] = U0[i * NB + j];
+    G[(size_t)(NB + j) * SB + NB + i] = u1(i, j);
+    G[(size_t)j * SB + NB + i] = 0.0;
   }
-  if (tid < NB) {
-    sx[tid] = tid < kb ? w[j0 + tid] : 0.0;
-    const double d = tid < kb ? (double)base[(j0 + tid) + (size_t)(j0 + tid) * lda] : 1.0;
-    sr[tid] = 1.0 / (d == 0.0 ? 1.0 : d);
+  d4v acc[2][2];
+  clear(acc);  // L10 L0^-1
+  product64(m0, n0, [&](int k, int i) { return l10(i, k); }, [&](int k, int n) { return L0[n * NB + k]; }, acc);
+  each(m0, n0, acc, [&](int i, int n, double v) { s_t[i][n] = v; });
+  __syncthreads();
+  clear(acc);
+  product64(m0, n0, [&](int k, int i) { return l1(i, k); }, [&](int k, int n) { return s_t[k][n]; }, acc);
+  each(m0, n0, acc, [&](int i, int n, double v) { F[(size_t)n * SB + NB + i] = -v; });
+  __syncthreads();
+  clear(acc);  // U0^-1 U01
+  product64(m0, n0, [&](int k, int i) { return U0[i * NB + k]; }, [&](int k, int n) { return u01(k, n); }, acc);
+  each(m0, n0, acc, [&](int i, int n, double v) { s_t[i][n] = v; });
+  __syncthreads();
+  clear(acc);
+  product64(m0, n0, [&](int k, int i) { return s_t[i][k]; }, [&](int k, int n) { return u1(k, n); }, acc);
+  each(m0, n0, acc, [&](int i, int n, double v) { G[(size_t)(NB + n) * SB + i] = -v; });
+}
+
+// One solve step over the pair of panels at s0, by every workgroup: its 128
+// values v = op w from one 128 x 128 operator (1024 threads: 128 rows x 8
+// column groups), then 64 rows per workgroup of the other unknowns it couples
+// to, w -= A v: the R rows below (forward) or above (UP).  Workgroup 0 writes
+// v to out; w of the pair itself is only read.  All of a thread's matrix
+// entries are loaded before anything waits: a step is one round of memory
+// latency and two LDS reductions (64-unknown blocks with the triangle solved
+// by one wave's shuffles took 13 us forward and 17 backward; this takes
+// 6.1 us for 128).
+template <typename T, bool UP>
+__global__ __launch_bounds__(1024) void k_band_step(int N, int s0, int R, const T *__restrict__ ab,
+                                                    long long off, long long lda, int band,
+                                                    const double *__restrict__ ops, double *__restrict__ w,
+                                                    double *__restrict__ out) {
+  __shared__ double s_w[SB], s_red[16][SB], s_v[SB];
+  const T *__restrict__ base = ab + off;
+  const int tid = threadIdx.x, i = tid & (SB - 1), g = tid >> 7;
+  const int ri = tid & 63, rg = tid >> 6;
+  const double *op = ops + (size_t)(s0 / SB) * OPS + (UP ? SB * SB : 0);
+  const int rr = blockIdx.x * 64 + ri, row = UP ? s0 - R + rr : s0 + SB + rr;
+  double m[16], a[8];
+#pragma unroll
+  for (int k = 0; k < 16; k++) m[k] = op[(size_t)(16 * g + k) * SB + i];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const int j = s0 + 8 * rg + k;
+    a[k] = rr < R && j < N && (UP ? j - row : row - j) <= band ? (double)base[(size_t)row + (size_t)j * lda] : 0.0;
+  }
+  if (tid < SB) s_w[tid] = s0 + tid < N ? w[s0 + tid] : 0.0;
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < 16; k++) s += m[k] * s_w[16 * g + k];
+  s_red[g][i] = s;
+  __syncthreads();
+  if (tid < SB) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) v += s_red[k][tid];
+    s_v[tid] = v;
+    if (blockIdx.x == 0 && s0 + tid < N) out[s0 + tid] = v;
   }
   __syncthreads();
-  if (tid < 64) {
-    double v = sx[lane];
-    for (int k = kb - 1; k >= 0; k--) {
-      if (lane == k) v *= sr[k];
-      const double vk = __shfl(v, k);
-      if (lane < k) v -= (double)sT[lane][k] * vk;
-    }
-    sx[lane] = v;
-    if (blockIdx.x == 0 && lane < kb) x[j0 + lane] = v;
-  }
+  s = 0.0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) s += a[k] * s_v[8 * rg + k];
+  s_red[rg][ri] = s;
   __syncthreads();
-  const int rr = blockIdx.x * 256 + tid;
-  if (rr >= R) return;
-  const size_t i = (size_t)j0 - R + rr;
-  const T *__restrict__ col = base + i + (size_t)j0 * lda;
-  double s0 = 0.0, s1 = 0.0;
-  int k = 0;
-#pragma unroll 8
-  for (; k + 1 < kb; k += 2) {
-    s0 += (double)col[(size_t)k * lda] * sx[k];
-    s1 += (double)col[(size_t)(k + 1) * lda] * sx[k + 1];
+  if (tid < 64 && rr < R) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; k++) v += s_red[k][tid];
+    w[row] -= v;
   }
-  if (k < kb) s0 += (double)col[(size_t)k * lda] * sx[k];
-  w[i] -= s0 + s1;
 }
 
 __global__ __launch_bounds__(256) void k_band_copy(int n, const double *__restrict__ a, double *__restrict__ b) {
@@ -338,6 +428,10 @@ static int band_plan(gm_ctx *c) {
   B.ld = (long long)kl + ku + 1 + 2 * MG;
   GM_HIP(hipMalloc(&B.d_w1, (size_t)c->N * sizeof(double)));
   GM_HIP(hipMalloc(&B.d_w2, (size_t)c->N * sizeof(double)));
+  const size_t np = (c->N + NB - 1) / NB;
+  // (one panel beyond the last, so that an update's successor is always inside)
+  GM_HIP(hipMalloc(&B.d_tri, (np + 1) * TRI * sizeof(double)));
+  GM_HIP(hipMalloc(&B.d_ops, (np + 1) / 2 * OPS * sizeof(double)));
   return GM_OK;
 }
 
@@ -352,38 +446,28 @@ static int band_factor_t(gm_ctx *c, const VT *val, T *ab) {
   k_band_load<VT, T><<<(N + 255) / 256, 256, 0, s>>>(N, val, c->d_bindx, ab, off, lda);
   GM_HIP(hipMemsetAsync(c->d_flag + 4, 0, sizeof(int), s));
   int *d_pivflag = c->d_flag + 4;
-  bool a11_done = false;  // the next panel's A11 was factored by the last update
-  auto panel = [&](int j0, int kb) {
+  const int np = (N + NB - 1) / NB;
+  for (int k = 0; k < np; k++) {
+    const int j0 = k * NB, kb = std::min(NB, N - j0);
     const int R = std::min(kl, N - j0 - kb), C = std::min(ku, N - j0 - kb);
-    const int nrb = (R + 255) / 256, ncb = (C + 255) / 256;
-    if (!a11_done)
-      gm_launch(c, GM_K_BAND_PANEL, 2.0 * kb * kb * sizeof(T), k_band_a11<T>, dim3(1), dim3(256), 0, s,
-                j0, kb, ab, off, lda, d_pivflag);
-    a11_done = false;
-    if (nrb + ncb > 0) {
-      const double pbytes = ((double)kb * kb + (double)(R + C) * kb * 2.0) * sizeof(T);
-      gm_launch(c, GM_K_BAND_PANEL, pbytes, k_band_panel<T>, dim3(nrb + ncb), dim3(256), 0, s, j0, kb,
-                R, C, nrb, ab, off, lda);
-    }
-  };
-  auto update = [&](int k0, int K, int rs, int re, int cs, int ce, int fuse) {
-    if (re <= rs || ce <= cs) return;
-    const double ubytes = ((double)(re - rs + ce - cs) * K + 2.0 * (re - rs) * (ce - cs)) * sizeof(T);
-    gm_launch(c, GM_K_BAND_UPDATE, ubytes, k_band_update<T>,
-              dim3((re - rs + NB - 1) / NB, (ce - cs + NB - 1) / NB), dim3(256), 0, s, k0, K, rs, re, cs, ce,
-              fuse, ab, off, lda, d_pivflag);
-    if (fuse) a11_done = true;
-  };
-  for (int j0 = 0; j0 < N;) {
-    const int kb = std::min(NB, N - j0);
-    const int R = std::min(kl, N - j0 - kb), C = std::min(ku, N - j0 - kb);
-    const int next_kb = std::min(NB, std::max(0, N - j0 - kb));
-    panel(j0, kb);
+    const int next = std::min(NB, N - j0 - kb);
+    double *tri = B.d_tri + (size_t)k * TRI;
+    // a panel whose predecessor's window held its diagonal block has its triangles already
+    const bool done = k > 0 && std::min(kl, N - j0) >= kb && std::min(ku, N - j0) >= kb;
+    if (!done)
+      gm_launch(c, GM_K_BAND_PANEL, 2.0 * kb * kb * sizeof(T), k_band_diag<T>, dim3(1), dim3(256), 0, s, j0,
+                kb, (const T *)ab, off, lda, tri, d_pivflag);
+    if (R <= 0 && C <= 0) continue;
+    const int rt = (R + NB - 1) / NB, ct = (C + NB - 1) / NB;
+    gm_launch(c, GM_K_BAND_PANEL, 2.0 * (R + C) * NB * sizeof(T), k_band_panel<T>, dim3(rt + ct), dim3(256), 0,
+              s, j0, j0 + kb + R, j0 + kb + C, rt, ab, off, lda, (const double *)tri);
     if (R > 0 && C > 0)
-      update(j0, kb, j0 + kb, j0 + kb + R, j0 + kb, j0 + kb + C,
-             (next_kb > 0 && R >= next_kb && C >= next_kb) ? next_kb : 0);
-    j0 += kb;
+      gm_launch(c, GM_K_BAND_UPDATE, ((double)(R + C) * NB + 2.0 * R * C) * sizeof(T), k_band_update<T>,
+                dim3(rt, ct), dim3(256), 0, s, j0, j0 + kb + R, j0 + kb + C, R >= next && C >= next ? next : 0,
+                ab, off, lda, tri + TRI, d_pivflag);
   }
+  k_band_ops<T><<<(N + SB - 1) / SB, 256, 0, s>>>(N, (const T *)ab, off, lda, kl, ku, np,
+                                                  (const double *)B.d_tri, B.d_ops);
   GM_HIP(hipGetLastError());
   int flag = 0;
   GM_HIP(hipMemcpyAsync(&flag, c->d_flag + 4, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -429,20 +513,18 @@ static void band_apply_t(gm_ctx *c, const T *ab, const double *in, double *out) 
   const long long off = MG + ku, lda = B.ld - 1;
   hipStream_t s = c->stream;
   k_band_copy<<<1024, 256, 0, s>>>(N, in, B.d_w1);
-  for (int j0 = 0; j0 < N; j0 += NB) {
-    const int kb = std::min(NB, N - j0);
-    const int R = std::min(kl, N - j0 - kb);
-    const double bytes = ((double)kb * (kb + R)) * sizeof(T) + 16.0 * (kb + R);
-    gm_launch(c, GM_K_BAND_SOLVE, bytes, k_band_fwd<T>, dim3(std::max(1, (R + 255) / 256)), dim3(256), 0,
-              s, j0, kb, R, ab, off, lda, B.d_w1, B.d_w2);
+  const int ns = (N + SB - 1) / SB;
+  for (int b = 0; b < ns; b++) {
+    const int s0 = b * SB, R = std::max(0, std::min(kl, N - s0 - SB));
+    const double bytes = (double)SB * R * sizeof(T) + SB * SB * 8.0 + 16.0 * (SB + R);
+    gm_launch(c, GM_K_BAND_SOLVE, bytes, k_band_step<T, false>, dim3(std::max(1, (R + 63) / 64)), dim3(1024), 0,
+              s, N, s0, R, ab, off, lda, kl, (const double *)B.d_ops, B.d_w1, B.d_w2);
   }
-  const int nblk = (N + NB - 1) / NB;
-  for (int b = nblk - 1; b >= 0; b--) {
-    const int j0 = b * NB, kb = std::min(NB, N - j0);
-    const int R = std::min(ku, j0);
-    const double bytes = ((double)kb * (kb + R)) * sizeof(T) + 16.0 * (kb + R);
-    gm_launch(c, GM_K_BAND_SOLVE, bytes, k_band_bwd<T>, dim3(std::max(1, (R + 255) / 256)), dim3(256), 0,
-              s, j0, kb, R, ab, off, lda, B.d_w2, out);
+  for (int b = ns - 1; b >= 0; b--) {
+    const int s0 = b * SB, R = std::min(ku, s0);
+    const double bytes = (double)SB * R * sizeof(T) + SB * SB * 8.0 + 16.0 * (SB + R);
+    gm_launch(c, GM_K_BAND_SOLVE, bytes, k_band_step<T, true>, dim3(std::max(1, (R + 63) / 64)), dim3(1024), 0,
+              s, N, s0, R, ab, off, lda, ku, (const double *)B.d_ops, B.d_w2, out);
   }
 }
 
@@ -460,7 +542,7 @@ int gm_band_apply(gm_ctx *c, const double *in, double *out) {
 
 void gm_band_free(gm_ctx *c) {
   BandLU &B = c->band;
-  void *p[] = {B.d_ab[0], B.d_ab[1], B.d_w1, B.d_w2};
+  void *p[] = {B.d_ab[0], B.d_ab[1], B.d_w1, B.d_w2, B.d_tri, B.d_ops};
   for (void *q : p)
     if (q) (void)hipFree(q);
   c->band = BandLU();

@@ -96,6 +96,8 @@ struct BandLU {
   int prec = -1;              // precision of the last factorisation (0 FP64, 1 FP32)
   void *d_ab[2] = {nullptr, nullptr};  // [N][ld] per precision
   double *d_w1 = nullptr, *d_w2 = nullptr;  // solve work vectors
+  double *d_tri = nullptr;   // [panels][2][64][64] inverse triangles of the diagonal blocks
+  double *d_ops = nullptr;   // per pair of panels: the solve's operators (k_band_ops)
 };
 
 struct gm_ctx;

@@ -392,9 +392,9 @@ int gm_mg_copy_coarse_inverse(const gm_ctx *ctx, double *out);
 #define GM_K_MG_DENSE 13  /* k_dense_gemv: exact solve on the coarsest level (dense inverse) */
 #define GM_K_GALERKIN 14  /* k_galerkin: coarse element matrices P^T K P of one level */
 #define GM_K_ELEM_SCATTER 15 /* k_elem_scatter: element matrices of one colour into MSR */
-#define GM_K_BAND_PANEL 16 /* k_band_a11 / k_band_panel: one 64-column panel of the banded LU */
+#define GM_K_BAND_PANEL 16 /* k_band_diag / k_band_panel: one 64-column panel of the banded LU */
 #define GM_K_BAND_UPDATE 17 /* k_band_update: trailing update of one panel */
-#define GM_K_BAND_SOLVE 18 /* k_band_fwd / k_band_bwd: one 64-row block of the triangular solves */
+#define GM_K_BAND_SOLVE 18 /* k_band_step: 128 unknowns of one direction of the banded solve */
 #define GM_K_VANKA_GATHER 19 /* k_vanka_gather: additive smoother, element corrections summed per unknown */
 #define GM_K_ROW_SCALE 20 /* k_row_sum_scale: row sums and scaling of the Jacobian and residual */
 #define GM_K_COARSE_INV 21 /* k_gjb_panel / k_gjb_swap / k_gjb_update: one panel of the coarsest level's dense inverse */

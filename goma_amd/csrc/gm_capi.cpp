@@ -109,10 +109,12 @@ static void free_ctx(gm_ctx *c) {
                   c->d_resid, c->d_dx,    c->d_scale, c->d_val32,    c->d_red,   c->d_xwork,
                   c->d_xsave, c->d_rtrial, c->d_w, c->d_mg_rows, c->d_mg_wmul, c->d_kel,
                   c->d_mg_gptr, c->d_mg_gent, c->d_mg_corr, c->d_stab, c->d_qs_ptr,
-                  c->d_qs_side, c->d_qs_q, c->d_rank, c->d_nn_ptr, c->d_nn_list};
+                  c->d_qs_side, c->d_qs_q, c->d_rank, c->d_nn_ptr, c->d_nn_list, c->d_pair,
+                  c->d_rank_t, c->d_src, c->d_re, c->d_ct};
   for (void *p : ptrs)
     if (p) hipFree(p);
   if (c->h_red) hipHostFree(c->h_red);
+  if (c->h_flag) hipHostFree(c->h_flag);
   for (int i = 0; i < GM_K_COUNT; i++) {
     for (hipEvent_t e : c->ev_b[i]) hipEventDestroy(e);
     for (hipEvent_t e : c->ev_e[i]) hipEventDestroy(e);
@@ -210,6 +212,7 @@ static int create_impl(const gm_mesh *m, const gm_physics *ph, const gm_bc *bc, 
   if ((rc = upload(&c->d_ecol_elems, c->ecol_elems.data(), c->ecol_elems.size()))) return rc;
   GM_HIP(hipMalloc(&c->d_flag, 8 * sizeof(int)));
   GM_HIP(hipMemset(c->d_flag, 0, 8 * sizeof(int)));
+  GM_HIP(hipHostMalloc(&c->h_flag, sizeof(int), hipHostMallocDefault));
   GM_HIP(hipMalloc(&c->d_red, 2 * 1024 * sizeof(double)));
   GM_HIP(hipHostMalloc(&c->h_red, 128 * 1024 * sizeof(double), hipHostMallocDefault));
   return gm_fill_setup_device(c);
@@ -368,10 +371,8 @@ static int set_transient(gm_ctx *c, const double *x_old, const double *xdot_old,
 extern "C" int gm_matrix_fill_full_assign_dev(gm_ctx *c, const double *x, double *resid,
                                               double *val) {
   if (!c || !x || !resid || !val) return GM_ERR_ARG;
-  int rc;
-  if (!c->d_rank && (rc = gm_zero(c, val, c->nval))) return rc;
   c->fill_overwrite = 1;
-  rc = gm_fill_launch(c, x, resid, val, nullptr);
+  const int rc = gm_fill_launch(c, x, resid, val, nullptr);
   c->fill_overwrite = 0;
   return rc;
 }
@@ -599,16 +600,9 @@ static int solve_impl(gm_ctx *c, double *x, const gm_solver_opts *o, gm_newton_r
     }
     if ((rc = gm_zero(c, c->d_resid, c->N))) return rc;
     if ((rc = gm_zero(c, c->d_dx, c->N))) return rc;
-    // the HEX27 assembly stores each node pair's first contribution, so the
-    // Jacobian needs no zeroing pass
-    const bool assign = c->d_rank != nullptr;
-    if (!assign) {
-      if (prec == GM_PREC_MIXED) rc = gm_zero32(c, c->d_val32, c->nval);
-      else rc = gm_zero(c, c->d_val, c->nval);
-      if (rc) return rc;
-    }
+    // the assembly stores the Jacobian, which needs no zeroing pass
     c->kel_on = galerkin;
-    c->fill_overwrite = assign;
+    c->fill_overwrite = 1;
     rc = gm_fill_launch(c, x, c->d_resid, c->d_val, prec == GM_PREC_MIXED ? c->d_val32 : nullptr);
     c->kel_on = 0;
     c->fill_overwrite = 0;

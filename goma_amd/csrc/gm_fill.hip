@@ -1,22 +1,24 @@
 // Element assembly (matrix_fill_full) for QUAD9 / HEX27 Q2-P1 Navier-Stokes
 // with optional energy, as HIP kernels for gfx950.
 //
-// One workgroup assembles one element.  Elements are launched one colour at a
-// time (no two elements of a colour share a node), so every element owns the
+// QUAD9: k_elem2 forms the element matrices and vectors, four elements per
+// workgroup, and k_gather (gm_gather.hip) sums them into the rows.  HEX27:
+// k_fill3m, one workgroup per element, elements launched one colour at a time
+// (no two elements of a colour share a node), so every element owns the
 // nonzeros it scatters into during its launch and the scatter is a plain
-// read-modify-write: deterministic, no atomics.
+// read-modify-write.  Either way: deterministic, no atomics.
 //
 // Per element:
 //   1. nodal coordinates / unknowns -> LDS
 //   2. per quadrature point: map Jacobian, inverse, dA = detJ*w  (beer_belly)
 //   3. physical basis gradients grad_phi[q][k][p]                (load_bf_grad)
 //   4. per quadrature point: v, grad v, T, grad T, P, mu(gammadot), body force
-//   5. residual rows, then the Jacobian: thread t owns node pair (i,j) and
-//      accumulates every (row variable, column variable) block of that pair;
-//      pressure couplings are separate task lists.
+//   5. residual rows, then the Jacobian: the node-by-node blocks as products
+//      over the quadrature points on the FP64 matrix cores, pressure couplings
+//      as separate tasks.
 //   6. Dirichlet rows: J row -> unit diagonal, R -> x - V (per element, as
-//      put_dirichlet_in_matrix does, src/bc_dirich.c:44-153).
-//   7. scatter through the element-to-nonzero map into the MSR arrays.
+//      put_dirichlet_in_matrix does, src/bc_dirich.c:44-153), in the scatter.
+//   7. scatter into the MSR arrays.
 //
 // Weak forms (Goma's, restated):
 //   momentum  (src/mm_fill_momentum.c:474-672, J_m_v 1564-1735, J_m_T 746-915,
@@ -58,6 +60,7 @@ struct FillArgs {
   const double *x;
   double *resid;
   void *val;
+  double *re, *ct;  // QUAD9: element residuals, PSPG continuity x temperature entries
   double *kel;  // optional [num_elems][E]: element matrices before the Dirichlet rows
                 // (for Galerkin multigrid coarse operators), in the e2nz layout
   int *flag;
@@ -156,175 +159,209 @@ __device__ inline void supg_params(double s, const XA &x, const double *vc, doub
   }
 }
 
-template <int DIM, int EN, int VISC, typename JT, int NT>
-__global__ __launch_bounds__(NT) void k_fill(FillArgs A, const int *__restrict__ elems) {
-  constexpr int NVE = El<DIM>::NVE, NQ = El<DIM>::NQ, NP = El<DIM>::NP;
-  constexpr int NV = DIM + EN;
-  constexpr int NVE2 = NVE * NVE;
-  using T = Tab<DIM>;
-  const int e = elems[xcd_block()];
-  const int tid = threadIdx.x;
+// ---------------------------------------------------------------------------
+// QUAD9 element matrices on the matrix cores, four elements per workgroup.
+//
+// The elements' maps, gradients, fields and residuals are worked out by the
+// whole workgroup (a thread per element and point, node or row: one element
+// would leave most of a wave idle) and staged in LDS; then each wave takes one
+// element, whose node-pair blocks are sums of products E(X, w, Y)[i][j] =
+// sum_q X[q][i] w[q] Y[q][j] of 9 x 9 operand tables (the same terms as the
+// HEX27 kernel below), one v_mfma_f64_16x16x4f64 tile each (nodes padded to
+// 16, the nine points to three k-steps of 4).  The wave writes its element's matrix
+// before Dirichlet rows (kel, in the e2nz layout), residual (re) and, with
+// PSPG and energy, the continuity x temperature entries (ct); k_gather sums
+// them into the MSR rows.  All elements are one launch.
+// Bound by the element matrices' traffic for large meshes and by the chain of
+// phases (about 10 us) for small ones.  Measured (assembly of 128 x 128
+// shear-thinning elements with energy, FP64): 215 us with k_gather
+// against 408 with four coloured launches of a workgroup per element, a
+// thread per node pair and += through the element-to-nonzero map; 16 x 16
+// cavity 61 us against 97.
+typedef double d4v __attribute__((ext_vector_type(4)));
+
+template <int EN>
+struct Quad9Lds {  // one element
+  static constexpr int NVE = 9, KP = 12, LD = 16, NV = 2 + EN, NSP = STab<2>::NSP;
+  double x[2][NVE], u[NV][NVE], ud[NV][NVE], p[3];
+  double B[NVE][2][2];
+  double dA[KP];
+  double G[2][KP][LD];
+  double v[KP][2], gv[KP][2][2], gT[KP][2];  // gv[p][a] = d v_a / d x_p
+  double P[KP], mu[KP], dmu[KP], div[KP], Td[KP], f[KP][2], vd[KP][2];
+  double ps[KP][2];  // PSPG: tau dA (rho v_dot + rho v.grad v + grad P - f)
+  double su[4];      // energy SUPG: s/h, s d(1/h)/d vc_b
+  double qw[GM_QS_MAX][NSP], qh[GM_QS_MAX][NSP];  // QSIDE / QCONV: w |J_s| (q + h (T_c - T)), w |J_s| h
+  int qsd[GM_QS_MAX];
+};
+
+template <int EN, int VISC>
+__global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, int num_elems) {
+  constexpr int DIM = 2, NVE = 9, NQ = 9, NP = 3, NV = DIM + EN, NVE2 = NVE * NVE;
+  constexpr int KP = 12, LD = 16, NL = NV * NVE + NP;
+  using T = Tab<2>;
+  constexpr int NSP = STab<2>::NSP, SREC = STab<2>::REC;
+  __shared__ double s_Phi[KP][LD], s_dphi[NQ][NVE][DIM], s_psi[NQ][NP], s_wt[NQ];
+  __shared__ Quad9Lds<EN> s_el[4];
   const double *__restrict__ tb = A.tables;
+  for (int t = threadIdx.x; t < KP * LD; t += 256) {
+    const int q = t / LD, i = t - q * LD;
+    s_Phi[q][i] = (q < NQ && i < NVE) ? tb[T::PHI + q * NVE + i] : 0.0;
+  }
+  for (int t = threadIdx.x; t < NQ * NVE * DIM; t += 256) (&s_dphi[0][0][0])[t] = tb[T::DPHI + t];
+  if (threadIdx.x < NQ * NP) (&s_psi[0][0])[threadIdx.x] = tb[T::PSI + threadIdx.x];
+  else if (threadIdx.x >= 64 && threadIdx.x < 64 + NQ) s_wt[threadIdx.x - 64] = tb[T::WT + threadIdx.x - 64];
+  const int tid = threadIdx.x, e0 = xcd_block() * 4, ne = min(4, num_elems - e0);
 
-  __shared__ double s_x[DIM][NVE];
-  __shared__ double s_u[NV][NVE];
-  __shared__ double s_p[NP];
-  __shared__ int s_gun[NV][NVE];
-  __shared__ int s_gp[NP];
-  __shared__ double s_B[NQ][DIM][DIM];
-  __shared__ double s_dA[NQ];
-  __shared__ double s_g[NQ][NVE][DIM];
-  __shared__ double s_v[NQ][DIM];
-  __shared__ double s_gv[NQ][DIM][DIM];  // gv[p][a] = d v_a / d x_p
-  __shared__ double s_gT[NQ][DIM];
-  __shared__ double s_P[NQ];
-  __shared__ double s_mu[NQ];
-  __shared__ double s_dmu[NQ];           // (dmu/dgammadot) / gammadot, 0 if gammadot == 0
-  __shared__ double s_f[NQ][DIM];
-  __shared__ double s_div[NQ];
-  __shared__ double s_ud[NV][NVE];       // nodal time derivatives (transient)
-  __shared__ double s_vd[NQ][DIM];       // v_dot at the quadrature points
-  __shared__ double s_Td[NQ];            // T_dot
-  __shared__ double s_ps[NQ][DIM];       // PSPG: tau dA (rho v_dot + rho v.grad v + grad P - f)
-  __shared__ double s_su[4];             // energy SUPG: s/h, s d(1/h)/d vc_b
-  constexpr int NSP = STab<DIM>::NSP, SREC = STab<DIM>::REC;
-  __shared__ double s_qw[GM_QS_MAX][NSP];  // QSIDE / QCONV: w |surface det| (q + h (T_c - T))
-  __shared__ double s_qh[GM_QS_MAX][NSP];  // QCONV: w |surface det| h (the Jacobian's weight)
-  __shared__ int s_qsd[GM_QS_MAX];         // side index (0-based) of each entry
-  const int qs0 = A.qs_ptr ? A.qs_ptr[e] : 0;
-  const int nqs = A.qs_ptr ? A.qs_ptr[e + 1] - qs0 : 0;
-
-  // 1. gather
-  if (tid < NVE) {
-    const int n = A.conn[(size_t)e * NVE + tid];
+  // 1. gather, a thread per element and node (the centroid carries the pressures)
+  if (tid < ne * NVE) {
+    const int el = tid / NVE, i = tid - el * NVE;
+    Quad9Lds<EN> &S = s_el[el];
+    const int n = A.conn[(size_t)e0 * NVE + tid];
     const int f = A.fu[n];
 #pragma unroll
-    for (int k = 0; k < DIM; k++) s_x[k][tid] = A.coor[(size_t)k * A.num_nodes + n];
+    for (int k = 0; k < DIM; k++) S.x[k][i] = A.coor[(size_t)k * A.num_nodes + n];
 #pragma unroll
     for (int a = 0; a < NV; a++) {
-      s_gun[a][tid] = f + a;
-      s_u[a][tid] = A.x[f + a];
+      const double xv = A.x[f + a];
+      S.u[a][i] = xv;
       // xdot as solve_nonlinear_problem forms it after each update (src/rf_solve.c:2848)
-      s_ud[a][tid] = A.x_old ? A.cmass * (A.x[f + a] - A.x_old[f + a]) - A.cold * A.xdot_old[f + a]
-                             : 0.0;
+      S.ud[a][i] = A.x_old ? A.cmass * (xv - A.x_old[f + a]) - A.cold * A.xdot_old[f + a] : 0.0;
     }
-  } else if (tid >= 64 && tid < 64 + NP) {
-    const int k = tid - 64;
-    const int g = A.fu[A.centroid[e]] + DIM + EN + k;
-    s_gp[k] = g;
-    s_p[k] = A.x[g];
+  } else if (tid >= 64 && tid < 64 + ne) {
+    const int f = A.fu[A.centroid[e0 + tid - 64]] + NV;
+#pragma unroll
+    for (int k = 0; k < NP; k++) s_el[tid - 64].p[k] = A.x[f + k];
   }
   __syncthreads();
 
-  // 2. map per quadrature point
-  if (tid < NQ) {
-    const int q = tid;
-    double J[DIM][DIM];
+  // 2. map per point (beer_belly): a thread per element, point and J[i][j]
+  if (tid < 36 * ne) {
+    const int el = tid / 36, t = tid - el * 36, q = t >> 2, i = (t >> 1) & 1, j = t & 1;
+    Quad9Lds<EN> &S = s_el[el];
+    double s = 0.0;
 #pragma unroll
-    for (int i = 0; i < DIM; i++)
-#pragma unroll
-      for (int j = 0; j < DIM; j++) {
-        double s = 0.0;
-        for (int k = 0; k < NVE; k++) s += s_x[j][k] * tb[T::DPHI + (q * NVE + k) * DIM + i];
-        J[i][j] = s;
-      }
-    double det;
-    if constexpr (DIM == 2) {
-      det = J[0][0] * J[1][1] - J[0][1] * J[1][0];
-      s_B[q][0][0] = J[1][1] / det;
-      s_B[q][0][1] = -J[0][1] / det;
-      s_B[q][1][0] = -J[1][0] / det;
-      s_B[q][1][1] = J[0][0] / det;
-    } else {
-      det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
-            J[0][1] * (J[1][0] * J[2][2] - J[2][0] * J[1][2]) +
-            J[0][2] * (J[1][0] * J[2][1] - J[2][0] * J[1][1]);
-      s_B[q][0][0] = (J[1][1] * J[2][2] - J[2][1] * J[1][2]) / det;
-      s_B[q][0][1] = -(J[0][1] * J[2][2] - J[2][1] * J[0][2]) / det;
-      s_B[q][0][2] = (J[0][1] * J[1][2] - J[1][1] * J[0][2]) / det;
-      s_B[q][1][0] = -(J[1][0] * J[2][2] - J[2][0] * J[1][2]) / det;
-      s_B[q][1][1] = (J[0][0] * J[2][2] - J[2][0] * J[0][2]) / det;
-      s_B[q][1][2] = -(J[0][0] * J[1][2] - J[1][0] * J[0][2]) / det;
-      s_B[q][2][0] = (J[1][0] * J[2][1] - J[2][0] * J[1][1]) / det;
-      s_B[q][2][1] = -(J[0][0] * J[2][1] - J[2][0] * J[0][1]) / det;
-      s_B[q][2][2] = (J[0][0] * J[1][1] - J[1][0] * J[0][1]) / det;
-    }
-    if (!(det > 0.0)) atomicOr(&A.flag[0], 1);
-    s_dA[q] = det * tb[T::WT + q];
-  } else if (tid == NQ) {
+    for (int k = 0; k < NVE; k++) s += S.x[j][k] * s_dphi[q][k][i];
+    S.B[q][i][j] = s;
+  } else if (tid >= 192 && tid < 192 + ne) {
+    Quad9Lds<EN> &S = s_el[tid - 192];
     double vc[DIM], su[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int p = 0; p < DIM; p++) vc[p] = s_u[p][NVE - 1];
-    if (EN && A.supg_e != 0.0) supg_params<DIM>(A.supg_e, s_x, vc, su);
+    for (int p = 0; p < DIM; p++) vc[p] = S.u[p][NVE - 1];
+    if (EN && A.supg_e != 0.0) supg_params<DIM>(A.supg_e, S.x, vc, su);
 #pragma unroll
-    for (int k = 0; k < 4; k++) s_su[k] = su[k];
+    for (int k = 0; k < 4; k++) S.su[k] = su[k];
+  } else if (EN && A.qs_ptr && tid >= 196 && tid < 196 + ne * GM_QS_MAX * NSP) {
+    // QSIDE (src/bc_integ.c:1518-1519, 2156-2157): w * |surface Jacobian| * q
+    // at one surface Gauss point of one side entry; the side's free reference
+    // axis gives the tangent, as get_side_info orders it
+    // (src/mm_fill_fill.c:3049-3072, 3182-3250)
+    const int el = (tid - 196) / (GM_QS_MAX * NSP), t = tid - 196 - el * GM_QS_MAX * NSP;
+    const int k = t / NSP, g = t - k * NSP, at = A.qs_ptr[e0 + el] + k;
+    if (at < A.qs_ptr[e0 + el + 1]) {
+      Quad9Lds<EN> &S = s_el[el];
+      const int sd = A.qs_side[at] - 1;
+      const double *st = A.stab + (size_t)(sd * NSP + g) * SREC;
+      const int fr = (sd == 0 || sd == 2) ? 0 : 1;
+      double t1[DIM], Tg = 0.0;
+#pragma unroll
+      for (int j = 0; j < DIM; j++) {
+        t1[j] = 0.0;
+        for (int i = 0; i < NVE; i++) t1[j] += S.x[j][i] * st[NVE + i * DIM + fr];
+      }
+      const double *qk = A.qs_q + 3 * at;
+      const double wd = st[NVE + NVE * DIM] * sqrt(t1[0] * t1[0] + t1[1] * t1[1]);
+      if constexpr (EN)
+        for (int j = 0; j < NVE; j++) Tg += st[j] * S.u[DIM][j];
+      S.qw[k][g] = wd * (qk[0] + qk[1] * (qk[2] - Tg));
+      S.qh[k][g] = wd * qk[1];
+      if (g == 0) S.qsd[k] = sd;
+    }
+  }
+  static_assert(196 + 4 * GM_QS_MAX * NSP <= 256, "side entries of four elements in one pass");
+  __syncthreads();
+  if (tid >= 64 && tid < 64 + ne * KP) {
+    const int el = (tid - 64) / KP, q = tid - 64 - el * KP;
+    Quad9Lds<EN> &S = s_el[el];
+    double dA = 0.0;
+    if (q < NQ) {
+      const double J00 = S.B[q][0][0], J01 = S.B[q][0][1], J10 = S.B[q][1][0], J11 = S.B[q][1][1];
+      const double det = J00 * J11 - J01 * J10;
+      S.B[q][0][0] = J11 / det;
+      S.B[q][0][1] = -J01 / det;
+      S.B[q][1][0] = -J10 / det;
+      S.B[q][1][1] = J00 / det;
+      if (!(det > 0.0)) *(volatile int *)A.flag = 1;
+      dA = det * s_wt[q];
+    }
+    S.dA[q] = dA;  // the padding points carry no weight
   }
   __syncthreads();
 
-  // 3. physical gradients
-  for (int idx = tid; idx < NQ * NVE; idx += NT) {
-    const int q = idx / NVE, k = idx - q * NVE;
-    double dxi[DIM];
-#pragma unroll
-    for (int r = 0; r < DIM; r++) dxi[r] = tb[T::DPHI + (q * NVE + k) * DIM + r];
-#pragma unroll
-    for (int p = 0; p < DIM; p++) {
-      double s = 0.0;
-#pragma unroll
-      for (int r = 0; r < DIM; r++) s += s_B[q][p][r] * dxi[r];
-      s_g[q][k][p] = s;
+  // 3. physical gradients into the padded operand tables (load_bf_grad)
+#pragma unroll 1
+  for (int t = tid; t < ne * KP * LD; t += 256) {
+    const int el = t / (KP * LD), r = t - el * KP * LD, q = r / LD, i = r - q * LD;
+    Quad9Lds<EN> &S = s_el[el];
+    double g0 = 0.0, g1 = 0.0;
+    if (q < NQ && i < NVE) {
+      const double d0 = s_dphi[q][i][0], d1 = s_dphi[q][i][1];
+      g0 = S.B[q][0][0] * d0 + S.B[q][0][1] * d1;
+      g1 = S.B[q][1][0] * d0 + S.B[q][1][1] * d1;
+    }
+    S.G[0][q][i] = g0;
+    S.G[1][q][i] = g1;
+  }
+  __syncthreads();
+
+  // 4. fields at the points (load_fv, load_fv_grads): a thread per element,
+  // point and variable
+  if (tid < ne * KP * NV) {
+    const int el = tid / (KP * NV), r = tid - el * KP * NV, q = r / NV, a = r - q * NV;
+    Quad9Lds<EN> &S = s_el[el];
+    double s = 0.0, sd = 0.0, g0 = 0.0, g1 = 0.0;
+    if (q < NQ) {
+#pragma unroll 3
+      for (int k = 0; k < NVE; k++) {
+        const double ua = S.u[a][k], ph = s_Phi[q][k];
+        s += ua * ph;
+        sd += S.ud[a][k] * ph;
+        g0 += ua * S.G[0][q][k];
+        g1 += ua * S.G[1][q][k];
+      }
+    }
+    if (a < DIM) {
+      S.v[q][a] = s;
+      S.vd[q][a] = sd;
+      S.gv[q][0][a] = g0;
+      S.gv[q][1][a] = g1;
+    } else {
+      S.f[q][0] = s;  // T, replaced by the body force below
+      S.Td[q] = sd;
+      S.gT[q][0] = g0;
+      S.gT[q][1] = g1;
     }
   }
   __syncthreads();
-
-  // 4. fields at quadrature points
-  if (tid < NQ) {
-    const int q = tid;
-    double v[DIM], gv[DIM][DIM], Tq = 0.0, gT[DIM];
+  if (tid >= 192 && tid < 192 + ne * KP) {
+    const int el = (tid - 192) / KP, q = tid - 192 - el * KP;
+    Quad9Lds<EN> &S = s_el[el];
+    const double Tq = EN ? S.f[q][0] : 0.0;
+    double gv[DIM][DIM], v[DIM];
 #pragma unroll
     for (int a = 0; a < DIM; a++) {
-      v[a] = 0.0;
-      gT[a] = 0.0;
+      v[a] = S.v[q][a];
 #pragma unroll
-      for (int p = 0; p < DIM; p++) gv[p][a] = 0.0;
+      for (int p = 0; p < DIM; p++) gv[p][a] = S.gv[q][p][a];
     }
-    for (int k = 0; k < NVE; k++) {
-      const double ph = tb[T::PHI + q * NVE + k];
+    double P = 0.0, mu = A.mu0, dmu = 0.0;
+    if (q < NQ)
 #pragma unroll
-      for (int a = 0; a < DIM; a++) {
-        const double ua = s_u[a][k];
-        v[a] += ua * ph;
-#pragma unroll
-        for (int p = 0; p < DIM; p++) gv[p][a] += ua * s_g[q][k][p];
-      }
-      if constexpr (EN) {
-        const double tk = s_u[DIM][k];
-        Tq += tk * ph;
-#pragma unroll
-        for (int p = 0; p < DIM; p++) gT[p] += tk * s_g[q][k][p];
-      }
-    }
-    double vd[DIM], Td = 0.0;
-#pragma unroll
-    for (int a = 0; a < DIM; a++) vd[a] = 0.0;
-    if (A.x_old) {
-      for (int k = 0; k < NVE; k++) {
-        const double ph = tb[T::PHI + q * NVE + k];
-#pragma unroll
-        for (int a = 0; a < DIM; a++) vd[a] += s_ud[a][k] * ph;
-        if constexpr (EN) Td += s_ud[DIM][k] * ph;
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < DIM; a++) s_vd[q][a] = vd[a];
-    s_Td[q] = Td;
-    double P = 0.0;
-#pragma unroll
-    for (int k = 0; k < NP; k++) P += s_p[k] * tb[T::PSI + q * NP + k];
-    double mu = A.mu0, dmu = 0.0;
+      for (int k = 0; k < NP; k++) P += S.p[k] * s_psi[q][k];
     if constexpr (VISC == 1) {
       // calc_shearrate + carreau_viscosity (src/mm_fill_util.c:4564,
-      // src/mm_viscosity.c:1065-1116)
+      // src/mm_viscosity.c:1065-1116); the derivative's powers are the
+      // viscosity's own over one factor each
       double gd = 0.0;
 #pragma unroll
       for (int a = 0; a < DIM; a++)
@@ -336,355 +373,263 @@ __global__ __launch_bounds__(NT) void k_fill(FillArgs A, const int *__restrict__
       gd = sqrt(0.5 * fabs(gd));
       const bool nz = fabs(gd) > 1.0e-298;
       const double val2 = nz ? pow(A.lam * gd, A.aexp) : 0.0;
-      mu = A.muinf + (A.mu0 - A.muinf) * pow(1.0 + val2, (A.nexp - 1.0) / A.aexp);
-      if (nz) {
-        const double val = pow(A.lam * gd, A.aexp - 1.0);
-        const double val1 = pow(1.0 + val2, (A.nexp - 1.0 - A.aexp) / A.aexp);
-        const double dmu_gd = (A.mu0 - A.muinf) * (A.nexp - 1.0) * A.lam * val * val1;
-        dmu = dmu_gd / gd;
-      }
+      const double pm = pow(1.0 + val2, (A.nexp - 1.0) / A.aexp);
+      mu = A.muinf + (A.mu0 - A.muinf) * pm;
+      if (nz) dmu = (A.mu0 - A.muinf) * (A.nexp - 1.0) * (val2 / gd) * (pm / (1.0 + val2)) / gd;
     }
-    double div = 0.0;
+    S.P[q] = P;
+    S.mu[q] = mu;
+    S.dmu[q] = dmu;
+    S.div[q] = gv[0][0] + gv[1][1];
+    if (!EN) {
+      S.Td[q] = 0.0;
+      S.gT[q][0] = S.gT[q][1] = 0.0;
+    }
+    const double wp = A.tau_pspg * S.dA[q];
 #pragma unroll
     for (int a = 0; a < DIM; a++) {
-      s_v[q][a] = v[a];
-      s_gT[q][a] = gT[a];
-      div += gv[a][a];
-#pragma unroll
-      for (int p = 0; p < DIM; p++) s_gv[q][p][a] = gv[p][a];
-      s_f[q][a] = EN ? A.rho * A.g[a] * (-A.beta * (Tq - A.Tref)) : 0.0;
-    }
-    s_P[q] = P;
-    s_mu[q] = mu;
-    s_dmu[q] = dmu;
-    s_div[q] = div;
-    const double w = A.tau_pspg * s_dA[q];
-#pragma unroll
-    for (int a = 0; a < DIM; a++) {
+      const double f = EN && q < NQ ? A.rho * A.g[a] * (-A.beta * (Tq - A.Tref)) : 0.0;
       double adv = 0.0, gP = 0.0;
 #pragma unroll
       for (int p = 0; p < DIM; p++) adv += v[p] * gv[p][a];
+      if (q < NQ)
 #pragma unroll
-      for (int k = 1; k < NP; k++) gP += s_p[k] * s_B[q][a][k - 1];
-      s_ps[q][a] = w * (A.rho * (adv + vd[a]) + gP - s_f[q][a]);
+        for (int k = 1; k < NP; k++) gP += S.p[k] * S.B[q][a][k - 1];
+      S.f[q][a] = f;
+      S.ps[q][a] = wp * (A.rho * (adv + S.vd[q][a]) + gP - f);
     }
-  } else if (EN && tid >= NT / 2 && tid < NT / 2 + nqs * NSP) {
-    // QSIDE (src/bc_integ.c:1518-1519, 2156-2157): w * |surface Jacobian| * q
-    // at one surface Gauss point of one side entry; the side's free reference
-    // axes give the tangents, as get_side_info orders them
-    // (src/mm_fill_fill.c:3049-3072, 3182-3250)
-    const int k = (tid - NT / 2) / NSP, g = tid - NT / 2 - k * NSP;
-    const int sd = A.qs_side[qs0 + k] - 1;
-    const double *st = A.stab + (size_t)(sd * NSP + g) * SREC;
-    const int ax = (sd == 0 || sd == 2) ? 1 : (sd == 1 || sd == 3) ? 0 : 2;
-    int fr[2], nf = 0;
-#pragma unroll
-    for (int a = 0; a < DIM; a++)
-      if (a != ax) fr[nf++] = a;
-    double t1[DIM], t2[DIM];
-#pragma unroll
-    for (int j = 0; j < DIM; j++) {
-      t1[j] = 0.0;
-      t2[j] = 0.0;
-      for (int i = 0; i < NVE; i++) {
-        t1[j] += s_x[j][i] * st[NVE + i * DIM + fr[0]];
-        if constexpr (DIM == 3) t2[j] += s_x[j][i] * st[NVE + i * DIM + fr[1]];
-      }
-    }
-    double sdet;
-    if constexpr (DIM == 2) {
-      sdet = sqrt(t1[0] * t1[0] + t1[1] * t1[1]);
-    } else {
-      const double c0 = t1[1] * t2[2] - t1[2] * t2[1], c1 = t1[2] * t2[0] - t1[0] * t2[2],
-                   c2 = t1[0] * t2[1] - t1[1] * t2[0];
-      sdet = sqrt(c0 * c0 + c1 * c1 + c2 * c2);
-    }
-    const double *qk = A.qs_q + 3 * (qs0 + k), wd = st[NVE + NVE * DIM] * sdet;
-    double Tg = 0.0;
-    if constexpr (EN)
-      for (int j = 0; j < NVE; j++) Tg += st[j] * s_u[DIM][j];
-    s_qw[k][g] = wd * (qk[0] + qk[1] * (qk[2] - Tg));
-    s_qh[k][g] = wd * qk[1];
-    if (g == 0) s_qsd[k] = sd;
   }
   __syncthreads();
 
   const double rho = A.rho, rCp = A.rho * A.Cp, kc = A.kcond;
   const double cm = A.x_old ? A.cmass : 0.0;  // d xdot / d x: the mass-matrix coefficient
-  JT *__restrict__ out = (JT *)A.val;
-  const int *__restrict__ map = A.e2nz + (size_t)e * A.E;
 
-  // 5a. residual rows
-  for (int t = tid; t < NV * NVE + NP; t += NT) {
-    int row;
+  // 5a. residual rows, a thread per element and row
+  if (tid < ne * NL) {
+    const int el = tid / NL, t = tid - el * NL, e = e0 + el;
+    const Quad9Lds<EN> &S = s_el[el];
     double R = 0.0;
     if (t < NV * NVE) {
       const int a = t / NVE, i = t - a * NVE;
-      row = s_gun[a][i];
       if (a < DIM) {
+#pragma unroll 1
         for (int q = 0; q < NQ; q++) {
-          const double ph = tb[T::PHI + q * NVE + i];
+          const double ph = s_Phi[q][i];
           double adv = 0.0, dif = 0.0;
 #pragma unroll
           for (int p = 0; p < DIM; p++) {
-            adv += s_v[q][p] * s_gv[q][p][a];
-            const double Pi_ap = (a == p ? -s_P[q] : 0.0) + s_mu[q] * (s_gv[q][a][p] + s_gv[q][p][a]);
-            dif += s_g[q][i][p] * Pi_ap;
+            adv += S.v[q][p] * S.gv[q][p][a];
+            const double Pi_ap = (a == p ? -S.P[q] : 0.0) + S.mu[q] * (S.gv[q][a][p] + S.gv[q][p][a]);
+            dif += S.G[p][q][i] * Pi_ap;
           }
-          R += s_dA[q] * (-rho * ph * adv - dif + ph * s_f[q][a] - rho * ph * s_vd[q][a]);
+          R += S.dA[q] * (-rho * ph * adv - dif + ph * S.f[q][a] - rho * ph * S.vd[q][a]);
         }
       } else {
-        const double sw = s_su[0];
+#pragma unroll 1
         for (int q = 0; q < NQ; q++) {
-          const double ph = tb[T::PHI + q * NVE + i];
+          const double ph = s_Phi[q][i];
           double adv = 0.0, dif = 0.0, vgi = 0.0;
 #pragma unroll
           for (int p = 0; p < DIM; p++) {
-            adv += s_v[q][p] * s_gT[q][p];
-            dif += s_g[q][i][p] * s_gT[q][p];
-            vgi += s_v[q][p] * s_g[q][i][p];
+            adv += S.v[q][p] * S.gT[q][p];
+            dif += S.G[p][q][i] * S.gT[q][p];
+            vgi += S.v[q][p] * S.G[p][q][i];
           }
-          R += s_dA[q] * (-rCp * (ph + sw * vgi) * adv - kc * dif + ph * A.hsrc - rCp * ph * s_Td[q]);
+          R += S.dA[q] * (-rCp * (ph + S.su[0] * vgi) * adv - kc * dif + ph * A.hsrc - rCp * ph * S.Td[q]);
         }
+        const int nqs = A.qs_ptr ? A.qs_ptr[e + 1] - A.qs_ptr[e] : 0;
         for (int k = 0; k < nqs; k++)
-          for (int g = 0; g < NSP; g++) R += s_qw[k][g] * A.stab[(size_t)(s_qsd[k] * NSP + g) * SREC + i];
+          for (int g = 0; g < NSP; g++) R += S.qw[k][g] * A.stab[(size_t)(S.qsd[k] * NSP + g) * SREC + i];
       }
     } else {
       const int k = t - NV * NVE;
-      row = s_gp[k];
-      for (int q = 0; q < NQ; q++) R += s_dA[q] * tb[T::PSI + q * NP + k] * s_div[q];
+#pragma unroll 1
+      for (int q = 0; q < NQ; q++) R += S.dA[q] * s_psi[q][k] * S.div[q];
       if (A.tau_pspg != 0.0 && k > 0)
+#pragma unroll 1
         for (int q = 0; q < NQ; q++)
 #pragma unroll
-          for (int a = 0; a < DIM; a++) R += s_B[q][a][k - 1] * s_ps[q][a];
+          for (int a = 0; a < DIM; a++) R += S.B[q][a][k - 1] * S.ps[q][a];
     }
-    if (A.dbc[row]) R = A.x[row] - A.dbc_val[row];
-    A.resid[row] += R;
+    A.re[(size_t)e0 * NL + tid] = R;
   }
-
   if (A.resid_only) return;
 
-  // 5b. nodal-variable blocks, one node pair (i,j) per task
-  for (int t = tid; t < NVE2; t += NT) {
-    const int i = t / NVE, j = t - i * NVE;
-    double acc[NV][NV];
+  // from here on a wave per element
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), e = e0 + w;
+  if (w >= ne) return;
+  const Quad9Lds<EN> &S = s_el[w];
+  const double sw = S.su[0];
+  const int qs0 = EN && A.qs_ptr ? A.qs_ptr[e] : 0;
+  const int nqs = EN && A.qs_ptr ? A.qs_ptr[e + 1] - qs0 : 0;
+  double *__restrict__ ke = A.kel + (size_t)e * A.E;
+
+  // 5b. nodal blocks: the lane's rows i = kk + 4 r and column j; operands at node j
+  const int j = lane & 15, kk = lane >> 4;
+#define GM_MFMA64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64((a), (b), (c), 0, 0, 0)
+  const d4v z = {0.0, 0.0, 0.0, 0.0};
+  auto store = [&](int a, int b, const d4v &D) {
+    if (j >= NVE) return;
 #pragma unroll
-    for (int a = 0; a < NV; a++)
+    for (int r = 0; r < 3; r++) {
+      const int i = kk + 4 * r;
+      if (i < NVE) ke[(a * NV + b) * NVE2 + i * NVE + j] = D[r];
+    }
+  };
+  // shared products: E(phi, dA, phi), and folded into the diagonal blocks
+  // E(phi, dA, v.G) and sum_p E(G_p, dA, G_p) (times mu, times k)
+  d4v A1 = z, Dm = z, Tt = z;
+  {
+    d4v Dadv = z, L1 = z, Lmu = z;
+#pragma unroll 1
+    for (int q = kk; q < KP; q += 4) {
+      const double dA = S.dA[q], ph = s_Phi[q][j], g0 = S.G[0][q][j], g1 = S.G[1][q][j];
+      const double vg = S.v[q][0] * g0 + S.v[q][1] * g1;
+      A1 = GM_MFMA64(ph * dA, ph, A1);
+      Dadv = GM_MFMA64(ph * dA, vg, Dadv);
+      L1 = GM_MFMA64(g0 * dA, g0, L1);
+      if constexpr (VISC == 1) Lmu = GM_MFMA64(g0 * dA * S.mu[q], g0, Lmu);
+      L1 = GM_MFMA64(g1 * dA, g1, L1);
+      if constexpr (VISC == 1) Lmu = GM_MFMA64(g1 * dA * S.mu[q], g1, Lmu);
+    }
+    if constexpr (VISC == 0) Lmu = A.mu0 * L1;
+    Dm = -(rho * Dadv + Lmu + (rho * cm) * A1);
+    if constexpr (EN) Tt = -(rCp * Dadv + kc * L1 + (rCp * cm) * A1);
+  }
+#pragma unroll 1
+  for (int a = 0; a < DIM; a++) {
+    d4v J[DIM];
 #pragma unroll
-      for (int b = 0; b < NV; b++) acc[a][b] = 0.0;
-    for (int q = 0; q < NQ; q++) {
-      const double dA = s_dA[q];
-      const double phi_i = tb[T::PHI + q * NVE + i];
-      const double phi_j = tb[T::PHI + q * NVE + j];
-      double Gi[DIM], gj[DIM];
-#pragma unroll
-      for (int p = 0; p < DIM; p++) {
-        Gi[p] = s_g[q][i][p];
-        gj[p] = s_g[q][j][p];
-      }
-      double advj = 0.0, GG = 0.0;
-#pragma unroll
-      for (int p = 0; p < DIM; p++) {
-        advj += s_v[q][p] * gj[p];
-        GG += Gi[p] * gj[p];
-      }
-      const double mu = s_mu[q];
-      const double pij = phi_i * phi_j;
-      double Gg[DIM], dmb[DIM];  // sum_p Gi[p] gamma[a][p], c * sum_p gj[p] gamma[b][p]
+    for (int b = 0; b < DIM; b++) J[b] = z;
+#pragma unroll 1
+    for (int q = kk; q < KP; q += 4) {
+      const double dA = S.dA[q], ph = s_Phi[q][j], g[DIM] = {S.G[0][q][j], S.G[1][q][j]};
+      const double ga = S.G[a][q][j], wmu = -dA * (VISC ? S.mu[q] : A.mu0);
+      double hA = 0.0;
       if constexpr (VISC == 1) {
-        const double c = s_dmu[q];
+        // Carreau: (d mu / d gammadot) / gammadot (G_i . gamma_a) (g_j . gamma_b)
 #pragma unroll
-        for (int a = 0; a < DIM; a++) {
-          double s1 = 0.0, s2 = 0.0;
+        for (int p = 0; p < DIM; p++) hA += g[p] * (S.gv[q][a][p] + S.gv[q][p][a]);
+        hA *= -dA * S.dmu[q];
+      }
 #pragma unroll
-          for (int p = 0; p < DIM; p++) {
-            const double gam = s_gv[q][a][p] + s_gv[q][p][a];
-            s1 += Gi[p] * gam;
-            s2 += gj[p] * gam;
-          }
-          Gg[a] = s1;
-          dmb[a] = c * s2;
+      for (int b = 0; b < DIM; b++) {
+        // advection through d_b v_a, then mu g_j,a G_i,b
+        J[b] = GM_MFMA64(ph * (-rho * dA) * S.gv[q][b][a], ph, J[b]);
+        J[b] = GM_MFMA64(g[b] * wmu, ga, J[b]);
+        if constexpr (VISC == 1) {
+          double hB = 0.0;
+#pragma unroll
+          for (int p = 0; p < DIM; p++) hB += g[p] * (S.gv[q][b][p] + S.gv[q][p][b]);
+          J[b] = GM_MFMA64(hA, hB, J[b]);
         }
       }
-      const double diag = rho * phi_i * advj + mu * GG + rho * cm * pij;
+    }
 #pragma unroll
-      for (int a = 0; a < DIM; a++) {
+    for (int b = 0; b < DIM; b++) store(a, b, a == b ? J[b] + Dm : J[b]);
+    if constexpr (EN) store(a, DIM, (-rho * A.g[a] * A.beta) * A1);
+  }
+  if constexpr (EN) {
+    d4v Jb[DIM];
+#pragma unroll
+    for (int b = 0; b < DIM; b++) Jb[b] = z;
+#pragma unroll 1
+    for (int q = kk; q < KP; q += 4) {
+      // (phi_i + sw v.G_i) d_b T + sw (v.grad T) G_b,i: the SUPG weight on
+      // the advection and its derivative in v at the column node; and the
+      // weight's part of J_TT, -rho Cp sw E(v.G_i dA, v.G_j)
+      const double ph = s_Phi[q][j], g[DIM] = {S.G[0][q][j], S.G[1][q][j]};
+      const double vg = S.v[q][0] * g[0] + S.v[q][1] * g[1];
+      const double wt = -rCp * S.dA[q], vgT = S.v[q][0] * S.gT[q][0] + S.v[q][1] * S.gT[q][1];
+#pragma unroll
+      for (int b = 0; b < DIM; b++)
+        Jb[b] = GM_MFMA64(wt * ((ph + sw * vg) * S.gT[q][b] + sw * vgT * g[b]), ph, Jb[b]);
+      if (sw != 0.0) Tt = GM_MFMA64(wt * sw * vg, vg, Tt);
+    }
+    if (sw != 0.0 && j == NVE - 1) {
+      // d(1/h)/dv at the last local node: -rho Cp s_b sum_q dA (v.grad T) v_b G_b,i
+#pragma unroll
+      for (int r = 0; r < 3; r++) {
+        const int i = kk + 4 * r;
+        if (i >= NVE) continue;
 #pragma unroll
         for (int b = 0; b < DIM; b++) {
-          double v = -rho * pij * s_gv[q][b][a] - mu * gj[a] * Gi[b];
-          if (a == b) v -= diag;
-          if constexpr (VISC == 1) v -= dmb[b] * Gg[a];
-          acc[a][b] += dA * v;
-        }
-      }
-      if constexpr (EN) {
-        // SUPG weight w_i = phi_i + sw (v.G_i) on the advection terms, and
-        // the weight's own derivative in v (d_wt_func)
-        const double sw = s_su[0];
-        double vgi = 0.0, vgT = 0.0;
-#pragma unroll
-        for (int p = 0; p < DIM; p++) {
-          vgi += s_v[q][p] * Gi[p];
-          vgT += s_v[q][p] * s_gT[q][p];
-        }
-        const double wi = phi_i + sw * vgi;
-#pragma unroll
-        for (int a = 0; a < DIM; a++) {
-          acc[a][DIM] += dA * (-rho * A.g[a] * A.beta * pij);
-          double dw = sw * phi_j * Gi[a];
-          if (j == NVE - 1) dw += s_su[1 + a] * s_v[q][a] * Gi[a];
-          acc[DIM][a] += dA * (-rCp * (wi * phi_j * s_gT[q][a] + dw * vgT));
-        }
-        acc[DIM][DIM] += dA * (-rCp * wi * advj - kc * GG - rCp * cm * pij);
-      }
-    }
-    if (A.kel) {
-      double *__restrict__ ke = A.kel + (size_t)e * A.E;
-#pragma unroll
-      for (int a = 0; a < NV; a++)
-#pragma unroll
-        for (int b = 0; b < NV; b++) ke[(a * NV + b) * NVE2 + t] = acc[a][b];
-    }
-#pragma unroll
-    for (int a = 0; a < NV; a++) {
-      const int row = s_gun[a][i];
-      const bool dir = A.dbc[row] != 0;
-#pragma unroll
-      for (int b = 0; b < NV; b++) {
-        double v = acc[a][b];
-        if (dir) {
-          if (a == b && i == j) v = 1.0;
-          else continue;
-        }
-        const int idx = map[(a * NV + b) * NVE2 + t];
-        out[idx] += (JT)v;
-      }
-    }
-  }
-
-  // QCONV: -h w |surface Jacobian| phi_i phi_j over the element's sides in the
-  // T-T block, on top of the entries scattered above
-  if constexpr (EN) {
-    bool conv = false;
-    for (int k = 0; k < nqs; k++) conv |= A.qs_q[3 * (qs0 + k) + 1] != 0.0;
-    if (conv) {
-      __syncthreads();
-      for (int t = tid; t < NVE2; t += NT) {
-        const int i = t / NVE, j = t - i * NVE;
-        double v = 0.0;
+          double c = 0.0;
 #pragma unroll 1
-        for (int k = 0; k < nqs; k++) {
-          if (A.qs_q[3 * (qs0 + k) + 1] == 0.0) continue;
-#pragma unroll 1
-          for (int g = 0; g < NSP; g++) {
-            const double *st = A.stab + (size_t)(s_qsd[k] * NSP + g) * SREC;
-            v -= s_qh[k][g] * st[i] * st[j];
-          }
+          for (int q = 0; q < NQ; q++)
+            c += S.dA[q] * (S.v[q][0] * S.gT[q][0] + S.v[q][1] * S.gT[q][1]) * S.v[q][b] * S.G[b][q][i];
+          Jb[b][r] -= rCp * S.su[1 + b] * c;
         }
-        if (v == 0.0) continue;  // a node pair off the sides
-        if (A.kel) A.kel[(size_t)e * A.E + (size_t)(DIM * NV + DIM) * NVE2 + t] += v;
-        if (A.dbc[s_gun[DIM][i]]) continue;  // a Dirichlet row keeps its unit diagonal only
-        out[map[(DIM * NV + DIM) * NVE2 + t]] += (JT)v;
       }
     }
-  }
-
-  // 5c. momentum x pressure (J_m_P): int grad_a phi_i psi_k dA
-  for (int t = tid; t < NVE * NP; t += NT) {
-    const int i = t / NP, k = t - i * NP;
-    double acc[DIM];
+    // QCONV: -h w |surface Jacobian| phi_i phi_j over the element's sides
+    for (int k = 0; k < nqs; k++) {
+      if (A.qs_q[3 * (qs0 + k) + 1] == 0.0 || j >= NVE) continue;
+      for (int g = 0; g < NSP; g++) {
+        const double *st = A.stab + (size_t)(S.qsd[k] * NSP + g) * SREC;
 #pragma unroll
-    for (int a = 0; a < DIM; a++) acc[a] = 0.0;
-    for (int q = 0; q < NQ; q++) {
-      const double w = s_dA[q] * tb[T::PSI + q * NP + k];
-#pragma unroll
-      for (int a = 0; a < DIM; a++) acc[a] += w * s_g[q][i][a];
+        for (int r = 0; r < 3; r++)
+          if (kk + 4 * r < NVE) Tt[r] -= S.qh[k][g] * st[kk + 4 * r] * st[j];
+      }
     }
 #pragma unroll
-    for (int a = 0; a < DIM; a++) {
-      if (A.kel) A.kel[(size_t)e * A.E + A.off_mp + a * NVE * NP + t] = acc[a];
-      if (A.dbc[s_gun[a][i]]) continue;
-      const int idx = map[A.off_mp + a * NVE * NP + t];
-      out[idx] += (JT)acc[a];
-    }
+    for (int b = 0; b < DIM; b++) store(DIM, b, Jb[b]);
+    store(DIM, DIM, Tt);
   }
+#undef GM_MFMA64
 
-  // 5d. continuity x velocity (J_c_v): int psi_k grad_b phi_j dA; PSPG adds
+  // 5c. momentum x pressure (J_m_P): int grad_a phi_i psi_k dA; 5d. continuity
+  // x velocity (J_c_v): int psi_k grad_b phi_j dA, plus PSPG's
   // tau rho [phi_j grad psi_k . d_b v + grad_b psi_k (v.grad phi_j + c phi_j)]
   // and continuity x temperature tau rho beta (grad psi_k . g) phi_j
   const bool ps = A.tau_pspg != 0.0;
-  for (int t = tid; t < NP * NVE; t += NT) {
-    const int k = t / NVE, j = t - k * NVE;
-    const bool dir = A.dbc[s_gp[k]] != 0;
-    if (dir && !A.kel) continue;
-    double acc[DIM], accT = 0.0;
-#pragma unroll
-    for (int b = 0; b < DIM; b++) acc[b] = 0.0;
+  if (lane < 2 * NVE * NP) {
+    const bool mp = lane < NVE * NP;
+    const int t = mp ? lane : lane - NVE * NP;
+    const int k = mp ? t % NP : t / NVE, i = mp ? t / NP : t % NVE;
+    double acc[DIM] = {0.0, 0.0}, accT = 0.0;
+#pragma unroll 3
     for (int q = 0; q < NQ; q++) {
-      const double w = s_dA[q] * tb[T::PSI + q * NP + k];
+      const double wq = S.dA[q] * s_psi[q][k];
 #pragma unroll
-      for (int b = 0; b < DIM; b++) acc[b] += w * s_g[q][j][b];
-      if (ps && k > 0) {
-        const double wp = A.tau_pspg * s_dA[q] * rho, phj = tb[T::PHI + q * NVE + j];
-        double vg = 0.0, gk[DIM], gkg = 0.0;
+      for (int a = 0; a < DIM; a++) acc[a] += wq * S.G[a][q][i];
+    }
+    if (ps && !mp && k > 0) {
+#pragma unroll 1
+      for (int q = 0; q < NQ; q++) {
+        const double wp = A.tau_pspg * S.dA[q] * rho, phj = s_Phi[q][i];
+        double vgj = 0.0, gk[DIM], gkg = 0.0;
 #pragma unroll
         for (int p = 0; p < DIM; p++) {
-          vg += s_v[q][p] * s_g[q][j][p];
-          gk[p] = s_B[q][p][k - 1];
+          vgj += S.v[q][p] * S.G[p][q][i];
+          gk[p] = S.B[q][p][k - 1];
           gkg += gk[p] * A.g[p];
         }
 #pragma unroll
         for (int b = 0; b < DIM; b++) {
           double gv = 0.0;
 #pragma unroll
-          for (int a = 0; a < DIM; a++) gv += gk[a] * s_gv[q][b][a];
-          acc[b] += wp * (phj * gv + gk[b] * (vg + cm * phj));
+          for (int a = 0; a < DIM; a++) gv += gk[a] * S.gv[q][b][a];
+          acc[b] += wp * (phj * gv + gk[b] * (vgj + cm * phj));
         }
         accT += wp * A.beta * gkg * phj;
       }
     }
 #pragma unroll
-    for (int b = 0; b < DIM; b++) {
-      if (A.kel) A.kel[(size_t)e * A.E + A.off_cv + b * NP * NVE + t] = acc[b];
-      if (dir) continue;
-      const int idx = map[A.off_cv + b * NP * NVE + t];
-      out[idx] += (JT)acc[b];
-    }
-    if (EN && ps && k > 0 && !dir) {
-      // the element layout holds no continuity x temperature entries: find
-      // the column in the row (sorted off-diagonal list)
-      const int row = s_gp[k], col = s_gun[DIM][j];
-      int lo = A.bindx[row], hi = A.bindx[row + 1] - 1;
-      while (lo <= hi) {
-        const int mid = (lo + hi) >> 1, v = A.bindx[mid];
-        if (v == col) {
-          out[mid] += (JT)accT;
-          break;
-        }
-        if (v < col) lo = mid + 1;
-        else hi = mid - 1;
-      }
-    }
+    for (int a = 0; a < DIM; a++) ke[(mp ? A.off_mp : A.off_cv) + a * NVE * NP + t] = acc[a];
+    if (EN && ps && !mp) A.ct[(size_t)e * NP * NVE + t] = accT;
   }
-
   // 5e. continuity x pressure: zero for Galerkin Q2-P1; PSPG adds
-  // tau grad psi_k . grad psi_l; a unit diagonal on a Dirichlet (datum) row
-  if (tid < NP * NP) {
-    const int k = tid / NP, k2 = tid - k * NP;
+  // tau grad psi_k . grad psi_l
+  if (lane < NP * NP) {
+    const int k = lane / NP, k2 = lane - k * NP;
     double acc = 0.0;
     if (ps && k > 0 && k2 > 0)
-      for (int q = 0; q < NQ; q++) {
-        double g2 = 0.0;
-#pragma unroll
-        for (int a = 0; a < DIM; a++) g2 += s_B[q][a][k - 1] * s_B[q][a][k2 - 1];
-        acc += A.tau_pspg * s_dA[q] * g2;
-      }
-    if (A.kel) A.kel[(size_t)e * A.E + A.off_cp + tid] = acc;
-    if (A.dbc[s_gp[k]]) {
-      if (k == k2) out[map[A.off_cp + tid]] += (JT)1.0;
-    } else if (acc != 0.0) {
-      out[map[A.off_cp + tid]] += (JT)acc;
-    }
+#pragma unroll 1
+      for (int q = 0; q < NQ; q++)
+        acc += A.tau_pspg * S.dA[q] *
+               (S.B[q][0][k - 1] * S.B[q][0][k2 - 1] + S.B[q][1][k - 1] * S.B[q][1][k2 - 1]);
+    ke[A.off_cp + lane] = acc;
   }
 }
 
@@ -717,7 +662,6 @@ __global__ __launch_bounds__(NT) void k_fill(FillArgs A, const int *__restrict__
 // bindx[row] + rank + b - (col > row).  With `overwrite` the first element
 // (in colour order) to touch a node pair stores its values, later ones add:
 // no zeroing pass and no read of the old value on first touch.
-typedef double d4v __attribute__((ext_vector_type(4)));
 
 template <int EN, int VISC, typename JT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VISC ? 3 : 4, VISC ? 3 : 4))) void k_fill3m(
@@ -808,7 +752,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VISC ? 3 : 
     s_B[q][2][0] = (J[1][0] * J[2][1] - J[2][0] * J[1][1]) / det;
     s_B[q][2][1] = -(J[0][0] * J[2][1] - J[2][0] * J[0][1]) / det;
     s_B[q][2][2] = (J[0][0] * J[1][1] - J[1][0] * J[0][1]) / det;
-    if (!(det > 0.0)) atomicOr(&A.flag[0], 1);
+    if (!(det > 0.0)) *(volatile int *)A.flag = 1;
     s_dA[q] = det * tb[T::WT + q];
   } else if (tid == NQ) {
     s_dA[NQ] = 0.0;  // the padding point carries no weight
@@ -1664,6 +1608,7 @@ int gm_fill_setup_device(gm_ctx *c) {
     gm_set_error("element-to-nonzero map: entry missing from the MSR graph");
     return GM_ERR_ARG;
   }
+  if (c->dim == 2) return gm_gather_setup(c);
   if (c->dim == 3) {
     // rank map and first touches (the HEX27 assembly kernel's scatter)
     const size_t nr = ne * 2 * (size_t)L.nve * L.nve;
@@ -1694,32 +1639,50 @@ int gm_fill_setup_device(gm_ctx *c) {
   return GM_OK;
 }
 
-template <int DIM, int EN, int VISC, typename JT>
-static void launch_fill(gm_ctx *c, FillArgs &a) {
-  constexpr int NT = DIM == 2 ? 128 : 256;
-  void (*kern)(FillArgs, const int *);
-  if constexpr (DIM == 3) kern = k_fill3m<EN, VISC, JT>;
-  else kern = k_fill<DIM, EN, VISC, JT, NT>;
+template <int EN, int VISC, typename JT>
+static void launch_fill3(gm_ctx *c, FillArgs &a) {
   for (int col = 0; col < c->n_ecol; col++) {
     const int cnt = c->ecol_ptr[col + 1] - c->ecol_ptr[col];
     if (cnt == 0) continue;
     // this colour's share of B_asm = nnz*s + 16 N + 8 dim n_nodes + 4 nve n_el
     const double share = (double)cnt / c->num_elems;
     const double basm = (double)(c->nval - 1) * sizeof(JT) + 16.0 * c->N +
-                        8.0 * DIM * c->num_nodes + 4.0 * El<DIM>::NVE * c->num_elems;
+                        24.0 * c->num_nodes + 4.0 * El<3>::NVE * c->num_elems;
     const int id = a.resid_only ? GM_K_FILL_RESID : GM_K_FILL;
     gm_launch(c, id, share * (a.resid_only ? basm - (double)(c->nval - 1) * sizeof(JT) : basm),
-              kern, dim3(cnt), dim3(NT), 0, c->stream, a, c->d_ecol_elems + c->ecol_ptr[col]);
+              k_fill3m<EN, VISC, JT>, dim3(cnt), dim3(256), 0, c->stream, a,
+              c->d_ecol_elems + c->ecol_ptr[col]);
   }
 }
 
-template <int DIM, typename JT>
-static void dispatch_fill(gm_ctx *c, FillArgs &a) {
+template <typename JT>
+static void dispatch_fill3(gm_ctx *c, FillArgs &a) {
   const int en = c->energy, vm = c->phys.visc_model;
-  if (en && vm) launch_fill<DIM, 1, 1, JT>(c, a);
-  else if (en) launch_fill<DIM, 1, 0, JT>(c, a);
-  else if (vm) launch_fill<DIM, 0, 1, JT>(c, a);
-  else launch_fill<DIM, 0, 0, JT>(c, a);
+  if (en && vm) launch_fill3<1, 1, JT>(c, a);
+  else if (en) launch_fill3<1, 0, JT>(c, a);
+  else if (vm) launch_fill3<0, 1, JT>(c, a);
+  else launch_fill3<0, 0, JT>(c, a);
+}
+
+static int fill2_buffers(gm_ctx *c) {
+  if (!c->d_re) GM_HIP(hipMalloc(&c->d_re, (size_t)c->num_elems * (c->nv * c->nve + c->np) * sizeof(double)));
+  if (!c->d_ct) GM_HIP(hipMalloc(&c->d_ct, (size_t)c->num_elems * c->np * c->nve * sizeof(double)));
+  return GM_OK;
+}
+
+// QUAD9: the element matrices and residuals of every element, then the rows.
+static int fill2(gm_ctx *c, FillArgs &a, double *val, float *val32) {
+  const int en = c->energy, vm = c->phys.visc_model;
+  auto kern = en ? (vm ? k_elem2<1, 1> : k_elem2<1, 0>) : (vm ? k_elem2<0, 1> : k_elem2<0, 0>);
+  const int id = a.resid_only ? GM_K_FILL_RESID : GM_K_FILL;
+  // coordinates, connectivity, the state; the element matrices and residuals written
+  const double bytes = 16.0 * c->num_nodes + 8.0 * c->N + 36.0 * c->num_elems +
+                       8.0 * c->num_elems * (c->nv * 9 + 3 + (a.resid_only ? 0.0 : (double)c->lay.total));
+  gm_launch(c, id, bytes, kern, dim3((c->num_elems + 3) / 4), dim3(256), 0, c->stream, a, c->num_elems);
+  GM_HIP(hipGetLastError());
+  const bool mat = !a.resid_only;
+  return gm_gather(c, id, c, c->stream, a.kel, en && a.tau_pspg != 0.0 ? a.ct : nullptr, mat ? val : nullptr,
+                   mat ? val32 : nullptr, c->fill_overwrite, a.re, a.x, a.resid);
 }
 
 int gm_fill_launch(gm_ctx *c, const double *x, double *resid, double *val, float *val32) {
@@ -1742,7 +1705,6 @@ int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, fl
   a.resid = resid;
   a.val = val32 ? (void *)val32 : (void *)val;
   a.kel = c->kel_on ? c->d_kel : nullptr;
-  a.flag = c->d_flag;
   a.x_old = c->tr_x_old;
   a.xdot_old = c->tr_xdot_old;
   a.cmass = c->tr_cmass;
@@ -1774,19 +1736,22 @@ int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, fl
   for (int k = 0; k < 3; k++) a.g[k] = p.g[k];
   a.beta = p.beta;
   a.Tref = p.Tref;
-  GM_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream));
+  *c->h_flag = 0;  // nothing that could set it is in flight: every call waits for its kernels
+  a.flag = c->h_flag;
   if (c->dim == 2) {
-    if (val32) dispatch_fill<2, float>(c, a);
-    else dispatch_fill<2, double>(c, a);
+    int rc = resid_only ? GM_OK : gm_mg_kel_alloc(c);
+    if (rc || (rc = fill2_buffers(c))) return rc;
+    a.kel = c->d_kel;
+    a.re = c->d_re;
+    a.ct = c->d_ct;
+    if ((rc = fill2(c, a, val, val32))) return rc;
   } else {
-    if (val32) dispatch_fill<3, float>(c, a);
-    else dispatch_fill<3, double>(c, a);
+    if (val32) dispatch_fill3<float>(c, a);
+    else dispatch_fill3<double>(c, a);
   }
   GM_HIP(hipGetLastError());
-  int flag = 0;
-  GM_HIP(hipMemcpyAsync(&flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   GM_HIP(hipStreamSynchronize(c->stream));
-  if (flag) {
+  if (*(volatile int *)c->h_flag) {
     gm_set_error("zero or negative element Jacobian determinant");
     return GM_ERR_ELEM;
   }

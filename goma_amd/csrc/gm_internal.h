@@ -178,6 +178,11 @@ struct gm_ctx {
   int *d_ecol_elems = nullptr;
   int *d_e2nz = nullptr;        // [num_elems * lay.total]
   int *d_flag = nullptr;        // device error flags
+  int *h_flag = nullptr;        // pinned: set by the assembly kernels on a bad element
+  // node pairs of the graph with the elements that hold them (k_gather)
+  int4 *d_pair = nullptr;       // [pairs + 1]
+  int *d_rank_t = nullptr, *d_src = nullptr;
+  double *d_re = nullptr, *d_ct = nullptr;  // QUAD9 assembly: element residuals; PSPG c x T entries
   double *d_tables = nullptr;   // reference basis tables
   double *d_stab = nullptr;     // side basis tables (surface integrals)
   unsigned short *d_rank = nullptr;  // HEX27: per element and node pair, the rank of the
@@ -243,6 +248,12 @@ int gm_fill_launch(gm_ctx *c, const double *x, double *resid, double *val, float
 void gm_q2_basis(int dim, const double *xi, double *phi);  // host: Q2 basis at one reference point
 int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, float *val32,
                       int resid_only);
+
+// element matrices to MSR rows (gm_gather.hip)
+int gm_gather_setup(gm_ctx *c);
+int gm_unknown_places(gm_ctx *c);
+int gm_gather(gm_ctx *prof, int id, gm_ctx *c, hipStream_t s, const double *kel, const double *ct, double *val,
+              float *val32, int assign, const double *re, const double *x, double *resid);
 
 // linear algebra (gm_linalg.hip)
 int gm_zero(gm_ctx *c, double *p, long long n);

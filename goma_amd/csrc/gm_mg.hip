@@ -997,61 +997,8 @@ __global__ __launch_bounds__(256) void k_galerkin(const double *__restrict__ kf,
   }
 }
 
-// Adds the element matrices of one element colour into an MSR matrix with
-// Goma's per-element Dirichlet rows (a Dirichlet row keeps only a unit
-// diagonal, src/bc_dirich.c:44-153), as the assembly kernel does.
-template <int DIM, typename JT>
-__global__ __launch_bounds__(256) void k_elem_scatter(const double *__restrict__ kel,
-                                                      const int *__restrict__ elems, int nv,
-                                                      const int *__restrict__ conn,
-                                                      const int *__restrict__ fu,
-                                                      const int *__restrict__ centroid,
-                                                      const signed char *__restrict__ dbc,
-                                                      const int *__restrict__ e2nz, long long E,
-                                                      long long off_mp, long long off_cv,
-                                                      long long off_cp, JT *__restrict__ val) {
-  constexpr int NVE = DIM == 2 ? 9 : 27, NP = DIM + 1, NVE2 = NVE * NVE;
-  const int e = elems[blockIdx.x];
-  __shared__ int s_f[NVE];
-  __shared__ int s_pc;
-  if (threadIdx.x < NVE) s_f[threadIdx.x] = fu[conn[(size_t)e * NVE + threadIdx.x]];
-  if (threadIdx.x == 0) s_pc = fu[centroid[e]] + nv;
-  __syncthreads();
-  const double *__restrict__ K = kel + (size_t)e * E;
-  const int *__restrict__ map = e2nz + (size_t)e * E;
-  for (long long idx = threadIdx.x; idx < E; idx += blockDim.x) {
-    int row;
-    bool diag;
-    if (idx < off_mp) {
-      const int blk = (int)(idx / NVE2), t = (int)(idx - (long long)blk * NVE2);
-      const int a = blk / nv, b = blk - a * nv, i = t / NVE, j = t - i * NVE;
-      row = s_f[i] + a;
-      diag = i == j && a == b;
-    } else if (idx < off_cv) {
-      const int r = (int)(idx - off_mp);
-      const int a = r / (NVE * NP), t = r - a * NVE * NP;
-      row = s_f[t / NP] + a;
-      diag = false;
-    } else if (idx < off_cp) {
-      const int t = (int)((idx - off_cv) % (NP * NVE));
-      row = s_pc + t / NVE;
-      diag = false;
-    } else {
-      const int r = (int)(idx - off_cp);
-      row = s_pc + r / NP;
-      diag = r / NP == r % NP;
-    }
-    double v = K[idx];
-    if (dbc[row]) {
-      if (!diag) continue;
-      v = 1.0;
-    }
-    val[map[idx]] += (JT)v;
-  }
-}
-
 template <typename JT>
-static void galerkin_level(gm_ctx *prof, const gm_ctx *above, MgLevel &L, JT *val) {
+static int galerkin_level(gm_ctx *prof, const gm_ctx *above, MgLevel &L, JT *val) {
   gm_ctx *lc = L.ctx;
   const ElemLayout &ly = lc->lay;
   const int nch = 1 << lc->dim;
@@ -1065,17 +1012,13 @@ static void galerkin_level(gm_ctx *prof, const gm_ctx *above, MgLevel &L, JT *va
   gm_launch(prof, GM_K_GALERKIN, gbytes, kern, dim3(lc->num_elems), dim3(256), 0, lc->stream,
             above->d_kel, L.d_child, L.d_Wp, L.d_Wi, L.d_Wv, L.W_stride, L.d_Q, ly.total, ly.off_mp,
             lc->d_kel);
-  for (int col = 0; col < lc->n_ecol; col++) {
-    const int cnt = lc->ecol_ptr[col + 1] - lc->ecol_ptr[col];
-    if (!cnt) continue;
-    const double sbytes = (double)cnt * ly.total * (8.0 + 4.0 + 2.0 * sizeof(JT));
-    auto kern = lc->dim == 2 ? k_elem_scatter<2, JT> : k_elem_scatter<3, JT>;
-    gm_launch(prof, GM_K_ELEM_SCATTER, sbytes, kern, dim3(cnt), dim3(256), 0, lc->stream,
-              (const double *)lc->d_kel, (const int *)(lc->d_ecol_elems + lc->ecol_ptr[col]), lc->nv,
-              (const int *)lc->d_conn, (const int *)lc->d_fu, (const int *)lc->d_centroid,
-              (const signed char *)lc->d_dbc, (const int *)lc->d_e2nz, ly.total, ly.off_mp,
-              ly.off_cv, ly.off_cp, val);
-  }
+  // with the coarse level's own Dirichlet rows
+  double *v64 = nullptr;
+  float *v32 = nullptr;
+  if constexpr (sizeof(JT) == 8) v64 = val;
+  else v32 = val;
+  return gm_gather(prof, GM_K_ELEM_SCATTER, lc, lc->stream, lc->d_kel, nullptr, v64, v32, 1, nullptr, nullptr,
+                   nullptr);
 }
 
 int gm_mg_kel_alloc(gm_ctx *c) {
@@ -1273,28 +1216,9 @@ static int build_colour_rows(gm_ctx *lc) {
   for (double &v : w) v = v > 0.0 ? 1.0 / v : 0.0;
   int rc = upv(&lc->d_mg_wmul, w.data(), w.size());
   if (rc) return rc;
-  // gather lists of the additive smoother: local dof li of element e (nodal
-  // variables node-blocked by variable, then the element's P1 dofs) is unknown
-  // g; its correction sits at e * nl + li
-  const int nl = lc->nv * nve + lc->np;
-  std::vector<int> gptr(lc->N + 1, 0), gent((size_t)lc->num_elems * nl);
-  auto dof = [&](int e, int li) {
-    if (li < lc->nv * nve) {
-      const int a = li / nve, i = li - a * nve;
-      return lc->first_unknown[lc->conn[(size_t)e * nve + i]] + a;
-    }
-    return lc->first_unknown[lc->elem_centroid[e]] + lc->dim + lc->energy + (li - lc->nv * nve);
-  };
-  for (int e = 0; e < lc->num_elems; e++)
-    for (int li = 0; li < nl; li++) gptr[dof(e, li) + 1]++;
-  for (int u = 0; u < lc->N; u++) gptr[u + 1] += gptr[u];
-  std::vector<int> fill(gptr.begin(), gptr.end() - 1);
-  for (int e = 0; e < lc->num_elems; e++)
-    for (int li = 0; li < nl; li++) gent[fill[dof(e, li)]++] = e * nl + li;
-  if ((rc = upv(&lc->d_mg_gptr, gptr.data(), gptr.size())) ||
-      (rc = upv(&lc->d_mg_gent, gent.data(), gent.size())))
-    return rc;
-  GM_HIP(hipMalloc(&lc->d_mg_corr, gent.size() * sizeof(double)));
+  // gather lists of the additive smoother
+  if ((rc = gm_unknown_places(lc))) return rc;
+  GM_HIP(hipMalloc(&lc->d_mg_corr, (size_t)lc->num_elems * nloc_of(lc) * sizeof(double)));
   return upv(&lc->d_mg_rows, rows.data(), rows.size());
 }
 
@@ -1465,13 +1389,10 @@ int gm_mg_setup(gm_ctx *c, const double *x, const double *val, const float *val3
         return GM_ERR_ARG;
       }
       if ((rc = alloc_level_vectors(L, lc, prec, true)) || (rc = gm_mg_kel_alloc(lc))) return rc;
-      if (prec == GM_PREC_MIXED) {
-        k_set<float><<<2048, 256, 0, lc->stream>>>((float *)L.d_val, lc->nval, 0.0f);
-        galerkin_level<float>(c, above, L, (float *)L.d_val);
-      } else {
-        k_set<double><<<2048, 256, 0, lc->stream>>>((double *)L.d_val, lc->nval, 0.0);
-        galerkin_level<double>(c, above, L, (double *)L.d_val);
-      }
+      if ((rc = gm_gather_setup(lc))) return rc;
+      rc = prec == GM_PREC_MIXED ? galerkin_level<float>(c, above, L, (float *)L.d_val)
+                                 : galerkin_level<double>(c, above, L, (double *)L.d_val);
+      if (rc) return rc;
       GM_HIP(hipGetLastError());
       GM_HIP(hipStreamSynchronize(lc->stream));
       above = lc;

@@ -207,7 +207,7 @@ int gm_matrix_fill_full_dev(gm_ctx *ctx, const double *x_dev, double *resid_dev,
 int gm_matrix_fill_full(gm_ctx *ctx, const double *x, double *resid, double *val);
 /* The same assembly, with the Jacobian stored rather than accumulated: val
  * needs no zeroing beforehand (the HEX27 kernel writes each entry's first
- * element contribution and adds the others; QUAD9 zeroes val first).  resid
+ * element contribution and adds the others; QUAD9 writes each sum once).  resid
  * is still accumulated.  Saves the caller's pass over val (8 GB at 48^3). */
 int gm_matrix_fill_full_assign_dev(gm_ctx *ctx, const double *x_dev, double *resid_dev,
                                    double *val_dev);
@@ -375,7 +375,7 @@ int gm_mg_copy_coarse_inverse(const gm_ctx *ctx, double *out);
  * is the kernel's execution alone; gm_prof_get returns the launch count, the
  * summed duration and the summed algorithmic HBM bytes (compulsory traffic,
  * each array counted once per launch) of those launches. */
-#define GM_K_FILL 0       /* k_fill: assembly + scatter of one element colour */
+#define GM_K_FILL 0       /* assembly: k_fill3m, one element colour (HEX27); k_elem2, k_gather (QUAD9) */
 #define GM_K_SPMV 1       /* k_spmv_msr: MSR matvec */
 #define GM_K_ILU_LOWER 2  /* k_ilu_sweep: forward sweep of one patch colour */
 #define GM_K_ILU_UPPER 3  /* k_ilu_sweep: backward sweep of one patch colour */
@@ -387,11 +387,11 @@ int gm_mg_copy_coarse_inverse(const gm_ctx *ctx, double *out);
                              k_vanka_corr: every element's correction (additive) */
 #define GM_K_TRANSFER 9   /* k_csr_apply: restriction or prolongation */
 #define GM_K_VANKA_INV 10 /* k_vanka_invert: element-block inverses of one level */
-#define GM_K_FILL_RESID 11 /* k_fill, residual only (line-search trial), one colour */
+#define GM_K_FILL_RESID 11 /* the same, residual only (line-search trial) */
 #define GM_K_MG_RESID_ROWS 12 /* k_mg_resid_rows: smoother residual on one element colour's rows */
 #define GM_K_MG_DENSE 13  /* k_dense_gemv: exact solve on the coarsest level (dense inverse) */
 #define GM_K_GALERKIN 14  /* k_galerkin: coarse element matrices P^T K P of one level */
-#define GM_K_ELEM_SCATTER 15 /* k_elem_scatter: element matrices of one colour into MSR */
+#define GM_K_ELEM_SCATTER 15 /* k_gather: a coarse level's element matrices into MSR */
 #define GM_K_BAND_PANEL 16 /* k_band_diag / k_band_panel: one 64-column panel of the banded LU */
 #define GM_K_BAND_UPDATE 17 /* k_band_update: trailing update of one panel */
 #define GM_K_BAND_SOLVE 18 /* k_band_step: 128 unknowns of one direction of the banded solve */

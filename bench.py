@@ -241,7 +241,7 @@ def kernel_roofline(name, k, prob, prec, workload):
         tr = recorded_traffic(workload, name) if prec == 0 else None
         return dict(kernel=name, bound="mfma", achieved=round(tf, 2), peak=peak, unit="TFLOP/s",
                     frac=round(tf / peak, 4), traffic=round(tr) if tr else None,
-                    flops_per_launch=round(flops),
+                    flops_per_assembly=round(flops),
                     avg_launch_ms=round(k["avg_ms"], 5),
                     precision="fp64" if prec == 0 else "fp32")
     a = k["GBps"] or 0.0
@@ -408,8 +408,8 @@ def headline(args, torch, capi):
 
     dom = max(kern, key=lambda k: kern[k]["total_ms"])
     roof = kernel_roofline(dom, kern[dom], prob, 0, prob.name)
-    # assembly: a Jacobian + residual assembly is one launch of k_fill per
-    # Newton pass (per element colour if the kernel is coloured)
+    # assembly: a Jacobian + residual assembly is one launch of the element
+    # kernel and one of the gather per Newton pass, both counted as k_fill
     nasm = prep.newton_its
     k_fill = kern.get("k_fill")
     asm_s = k_fill["total_ms"] * 1e-3 / max(nasm, 1) if k_fill else None
@@ -418,20 +418,20 @@ def headline(args, torch, capi):
     if asm_roof:
         asm_roof["per_assembly_s"] = round(asm_s, 6)
         if prob.mesh.dim == 3:
-            # HEX27 node-pair blocks on the FP64 matrix cores (k_fill3m): per
+            # HEX27 node-pair blocks on the FP64 matrix cores (k_elem3): per
             # element and wave, 7 k-steps of 5 shared products (3 more with
-            # Carreau), 6 per momentum block row and 3 for the energy row;
-            # four waves; 2 * 16 * 16 * 4 flop per v_mfma_f64_16x16x4f64
+            # Carreau), 6 per momentum block row and 3 for the energy row, and
+            # 14 for the state at the points; four waves; 2 * 16 * 16 * 4 flop
+            # per v_mfma_f64_16x16x4f64
             en, vm = int(prob.phys.energy), int(prob.phys.visc_model)
-            per_wave = 7 * ((5 + 3 * vm) + 3 * (6 + 3 * vm) + 3 * en)
-            ncol = int(ctx.elem_colours().max()) + 1
-            flops = 4 * per_wave * 2048.0 * prob.mesh.num_elems / ncol
-            tf = flops / (k_fill["avg_ms"] * 1e-3) / 1e12
+            per_wave = 7 * ((5 + 3 * vm) + 3 * (6 + 3 * vm) + 3 * en) + 14
+            flops = 4 * per_wave * 2048.0 * prob.mesh.num_elems
+            tf = flops / asm_s / 1e12
             asm_roof["mfma"] = dict(bound="mfma", achieved=round(tf, 2), peak=FP64_PEAK_TFS,
                                     unit="TFLOP/s", frac=round(tf / FP64_PEAK_TFS, 4),
-                                    flops_per_launch=round(flops),
-                                    note="padded 32 x 32 x 28 products; the map, field, "
-                                         "residual and scatter phases run beside them")
+                                    flops_per_assembly=round(flops),
+                                    note="padded 32 x 32 x 28 products over the time of the assembly (element "
+                                         "matrices and gather)")
     out = {
         "metric": METRIC,
         "value": round(t_plain, 4),

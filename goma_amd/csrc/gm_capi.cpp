@@ -109,7 +109,7 @@ static void free_ctx(gm_ctx *c) {
                   c->d_resid, c->d_dx,    c->d_scale, c->d_val32,    c->d_red,   c->d_xwork,
                   c->d_xsave, c->d_rtrial, c->d_w, c->d_mg_rows, c->d_mg_wmul, c->d_kel,
                   c->d_mg_gptr, c->d_mg_gent, c->d_mg_corr, c->d_stab, c->d_qs_ptr,
-                  c->d_qs_side, c->d_qs_q, c->d_rank, c->d_nn_ptr, c->d_nn_list, c->d_pair,
+                  c->d_qs_side, c->d_qs_q, c->d_nn_ptr, c->d_nn_list, c->d_pair,
                   c->d_rank_t, c->d_src, c->d_re, c->d_ct};
   for (void *p : ptrs)
     if (p) hipFree(p);
@@ -589,7 +589,6 @@ static int solve_impl(gm_ctx *c, double *x, const gm_solver_opts *o, gm_newton_r
   int its_ref = 0, last_its = 0;
   double eta = 0.1, L2_prev = -1.0;  // Eisenstat-Walker forcing term and the last scaled norm
   const bool galerkin = o->precond == GM_PC_MG && o->mg_galerkin && !c->mg.empty();
-  if (galerkin && (rc = gm_mg_kel_alloc(c))) return rc;
   while (!converged && inewton < o->max_newton) {
     double ta = now_s();
     // the PSPG velocity norm of this pass (src/mm_sol_nonlinear.c:1183-1192);
@@ -601,10 +600,8 @@ static int solve_impl(gm_ctx *c, double *x, const gm_solver_opts *o, gm_newton_r
     if ((rc = gm_zero(c, c->d_resid, c->N))) return rc;
     if ((rc = gm_zero(c, c->d_dx, c->N))) return rc;
     // the assembly stores the Jacobian, which needs no zeroing pass
-    c->kel_on = galerkin;
     c->fill_overwrite = 1;
     rc = gm_fill_launch(c, x, c->d_resid, c->d_val, prec == GM_PREC_MIXED ? c->d_val32 : nullptr);
-    c->kel_on = 0;
     c->fill_overwrite = 0;
     if (rc) return rc;
     double un, unoo;

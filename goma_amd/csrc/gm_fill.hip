@@ -1,12 +1,9 @@
 // Element assembly (matrix_fill_full) for QUAD9 / HEX27 Q2-P1 Navier-Stokes
 // with optional energy, as HIP kernels for gfx950.
 //
-// QUAD9: k_elem2 forms the element matrices and vectors, four elements per
-// workgroup, and k_gather (gm_gather.hip) sums them into the rows.  HEX27:
-// k_fill3m, one workgroup per element, elements launched one colour at a time
-// (no two elements of a colour share a node), so every element owns the
-// nonzeros it scatters into during its launch and the scatter is a plain
-// read-modify-write.  Either way: deterministic, no atomics.
+// k_elem2 (QUAD9, four elements per workgroup) and k_elem3 (HEX27, one) form
+// the element matrices and vectors; k_gather (gm_gather.hip) sums them into
+// the rows: deterministic, no atomics.
 //
 // Per element:
 //   1. nodal coordinates / unknowns -> LDS
@@ -53,16 +50,11 @@ struct FillArgs {
   const int *conn;          // [num_elems][nve]
   const int *fu;            // first unknown per node
   const int *centroid;      // centroid node per element
-  const signed char *dbc;   // [N]
-  const double *dbc_val;    // [N]
   const double *tables;     // phi, dphidxi, psi, wt
-  const int *e2nz;          // [num_elems][E]
   const double *x;
-  double *resid;
-  void *val;
-  double *re, *ct;  // QUAD9: element residuals, PSPG continuity x temperature entries
-  double *kel;  // optional [num_elems][E]: element matrices before the Dirichlet rows
-                // (for Galerkin multigrid coarse operators), in the e2nz layout
+  double *re, *ct;  // element residuals, PSPG continuity x temperature entries
+  double *kel;  // [num_elems][E]: element matrices before the Dirichlet rows (also for
+                // the Galerkin multigrid coarse operators), in the e2nz layout
   int *flag;
   // theta-method time step (nullptr x_old: steady): at each node
   // xdot = cmass (x - x_old) - cold xdot_old, cmass = (1 + 2 theta) / dt, cold = 2 theta
@@ -74,9 +66,6 @@ struct FillArgs {
   const int *qs_ptr, *qs_side;
   const double *qs_q;
   const double *stab;  // side tables: [side][point] phi[NVE], dphidxi[NVE][DIM], weight
-  const int *bindx;                 // MSR graph
-  const unsigned short *rank;       // rank map [num_elems][2][nve * nve] (k_build_ranks)
-  int overwrite;                    // 1: first touch of a node pair stores (no zeroing needed)
   int num_nodes;
   double tau_pspg;  // global PSPG tau, 0: no pressure stabilisation
   double supg_e;    // energy SUPG coefficient, 0: Galerkin weights
@@ -634,10 +623,9 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
 }
 
 // ---------------------------------------------------------------------------
-// HEX27 assembly on the matrix cores.
+// HEX27 element matrices on the matrix cores.
 //
-// One workgroup (four waves) per element.  The basis tables, the physical
-// gradients and the quadrature-point fields are staged in LDS; every
+// One workgroup (four waves) per element, all elements in one launch.  Every
 // node-pair block of the element Jacobian is a sum of products
 //   E(X, w, Y)[i][j] = sum_q X[q][i] w[q] Y[q][j]
 // of 27 x 27 operand tables (X, Y in {phi, d phi / d x_p}, weights from the
@@ -656,133 +644,143 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
 // MFMA lane layout (checked on the device): lane l supplies A[l%16][l/16]
 // and B[l/16][l%16] and holds D[l/16 + 4r][l%16], r = 0..3 (rows interleaved).
 //
-// Scatter: each entry's MSR position comes from the element's rank map
-// (rank of node j's first column in the rows of node i, see
-// k_build_ranks), so a node pair's NV x NV block lands at
-// bindx[row] + rank + b - (col > row).  With `overwrite` the first element
-// (in colour order) to touch a node pair stores its values, later ones add:
-// no zeroing pass and no read of the old value on first touch.
+// The products that are not node by node ride along.  The state at the points
+// is one product of the reference tables {d phi / d xi_r, phi} with the nodes'
+// (x, u, xdot) as columns.  Columns 27..30 of the padded tables carry the
+// residual rows' weights W_a(q) (beside phi) and fluxes -Pi_ap(q) (beside
+// d phi / d x_p), so E(phi, dA, phi) + sum_p E(G_p, dA, G_p) holds the
+// residual in columns 27 + a; and dA psi_k in those columns of the products
+// with G_b gives momentum x pressure, whose transpose is continuity x velocity.
+//
+// The workgroup writes the element's matrix before Dirichlet rows (kel, in the
+// e2nz layout), residual (re) and, with PSPG and energy, the continuity x
+// temperature entries (ct); k_gather sums them into the MSR rows.
+// Bound by the element matrices' bytes (98 KB an element with energy) and the
+// 182 products a wave (64 cycles each).  Measured, with k_gather (16^3
+// elements with energy, FP64): 508 us against 716 with eight coloured
+// launches that staged the state by threads and added into the rows through a
+// rank map; 11^3 shear-thinning, FP32 matrix: 217 against 629.
 
-template <int EN, int VISC, typename JT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VISC ? 3 : 4, VISC ? 3 : 4))) void k_fill3m(
-    FillArgs A, const int *__restrict__ elems) {
+struct NodeCols {  // coordinates as x[a][i] from rows of 16 doubles a node
+  const double *p;
+  struct Col {
+    const double *p;
+    __device__ double operator[](int i) const { return p[i * 16]; }
+  };
+  __device__ Col operator[](int a) const { return Col{p + a}; }
+};
+
+template <int EN, int VISC>
+__global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
   constexpr int DIM = 3, NVE = 27, NQ = 27, NP = 4, NV = DIM + EN, NVE2 = NVE * NVE;
-  constexpr int KP = 28, LD = 32, NT = 256, CL = 20;
+  constexpr int KP = 28, LD = 32, NL = NV * NVE + NP, NCOL = DIM + 2 * NV, NG = (KP * LD + 255) / 256;
   using T = Tab<3>;
   constexpr int NSP = STab<3>::NSP, SREC = STab<3>::REC;
-  const int e = elems[xcd_block()];
-  const int tid = threadIdx.x;
+  const int e = xcd_block(), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, kk = lane >> 4;
   const double *__restrict__ tb = A.tables;
 
-  __shared__ double s_x[DIM][NVE];
-  __shared__ double s_u[NV][NVE];
-  __shared__ double s_ud[NV][NVE];
+  __shared__ double s_nod[KP][16];  // columns x, u, xdot of each node
   __shared__ double s_p[NP];
-  __shared__ int s_gun[NV][NVE];   // global row of each nodal unknown
-  __shared__ int s_brow[NV][NVE];  // bindx[row]: start of its off-diagonal list
-  __shared__ signed char s_dir[NV][NVE];
-  __shared__ int s_gp[NP], s_bp[NP];
-  __shared__ signed char s_dirp[NP];
   __shared__ double s_B[NQ][DIM][DIM];
-  __shared__ double s_dA[KP];
+  __shared__ double s_dA[KP], s_mu[KP], s_dmu[KP], s_wpsi[KP][NP];
   __shared__ double s_Phi[KP][LD];
   __shared__ double s_G[DIM][KP][LD];
   __shared__ double s_v[KP][DIM];
   __shared__ double s_gv[KP][DIM][DIM];  // gv[p][a] = d v_a / d x_p
   __shared__ double s_gT[KP][DIM];
-  __shared__ double s_P[KP], s_mu[KP], s_dmu[KP], s_div[KP], s_Td[KP];
-  __shared__ double s_f[KP][DIM], s_vd[KP][DIM];
+  __shared__ double s_m[NQ][DIM];  // PSPG: rho v_dot + rho v.grad v + grad P - f
+  __shared__ double s_rk[2][NP];
   __shared__ double s_su[4];  // energy SUPG: s/h, s d(1/h)/d vc_b
   __shared__ double s_qw[GM_QS_MAX][NSP], s_qh[GM_QS_MAX][NSP];
   __shared__ int s_qsd[GM_QS_MAX];
-  const int qs0 = A.qs_ptr ? A.qs_ptr[e] : 0;
-  const int nqs = A.qs_ptr ? A.qs_ptr[e + 1] - qs0 : 0;
+  // d(column)/d(xi_r) (r < 3) and the column's value (r = 3) at the points,
+  // until the gradients take the space
+  double(*s_F)[NQ][12] = (double(*)[NQ][12])&s_G[0][0][0];
+  static_assert(4 * NQ * 12 <= DIM * KP * LD && NCOL <= 12, "point fields fit the gradient table");
+#define GM_MFMA64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64((a), (b), (c), 0, 0, 0)
+  const d4v z = {0.0, 0.0, 0.0, 0.0};
+  const int qs0 = EN && A.qs_ptr ? A.qs_ptr[e] : 0;
+  const int nqs = EN && A.qs_ptr ? A.qs_ptr[e + 1] - qs0 : 0;
 
-  // 1. gather; basis values into the padded operand table
-  if (tid < NVE) {
-    const int n = A.conn[(size_t)e * NVE + tid];
-    const int f = A.fu[n];
-#pragma unroll
-    for (int k = 0; k < DIM; k++) s_x[k][tid] = A.coor[(size_t)k * A.num_nodes + n];
-#pragma unroll
-    for (int a = 0; a < NV; a++) {
-      const int g = f + a;
-      s_gun[a][tid] = g;
-      s_brow[a][tid] = A.bindx[g];
-      s_dir[a][tid] = A.dbc[g];
-      s_u[a][tid] = A.x[g];
-      s_ud[a][tid] = A.x_old ? A.cmass * (A.x[g] - A.x_old[g]) - A.cold * A.xdot_old[g] : 0.0;
+  // 1. gather: 32 threads per column, node by node; this wave's reference
+  // table (operand of step 2) and this thread's share of the others
+  {
+    const int k = tid & 31, c = tid >> 5;
+    if (c < DIM + NV) {
+      double v = 0.0, vd = 0.0;
+      if (k < NVE) {
+        const int n = A.conn[(size_t)e * NVE + k];
+        if (c < DIM) v = A.coor[(size_t)c * A.num_nodes + n];
+        else {
+          const int g = A.fu[n] + c - DIM;
+          v = A.x[g];
+          // xdot as solve_nonlinear_problem forms it after each update (src/rf_solve.c:2848)
+          if (A.x_old) vd = A.cmass * (v - A.x_old[g]) - A.cold * A.xdot_old[g];
+        }
+      }
+      if (k < KP) {
+        s_nod[k][c] = v;
+        if (c >= DIM) s_nod[k][c + NV] = vd;
+      }
+    } else if (c == 7 && k < NP) {
+      s_p[k] = A.x[A.fu[A.centroid[e]] + NV + k];
     }
-  } else if (tid >= 64 && tid < 64 + NP) {
-    const int k = tid - 64;
-    const int g = A.fu[A.centroid[e]] + DIM + EN + k;
-    s_gp[k] = g;
-    s_bp[k] = A.bindx[g];
-    s_dirp[k] = A.dbc[g];
-    s_p[k] = A.x[g];
   }
-  for (int idx = tid; idx < KP * LD; idx += NT) {
-    const int q = idx / LD, i = idx - q * LD;
-    s_Phi[q][i] = (q < NQ && i < NVE) ? tb[T::PHI + q * NVE + i] : 0.0;
+  double ref[2][KP / 4], dph[NG][DIM];
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int s = 0; s < KP / 4; s++) {
+      const int q = 16 * t + r16, k = 4 * s + kk;
+      ref[t][s] = q < NQ && k < NVE ? tb[wave < 3 ? T::DPHI + (q * NVE + k) * DIM + wave : T::PHI + q * NVE + k] : 0.0;
+    }
+#pragma unroll
+  for (int n = 0; n < NG; n++) {
+    const int t = tid + 256 * n, q = t / LD, i = t - q * LD;
+    const bool in = q < NQ && i < NVE;
+#pragma unroll
+    for (int r = 0; r < DIM; r++) dph[n][r] = in ? tb[T::DPHI + (q * NVE + i) * DIM + r] : 0.0;
+    if (q < KP) s_Phi[q][i] = in ? tb[T::PHI + q * NVE + i] : 0.0;
   }
   __syncthreads();
 
-  // 2. map per quadrature point (beer_belly)
-  if (tid < NQ) {
-    const int q = tid;
-    double J[DIM][DIM];
+  // 2. the columns at the points: wave w takes table w
 #pragma unroll
-    for (int i = 0; i < DIM; i++)
+  for (int t = 0; t < 2; t++) {
+    d4v D = z;
 #pragma unroll
-      for (int j = 0; j < DIM; j++) {
-        double s = 0.0;
-#pragma unroll 3
-        for (int k = 0; k < NVE; k++) s += s_x[j][k] * tb[T::DPHI + (q * NVE + k) * DIM + i];
-        J[i][j] = s;
-      }
-    const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
-                       J[0][1] * (J[1][0] * J[2][2] - J[2][0] * J[1][2]) +
-                       J[0][2] * (J[1][0] * J[2][1] - J[2][0] * J[1][1]);
-    s_B[q][0][0] = (J[1][1] * J[2][2] - J[2][1] * J[1][2]) / det;
-    s_B[q][0][1] = -(J[0][1] * J[2][2] - J[2][1] * J[0][2]) / det;
-    s_B[q][0][2] = (J[0][1] * J[1][2] - J[1][1] * J[0][2]) / det;
-    s_B[q][1][0] = -(J[1][0] * J[2][2] - J[2][0] * J[1][2]) / det;
-    s_B[q][1][1] = (J[0][0] * J[2][2] - J[2][0] * J[0][2]) / det;
-    s_B[q][1][2] = -(J[0][0] * J[1][2] - J[1][0] * J[0][2]) / det;
-    s_B[q][2][0] = (J[1][0] * J[2][1] - J[2][0] * J[1][1]) / det;
-    s_B[q][2][1] = -(J[0][0] * J[2][1] - J[2][0] * J[0][1]) / det;
-    s_B[q][2][2] = (J[0][0] * J[1][1] - J[1][0] * J[0][1]) / det;
-    if (!(det > 0.0)) *(volatile int *)A.flag = 1;
-    s_dA[q] = det * tb[T::WT + q];
-  } else if (tid == NQ) {
-    s_dA[NQ] = 0.0;  // the padding point carries no weight
-  } else if (tid == NQ + 1) {
+    for (int s = 0; s < KP / 4; s++) D = GM_MFMA64(ref[t][s], s_nod[4 * s + kk][r16], D);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int q = 16 * t + kk + 4 * r;
+      if (q < NQ && r16 < NCOL) s_F[wave][q][r16] = D[r];
+    }
+  }
+  if (EN && tid == 255) {
     double vc[DIM], su[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int p = 0; p < DIM; p++) vc[p] = s_u[p][NVE - 1];
-    if (EN && A.supg_e != 0.0) supg_params<DIM>(A.supg_e, s_x, vc, su);
+    for (int p = 0; p < DIM; p++) vc[p] = s_nod[NVE - 1][DIM + p];
+    if (A.supg_e != 0.0) supg_params<DIM>(A.supg_e, NodeCols{&s_nod[0][0]}, vc, su);
 #pragma unroll
     for (int k = 0; k < 4; k++) s_su[k] = su[k];
-  } else if (EN && tid >= 64 && tid < 64 + nqs * NSP) {
+  } else if (EN && tid < nqs * NSP) {
     // QSIDE (src/bc_integ.c:1518-1519, 2156-2157): w |surface Jacobian| q at
     // one surface Gauss point of one side entry
-    const int t2 = tid - 64;
-    const int k = t2 / NSP, g = t2 - k * NSP;
+    const int k = tid / NSP, g = tid - k * NSP;
     const int sd = A.qs_side[qs0 + k] - 1;
     const double *st = A.stab + (size_t)(sd * NSP + g) * SREC;
     const int ax = (sd == 0 || sd == 2) ? 1 : (sd == 1 || sd == 3) ? 0 : 2;
-    int fr[2], nf = 0;
-#pragma unroll
-    for (int a = 0; a < DIM; a++)
-      if (a != ax) fr[nf++] = a;
+    const int fr[2] = {ax == 0 ? 1 : 0, ax == 2 ? 1 : 2};
     double t1[DIM], tt2[DIM];
 #pragma unroll
     for (int j = 0; j < DIM; j++) {
       t1[j] = 0.0;
       tt2[j] = 0.0;
+#pragma unroll 1
       for (int i = 0; i < NVE; i++) {
-        t1[j] += s_x[j][i] * st[NVE + i * DIM + fr[0]];
-        tt2[j] += s_x[j][i] * st[NVE + i * DIM + fr[1]];
+        t1[j] += s_nod[i][j] * st[NVE + i * DIM + fr[0]];
+        tt2[j] += s_nod[i][j] * st[NVE + i * DIM + fr[1]];
       }
     }
     const double c0 = t1[1] * tt2[2] - t1[2] * tt2[1], c1 = t1[2] * tt2[0] - t1[0] * tt2[2],
@@ -790,76 +788,95 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VISC ? 3 : 
     const double *qk = A.qs_q + 3 * (qs0 + k);
     const double wd = st[NVE + NVE * DIM] * sqrt(c0 * c0 + c1 * c1 + c2 * c2);
     double Tg = 0.0;
-    if constexpr (EN)
-      for (int j = 0; j < NVE; j++) Tg += st[j] * s_u[DIM][j];
+#pragma unroll 1
+    for (int j = 0; j < NVE; j++) Tg += st[j] * s_nod[j][2 * DIM];
     s_qw[k][g] = wd * (qk[0] + qk[1] * (qk[2] - Tg));
     s_qh[k][g] = wd * qk[1];
     if (g == 0) s_qsd[k] = sd;
   }
+  static_assert(GM_QS_MAX * NSP <= 255, "a thread per surface point");
   __syncthreads();
 
-  // 3. physical gradients into the padded operand tables (load_bf_grad)
-  for (int idx = tid; idx < DIM * KP * LD; idx += NT) {
-    const int p = idx / (KP * LD), r0 = idx - p * KP * LD, q = r0 / LD, i = r0 - q * LD;
-    double s = 0.0;
-    if (q < NQ && i < NVE) {
+  // 3. map (beer_belly) and physical gradients of the fields (load_fv,
+  // load_fv_grads): a thread per point and variable, each forming the inverse
+  const int pq = tid >> 2, pa = tid & 3;
+  const bool point = pq < NQ;
+  double g[DIM] = {0.0, 0.0, 0.0}, v[DIM] = {0.0, 0.0, 0.0}, uda = 0.0, Tq = 0.0, dA = 0.0;
+  if (point) {
+    const int q = pq;
+    double J[DIM][DIM], B[DIM][DIM];
 #pragma unroll
-      for (int r = 0; r < DIM; r++) s += s_B[q][p][r] * tb[T::DPHI + (q * NVE + i) * DIM + r];
+    for (int i = 0; i < DIM; i++)
+#pragma unroll
+      for (int j = 0; j < DIM; j++) J[i][j] = s_F[i][q][j];
+    const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
+                       J[0][1] * (J[1][0] * J[2][2] - J[2][0] * J[1][2]) +
+                       J[0][2] * (J[1][0] * J[2][1] - J[2][0] * J[1][1]);
+    B[0][0] = (J[1][1] * J[2][2] - J[2][1] * J[1][2]) / det;
+    B[0][1] = -(J[0][1] * J[2][2] - J[2][1] * J[0][2]) / det;
+    B[0][2] = (J[0][1] * J[1][2] - J[1][1] * J[0][2]) / det;
+    B[1][0] = -(J[1][0] * J[2][2] - J[2][0] * J[1][2]) / det;
+    B[1][1] = (J[0][0] * J[2][2] - J[2][0] * J[0][2]) / det;
+    B[1][2] = -(J[0][0] * J[1][2] - J[1][0] * J[0][2]) / det;
+    B[2][0] = (J[1][0] * J[2][1] - J[2][0] * J[1][1]) / det;
+    B[2][1] = -(J[0][0] * J[2][1] - J[2][0] * J[0][1]) / det;
+    B[2][2] = (J[0][0] * J[1][1] - J[1][0] * J[0][1]) / det;
+    dA = det * tb[T::WT + q];
+    if (pa < NV) {
+#pragma unroll
+      for (int p = 0; p < DIM; p++)
+#pragma unroll
+        for (int r = 0; r < DIM; r++) g[p] += B[p][r] * s_F[r][q][DIM + pa];
+      uda = s_F[3][q][DIM + NV + pa];
     }
-    s_G[p][q][i] = s;
+#pragma unroll
+    for (int p = 0; p < DIM; p++) v[p] = s_F[3][q][DIM + p];
+    if constexpr (EN) Tq = s_F[3][q][2 * DIM];
+    if (pa == 0) {
+      if (!(det > 0.0)) *(volatile int *)A.flag = 1;
+#pragma unroll
+      for (int p = 0; p < DIM; p++) {
+        s_v[q][p] = v[p];
+#pragma unroll
+        for (int r = 0; r < DIM; r++) s_B[q][p][r] = B[p][r];
+      }
+      s_dA[q] = dA;
+    }
+  }
+  if (pq < KP) {  // zeros at the padding point
+#pragma unroll
+    for (int p = 0; p < DIM; p++) {
+      if (pa < DIM) s_gv[pq][p][pa] = g[p];
+      else s_gT[pq][p] = g[p];
+      if (pq == NQ) s_v[NQ][p] = 0.0;
+    }
+    if (pq == NQ) s_dA[NQ] = s_mu[NQ] = s_dmu[NQ] = s_wpsi[NQ][pa] = 0.0;
   }
   __syncthreads();
 
-  // 4. fields at the quadrature points (load_fv, load_fv_grads): eight
-  // threads per point, each summing a quarter of the nodes, then a
-  // butterfly over the eight
-  if (tid < NQ * 8) {
-    const int q = tid >> 3, sub = tid & 7;
-    double v[DIM] = {0.0, 0.0, 0.0}, gv[DIM][DIM], Tq = 0.0, gT[DIM] = {0.0, 0.0, 0.0};
-    double vd[DIM] = {0.0, 0.0, 0.0}, Td = 0.0;
+  // 4. physical gradients of the basis into the padded tables (load_bf_grad);
+  // viscosity, stress and sources at the points into columns 27 + a
 #pragma unroll
-    for (int a = 0; a < DIM; a++)
+  for (int n = 0; n < NG; n++) {
+    const int t = tid + 256 * n, q = t / LD, i = t - q * LD;
+    if (q >= KP || (i >= NVE && i < NVE + NV && q < NQ)) continue;
 #pragma unroll
-      for (int p = 0; p < DIM; p++) gv[p][a] = 0.0;
-#pragma unroll 1
-    for (int k = sub; k < NVE; k += 8) {
-      const double ph = s_Phi[q][k];
-      double g[DIM];
+    for (int p = 0; p < DIM; p++) {
+      double s = 0.0;
+      if (q < NQ && i < NVE) {
 #pragma unroll
-      for (int p = 0; p < DIM; p++) g[p] = s_G[p][q][k];
-#pragma unroll
-      for (int a = 0; a < DIM; a++) {
-        const double ua = s_u[a][k];
-        v[a] += ua * ph;
-        vd[a] += s_ud[a][k] * ph;
-#pragma unroll
-        for (int p = 0; p < DIM; p++) gv[p][a] += ua * g[p];
+        for (int r = 0; r < DIM; r++) s += s_B[q][p][r] * dph[n][r];
       }
-      if constexpr (EN) {
-        const double tk = s_u[DIM][k];
-        Tq += tk * ph;
-        Td += s_ud[DIM][k] * ph;
-#pragma unroll
-        for (int p = 0; p < DIM; p++) gT[p] += tk * g[p];
-      }
+      s_G[p][q][i] = s;
     }
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1) {
-#pragma unroll
-      for (int a = 0; a < DIM; a++) {
-        v[a] += __shfl_xor(v[a], o, 8);
-        vd[a] += __shfl_xor(vd[a], o, 8);
-        gT[a] += __shfl_xor(gT[a], o, 8);
-#pragma unroll
-        for (int p = 0; p < DIM; p++) gv[p][a] += __shfl_xor(gv[p][a], o, 8);
-      }
-      Tq += __shfl_xor(Tq, o, 8);
-      Td += __shfl_xor(Td, o, 8);
-    }
-    if (sub == 0) {
-      double P = 0.0;
-#pragma unroll
-      for (int k = 0; k < NP; k++) P += s_p[k] * tb[T::PSI + q * NP + k];
+  }
+  const double rho = A.rho, rCp = A.rho * A.Cp, kc = A.kcond;
+  const double cm = A.x_old ? A.cmass : 0.0;
+  const bool ps = A.tau_pspg != 0.0;
+  if (tid < 128) {
+    double ck = 0.0;
+    if (point) {
+      const int q = pq;
       double mu = A.mu0, dmu = 0.0;
       if constexpr (VISC == 1) {
         // calc_shearrate + carreau_viscosity (src/mm_fill_util.c:4564,
@@ -869,386 +886,271 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VISC ? 3 : 
         for (int a = 0; a < DIM; a++)
 #pragma unroll
           for (int b = 0; b < DIM; b++) {
-            const double gab = gv[a][b] + gv[b][a];
+            const double gab = s_gv[q][a][b] + s_gv[q][b][a];
             gd += gab * gab;
           }
         gd = sqrt(0.5 * fabs(gd));
         const bool nz = fabs(gd) > 1.0e-298;
         const double val2 = nz ? pow(A.lam * gd, A.aexp) : 0.0;
-        mu = A.muinf + (A.mu0 - A.muinf) * pow(1.0 + val2, (A.nexp - 1.0) / A.aexp);
-        if (nz) {
-          const double val = pow(A.lam * gd, A.aexp - 1.0);
-          const double val1 = pow(1.0 + val2, (A.nexp - 1.0 - A.aexp) / A.aexp);
-          dmu = (A.mu0 - A.muinf) * (A.nexp - 1.0) * A.lam * val * val1 / gd;
+        const double pm = pow(1.0 + val2, (A.nexp - 1.0) / A.aexp);
+        mu = A.muinf + (A.mu0 - A.muinf) * pm;
+        // d mu / d gammadot / gammadot; lam^a gd^(a-1) = val2 / gd
+        if (nz) dmu = (A.mu0 - A.muinf) * (A.nexp - 1.0) * (val2 / gd) * (pm / (1.0 + val2)) / gd;
+      }
+      double P = 0.0;
+#pragma unroll
+      for (int k = 0; k < NP; k++) P += s_p[k] * tb[T::PSI + q * NP + k];
+      double adv = 0.0;
+#pragma unroll
+      for (int p = 0; p < DIM; p++) adv += v[p] * g[p];
+      if (pa < DIM) {
+        const double f = EN ? rho * A.g[pa] * (-A.beta * (Tq - A.Tref)) : 0.0;
+        s_Phi[q][NVE + pa] = f - rho * (adv + uda);
+#pragma unroll
+        for (int p = 0; p < DIM; p++)
+          s_G[p][q][NVE + pa] = (pa == p ? P : 0.0) - mu * (g[p] + s_gv[q][pa][p]);
+        if (ps) {
+          double gP = 0.0;
+#pragma unroll
+          for (int l = 1; l < NP; l++) gP += s_p[l] * s_B[q][pa][l - 1];
+          s_m[q][pa] = rho * (adv + uda) + gP - f;
         }
+      } else if constexpr (EN) {
+        s_Phi[q][NVE + DIM] = A.hsrc - rCp * (adv + uda);
+#pragma unroll
+        for (int p = 0; p < DIM; p++) s_G[p][q][NVE + DIM] = -kc * g[p] - rCp * s_su[0] * adv * v[p];
       }
-      double div = 0.0;
-#pragma unroll
-      for (int a = 0; a < DIM; a++) {
-        s_v[q][a] = v[a];
-        s_vd[q][a] = vd[a];
-        s_gT[q][a] = gT[a];
-        div += gv[a][a];
-#pragma unroll
-        for (int p = 0; p < DIM; p++) s_gv[q][p][a] = gv[p][a];
-        s_f[q][a] = EN ? A.rho * A.g[a] * (-A.beta * (Tq - A.Tref)) : 0.0;
+      if (pa == 0) {
+        s_mu[q] = mu;
+        s_dmu[q] = dmu;
       }
-      s_P[q] = P;
-      s_mu[q] = mu;
-      s_dmu[q] = dmu;
-      s_div[q] = div;
-      s_Td[q] = Td;
+      const double wp = dA * tb[T::PSI + q * NP + pa];
+      s_wpsi[q][pa] = wp;
+      ck = wp * (s_gv[q][0][0] + s_gv[q][1][1] + s_gv[q][2][2]);
     }
-  } else if (tid == NT - 1) {
-    // the padding point: finite zeros for the weights read by the products
+    // continuity residual: psi_k div v over this wave's points
 #pragma unroll
-    for (int a = 0; a < DIM; a++) {
-      s_v[NQ][a] = 0.0;
-      s_vd[NQ][a] = 0.0;
-      s_gT[NQ][a] = 0.0;
-      s_f[NQ][a] = 0.0;
-#pragma unroll
-      for (int p = 0; p < DIM; p++) s_gv[NQ][p][a] = 0.0;
-    }
-    s_P[NQ] = s_mu[NQ] = s_dmu[NQ] = s_div[NQ] = s_Td[NQ] = 0.0;
+    for (int o = 4; o < 64; o <<= 1) ck += __shfl_xor(ck, o);
+    if (lane < NP) s_rk[wave][lane] = ck;
   }
   __syncthreads();
 
-  const double rho = A.rho, rCp = A.rho * A.Cp, kc = A.kcond;
-  const double cm = A.x_old ? A.cmass : 0.0;
-  JT *__restrict__ out = (JT *)A.val;
-  const bool ow = A.overwrite != 0;
-  const unsigned short *__restrict__ rk = A.rank + (size_t)e * 2 * NVE2;
-
-  // 5a. residual rows
-  for (int t = tid; t < NV * NVE + NP; t += NT) {
-    int row;
-    double R = 0.0;
-    if (t < NV * NVE) {
-      const int a = t / NVE, i = t - a * NVE;
-      row = s_gun[a][i];
-      if (a < DIM) {
+  // 5a. shared products: E(phi, dA, phi), E(phi, dA, v.G), sum_p E(G_p, dA,
+  // G_p) and (Carreau) its mu-weighted form; the residual in columns 27 + a.
+  // Wave w: rows 16 (w >> 1) .. +15, columns 16 (w & 1) .. +15 of every block
+  const int i0 = 16 * (wave >> 1), ii = i0 + r16;  // row operand (A)
+  const int j = 16 * (wave & 1) + r16;             // column operand (B) and column
+  const bool node = j < NVE;
+  double *__restrict__ re = A.re + (size_t)e * NL;
+  double *__restrict__ K = A.kel + (size_t)e * A.E;
+  d4v A1 = z, L1 = z, Dadv = z, Lmu = z;
+  if (!A.resid_only) {
 #pragma unroll 1
-        for (int q = 0; q < NQ; q++) {
-          const double ph = s_Phi[q][i];
-          double adv = 0.0, dif = 0.0;
-#pragma unroll
-          for (int p = 0; p < DIM; p++) {
-            adv += s_v[q][p] * s_gv[q][p][a];
-            const double Pi_ap = (a == p ? -s_P[q] : 0.0) + s_mu[q] * (s_gv[q][a][p] + s_gv[q][p][a]);
-            dif += s_G[p][q][i] * Pi_ap;
-          }
-          R += s_dA[q] * (-rho * ph * adv - dif + ph * s_f[q][a] - rho * ph * s_vd[q][a]);
-        }
-      } else {
-        const double sw = s_su[0];
-#pragma unroll 1
-        for (int q = 0; q < NQ; q++) {
-          const double ph = s_Phi[q][i];
-          double adv = 0.0, dif = 0.0;
-#pragma unroll
-          for (int p = 0; p < DIM; p++) {
-            adv += s_v[q][p] * s_gT[q][p];
-            dif += s_G[p][q][i] * s_gT[q][p];
-          }
-          double wi = ph;
-          if (sw != 0.0) {
-            double vgi = 0.0;
-#pragma unroll
-            for (int p = 0; p < DIM; p++) vgi += s_v[q][p] * s_G[p][q][i];
-            wi += sw * vgi;
-          }
-          R += s_dA[q] * (-rCp * wi * adv - kc * dif + ph * A.hsrc - rCp * ph * s_Td[q]);
-        }
-        for (int k = 0; k < nqs; k++)
-          for (int g = 0; g < NSP; g++) R += s_qw[k][g] * A.stab[(size_t)(s_qsd[k] * NSP + g) * SREC + i];
-      }
-      if (s_dir[a][i]) R = s_u[a][i] - A.dbc_val[row];
-    } else {
-      const int k = t - NV * NVE;
-      row = s_gp[k];
-#pragma unroll 1
-      for (int q = 0; q < NQ; q++) R += s_dA[q] * tb[T::PSI + q * NP + k] * s_div[q];
-      if (A.tau_pspg != 0.0 && k > 0) {
-        // PSPG: grad psi_k . tau (rho v_dot + rho v.grad v + grad P - f) dA,
-        // formed per point from the staged fields (four threads do this)
-#pragma unroll 1
-        for (int q = 0; q < NQ; q++) {
-          double r = 0.0;
-#pragma unroll
-          for (int a = 0; a < DIM; a++) {
-            double adv = 0.0, gP = 0.0;
-#pragma unroll
-            for (int p = 0; p < DIM; p++) adv += s_v[q][p] * s_gv[q][p][a];
-#pragma unroll
-            for (int l = 1; l < NP; l++) gP += s_p[l] * s_B[q][a][l - 1];
-            r += s_B[q][a][k - 1] * (rho * (adv + s_vd[q][a]) + gP - s_f[q][a]);
-          }
-          R += A.tau_pspg * s_dA[q] * r;
-        }
-      }
-      if (s_dirp[k]) R = s_p[k] - A.dbc_val[row];
-    }
-    A.resid[row] += R;
-  }
-
-  if (A.resid_only) return;
-
-  // 5b. nodal blocks on the matrix cores: wave w computes rows 16 (w >> 1) ..
-  // +15 and columns 16 (w & 1) .. +15 of every block
-  {
-    const int lane = tid & 63, wave = tid >> 6;
-    const int r16 = lane & 15, kk = lane >> 4;
-    const int ii = 16 * (wave >> 1) + r16;  // row operand index (A)
-    const int jj = 16 * (wave & 1) + r16;   // column operand index (B)
-#define GM_MFMA64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64((a), (b), (c), 0, 0, 0)
-    const d4v z = {0.0, 0.0, 0.0, 0.0};
-    // shared products, four independent chains per k-step: E(phi, dA, phi),
-    // E(phi, dA, v.G), sum_p E(G_p, dA, G_p) and (Carreau) its mu-weighted
-    // form, folded into the diagonal-block terms
-    d4v A1 = z, Dadv = z, L1 = z, Lmu = z;
-    const bool supg = EN && s_su[0] != 0.0;
-#pragma unroll 1
-    for (int q0 = 0; q0 < KP; q0 += 4) {
-      const int q = q0 + kk;
-      const double dA = s_dA[q];
-      const double phA = s_Phi[q][ii] * dA, phB = s_Phi[q][jj];
+    for (int q = kk; q < KP; q += 4) {
+      const double dAq = s_dA[q], phA = s_Phi[q][ii] * dAq;
       double vB = 0.0;
 #pragma unroll
-      for (int p = 0; p < DIM; p++) vB += s_v[q][p] * s_G[p][q][jj];
-      A1 = GM_MFMA64(phA, phB, A1);
+      for (int p = 0; p < DIM; p++) vB += s_v[q][p] * s_G[p][q][j];
+      A1 = GM_MFMA64(phA, s_Phi[q][j], A1);
       Dadv = GM_MFMA64(phA, vB, Dadv);
 #pragma unroll
       for (int p = 0; p < DIM; p++) {
-        const double gA = s_G[p][q][ii] * dA, gB = s_G[p][q][jj];
+        const double gA = s_G[p][q][ii] * dAq, gB = s_G[p][q][j];
         L1 = GM_MFMA64(gA, gB, L1);
         if constexpr (VISC == 1) Lmu = GM_MFMA64(gA * s_mu[q], gB, Lmu);
       }
     }
-    if constexpr (VISC == 0) Lmu = A.mu0 * L1;
-    const d4v Dm = -(rho * Dadv + Lmu + (rho * cm) * A1);
-    const d4v Tt = -(rCp * Dadv + kc * L1 + (rCp * cm) * A1);
-
-    // this lane's rows i = 16 (wave >> 1) + kk + 4 r, column j = jj: rank
-    // words of the four node pairs
-    const int j = jj;
-    unsigned rmw[4], rew[4];
+  } else if (wave & 1) {
+#pragma unroll 1
+    for (int q = kk; q < KP; q += 4) {
+      const double dAq = s_dA[q];
+      A1 = GM_MFMA64(s_Phi[q][ii] * dAq, s_Phi[q][j], A1);
+#pragma unroll
+      for (int p = 0; p < DIM; p++) L1 = GM_MFMA64(s_G[p][q][ii] * dAq, s_G[p][q][j], L1);
+    }
+  }
+  if (j >= NVE && j < NVE + NV) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int i = 16 * (wave >> 1) + kk + 4 * r;
-      const bool in = i < NVE && j < NVE;
-      rmw[r] = in ? rk[i * NVE + j] : 0u;
-      rew[r] = (in && EN) ? rk[NVE2 + i * NVE + j] : 0u;
+      const int i = i0 + kk + 4 * r;
+      if (i >= NVE) continue;
+      double R = A1[r] + L1[r];
+      if (EN && j == NVE + DIM)
+        for (int k = 0; k < nqs; k++)
+#pragma unroll 1
+          for (int s = 0; s < NSP; s++) R += s_qw[k][s] * A.stab[(size_t)(s_qsd[k] * NSP + s) * SREC + i];
+      re[(j - NVE) * NVE + i] = R;
     }
-    // scatter of one block row a (put_dirichlet_in_matrix, load_lec)
-    auto scatter_row = [&](int a, const d4v *Jr) {
+  }
+  if (tid < NP) {
+    double R = s_rk[0][tid] + s_rk[1][tid];
+    if (ps && tid > 0) {
+      // PSPG: grad psi_k . tau (rho v_dot + rho v.grad v + grad P - f) dA
+#pragma unroll 1
+      for (int q = 0; q < NQ; q++) {
+        double r = 0.0;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int i = 16 * (wave >> 1) + kk + 4 * r;
-        if (i >= NVE || j >= NVE) continue;
-        const int t = i * NVE + j;
-        const bool first = ow && (rmw[r] & 0x8000u);
-        const int row = s_gun[a][i];
-        const bool dir = s_dir[a][i] != 0;
-        const int base = s_brow[a][i] + (a < DIM ? (int)(rmw[r] & 0x7fffu) : (int)rew[r]);
-#pragma unroll
-        for (int b = 0; b < NV; b++) {
-          double v = Jr[b][r];
-          if (A.kel) A.kel[(size_t)e * A.E + (size_t)(a * NV + b) * NVE2 + t] = v;
-          if (dir) {
-            if (a == b && i == j) v = 1.0;
-            else if (first) v = 0.0;
-            else continue;
-          }
-          const int col = s_gun[b][j];
-          const long long pos = row == col ? row : base + b - (col > row ? 1 : 0);
-          if (first) out[pos] = (JT)v;
-          else out[pos] += (JT)v;
-        }
+        for (int a = 0; a < DIM; a++) r += s_B[q][a][tid - 1] * s_m[q][a];
+        R += A.tau_pspg * s_dA[q] * r;
       }
-    };
-    // block row a of the momentum equation: three independent chains (b)
-#pragma unroll 1
-    for (int a = 0; a < DIM; a++) {
-      d4v Jr[NV];
+    }
+    re[NV * NVE + tid] = R;
+  }
+  if (A.resid_only) return;
+
+  // 5b. nodal blocks: rows i0 + kk + 4 r, column j
+  auto store = [&](int a, int b, const d4v &D) {
+    double *__restrict__ k = K + (size_t)(a * NV + b) * NVE2 + j;
 #pragma unroll
-      for (int b = 0; b < DIM; b++) Jr[b] = a == b ? Dm : z;
+    for (int r = 0; r < 4; r++) {
+      const int i = i0 + kk + 4 * r;
+      if (i < NVE && node) k[i * NVE] = D[r];
+    }
+  };
+  if constexpr (VISC == 0) Lmu = A.mu0 * L1;
+  const d4v Dm = -(rho * Dadv + Lmu + (rho * cm) * A1);
+  d4v Tt = -(rCp * Dadv + kc * L1 + (rCp * cm) * A1);
 #pragma unroll 1
-      for (int q0 = 0; q0 < KP; q0 += 4) {
-        const int q = q0 + kk;
-        const double dA = s_dA[q];
-        const double phA = s_Phi[q][ii] * (-rho * dA), phB = s_Phi[q][jj];
-        const double gaB = s_G[a][q][jj];
-        const double wmu = -dA * (VISC ? s_mu[q] : A.mu0);
+  for (int a = 0; a < DIM; a++) {
+    d4v J[DIM];
+#pragma unroll
+    for (int b = 0; b < DIM; b++) J[b] = z;
+#pragma unroll 1
+    for (int q = kk; q < KP; q += 4) {
+      const double dAq = s_dA[q], phA = s_Phi[q][ii] * (-rho * dAq), phB = node ? s_Phi[q][j] : 0.0;
+      double gA[DIM];
+#pragma unroll
+      for (int b = 0; b < DIM; b++) gA[b] = s_G[b][q][ii];
+      // columns 27 + k: dA psi_k, momentum x pressure
+      const double gB = node ? s_G[a][q][j] * (-dAq * (VISC ? s_mu[q] : A.mu0)) : s_wpsi[q][(j - NVE) & 3];
+#pragma unroll
+      for (int b = 0; b < DIM; b++) J[b] = GM_MFMA64(phA * s_gv[q][b][a], phB, J[b]);
+#pragma unroll
+      for (int b = 0; b < DIM; b++) J[b] = GM_MFMA64(gA[b], gB, J[b]);
+      if constexpr (VISC == 1) {
+        // Carreau: (d mu / d gammadot) / gammadot (G_i . gamma_a) (g_j . gamma_b)
         double hA = 0.0;
-        if constexpr (VISC == 1) {
-          // Carreau: (d mu / d gammadot) / gammadot (G_i . gamma_a) (g_j . gamma_b)
 #pragma unroll
-          for (int p = 0; p < DIM; p++) hA += s_G[p][q][ii] * (s_gv[q][a][p] + s_gv[q][p][a]);
-          hA *= -dA * s_dmu[q];
-        }
+        for (int p = 0; p < DIM; p++) hA += gA[p] * (s_gv[q][a][p] + s_gv[q][p][a]);
+        hA *= -dAq * s_dmu[q];
 #pragma unroll
         for (int b = 0; b < DIM; b++) {
-          // advection through d_b v_a, then mu g_j,a G_i,b
-          Jr[b] = GM_MFMA64(phA * s_gv[q][b][a], phB, Jr[b]);
-          Jr[b] = GM_MFMA64(s_G[b][q][ii] * wmu, gaB, Jr[b]);
-          if constexpr (VISC == 1) {
-            double hB = 0.0;
+          double hB = 0.0;
 #pragma unroll
-            for (int p = 0; p < DIM; p++) hB += s_G[p][q][jj] * (s_gv[q][b][p] + s_gv[q][p][b]);
-            Jr[b] = GM_MFMA64(hA, hB, Jr[b]);
+          for (int p = 0; p < DIM; p++) hB += s_G[p][q][j] * (s_gv[q][b][p] + s_gv[q][p][b]);
+          J[b] = GM_MFMA64(hA, node ? hB : 0.0, J[b]);
+        }
+      }
+    }
+    if (a == 0 && j >= NVE && j < NVE + NP) {
+      // momentum x pressure (J_m_P): int grad_b phi_i psi_k dA, and its
+      // transpose, continuity x velocity (J_c_v)
+      const int k = j - NVE;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int i = i0 + kk + 4 * r;
+        if (i >= NVE) continue;
+#pragma unroll
+        for (int b = 0; b < DIM; b++) {
+          K[A.off_mp + (b * NVE + i) * NP + k] = J[b][r];
+          if (!ps) K[A.off_cv + (b * NP + k) * NVE + i] = J[b][r];
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < DIM; b++) store(a, b, a == b ? J[b] + Dm : J[b]);
+    if constexpr (EN) store(a, DIM, (-rho * A.g[a] * A.beta) * A1);
+  }
+  if constexpr (EN) {
+    const double sw = s_su[0];
+    d4v J[DIM];
+#pragma unroll
+    for (int b = 0; b < DIM; b++) J[b] = z;
+    if (sw != 0.0) {
+#pragma unroll 1
+      for (int q = kk; q < KP; q += 4) {
+        const double w = -rCp * s_dA[q], phB = s_Phi[q][j];
+        // (phi_i + sw v.G_i) d_b T + sw (v.grad T) G_b,i: the SUPG weight on
+        // the advection and its derivative in v at the column node; and the
+        // weight's part of J_TT, -rho Cp sw E(v.G_i dA, v.G_j)
+        double vA = 0.0, vgT = 0.0, vB = 0.0;
+#pragma unroll
+        for (int p = 0; p < DIM; p++) {
+          vA += s_v[q][p] * s_G[p][q][ii];
+          vgT += s_v[q][p] * s_gT[q][p];
+          vB += s_v[q][p] * s_G[p][q][j];
+        }
+        const double wi = s_Phi[q][ii] + sw * vA;
+#pragma unroll
+        for (int b = 0; b < DIM; b++)
+          J[b] = GM_MFMA64(w * (wi * s_gT[q][b] + sw * vgT * s_G[b][q][ii]), phB, J[b]);
+        Tt = GM_MFMA64(w * sw * vA, vB, Tt);
+      }
+      if (j == NVE - 1) {
+        // d(1/h)/dv at the last local node: -rho Cp s_b sum_q dA (v.grad T) v_b G_b,i
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int i = i0 + kk + 4 * r;
+          if (i >= NVE) continue;
+#pragma unroll
+          for (int b = 0; b < DIM; b++) {
+            double c = 0.0;
+#pragma unroll 1
+            for (int q = 0; q < NQ; q++) {
+              double vgT = 0.0;
+#pragma unroll
+              for (int p = 0; p < DIM; p++) vgT += s_v[q][p] * s_gT[q][p];
+              c += s_dA[q] * vgT * s_v[q][b] * s_G[b][q][i];
+            }
+            J[b][r] -= rCp * s_su[1 + b] * c;
           }
         }
       }
-      if constexpr (EN) Jr[DIM] = (-rho * A.g[a] * A.beta) * A1;
-      scatter_row(a, Jr);
+    } else {
+#pragma unroll 1
+      for (int q = kk; q < KP; q += 4) {
+        const double phA = s_Phi[q][ii] * (-rCp * s_dA[q]), phB = s_Phi[q][j];
+#pragma unroll
+        for (int b = 0; b < DIM; b++) J[b] = GM_MFMA64(phA * s_gT[q][b], phB, J[b]);
+      }
     }
-    if constexpr (EN) {
-      d4v Jr[NV];
-#pragma unroll
-      for (int b = 0; b < DIM; b++) Jr[b] = z;
-      const double sw = s_su[0];
-      Jr[DIM] = Tt;
-      if (supg) {
+    // QCONV: -h w |surface Jacobian| phi_i phi_j over the element's sides
+    for (int k = 0; k < nqs; k++) {
+      if (A.qs_q[3 * (qs0 + k) + 1] == 0.0 || !node) continue;
 #pragma unroll 1
-        for (int q0 = 0; q0 < KP; q0 += 4) {
-          const int q = q0 + kk;
-          const double w = -rCp * s_dA[q], phB = s_Phi[q][jj];
-          // (phi_i + sw v.G_i) d_b T + sw (v.grad T) G_b,i: the SUPG weight on
-          // the advection and its derivative in v at the column node; and
-          // the weight's part of J_TT, -rho Cp sw E(v.G_i dA, v.G_j)
-          double vA = 0.0, vgT = 0.0, vB = 0.0;
+      for (int s = 0; s < NSP; s++) {
+        const double *st = A.stab + (size_t)(s_qsd[k] * NSP + s) * SREC;
 #pragma unroll
-          for (int p = 0; p < DIM; p++) {
-            vA += s_v[q][p] * s_G[p][q][ii];
-            vgT += s_v[q][p] * s_gT[q][p];
-            vB += s_v[q][p] * s_G[p][q][jj];
-          }
-          const double wi = s_Phi[q][ii] + sw * vA;
-#pragma unroll
-          for (int b = 0; b < DIM; b++)
-            Jr[b] = GM_MFMA64(w * (wi * s_gT[q][b] + sw * vgT * s_G[b][q][ii]), phB, Jr[b]);
-          Jr[DIM] = GM_MFMA64(w * sw * vA, vB, Jr[DIM]);
-        }
-      } else {
-#pragma unroll 1
-        for (int q0 = 0; q0 < KP; q0 += 4) {
-          const int q = q0 + kk;
-          const double phA = s_Phi[q][ii] * (-rCp * s_dA[q]), phB = s_Phi[q][jj];
-#pragma unroll
-          for (int b = 0; b < DIM; b++) Jr[b] = GM_MFMA64(phA * s_gT[q][b], phB, Jr[b]);
+        for (int r = 0; r < 4; r++) {
+          const int i = i0 + kk + 4 * r;
+          if (i < NVE) Tt[r] -= s_qh[k][s] * st[i] * st[j];
         }
       }
-      scatter_row(DIM, Jr);
     }
+#pragma unroll
+    for (int b = 0; b < DIM; b++) store(DIM, b, J[b]);
+    store(DIM, DIM, Tt);
+  }
 #undef GM_MFMA64
-  }
 
-  // energy SUPG: d(1/h)/dv at the last local node adds
-  // -rho Cp s_d,b sum_q dA (v.grad T) v_b G_b,i to the energy rows' columns of
-  // that node's velocities, on top of the entries scattered above
-  if (EN && s_su[0] != 0.0) {
-    __syncthreads();
-    for (int t = tid; t < DIM * NVE; t += NT) {
-      const int b = t / NVE, i = t - b * NVE;
-      double c = 0.0;
+  // 5c. PSPG: continuity x velocity gains tau rho [phi_j grad psi_k . d_b v +
+  // grad_b psi_k (v.grad phi_j + c phi_j)], continuity x temperature is tau rho
+  // beta (grad psi_k . g) phi_j, continuity x pressure tau grad psi_k . grad psi_l
+  if (ps)
+    for (int t = tid; t < NP * NVE; t += 256) {
+      const int k = t / NVE, n = t - k * NVE;
+      double acc[DIM] = {0.0, 0.0, 0.0}, accT = 0.0;
 #pragma unroll 1
       for (int q = 0; q < NQ; q++) {
-        double vgT = 0.0;
+        const double w = s_wpsi[q][k];
 #pragma unroll
-        for (int p = 0; p < DIM; p++) vgT += s_v[q][p] * s_gT[q][p];
-        c += s_dA[q] * vgT * s_v[q][b] * s_G[b][q][i];
-      }
-      const double v = -rCp * s_su[1 + b] * c;
-      const int ij = i * NVE + (NVE - 1);
-      if (A.kel) A.kel[(size_t)e * A.E + (size_t)(DIM * NV + b) * NVE2 + ij] += v;
-      if (s_dir[DIM][i]) continue;  // a Dirichlet row keeps its unit diagonal only
-      const int row = s_gun[DIM][i], col = s_gun[b][NVE - 1];
-      const long long pos = s_brow[DIM][i] + (int)rk[NVE2 + ij] + b - (col > row ? 1 : 0);
-      out[pos] += (JT)v;
-    }
-  }
-
-  // QCONV: -h w |surface Jacobian| phi_i phi_j over the element's sides in the
-  // T-T block, on top of the entries scattered above
-  if (EN && nqs > 0) {
-    bool conv = false;
-    for (int k = 0; k < nqs; k++) conv |= A.qs_q[3 * (qs0 + k) + 1] != 0.0;
-    if (conv) {
-      __syncthreads();
-      for (int t = tid; t < NVE2; t += NT) {
-        const int i = t / NVE, j = t - i * NVE;
-        double v = 0.0;
-#pragma unroll 1
-        for (int k = 0; k < nqs; k++) {
-          if (A.qs_q[3 * (qs0 + k) + 1] == 0.0) continue;
-#pragma unroll 1
-          for (int g = 0; g < NSP; g++) {
-            const double *st = A.stab + (size_t)(s_qsd[k] * NSP + g) * SREC;
-            v -= s_qh[k][g] * st[i] * st[j];
-          }
-        }
-        if (v == 0.0) continue;  // a node pair off the sides
-        if (A.kel) A.kel[(size_t)e * A.E + (size_t)(DIM * NV + DIM) * NVE2 + t] += v;
-        if (s_dir[DIM][i]) continue;  // a Dirichlet row keeps its unit diagonal only
-        const int row = s_gun[DIM][i], col = s_gun[DIM][j];
-        const long long pos =
-            row == col ? row : s_brow[DIM][i] + (int)rk[NVE2 + t] + DIM - (col > row ? 1 : 0);
-        out[pos] += (JT)v;
-      }
-    }
-  }
-
-  // 5c. momentum x pressure (J_m_P): int grad_a phi_i psi_k dA
-  for (int t = tid; t < NVE * NP; t += NT) {
-    const int i = t / NP, k = t - i * NP;
-    double acc[DIM] = {0.0, 0.0, 0.0};
-#pragma unroll 1
-    for (int q = 0; q < NQ; q++) {
-      const double w = s_dA[q] * tb[T::PSI + q * NP + k];
-#pragma unroll
-      for (int a = 0; a < DIM; a++) acc[a] += w * s_G[a][q][i];
-    }
-    const unsigned rm = rk[i * NVE + CL];
-    const bool first = ow && (rm & 0x8000u);
-    const int col = s_gp[k];
-#pragma unroll
-    for (int a = 0; a < DIM; a++) {
-      if (A.kel) A.kel[(size_t)e * A.E + A.off_mp + a * NVE * NP + t] = acc[a];
-      double v = acc[a];
-      if (s_dir[a][i]) {
-        if (!first) continue;
-        v = 0.0;
-      }
-      const int row = s_gun[a][i];
-      const long long pos = s_brow[a][i] + (int)(rm & 0x7fffu) + NV + k - (col > row ? 1 : 0);
-      if (first) out[pos] = (JT)v;
-      else out[pos] += (JT)v;
-    }
-  }
-
-  // 5d. continuity x velocity (J_c_v): int psi_k grad_b phi_j dA; PSPG adds
-  // tau rho [phi_j grad psi_k . d_b v + grad_b psi_k (v.grad phi_j + c phi_j)]
-  // and continuity x temperature tau rho beta (grad psi_k . g) phi_j
-  const bool ps = A.tau_pspg != 0.0;
-  for (int t = tid; t < NP * NVE; t += NT) {
-    const int k = t / NVE, j = t - k * NVE;
-    const bool dir = s_dirp[k] != 0;
-    double acc[DIM] = {0.0, 0.0, 0.0}, accT = 0.0;
-#pragma unroll 1
-    for (int q = 0; q < NQ; q++) {
-      const double w = s_dA[q] * tb[T::PSI + q * NP + k];
-#pragma unroll
-      for (int b = 0; b < DIM; b++) acc[b] += w * s_G[b][q][j];
-    }
-    if (ps && k > 0) {
-#pragma unroll 1
-      for (int q = 0; q < NQ; q++) {
-        const double wp = A.tau_pspg * s_dA[q] * rho, phj = s_Phi[q][j];
+        for (int b = 0; b < DIM; b++) acc[b] += w * s_G[b][q][n];
+        if (k == 0) continue;
+        const double wp = A.tau_pspg * s_dA[q] * rho, phj = s_Phi[q][n];
         double vg = 0.0, gk[DIM], gkg = 0.0;
 #pragma unroll
         for (int p = 0; p < DIM; p++) {
-          vg += s_v[q][p] * s_G[p][q][j];
+          vg += s_v[q][p] * s_G[p][q][n];
           gk[p] = s_B[q][p][k - 1];
           gkg += gk[p] * A.g[p];
         }
@@ -1261,37 +1163,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VISC ? 3 : 
         }
         accT += wp * A.beta * gkg * phj;
       }
-    }
-    const unsigned rm = rk[CL * NVE + j];
-    const bool first = ow && (rm & 0x8000u);
-    const int row = s_gp[k];
 #pragma unroll
-    for (int b = 0; b < DIM; b++) {
-      if (A.kel) A.kel[(size_t)e * A.E + A.off_cv + b * NP * NVE + t] = acc[b];
-      double v = acc[b];
-      if (dir) {
-        if (!first) continue;
-        v = 0.0;
-      }
-      const int col = s_gun[b][j];
-      const long long pos = s_bp[k] + (int)(rm & 0x7fffu) + b - (col > row ? 1 : 0);
-      if (first) out[pos] = (JT)v;
-      else out[pos] += (JT)v;
+      for (int b = 0; b < DIM; b++) K[A.off_cv + b * NP * NVE + t] = acc[b];
+      if constexpr (EN) A.ct[(size_t)e * NP * NVE + t] = accT;
     }
-    // continuity x temperature: in the graph (the continuity rows couple to
-    // every unknown of the element's nodes); zero in the Galerkin weak form,
-    // PSPG's Boussinesq term otherwise
-    if (EN && (first || (ps && !dir))) {
-      const int col = s_gun[DIM][j];
-      const long long pos = s_bp[k] + (int)(rm & 0x7fffu) + DIM - (col > row ? 1 : 0);
-      const double v = dir ? 0.0 : accT;
-      if (first) out[pos] = (JT)v;
-      else out[pos] += (JT)v;
-    }
-  }
-
-  // 5e. continuity x pressure: zero for Galerkin Q2-P1; PSPG adds
-  // tau grad psi_k . grad psi_l; a unit diagonal on a Dirichlet (datum) row
   if (tid < NP * NP) {
     const int k = tid / NP, k2 = tid - k * NP;
     double acc = 0.0;
@@ -1303,91 +1178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VISC ? 3 : 
         for (int a = 0; a < DIM; a++) g2 += s_B[q][a][k - 1] * s_B[q][a][k2 - 1];
         acc += A.tau_pspg * s_dA[q] * g2;
       }
-    if (A.kel) A.kel[(size_t)e * A.E + A.off_cp + tid] = acc;
-    const unsigned rm = rk[CL * NVE + CL];
-    const bool first = ow && (rm & 0x8000u);
-    const double v = s_dirp[k] ? (k == k2 ? 1.0 : 0.0) : acc;
-    const long long pos = k == k2 ? (long long)s_gp[k] : s_bp[k] + (int)(rm & 0x7fffu) + NV + k2 - (k2 > k ? 1 : 0);
-    if (first) out[pos] = (JT)v;
-    else if (v != 0.0) out[pos] += (JT)v;
-  }
-}
-
-// Rank map of every element: for node pair (i, j) (local order, i row node),
-//   rank[e][0][i*nve + j] = number of columns below fu[n_j] in the full column
-//     set (off-diagonals and the diagonal) of the momentum rows of node n_i,
-//     with bit 15 set when e is the first element, in colour order, holding
-//     both nodes (filled in by k_first_touch);
-//   rank[e][1][i*nve + j] = the same for the energy row (no pressure columns).
-// Every momentum row of a node has the same full column set, so the off-
-// diagonal position of column fu[n_j] + b in row fu[n_i] + a is
-// bindx[row] + rank + b - (col > row).  Continuity rows live on the centroid
-// node, whose neighbours are the element's own nodes, so they share the
-// column set of the centroid's momentum rows.
-template <int DIM>
-__global__ __launch_bounds__(256) void k_build_ranks(const int *__restrict__ conn,
-                                                     const int *__restrict__ fu,
-                                                     const int *__restrict__ bindx, int en,
-                                                     unsigned short *__restrict__ rank, int *flag) {
-  constexpr int NVE = El<DIM>::NVE, NVE2 = NVE * NVE;
-  const int e = blockIdx.x;
-  __shared__ int s_f[NVE];
-  if (threadIdx.x < NVE) s_f[threadIdx.x] = fu[conn[(size_t)e * NVE + threadIdx.x]];
-  __syncthreads();
-  for (int t = threadIdx.x; t < NVE2; t += blockDim.x) {
-    const int i = t / NVE, j = t - i * NVE;
-    const int col = s_f[j];
-    for (int w = 0; w < 1 + en; w++) {
-      const int row = s_f[i] + (w ? DIM : 0);
-      // lower bound of col in the sorted off-diagonal list of row
-      int lo = bindx[row], hi = bindx[row + 1];
-      const int start = lo;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (bindx[mid] < col) lo = mid + 1;
-        else hi = mid;
-      }
-      const int r = lo - start + (row < col ? 1 : 0);
-      if (r > 0x7fff) atomicOr(&flag[1], 1);
-      rank[(size_t)e * 2 * NVE2 + w * NVE2 + t] = (unsigned short)r;
-    }
-    if (!en) rank[(size_t)e * 2 * NVE2 + NVE2 + t] = 0;
-  }
-}
-
-// First touch, one element colour per launch (colours in order): the element
-// of this colour holding both nodes of a pair marks it when no earlier colour
-// has; `touched` is indexed by the MSR position of the pair's (U1, U1) entry.
-template <int DIM>
-__global__ __launch_bounds__(256) void k_first_touch(const int *__restrict__ elems,
-                                                     const int *__restrict__ conn,
-                                                     const int *__restrict__ fu,
-                                                     const int *__restrict__ bindx,
-                                                     unsigned short *__restrict__ rank,
-                                                     unsigned char *__restrict__ touched,
-                                                     int *flag) {
-  constexpr int NVE = El<DIM>::NVE, NVE2 = NVE * NVE;
-  const int e = elems[blockIdx.x];
-  __shared__ int s_f[NVE];
-  if (threadIdx.x < NVE) s_f[threadIdx.x] = fu[conn[(size_t)e * NVE + threadIdx.x]];
-  __syncthreads();
-  for (int t = threadIdx.x; t < NVE2; t += blockDim.x) {
-    const int i = t / NVE, j = t - i * NVE;
-    const int row = s_f[i], col = s_f[j];
-    unsigned short *rp = rank + (size_t)e * 2 * NVE2 + t;
-    const int r = *rp & 0x7fff;
-    long long pos = row;
-    if (row != col) {
-      pos = (long long)bindx[row] + r - (col > row ? 1 : 0);
-      if (pos < bindx[row] || pos >= bindx[row + 1] || bindx[pos] != col) {
-        atomicOr(&flag[1], 1);
-        continue;
-      }
-    }
-    if (!touched[pos]) {
-      touched[pos] = 1;
-      *rp = (unsigned short)(r | 0x8000);
-    }
+    K[A.off_cp + tid] = acc;
   }
 }
 
@@ -1608,81 +1399,32 @@ int gm_fill_setup_device(gm_ctx *c) {
     gm_set_error("element-to-nonzero map: entry missing from the MSR graph");
     return GM_ERR_ARG;
   }
-  if (c->dim == 2) return gm_gather_setup(c);
-  if (c->dim == 3) {
-    // rank map and first touches (the HEX27 assembly kernel's scatter)
-    const size_t nr = ne * 2 * (size_t)L.nve * L.nve;
-    GM_HIP(hipMalloc(&c->d_rank, nr * sizeof(unsigned short)));
-    k_build_ranks<3><<<c->num_elems, 256, 0, c->stream>>>(c->d_conn, c->d_fu, c->d_bindx, c->energy,
-                                                         c->d_rank, c->d_flag);
-    GM_HIP(hipGetLastError());
-    unsigned char *touched = nullptr;
-    GM_HIP(hipMalloc(&touched, (size_t)c->nval));
-    GM_HIP(hipMemsetAsync(touched, 0, (size_t)c->nval, c->stream));
-    for (int col = 0; col < c->n_ecol; col++) {
-      const int cnt = c->ecol_ptr[col + 1] - c->ecol_ptr[col];
-      if (cnt)
-        k_first_touch<3><<<cnt, 256, 0, c->stream>>>(c->d_ecol_elems + c->ecol_ptr[col], c->d_conn,
-                                                    c->d_fu, c->d_bindx, c->d_rank, touched,
-                                                    c->d_flag);
-    }
-    const hipError_t le = hipGetLastError();
-    GM_HIP(hipMemcpyAsync(flag, c->d_flag, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    GM_HIP(hipStreamSynchronize(c->stream));
-    (void)hipFree(touched);
-    GM_HIP(le);
-    if (flag[1]) {
-      gm_set_error("rank map: a node pair's position does not match the MSR graph");
-      return GM_ERR_ARG;
-    }
-  }
-  return GM_OK;
+  return gm_gather_setup(c);
 }
 
-template <int EN, int VISC, typename JT>
-static void launch_fill3(gm_ctx *c, FillArgs &a) {
-  for (int col = 0; col < c->n_ecol; col++) {
-    const int cnt = c->ecol_ptr[col + 1] - c->ecol_ptr[col];
-    if (cnt == 0) continue;
-    // this colour's share of B_asm = nnz*s + 16 N + 8 dim n_nodes + 4 nve n_el
-    const double share = (double)cnt / c->num_elems;
-    const double basm = (double)(c->nval - 1) * sizeof(JT) + 16.0 * c->N +
-                        24.0 * c->num_nodes + 4.0 * El<3>::NVE * c->num_elems;
-    const int id = a.resid_only ? GM_K_FILL_RESID : GM_K_FILL;
-    gm_launch(c, id, share * (a.resid_only ? basm - (double)(c->nval - 1) * sizeof(JT) : basm),
-              k_fill3m<EN, VISC, JT>, dim3(cnt), dim3(256), 0, c->stream, a,
-              c->d_ecol_elems + c->ecol_ptr[col]);
-  }
-}
-
-template <typename JT>
-static void dispatch_fill3(gm_ctx *c, FillArgs &a) {
-  const int en = c->energy, vm = c->phys.visc_model;
-  if (en && vm) launch_fill3<1, 1, JT>(c, a);
-  else if (en) launch_fill3<1, 0, JT>(c, a);
-  else if (vm) launch_fill3<0, 1, JT>(c, a);
-  else launch_fill3<0, 0, JT>(c, a);
-}
-
-static int fill2_buffers(gm_ctx *c) {
+static int elem_buffers(gm_ctx *c) {
   if (!c->d_re) GM_HIP(hipMalloc(&c->d_re, (size_t)c->num_elems * (c->nv * c->nve + c->np) * sizeof(double)));
   if (!c->d_ct) GM_HIP(hipMalloc(&c->d_ct, (size_t)c->num_elems * c->np * c->nve * sizeof(double)));
   return GM_OK;
 }
 
-// QUAD9: the element matrices and residuals of every element, then the rows.
-static int fill2(gm_ctx *c, FillArgs &a, double *val, float *val32) {
+// The element matrices and residuals of every element, then the rows.
+static int assemble(gm_ctx *c, const FillArgs &a, double *resid, double *val, float *val32) {
   const int en = c->energy, vm = c->phys.visc_model;
-  auto kern = en ? (vm ? k_elem2<1, 1> : k_elem2<1, 0>) : (vm ? k_elem2<0, 1> : k_elem2<0, 0>);
   const int id = a.resid_only ? GM_K_FILL_RESID : GM_K_FILL;
   // coordinates, connectivity, the state; the element matrices and residuals written
-  const double bytes = 16.0 * c->num_nodes + 8.0 * c->N + 36.0 * c->num_elems +
-                       8.0 * c->num_elems * (c->nv * 9 + 3 + (a.resid_only ? 0.0 : (double)c->lay.total));
-  gm_launch(c, id, bytes, kern, dim3((c->num_elems + 3) / 4), dim3(256), 0, c->stream, a, c->num_elems);
+  const double bytes = 8.0 * c->dim * c->num_nodes + 8.0 * c->N + 4.0 * c->nve * c->num_elems +
+                       8.0 * c->num_elems * (c->nv * c->nve + c->np + (a.resid_only ? 0.0 : (double)c->lay.total));
+  if (c->dim == 2)
+    gm_launch(c, id, bytes, en ? (vm ? k_elem2<1, 1> : k_elem2<1, 0>) : (vm ? k_elem2<0, 1> : k_elem2<0, 0>),
+              dim3((c->num_elems + 3) / 4), dim3(256), 0, c->stream, a, c->num_elems);
+  else
+    gm_launch(c, id, bytes, en ? (vm ? k_elem3<1, 1> : k_elem3<1, 0>) : (vm ? k_elem3<0, 1> : k_elem3<0, 0>),
+              dim3(c->num_elems), dim3(256), 0, c->stream, a);
   GM_HIP(hipGetLastError());
   const bool mat = !a.resid_only;
-  return gm_gather(c, id, c, c->stream, a.kel, en && a.tau_pspg != 0.0 ? a.ct : nullptr, mat ? val : nullptr,
-                   mat ? val32 : nullptr, c->fill_overwrite, a.re, a.x, a.resid);
+  return gm_gather(c, id, c, c->stream, a.kel, en && a.tau_pspg != 0.0 ? a.ct : nullptr, mat && !val32 ? val : nullptr,
+                   mat ? val32 : nullptr, c->fill_overwrite, a.re, a.x, resid);
 }
 
 int gm_fill_launch(gm_ctx *c, const double *x, double *resid, double *val, float *val32) {
@@ -1697,14 +1439,8 @@ int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, fl
   a.conn = c->d_conn;
   a.fu = c->d_fu;
   a.centroid = c->d_centroid;
-  a.dbc = c->d_dbc;
-  a.dbc_val = c->d_dbc_val;
   a.tables = c->d_tables;
-  a.e2nz = c->d_e2nz;
   a.x = x;
-  a.resid = resid;
-  a.val = val32 ? (void *)val32 : (void *)val;
-  a.kel = c->kel_on ? c->d_kel : nullptr;
   a.x_old = c->tr_x_old;
   a.xdot_old = c->tr_xdot_old;
   a.cmass = c->tr_cmass;
@@ -1713,9 +1449,6 @@ int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, fl
   a.qs_side = c->d_qs_side;
   a.qs_q = c->d_qs_q;
   a.stab = c->d_stab;
-  a.bindx = c->d_bindx;
-  a.rank = c->d_rank;
-  a.overwrite = c->fill_overwrite && c->d_rank ? 1 : 0;
   a.num_nodes = c->num_nodes;
   a.tau_pspg = c->phys.pspg ? gm_pspg_tau(c) : 0.0;
   a.supg_e = c->energy ? c->phys.energy_supg : 0.0;
@@ -1738,17 +1471,12 @@ int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, fl
   a.Tref = p.Tref;
   *c->h_flag = 0;  // nothing that could set it is in flight: every call waits for its kernels
   a.flag = c->h_flag;
-  if (c->dim == 2) {
-    int rc = resid_only ? GM_OK : gm_mg_kel_alloc(c);
-    if (rc || (rc = fill2_buffers(c))) return rc;
-    a.kel = c->d_kel;
-    a.re = c->d_re;
-    a.ct = c->d_ct;
-    if ((rc = fill2(c, a, val, val32))) return rc;
-  } else {
-    if (val32) dispatch_fill3<float>(c, a);
-    else dispatch_fill3<double>(c, a);
-  }
+  int rc = resid_only ? GM_OK : gm_mg_kel_alloc(c);
+  if (rc || (rc = elem_buffers(c))) return rc;
+  a.kel = c->d_kel;
+  a.re = c->d_re;
+  a.ct = c->d_ct;
+  if ((rc = assemble(c, a, resid, val, val32))) return rc;
   GM_HIP(hipGetLastError());
   GM_HIP(hipStreamSynchronize(c->stream));
   if (*(volatile int *)c->h_flag) {

@@ -1,15 +1,15 @@
-// Element matrices -> MSR matrix, one thread per pair of coupled nodes.
+// Element matrices -> MSR matrix, a thread per pair of coupled nodes and row.
 //
 // The node graph's pairs (row node n, column node m, in the graph's order) are
 // the blocks of the matrix: pair p holds the MSR offset of m's first column in
 // the rows of n and the list of elements that contain both nodes, each with
-// the pair's local position.  A thread sums its pair's block over that list,
-// in element order, and writes it once: no colours, no zeroing, no
+// the pair's local position.  A thread sums its row of the pair's block over that
+// list, in element order, and writes it once: no colours, no zeroing, no
 // read-modify-write, and the same bits every time.  Neighbouring threads write
 // neighbouring columns of the same rows.
 //
-// It is the second half of the QUAD9 assembly (gm_fill.hip) and the scatter
-// of the Galerkin coarse levels (gm_mg.hip).
+// It is the second half of the assembly (gm_fill.hip) and the scatter of the
+// Galerkin coarse levels (gm_mg.hip).
 #include <algorithm>
 #include <vector>
 
@@ -43,10 +43,50 @@ struct GatherArgs {
 constexpr int HAS_P_COL = 1 << 30;  // m carries pressure unknowns
 constexpr int HAS_P_ROW = 1 << 29;  // n does
 
-template <typename JT>
-__device__ inline void put(JT *val, long long pos, double v, bool assign) {
-  if (assign) val[pos] = (JT)v;
-  else val[pos] += (JT)v;
+// n values at val[pos ..], stored or added.  Stores go out 16 bytes at a time
+// (aligned to the value only).
+template <int n, typename JT>
+__device__ inline void put(JT *val, long long pos, const double *v, bool assign) {
+  constexpr int W = 16 / sizeof(JT), M = n / W * W;
+  if (!assign) {
+#pragma unroll
+    for (int k = 0; k < n; k++) val[pos + k] += (JT)v[k];
+    return;
+  }
+  typedef JT Wide __attribute__((ext_vector_type(W), aligned(sizeof(JT))));
+#pragma unroll
+  for (int k = 0; k < M; k += W) {
+    Wide w;
+#pragma unroll
+    for (int l = 0; l < W; l++) w[l] = (JT)v[k + l];
+    *(Wide *)(val + pos + k) = w;
+  }
+#pragma unroll
+  for (int k = M; k < n; k++) val[pos + k] = (JT)v[k];
+}
+
+// columns fm .. fm + n - 1 of a row, whose place among the off-diagonals is
+// base; the diagonal stands apart and those after it one place earlier
+template <int n, typename JT>
+__device__ inline void put_row(JT *val, int row, long long base, int fm, const double *v, bool dir, double unit,
+                               bool assign) {
+  double w[n];
+#pragma unroll
+  for (int k = 0; k < n; k++) w[k] = dir ? 0.0 : v[k];
+  if (row < fm || row >= fm + n) {
+    if (assign || !dir) put<n>(val, base - (fm > row ? 1 : 0), w, assign);
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < n; k++) {
+    const int col = fm + k;
+    if (row == col) {
+      const double d = dir ? unit : w[k];
+      put<1>(val, row, &d, assign);
+    } else if (assign || !dir) {
+      put<1>(val, base + k - (col > row ? 1 : 0), &w[k], assign);
+    }
+  }
 }
 
 // A Dirichlet row keeps the unit diagonal of each element at its node
@@ -54,14 +94,18 @@ __device__ inline void put(JT *val, long long pos, double v, bool assign) {
 // is that many times x - V.
 //
 // Bound by memory: every element-matrix entry read once (8 bytes) and every
-// nonzero written once.  A thread takes its pair through all the rows of n,
-// so the pair's description is read once and its loads are independent.
+// nonzero written once.  Wave a of a workgroup takes row a of the block's 64
+// pairs (and the continuity rows a, a + NV, ..): with a thread for all the
+// rows of its pair there are a quarter of the waves, and those of the corner
+// nodes, eight dependent sources long, are waited for (11^3 elements with
+// energy, FP32: 70 us against 86; 16 x 16 QUAD9: 5.9 against 8.0; 16^3 FP64,
+// where the traffic counts, 300 against 297).
 template <int DIM, int EN, typename JT>
-__global__ __launch_bounds__(256) void k_gather(GatherArgs A, JT *__restrict__ val) {
-  constexpr int NVE = DIM == 2 ? 9 : 27, NP = DIM + 1, NV = DIM + EN, NVE2 = NVE * NVE;
+__global__ __launch_bounds__(64 * (DIM + EN)) void k_gather(GatherArgs A, JT *__restrict__ val) {
+  constexpr int NVE = DIM == 2 ? 9 : 27, NP = DIM + 1, NV = DIM + EN, NVE2 = NVE * NVE, NT = 64 * NV;
   constexpr int CL = DIM == 2 ? 8 : 20;
   if ((int)blockIdx.x >= A.nb_pairs) {
-    const int u = ((int)blockIdx.x - A.nb_pairs) * 256 + threadIdx.x;
+    const int u = ((int)blockIdx.x - A.nb_pairs) * NT + threadIdx.x;
     if (u >= A.N) return;
     const int k0 = A.gptr[u], k1 = A.gptr[u + 1];
     double s = 0.0;
@@ -71,93 +115,88 @@ __global__ __launch_bounds__(256) void k_gather(GatherArgs A, JT *__restrict__ v
     A.resid[u] += s;
     return;
   }
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p == 0 && A.assign) val[A.N] = (JT)0;  // the unused entry between diagonal and rows
+  const int a = threadIdx.x >> 6, p = blockIdx.x * 64 + (threadIdx.x & 63);
+  if (p == 0 && a == 0 && A.assign) val[A.N] = (JT)0;  // the unused entry between diagonal and rows
   if (p >= A.npairs) return;
   const int4 P = A.pair[p];
   const int s0 = P.w, s1 = A.pair[p + 1].w, fn = P.x, fm = P.y, ra = P.z & (HAS_P_ROW - 1);
-  const int rt = EN ? A.rank_t[p] : 0;
   const bool pc = P.z & HAS_P_COL, pr = P.z & HAS_P_ROW, as = A.assign != 0;
-  double acc[NV][NV], accp[DIM][NP];
-#pragma unroll
-  for (int a = 0; a < NV; a++)
-#pragma unroll
-    for (int b = 0; b < NV; b++) acc[a][b] = 0.0;
-#pragma unroll
-  for (int a = 0; a < DIM; a++)
-#pragma unroll
-    for (int k = 0; k < NP; k++) accp[a][k] = 0.0;
-  for (int s = s0; s < s1; s++) {
-    const int sv = A.src[s], e = sv / NVE2, t = sv - e * NVE2;
-    const double *__restrict__ K = A.kel + (size_t)e * A.E;
-#pragma unroll
-    for (int a = 0; a < NV; a++)
-#pragma unroll
-      for (int b = 0; b < NV; b++) acc[a][b] += K[(a * NV + b) * NVE2 + t];
-    if (pc && t % NVE == CL) {
-      const double *__restrict__ Q = K + A.off_mp + (t / NVE) * NP;
-#pragma unroll
-      for (int a = 0; a < DIM; a++)
-#pragma unroll
-        for (int k = 0; k < NP; k++) accp[a][k] += Q[a * NVE * NP + k];
-    }
-  }
-#pragma unroll
-  for (int a = 0; a < NV; a++) {
+  {
     const int row = fn + a;
     const bool dir = A.dbc[row] != 0;
-    const long long base = (long long)A.bindx[row] + (a < DIM ? ra : rt) - (fm > row ? 1 : 0);
+    const long long base = (long long)A.bindx[row] + (a < DIM ? ra : A.rank_t[p]);
+    double acc[NV + NP];
 #pragma unroll
-    for (int b = 0; b < NV; b++) {
-      const int col = fm + b;
-      const bool diag = row == col;
-      if (dir && !diag && !as) continue;
-      const double v = dir ? (diag ? (double)(s1 - s0) : 0.0) : acc[a][b];
-      // the columns of m after the row's own unknown stand one place earlier
-      const long long pos = diag ? row : base + b - (fm <= row && col > row ? 1 : 0);
-      put(val, pos, v, as);
-    }
-    if (pc && a < DIM) {
+    for (int b = 0; b < NV + NP; b++) acc[b] = 0.0;
+    if (!dir)
+#pragma unroll 2
+      for (int s = s0; s < s1; s++) {
+        const int sv = A.src[s], e = sv / NVE2, t = sv - e * NVE2;
+        const double *__restrict__ K = A.kel + (size_t)e * A.E;
 #pragma unroll
-      for (int k = 0; k < NP; k++) {
-        if (dir && !as) continue;
-        put(val, base + NV + k - (fm <= row && fm + NV + k > row ? 1 : 0), dir ? 0.0 : accp[a < DIM ? a : 0][k], as);
+        for (int b = 0; b < NV; b++) acc[b] += K[(a * NV + b) * NVE2 + t];
+        if (pc && a < DIM && t % NVE == CL) {
+          const double *__restrict__ Q = K + A.off_mp + (a * NVE + t / NVE) * NP;
+#pragma unroll
+          for (int k = 0; k < NP; k++) acc[NV + k] += Q[k];
+        }
       }
-    }
+    if (pc && a < DIM) put_row<NV + NP>(val, row, base, fm, acc, dir, (double)(s1 - s0), as);
+    else put_row<NV>(val, row, base, fm, acc, dir, (double)(s1 - s0), as);
   }
   if (!pr) return;
   // continuity rows: velocities, temperature (PSPG only), pressures
 #pragma unroll 1
-  for (int k = 0; k < NP; k++) {
+  for (int k = a; k < NP; k += NV) {
     const int row = fn + NV + k;
     const bool dir = A.dbc[row] != 0;
-    double c[NV], q[NP], nd = 0.0;
+    double acc[NV + NP], nd = 0.0;
 #pragma unroll
-    for (int b = 0; b < NV; b++) c[b] = 0.0;
-#pragma unroll
-    for (int b = 0; b < NP; b++) q[b] = 0.0;
+    for (int b = 0; b < NV + NP; b++) acc[b] = 0.0;
     for (int s = s0; s < s1; s++) {
       const int sv = A.src[s], e = sv / NVE2, t = sv - e * NVE2, i = t / NVE, j = t - i * NVE;
       if (i != CL) continue;
       nd += 1.0;
       const double *__restrict__ K = A.kel + (size_t)e * A.E;
 #pragma unroll
-      for (int b = 0; b < DIM; b++) c[b] += K[A.off_cv + (b * NP + k) * NVE + j];
-      if (EN && A.ct) c[NV - 1] += A.ct[(size_t)e * NP * NVE + k * NVE + j];
+      for (int b = 0; b < DIM; b++) acc[b] += K[A.off_cv + (b * NP + k) * NVE + j];
+      if (EN && A.ct) acc[NV - 1] += A.ct[(size_t)e * NP * NVE + k * NVE + j];
       if (j == CL)
 #pragma unroll
-        for (int b = 0; b < NP; b++) q[b] += K[A.off_cp + k * NP + b];
+        for (int b = 0; b < NP; b++) acc[NV + b] += K[A.off_cp + k * NP + b];
     }
-    const long long base = (long long)A.bindx[row] + ra - (fm > row ? 1 : 0);
-#pragma unroll
-    for (int b = 0; b < NV + NP; b++) {
-      if (b >= NV && !pc) continue;
-      const int col = fm + b;
-      const bool diag = row == col;
-      if (dir && !diag && !as) continue;
-      const double v = dir ? (diag ? nd : 0.0) : (b < NV ? c[b < NV ? b : 0] : q[b >= NV ? b - NV : 0]);
-      const long long pos = diag ? row : base + b - (fm <= row && col > row ? 1 : 0);
-      put(val, pos, v, as);
+    const long long base = (long long)A.bindx[row] + ra;
+    if (pc) put_row<NV + NP>(val, row, base, fm, acc, dir, nd, as);
+    else put_row<NV>(val, row, base, fm, acc, dir, nd, as);
+  }
+}
+
+// The pairs' descriptions, one thread per row node: pair p's sources are the
+// (k, l) places of its two nodes in a common element, element by element; the
+// pairs of node n hold nve of them for each of its places.
+__global__ __launch_bounds__(256) void k_pairs(int nn, int nve, int nv, const int *__restrict__ fu,
+                                               const int *__restrict__ nn_ptr, const int *__restrict__ nn_list,
+                                               const int *__restrict__ eptr, const int *__restrict__ elist,
+                                               int4 *__restrict__ pair, int *__restrict__ rank_t,
+                                               int *__restrict__ src) {
+  const int n = blockIdx.x * 256 + threadIdx.x;
+  if (n > nn) return;
+  if (n == nn) {
+    pair[nn_ptr[nn]] = make_int4(0, 0, 0, eptr[nn] * nve);
+    return;
+  }
+  const int k0 = eptr[n], k1 = eptr[n + 1], fn = fu[n], pr = fu[n + 1] - fn > nv ? HAS_P_ROW : 0;
+  int ra = 0, rt = 0, at = k0 * nve;
+  for (int p = nn_ptr[n]; p < nn_ptr[n + 1]; p++) {
+    const int m = nn_list[p], l = fu[m + 1] - fu[m];
+    pair[p] = make_int4(fn, fu[m], ra | (l > nv ? HAS_P_COL : 0) | pr, at);
+    rank_t[p] = rt;
+    ra += l;
+    rt += min(l, nv);
+    for (int k = k0; k < k1; k++) {
+      const int e = elist[k] / nve, i = elist[k] - e * nve;
+      for (int q = eptr[m]; q < eptr[m + 1]; q++)
+        if (elist[q] / nve == e) src[at++] = e * nve * nve + i * nve + elist[q] - e * nve;
     }
   }
 }
@@ -169,61 +208,40 @@ __global__ __launch_bounds__(256) void k_gather(GatherArgs A, JT *__restrict__ v
 // the additive smoother).
 int gm_gather_setup(gm_ctx *c) {
   if (c->d_pair) return GM_OK;
-  const int nn = c->num_nodes, ne = c->num_elems, nve = c->nve, nve2 = nve * nve, nv = c->nv, np = c->np;
-  const size_t npairs = c->nn_list.size();
-  if ((long long)ne * nve2 >= (1LL << 31) || npairs >= (1ull << 31) - 512) {
+  const int nn = c->num_nodes, ne = c->num_elems, nve = c->nve;
+  const size_t npairs = c->nn_list.size(), places = (size_t)ne * nve;
+  // (the 32-bit row pointers of the matrix end far below this)
+  if (places * nve >= (1ull << 31) || npairs >= (1ull << 31) - 512) {
     gm_set_error("too many elements for the assembly's pair lists (%d)", ne);
     return GM_ERR_ARG;
   }
-  std::vector<int> eptr(nn + 1, 0), elist((size_t)ne * nve);
-  for (size_t k = 0; k < (size_t)ne * nve; k++) eptr[c->conn[k] + 1]++;
+  std::vector<int> eptr(nn + 1, 0), elist(places);
+  for (size_t k = 0; k < places; k++) eptr[c->conn[k] + 1]++;
   for (int n = 0; n < nn; n++) eptr[n + 1] += eptr[n];
   {
-    std::vector<int> fp(eptr.begin(), eptr.end() - 1);
-    for (int e = 0; e < ne; e++)
-      for (int i = 0; i < nve; i++) elist[fp[c->conn[(size_t)e * nve + i]]++] = e * nve + i;
+    std::vector<int> at(eptr.begin(), eptr.end() - 1);
+    for (size_t k = 0; k < places; k++) elist[at[c->conn[k]]++] = (int)k;
   }
-  std::vector<int4> pair(npairs + 1);
-  std::vector<int> rank_t(npairs), cnt(npairs, 0);
-  auto find = [&](int n, int m) {
-    return (size_t)(std::lower_bound(c->nn_list.begin() + c->nn_ptr[n], c->nn_list.begin() + c->nn_ptr[n + 1], m) -
-                    c->nn_list.begin());
+  int *d_eptr = nullptr, *d_elist = nullptr;
+  int4 *pair = nullptr;
+  auto build = [&]() -> int {
+    int rc;
+    if ((rc = up(&d_eptr, eptr)) || (rc = up(&d_elist, elist)) || (rc = gm_unknown_places(c))) return rc;
+    GM_HIP(hipMalloc(&pair, (npairs + 1) * sizeof(int4)));
+    if (!c->d_rank_t) GM_HIP(hipMalloc(&c->d_rank_t, std::max<size_t>(npairs, 1) * sizeof(int)));
+    if (!c->d_src) GM_HIP(hipMalloc(&c->d_src, places * nve * sizeof(int)));
+    k_pairs<<<nn / 256 + 1, 256, 0, c->stream>>>(nn, nve, c->nv, c->d_fu, c->d_nn_ptr, c->d_nn_list, d_eptr, d_elist,
+                                                 pair, c->d_rank_t, c->d_src);
+    GM_HIP(hipGetLastError());
+    GM_HIP(hipStreamSynchronize(c->stream));
+    return GM_OK;
   };
-  auto len = [&](int n) { return c->first_unknown[n + 1] - c->first_unknown[n]; };
-#pragma omp parallel for schedule(dynamic, 1024)
-  for (int n = 0; n < nn; n++) {
-    int ra = 0, rt = 0;
-    for (int p = c->nn_ptr[n]; p < c->nn_ptr[n + 1]; p++) {
-      const int m = c->nn_list[p], l = len(m);
-      pair[p] = make_int4(c->first_unknown[n], c->first_unknown[m],
-                          ra | (l > nv ? HAS_P_COL : 0) | (len(n) > nv ? HAS_P_ROW : 0), 0);
-      rank_t[p] = rt;
-      ra += l;
-      rt += std::min(l, nv);
-    }
-    for (int k = eptr[n]; k < eptr[n + 1]; k++)
-      for (int j = 0; j < nve; j++) cnt[find(n, c->conn[(size_t)(elist[k] / nve) * nve + j])]++;
-  }
-  int total = 0;
-  for (size_t p = 0; p < npairs; p++) {
-    pair[p].w = total;
-    total += cnt[p];
-  }
-  pair[npairs] = make_int4(0, 0, 0, total);
-  std::vector<int> src(total);
-#pragma omp parallel for schedule(dynamic, 1024)
-  for (int n = 0; n < nn; n++) {
-    for (int p = c->nn_ptr[n]; p < c->nn_ptr[n + 1]; p++) cnt[p] = pair[p].w;
-    for (int k = eptr[n]; k < eptr[n + 1]; k++) {
-      const int e = elist[k] / nve, i = elist[k] - e * nve;
-      for (int j = 0; j < nve; j++) src[cnt[find(n, c->conn[(size_t)e * nve + j])]++] = e * nve2 + i * nve + j;
-    }
-  }
-  int rc;
-  if ((rc = up(&c->d_src, src)) || (rc = up(&c->d_rank_t, rank_t)) || (rc = gm_unknown_places(c)) ||
-      (rc = up(&c->d_pair, pair)))
-    return rc;
-  return GM_OK;
+  const int rc = build();
+  (void)hipFree(d_eptr);
+  (void)hipFree(d_elist);
+  if (rc) (void)hipFree(pair);
+  else c->d_pair = pair;
+  return rc;
 }
 
 // Local dof li of element e (nodal variables node-blocked by variable, then
@@ -278,15 +296,16 @@ int gm_gather(gm_ctx *prof, int id, gm_ctx *c, hipStream_t s, const double *kel,
   A.resid = resid;
   const bool mat = val || val32;
   A.npairs = mat ? (int)c->nn_list.size() : 0;
-  A.nb_pairs = (A.npairs + 255) / 256;
-  const int blocks = A.nb_pairs + (re ? (c->N + 255) / 256 : 0);
+  const int nt = 64 * c->nv;
+  A.nb_pairs = (A.npairs + 63) / 64;
+  const int blocks = A.nb_pairs + (re ? (c->N + nt - 1) / nt : 0);
   if (!blocks) return GM_OK;
   const double nnz = (double)c->nval - 1.0, vs = val32 ? 4.0 : 8.0;
   const double bytes = (mat ? (double)c->num_elems * c->lay.total * 8.0 + nnz * vs * (assign ? 1.0 : 2.0) +
                                   20.0 * A.npairs + 4.0 * c->num_elems * c->nve * c->nve
                             : 0.0) +
                        (re ? (double)c->num_elems * (c->nv * c->nve + c->np) * 12.0 + 20.0 * c->N : 0.0);
-  auto go = [&](auto kern, auto *v) { gm_launch(prof, id, bytes, kern, dim3(blocks), dim3(256), 0, s, A, v); };
+  auto go = [&](auto kern, auto *v) { gm_launch(prof, id, bytes, kern, dim3(blocks), dim3(nt), 0, s, A, v); };
   if (val32) {
     if (c->dim == 2) go(c->energy ? k_gather<2, 1, float> : k_gather<2, 0, float>, val32);
     else go(c->energy ? k_gather<3, 1, float> : k_gather<3, 0, float>, val32);

@@ -182,12 +182,10 @@ struct gm_ctx {
   // node pairs of the graph with the elements that hold them (k_gather)
   int4 *d_pair = nullptr;       // [pairs + 1]
   int *d_rank_t = nullptr, *d_src = nullptr;
-  double *d_re = nullptr, *d_ct = nullptr;  // QUAD9 assembly: element residuals; PSPG c x T entries
+  double *d_re = nullptr, *d_ct = nullptr;  // element residuals; PSPG c x T entries
   double *d_tables = nullptr;   // reference basis tables
   double *d_stab = nullptr;     // side basis tables (surface integrals)
-  unsigned short *d_rank = nullptr;  // HEX27: per element and node pair, the rank of the
-                                     // column node in the row node's rows (+ first-touch bit)
-  int fill_overwrite = 0;       // the next assembly stores first touches instead of adding
+  int fill_overwrite = 0;       // the next assembly stores the Jacobian instead of adding
 
   // theta-method state of the next assemblies (tr_x_old == nullptr: steady):
   // xdot = tr_cmass (x - x_old) - tr_cold xdot_old
@@ -202,8 +200,7 @@ struct gm_ctx {
 
   // Newton work vectors
   double *d_val = nullptr, *d_resid = nullptr, *d_dx = nullptr, *d_scale = nullptr;
-  double *d_kel = nullptr;  // element matrices before Dirichlet rows [num_elems][lay.total]
-  int kel_on = 0;           // the next assembly also writes d_kel
+  double *d_kel = nullptr;  // the last assembly's element matrices before Dirichlet rows [num_elems][lay.total]
   float *d_val32 = nullptr;
   double *d_red = nullptr;      // reduction scratch
   double *h_red = nullptr;      // pinned host mirror

@@ -206,8 +206,7 @@ int gm_set_velocity_norm(gm_ctx *ctx, double U_norm);
 int gm_matrix_fill_full_dev(gm_ctx *ctx, const double *x_dev, double *resid_dev, double *val_dev);
 int gm_matrix_fill_full(gm_ctx *ctx, const double *x, double *resid, double *val);
 /* The same assembly, with the Jacobian stored rather than accumulated: val
- * needs no zeroing beforehand (the HEX27 kernel writes each entry's first
- * element contribution and adds the others; QUAD9 writes each sum once).  resid
+ * needs no zeroing beforehand (each entry's sum is written once).  resid
  * is still accumulated.  Saves the caller's pass over val (8 GB at 48^3). */
 int gm_matrix_fill_full_assign_dev(gm_ctx *ctx, const double *x_dev, double *resid_dev,
                                    double *val_dev);
@@ -375,7 +374,7 @@ int gm_mg_copy_coarse_inverse(const gm_ctx *ctx, double *out);
  * is the kernel's execution alone; gm_prof_get returns the launch count, the
  * summed duration and the summed algorithmic HBM bytes (compulsory traffic,
  * each array counted once per launch) of those launches. */
-#define GM_K_FILL 0       /* assembly: k_fill3m, one element colour (HEX27); k_elem2, k_gather (QUAD9) */
+#define GM_K_FILL 0       /* assembly: k_elem2 / k_elem3, the element matrices, and k_gather, the rows */
 #define GM_K_SPMV 1       /* k_spmv_msr: MSR matvec */
 #define GM_K_ILU_LOWER 2  /* k_ilu_sweep: forward sweep of one patch colour */
 #define GM_K_ILU_UPPER 3  /* k_ilu_sweep: backward sweep of one patch colour */

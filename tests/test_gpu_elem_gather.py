@@ -1,6 +1,6 @@
-"""QUAD9 assembly at the edges of its workgroups, and its order.
+"""Element assembly at the edges of its workgroups, and its order.
 
-Four elements share a workgroup and a thread sums a pair of nodes: one to five
+Four QUAD9 elements share a workgroup (one HEX27) and a thread sums a pair of nodes: one to five
 elements leave every remainder of a workgroup, a renumbered mesh every order of
 a pair's two nodes (columns before and after the row's own unknown).  Every
 form of the kernel (energy or not, constant or shear-thinning viscosity), with
@@ -57,9 +57,30 @@ def _make(kind, ne):
 @pytest.mark.parametrize("kind", ["flow", "energy", "carreau", "stabilised"])
 @pytest.mark.parametrize("ne", [1, 2, 3, 5])
 def test_assembly_at_workgroup_edges(kind, ne, oracle_mod):
+    _check(_make(kind, ne), kind, ne, oracle_mod)
+
+
+@pytest.mark.parametrize("kind", ["flow", "energy", "carreau", "stabilised", "carreau_flow"])
+@pytest.mark.parametrize("ne", [1, 3])
+def test_hex_assembly(kind, ne, oracle_mod):
+    n = 2 if ne > 1 else 1
+    if kind in ("flow", "carreau_flow"):
+        p = problems.lid_cavity(n=n, Re=100.0, dim=3, jitter=0.1)
+        if kind == "carreau_flow":
+            q = problems.natural_convection(n=1, Ra=1e4, dim=3, carreau=True).phys
+            p = replace(p, phys=replace(q, energy=p.phys.energy))
+    elif kind == "carreau":
+        p = problems.natural_convection(n=n, Ra=1e4, dim=3, carreau=True, jitter=0.1)
+    else:
+        p = problems.lid_cavity(n=n, Re=100.0, dim=3, energy=True, Ra=1e3, jitter=0.1)
+    if kind == "stabilised":
+        p = replace(p, phys=replace(p.phys, pspg=1, ps_scaling=0.5, energy_supg=1.0))
+    _check(_cut(p, ne), kind, ne, oracle_mod)
+
+
+def _check(prob, kind, ne, oracle_mod):
     from goma_amd import capi
 
-    prob = _make(kind, ne)
     ctx, orc = capi.Context(prob), oracle_mod.Oracle(prob)
     print(f"[case] element gather {kind} ne={ne} N={ctx.N}", flush=True)
     assert prob.mesh.connect.shape[0] == ne

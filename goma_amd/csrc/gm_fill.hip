@@ -53,8 +53,11 @@ struct FillArgs {
   const double *tables;     // phi, dphidxi, psi, wt
   const double *x;
   double *re, *ct;  // element residuals, PSPG continuity x temperature entries
-  double *kel;  // [num_elems][E]: element matrices before the Dirichlet rows (also for
-                // the Galerkin multigrid coarse operators), in the e2nz layout
+  // [num_elems][E]: element matrices before the Dirichlet rows (also for the
+  // Galerkin multigrid coarse operators): nodal blocks [a][i][j][b] (variable b
+  // innermost: a node pair's row a is one access of the kernels that read it),
+  // then momentum x P, continuity x velocity, P x P as in the e2nz map
+  double *kel;
   int *flag;
   // theta-method time step (nullptr x_old: steady): at each node
   // xdot = cmass (x - x_old) - cold xdot_old, cmass = (1 + 2 theta) / dt, cold = 2 theta
@@ -158,16 +161,25 @@ __device__ inline void supg_params(double s, const XA &x, const double *vc, doub
 // sum_q X[q][i] w[q] Y[q][j] of 9 x 9 operand tables (the same terms as the
 // HEX27 kernel below), one v_mfma_f64_16x16x4f64 tile each (nodes padded to
 // 16, the nine points to three k-steps of 4).  The wave writes its element's matrix
-// before Dirichlet rows (kel, in the e2nz layout), residual (re) and, with
+// before Dirichlet rows (kel), residual (re) and, with
 // PSPG and energy, the continuity x temperature entries (ct); k_gather sums
 // them into the MSR rows.  All elements are one launch.
 // Bound by the element matrices' traffic for large meshes and by the chain of
 // phases (about 10 us) for small ones.  Measured (assembly of 128 x 128
-// shear-thinning elements with energy, FP64): 215 us with k_gather
+// shear-thinning elements with energy, FP64): 209 us with k_gather
 // against 408 with four coloured launches of a workgroup per element, a
 // thread per node pair and += through the element-to-nonzero map; 16 x 16
-// cavity 61 us against 97.
+// cavity 59 us against 98.
 typedef double d4v __attribute__((ext_vector_type(4)));
+
+// entry r of n tiles to n neighbouring places, 16 bytes at a time
+template <int n>
+__device__ inline void put_cols(double *p, const d4v *D, int r) {
+  typedef double Two __attribute__((ext_vector_type(2), aligned(8)));
+#pragma unroll
+  for (int b = 0; b < n / 2 * 2; b += 2) *(Two *)(p + b) = Two{D[b][r], D[b + 1][r]};
+  if constexpr (n & 1) p[n - 1] = D[n - 1][r];
+}
 
 template <int EN>
 struct Quad9Lds {  // one element
@@ -457,12 +469,12 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
   const int j = lane & 15, kk = lane >> 4;
 #define GM_MFMA64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64((a), (b), (c), 0, 0, 0)
   const d4v z = {0.0, 0.0, 0.0, 0.0};
-  auto store = [&](int a, int b, const d4v &D) {
+  auto store = [&](int a, const d4v *D) {  // block row a
     if (j >= NVE) return;
 #pragma unroll
     for (int r = 0; r < 3; r++) {
       const int i = kk + 4 * r;
-      if (i < NVE) ke[(a * NV + b) * NVE2 + i * NVE + j] = D[r];
+      if (i < NVE) put_cols<NV>(ke + (a * NVE2 + i * NVE + j) * NV, D, r);
     }
   };
   // shared products: E(phi, dA, phi), and folded into the diagonal blocks
@@ -487,7 +499,7 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
   }
 #pragma unroll 1
   for (int a = 0; a < DIM; a++) {
-    d4v J[DIM];
+    d4v J[NV];
 #pragma unroll
     for (int b = 0; b < DIM; b++) J[b] = z;
 #pragma unroll 1
@@ -515,11 +527,12 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
       }
     }
 #pragma unroll
-    for (int b = 0; b < DIM; b++) store(a, b, a == b ? J[b] + Dm : J[b]);
-    if constexpr (EN) store(a, DIM, (-rho * A.g[a] * A.beta) * A1);
+    for (int b = 0; b < DIM; b++) J[b] = a == b ? J[b] + Dm : J[b];
+    if constexpr (EN) J[DIM] = (-rho * A.g[a] * A.beta) * A1;
+    store(a, J);
   }
   if constexpr (EN) {
-    d4v Jb[DIM];
+    d4v Jb[NV];
 #pragma unroll
     for (int b = 0; b < DIM; b++) Jb[b] = z;
 #pragma unroll 1
@@ -561,9 +574,8 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
           if (kk + 4 * r < NVE) Tt[r] -= S.qh[k][g] * st[kk + 4 * r] * st[j];
       }
     }
-#pragma unroll
-    for (int b = 0; b < DIM; b++) store(DIM, b, Jb[b]);
-    store(DIM, DIM, Tt);
+    Jb[DIM] = Tt;
+    store(DIM, Jb);
   }
 #undef GM_MFMA64
 
@@ -652,14 +664,14 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
 // residual in columns 27 + a; and dA psi_k in those columns of the products
 // with G_b gives momentum x pressure, whose transpose is continuity x velocity.
 //
-// The workgroup writes the element's matrix before Dirichlet rows (kel, in the
-// e2nz layout), residual (re) and, with PSPG and energy, the continuity x
-// temperature entries (ct); k_gather sums them into the MSR rows.
+// The workgroup writes the element's matrix before Dirichlet rows (kel),
+// residual (re) and, with PSPG and energy, the continuity x temperature entries
+// (ct); k_gather sums them into the MSR rows.
 // Bound by the element matrices' bytes (98 KB an element with energy) and the
 // 182 products a wave (64 cycles each).  Measured, with k_gather (16^3
-// elements with energy, FP64): 508 us against 716 with eight coloured
+// elements with energy, FP64): 449 us against 743 with eight coloured
 // launches that staged the state by threads and added into the rows through a
-// rank map; 11^3 shear-thinning, FP32 matrix: 217 against 629.
+// rank map; 11^3 shear-thinning, FP32 matrix: 198 against 629.
 
 struct NodeCols {  // coordinates as x[a][i] from rows of 16 doubles a node
   const double *p;
@@ -999,12 +1011,12 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
   if (A.resid_only) return;
 
   // 5b. nodal blocks: rows i0 + kk + 4 r, column j
-  auto store = [&](int a, int b, const d4v &D) {
-    double *__restrict__ k = K + (size_t)(a * NV + b) * NVE2 + j;
+  auto store = [&](int a, const d4v *D) {  // block row a
+    double *__restrict__ k = K + (size_t)(a * NVE2 + j) * NV;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int i = i0 + kk + 4 * r;
-      if (i < NVE && node) k[i * NVE] = D[r];
+      if (i < NVE && node) put_cols<NV>(k + i * NVE * NV, D, r);
     }
   };
   if constexpr (VISC == 0) Lmu = A.mu0 * L1;
@@ -1012,7 +1024,7 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
   d4v Tt = -(rCp * Dadv + kc * L1 + (rCp * cm) * A1);
 #pragma unroll 1
   for (int a = 0; a < DIM; a++) {
-    d4v J[DIM];
+    d4v J[NV];
 #pragma unroll
     for (int b = 0; b < DIM; b++) J[b] = z;
 #pragma unroll 1
@@ -1058,12 +1070,13 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
       }
     }
 #pragma unroll
-    for (int b = 0; b < DIM; b++) store(a, b, a == b ? J[b] + Dm : J[b]);
-    if constexpr (EN) store(a, DIM, (-rho * A.g[a] * A.beta) * A1);
+    for (int b = 0; b < DIM; b++) J[b] = a == b ? J[b] + Dm : J[b];
+    if constexpr (EN) J[DIM] = (-rho * A.g[a] * A.beta) * A1;
+    store(a, J);
   }
   if constexpr (EN) {
     const double sw = s_su[0];
-    d4v J[DIM];
+    d4v J[NV];
 #pragma unroll
     for (int b = 0; b < DIM; b++) J[b] = z;
     if (sw != 0.0) {
@@ -1127,9 +1140,8 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
         }
       }
     }
-#pragma unroll
-    for (int b = 0; b < DIM; b++) store(DIM, b, J[b]);
-    store(DIM, DIM, Tt);
+    J[DIM] = Tt;
+    store(DIM, J);
   }
 #undef GM_MFMA64
 

@@ -763,6 +763,10 @@ static int upv(T **d, const T *h, size_t n) {
 template <int DIM>
 constexpr int gal_ws_max() { return DIM == 2 ? 32 : 128; }
 
+// Block rows per workgroup of the Galerkin kernel
+template <int DIM, int EN>
+constexpr int gal_rows() { return DIM == 2 ? DIM + EN : 1; }
+
 // Galerkin coarse operators.  When every finer element lies inside one
 // coarser element (its parent) and P maps the parent's unknowns to the
 // element's unknowns, R A P = sum over finer elements of P_e^T K_e P_e, with K_e
@@ -853,8 +857,42 @@ static std::string build_galerkin_maps(const gm_ctx *f, const gm_ctx *c, const i
 }
 
 // Coarse element matrices P_e^T K_e P_e summed over the children of each coarse
-// element (one workgroup per coarse element), in the e2nz layout: nodal blocks
-// (a, b) as [i][j], then momentum x P, continuity x velocity, P x P.
+// element, in the element matrices' layout: nodal block rows a as [i][j][b],
+// then momentum x P, continuity x velocity, P x P.
+//
+// A workgroup takes RW block rows of one coarse element (HEX27: one, QUAD9:
+// all), another its pressure couplings: the blocks are independent, and with
+// one workgroup for all of them the levels of up to a few hundred elements
+// leave most of the chip idle behind 128 rounds of three barriers (64 coarse
+// elements with energy, FP64: 57 us against 580).  Per child: K_e's rows from
+// memory a child ahead, T = K W over them in LDS, W^T T summed in registers.
+// Larger levels are bound by reading the finer element matrices once (1728
+// coarse elements with energy, FP32 products: 353 us for 1.4 GB).
+// One weight of a child's nodal interpolation and the finer node it is for
+template <typename CT>
+struct alignas(2 * sizeof(CT)) GalW {
+  CT w;
+  int i;
+};
+
+// the n entries of a node pair's row, in 16-byte reads where n allows
+template <int n, typename CT>
+__device__ inline void load_cols(const CT *p, CT *v) {
+  constexpr int W = n * sizeof(CT) % 16 == 0 ? 16 / sizeof(CT) : 1;
+  if constexpr (W > 1) {
+    typedef CT Wide __attribute__((ext_vector_type(W)));
+#pragma unroll
+    for (int b = 0; b < n; b += W) {
+      const Wide w = *(const Wide *)(p + b);
+#pragma unroll
+      for (int l = 0; l < W; l++) v[b + l] = w[l];
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < n; b++) v[b] = p[b];
+  }
+}
+
 template <int DIM, int EN, typename CT>
 __global__ __launch_bounds__(256) void k_galerkin(const double *__restrict__ kf,
                                                   const int *__restrict__ child,
@@ -864,21 +902,39 @@ __global__ __launch_bounds__(256) void k_galerkin(const double *__restrict__ kf,
                                                   const double *__restrict__ Q, long long E,
                                                   long long off_mp, double *__restrict__ kc) {
   constexpr int NVE = DIM == 2 ? 9 : 27, NP = DIM + 1, NV = DIM + EN, NCH = 1 << DIM, NT = 256;
-  constexpr int NVE2 = NVE * NVE;
-  constexpr int RN = (NVE2 + NT - 1) / NT;
+  constexpr int NVE2 = NVE * NVE, RW = gal_rows<DIM, EN>(), PARTS = NV / RW + 1;
+  constexpr int ROW = NVE * NV, LROW = ROW + (DIM == 3 && sizeof(CT) == 8 ? 2 : 0);  // padded against bank conflicts
+  constexpr int NK = RW * NVE2 * NV, RK = (NK + NT - 1) / NT;    // entries of the block rows
+  constexpr int NI = RW * NVE2, RN = (NI + NT - 1) / NT;         // node pairs of the block rows
   constexpr int NMP = DIM * NVE * NP;          // momentum x P (= continuity x velocity) entries
   constexpr int NPC = 2 * NMP + NP * NP;       // pressure couplings, contiguous from off_mp
   constexpr int RP = (NPC + NT - 1) / NT;
   constexpr int WSM = gal_ws_max<DIM>();
   // W of every child by columns, loaded once: s_wp[c][m] .. s_wp[c][m + 1]
-  // index the finer nodes s_wi (ascending) interpolating from coarse node m
-  // and their weights s_wv; only these terms of the dense sums are nonzero,
-  // taken in the same order
-  __shared__ CT sK[NVE2], sT[NVE2], sQ[NP * NP], sKp[NPC], s_wv[NCH * WSM];
-  __shared__ int s_wp[NCH][NVE + 1], s_wi[NCH * WSM];
-  const int ec = blockIdx.x, tid = threadIdx.x;
+  // index the finer nodes (ascending) interpolating from coarse node m and
+  // their weights, s_w; only these terms of the dense sums are nonzero
+  __shared__ alignas(16) CT sK[RW * NVE * LROW];
+  __shared__ GalW<CT> s_w[NCH * WSM];
+  __shared__ CT sQ[NP * NP];
+  __shared__ int s_wp[NCH][NVE + 1];
+  static_assert(NPC <= RW * NVE * LROW, "the pressure couplings fit the block rows' space");
+  const int ec = blockIdx.x / PARTS, part = blockIdx.x - ec * PARTS, tid = threadIdx.x;
   const int *ch = child + (size_t)ec * NCH;
   double *__restrict__ out = kc + (size_t)ec * E;
+  const bool press = part == PARTS - 1;
+  const size_t off = press ? (size_t)off_mp : (size_t)part * NK;
+  const int cnt = press ? NPC : NK;
+  double kr[RK];
+  static_assert(RP <= RK, "registers for the pressure couplings");
+  auto fetch = [&](int c) {
+    const double *Kf = kf + (size_t)ch[c] * E + off;
+#pragma unroll
+    for (int r = 0; r < RK; r++) {
+      const int t = tid + r * NT;
+      kr[r] = t < cnt ? Kf[t] : 0.0;
+    }
+  };
+  fetch(0);
   for (int t = tid; t < NCH * (NVE + 1); t += NT) {
     const int c = t / (NVE + 1), m = t - c * (NVE + 1);
     s_wp[c][m] = Wp[(size_t)ch[c] * (NVE + 1) + m];
@@ -886,73 +942,113 @@ __global__ __launch_bounds__(256) void k_galerkin(const double *__restrict__ kf,
   for (int t = tid; t < NCH * WSM; t += NT) {
     const int c = t / WSM, k = t - c * WSM;
     if (k < ws) {
-      s_wi[t] = Wi[(size_t)ch[c] * ws + k];
-      s_wv[t] = (CT)Wv[(size_t)ch[c] * ws + k];
+      s_w[t].i = Wi[(size_t)ch[c] * ws + k];
+      s_w[t].w = (CT)Wv[(size_t)ch[c] * ws + k];
     }
   }
-  // The finer element matrices' blocks, (variable block, child) in turn: the
-  // next one is loaded into registers while the current one is reduced.
-  double kr[RN];
-  auto fetch = [&](int it) {
-    const int blk = it / NCH, f = ch[it - blk * NCH];
-    const double *Kf = kf + (size_t)f * E + (size_t)blk * NVE2;
+  if (!press) {
+    CT acc[RN][NV];
 #pragma unroll
-    for (int r = 0; r < RN; r++) {
-      const int t = tid + r * NT;
-      kr[r] = t < NVE2 ? Kf[t] : 0.0;
-    }
-  };
-  fetch(0);
-  for (int blk = 0; blk < NV * NV; blk++) {
-    CT acc[RN];
+    for (int r = 0; r < RN; r++)
 #pragma unroll
-    for (int r = 0; r < RN; r++) acc[r] = 0.0;
-    for (int sidx = 0; sidx < NCH; sidx++) {
+      for (int b = 0; b < NV; b++) acc[r][b] = 0;
+#pragma unroll 1
+    for (int c = 0; c < NCH; c++) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < RK; r++) {
+        const int t = tid + r * NT, i = t / ROW;
+        if (t < NK) sK[i * LROW + t - i * ROW] = (CT)kr[r];
+      }
+      if (c + 1 < NCH) fetch(c + 1);
+      const int *wp = s_wp[c];
+      const GalW<CT> *w = s_w + c * WSM;
+      __syncthreads();
+      CT T[RN][NV];  // T = K W: row i, column m of W
 #pragma unroll
       for (int r = 0; r < RN; r++) {
-        const int t = tid + r * NT;
-        if (t < NVE2) sK[t] = (CT)kr[r];
-      }
-      const int it = blk * NCH + sidx;
-      if (it + 1 < NV * NV * NCH) fetch(it + 1);
-      const int *wp = s_wp[sidx], *wi = s_wi + sidx * WSM;
-      const CT *wv = s_wv + sidx * WSM;
-      __syncthreads();
-      for (int t = tid; t < NVE2; t += NT) {  // T = K W, column m of W
-        const int m = t / NVE, i = t - m * NVE;
-        CT v = 0;
-        for (int k = wp[m]; k < wp[m + 1]; k++) v += sK[i * NVE + wi[k]] * wv[k];
-        sT[i * NVE + m] = v;
+        const int t = tid + r * NT, a = t / NVE2, t2 = t - a * NVE2, m = t2 / NVE, i = t2 - m * NVE;
+#pragma unroll
+        for (int b = 0; b < NV; b++) T[r][b] = 0;
+        if (t < NI)
+          for (int k = wp[m]; k < wp[m + 1]; k++) {
+            const GalW<CT> x = w[k];
+            CT y[NV];
+            load_cols<NV>(sK + (a * NVE + i) * LROW + x.i * NV, y);
+#pragma unroll
+            for (int b = 0; b < NV; b++) T[r][b] += y[b] * x.w;
+          }
       }
       __syncthreads();
 #pragma unroll
-      for (int r = 0; r < RN; r++) {  // acc += W^T T
-        const int t = tid + r * NT;
-        if (t < NVE2) {
-          const int m = t / NVE, n = t - m * NVE;
-          CT v = 0;
-          for (int k = wp[m]; k < wp[m + 1]; k++) v += wv[k] * sT[wi[k] * NVE + n];
-          acc[r] += v;
-        }
+      for (int r = 0; r < RN; r++) {
+        const int t = tid + r * NT, a = t / NVE2, t2 = t - a * NVE2, m = t2 / NVE, i = t2 - m * NVE;
+        if (t < NI)
+#pragma unroll
+          for (int b = 0; b < NV; b++) sK[(a * NVE + i) * LROW + m * NV + b] = T[r][b];
       }
       __syncthreads();
+#pragma unroll
+      for (int r = 0; r < RN; r++) {  // acc += W^T T: row m, column n
+        const int t = tid + r * NT, a = t / NVE2, t2 = t - a * NVE2, m = t2 / NVE, n = t2 - m * NVE;
+        if (t >= NI) continue;
+        CT v[NV];
+#pragma unroll
+        for (int b = 0; b < NV; b++) v[b] = 0;
+        for (int k = wp[m]; k < wp[m + 1]; k++) {
+          const GalW<CT> x = w[k];
+          CT y[NV];
+          load_cols<NV>(sK + (a * NVE + x.i) * LROW + n * NV, y);
+#pragma unroll
+          for (int b = 0; b < NV; b++) v[b] += x.w * y[b];
+        }
+#pragma unroll
+        for (int b = 0; b < NV; b++) acc[r][b] += v[b];
+      }
     }
 #pragma unroll
     for (int r = 0; r < RN; r++) {
       const int t = tid + r * NT;
-      if (t < NVE2) out[(size_t)blk * NVE2 + t] = acc[r];
+      if (t < NI)
+#pragma unroll
+        for (int b = 0; b < NV; b++) out[off + (size_t)t * NV + b] = acc[r][b];
     }
+    return;
   }
   CT accp[RP];
 #pragma unroll
   for (int r = 0; r < RP; r++) accp[r] = 0.0;
-  for (int sidx = 0; sidx < NCH; sidx++) {
-    const int f = ch[sidx];
-    const double *Kf = kf + (size_t)f * E + off_mp;
-    const int *wp = s_wp[sidx], *wi = s_wi + sidx * WSM;
-    const CT *wv = s_wv + sidx * WSM;
-    if (tid < NP * NP) sQ[tid] = (CT)Q[(size_t)f * NP * NP + tid];
-    for (int t = tid; t < NPC; t += NT) sKp[t] = (CT)Kf[t];
+#pragma unroll 1
+  for (int c = 0; c < NCH; c++) {
+    __syncthreads();
+    if (tid < NP * NP) sQ[tid] = (CT)Q[(size_t)ch[c] * NP * NP + tid];
+#pragma unroll
+    for (int r = 0; r < RP; r++) {
+      const int t = tid + r * NT;
+      if (t < NPC) sK[t] = (CT)kr[r];
+    }
+    if (c + 1 < NCH) fetch(c + 1);
+    const int *wp = s_wp[c];
+    const GalW<CT> *w = s_w + c * WSM;
+    __syncthreads();
+    // over the nodes first (W^T K, K W; nothing for P x P), then over the P1 dofs
+    CT T[RP];
+#pragma unroll
+    for (int r = 0; r < RP; r++) {
+      const int t = tid + r * NT;
+      T[r] = 0;
+      if (t >= 2 * NMP) continue;
+      const bool mp = t < NMP;
+      const int node = mp ? t / NP % NVE : (t - NMP) % NVE;
+      const int base = mp ? t - node * NP : t - node, step = mp ? NP : 1;
+      for (int k = wp[node]; k < wp[node + 1]; k++) T[r] += w[k].w * sK[base + w[k].i * step];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RP; r++) {
+      const int t = tid + r * NT;
+      if (t < 2 * NMP) sK[t] = T[r];
+    }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < RP; r++) {
@@ -960,35 +1056,23 @@ __global__ __launch_bounds__(256) void k_galerkin(const double *__restrict__ kf,
       if (t >= NPC) continue;
       CT v = 0;
       if (t < NMP) {  // row (a, m) momentum, column l pressure
-        const int a = t / (NVE * NP), rem = t - a * NVE * NP, m = rem / NP, l = rem - m * NP;
-        for (int k2 = wp[m]; k2 < wp[m + 1]; k2++) {
-          const int i = wi[k2];
-          CT q = 0;
+        const int l = t % NP;
 #pragma unroll
-          for (int k = 0; k < NP; k++) q += sKp[a * NVE * NP + i * NP + k] * sQ[k * NP + l];
-          v += wv[k2] * q;
-        }
+        for (int k = 0; k < NP; k++) v += sK[t - l + k] * sQ[k * NP + l];
       } else if (t < 2 * NMP) {  // row l continuity, column (b, n) velocity
-        const int t2 = t - NMP, b = t2 / (NP * NVE), rem = t2 - b * NP * NVE;
-        const int l = rem / NVE, n = rem - l * NVE;
+        const int t2 = t - NMP, l = t2 / NVE % NP;
 #pragma unroll
-        for (int k = 0; k < NP; k++) {
-          CT q = 0;
-          for (int k2 = wp[n]; k2 < wp[n + 1]; k2++)
-            q += sKp[NMP + b * NP * NVE + k * NVE + wi[k2]] * wv[k2];
-          v += sQ[k * NP + l] * q;
-        }
+        for (int k = 0; k < NP; k++) v += sQ[k * NP + l] * sK[t + (k - l) * NVE];
       } else {  // P x P
         const int t3 = t - 2 * NMP, l = t3 / NP, l2 = t3 - l * NP;
 #pragma unroll
         for (int k = 0; k < NP; k++)
 #pragma unroll
           for (int k2 = 0; k2 < NP; k2++)
-            v += sQ[k * NP + l] * sKp[2 * NMP + k * NP + k2] * sQ[k2 * NP + l2];
+            v += sQ[k * NP + l] * sK[2 * NMP + k * NP + k2] * sQ[k2 * NP + l2];
       }
       accp[r] += v;
     }
-    __syncthreads();
   }
 #pragma unroll
   for (int r = 0; r < RP; r++) {
@@ -1009,7 +1093,8 @@ static int galerkin_level(gm_ctx *prof, const gm_ctx *above, MgLevel &L, JT *val
   using CT = JT;
   auto kern = lc->dim == 2 ? (lc->energy ? k_galerkin<2, 1, CT> : k_galerkin<2, 0, CT>)
                            : (lc->energy ? k_galerkin<3, 1, CT> : k_galerkin<3, 0, CT>);
-  gm_launch(prof, GM_K_GALERKIN, gbytes, kern, dim3(lc->num_elems), dim3(256), 0, lc->stream,
+  const int parts = (lc->dim == 2 ? 1 : lc->nv) + 1;  // workgroups per coarse element
+  gm_launch(prof, GM_K_GALERKIN, gbytes, kern, dim3(lc->num_elems * parts), dim3(256), 0, lc->stream,
             above->d_kel, L.d_child, L.d_Wp, L.d_Wi, L.d_Wv, L.W_stride, L.d_Q, ly.total, ly.off_mp,
             lc->d_kel);
   // with the coarse level's own Dirichlet rows

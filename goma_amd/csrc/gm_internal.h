@@ -131,9 +131,9 @@ struct MgLevel {
   int vec_prec = -1;
   int nnz = 0;                // entries of P
   // coarsest level only: dense FP64 inverse for the exact coarse solve
-  double *d_dense = nullptr;  // [n][n]
-  double *d_pcol = nullptr;  // pivot rows of one panel of the coarsest inverse [GJ_NB][n]
-  int *d_perm = nullptr;      // row interchange of each step
+  double *d_dense = nullptr, *d_dense2 = nullptr;  // [n][n] the coarsest inverse; elimination workspace
+  double *d_pcol = nullptr;  // two panels of the elimination [2][GJ_NB][n]
+  int *d_perm = nullptr;      // pivot row of each step, then step of each row
   int dense_n = 0;
   // host copy of P, kept by gm_mg_build (gm_mg_copy_prolongation)
   std::vector<int> P_host_rowptr, P_host_col;

@@ -369,8 +369,42 @@ __global__ __launch_bounds__(256) void k_mg_resid_rows(int nrows, const int *__r
   if (lane == 0) r[row] = (BT)((AT)b[row] - s - (AT)a[row] * (AT)x[row]);
 }
 
-// ---- exact coarse solve: dense inverse by in-place Gauss-Jordan with
-// partial pivoting (two launches per pivot), applied as a dense GEMV.
+// ---- exact coarse solve: dense inverse by Gauss-Jordan with partial
+// pivoting, applied as a dense GEMV.
+
+// maximum over the 16 lanes of a DPP row, in every lane
+__device__ inline unsigned row_max16(unsigned v) {
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));  // row_ror:8
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false));
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
+}
+
+// the value of lane j of each DPP row of 16, in all of its lanes (row_newbcast)
+template <int j>
+__device__ inline double row_bcast_c(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  return __builtin_bit_cast(double, (unsigned long long)__builtin_amdgcn_update_dpp(0ull, b, 0x150 + j, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double row_bcast(double v, int j) {
+  switch (j) {
+#define GM_B(k) case k: return row_bcast_c<k>(v);
+    GM_B(0) GM_B(1) GM_B(2) GM_B(3) GM_B(4) GM_B(5) GM_B(6) GM_B(7)
+    GM_B(8) GM_B(9) GM_B(10) GM_B(11) GM_B(12) GM_B(13) GM_B(14)
+#undef GM_B
+    default: return row_bcast_c<15>(v);
+  }
+}
+
+// 1 / v to the last bit but one, 0 for 0: the hardware's estimate and two Newton
+// steps, half the chain of the correctly rounded division
+__device__ inline double reciprocal(double v) {
+  double y = __builtin_amdgcn_rcp(v);
+  y = fma(fma(-v, y, 1.0), y, y);
+  y = fma(fma(-v, y, 1.0), y, y);
+  return v != 0.0 ? y : 0.0;
+}
+
 template <typename VT>
 __global__ void k_msr_to_dense(int n, const VT *__restrict__ a, const int *__restrict__ bindx,
                                double *__restrict__ D) {
@@ -381,220 +415,287 @@ __global__ void k_msr_to_dense(int n, const VT *__restrict__ a, const int *__res
 }
 
 // Dense Gauss-Jordan inverse of the coarsest level with partial pivoting,
-// blocked in panels of at most GJ_NB columns (same pivots and interchanges as
-// the column-at-a-time algorithm).  For panel K:
-//   k_gjb_panel    one workgroup runs the panel's column steps on the panel
-//                  columns only, the panel in registers (pivot: largest
-//                  |entry| at or below the diagonal, first on ties; whole
-//                  panel rows interchanged);
-//   k_gjb_swap     the panel's interchanges on every other column, in order,
-//                  and a copy of the pivot rows B_K of those columns;
-//   k_gjb_update   every other column: B <- B' + Pan B_K, B' = B with the
-//                  pivot rows zeroed (the panel now holds the K columns of
-//                  the accumulated elimination, so pivot rows become
-//                  A_KK^-1 B_K and the others B_R - A_RK A_KK^-1 B_K).
-// D is row-major n x n.  perm[k] = the row interchanged with k at step k.
-constexpr int GJ_NB = 32;
+// blocked in panels of NB columns.  Rows stay where they are: step k takes as
+// pivot the unused row with the largest entry of column k (to 20 bits; the
+// first on ties), and the finished array holds inverse row k in the row that
+// was step k's pivot, its columns in pivot order too (k_gj_permute).
+//
+// One launch per panel, from one copy D of the array into the other, O:
+//   the tiles apply panel K to the other columns, O = D' + Pan D_K: Pan the
+//     panel's columns after its steps, D_K its pivot rows, D' = D with those
+//     rows zeroed; panel K's own columns become Pan;
+//   the first workgroup meanwhile brings panel K + 1 up to date in registers
+//     and runs its column steps.
+// The panel workgroup is a chain of dependent steps that the tiles hide behind
+// (for 1480 unknowns they take 17 us of the launch): thread t owns rows
+// t + NT r of the panel.  Per step each group of 16 lanes finds its candidate
+// with a 32-bit maximum (DPP rotations); the lane that holds it puts its key,
+// its reciprocal and its row into LDS, and after the step's only barrier every
+// wave picks the winner.  The buffers alternate by step parity, so no second
+// barrier guards their reuse.  Few waves with several rows a thread: the step
+// is latency, not work.
+// Measured: 32 us a panel of 16 for 1480 unknowns, 22 for 532, 14 for 87,
+// against 80, 59 and 46 with row interchanges, two barriers a step and launches
+// of their own for the panel, the interchanges and the update; the rows'
+// final order costs 9 us instead of 295.
+constexpr int GJ_NB = 16;  // widest panel
 
-// The panel lives in registers for its column steps: thread t of 512 owns
-// rows t + 512 r (r < RPT) of the NB panel columns (RPT NB <= 64 doubles),
-// so D is read and written once per panel.  Per step: the pivot candidate of
-// each wave (DPP row rotations, then the wave's four rows by readlane) goes to
-// LDS; after one barrier every thread merges the eight candidates itself; the
-// pivot row and row k pass through LDS; a second barrier.  The LDS buffers
-// alternate by step parity, so no third barrier guards their reuse.
-template <int NB, int RPT>
-__global__ __launch_bounds__(512) void k_gjb_panel(int n, int kb0, int nb, double *__restrict__ D,
-                                                    int *__restrict__ perm, int *__restrict__ flag) {
-  __shared__ double s_rk[2][NB], s_rp[2][NB];
-  __shared__ double sv[2][8];
-  __shared__ int si[2][8];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  double P[RPT][NB];
+template <int NB, int RPT, int NT>
+__global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2, int nb2,
+                                                 const double *__restrict__ D, double *__restrict__ O,
+                                                 const double *__restrict__ pan, double *__restrict__ pan2,
+                                                 const int *__restrict__ piv, int *__restrict__ piv2,
+                                                 int *stepof, int *__restrict__ flag) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+  constexpr int NW = NT / 64;
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  if (blockIdx.x == 0) {
+    if (nb2 == 0) return;
+    constexpr int NG = 4 * NW, NK = NG / 16;  // groups of 16 lanes, keys per lane
+    struct Cand {
+      double v[4], inv;
+      int row;
+    };
+    __shared__ Cand s_cand[2][NG];
+    __shared__ unsigned s_key[2][NG];
+    __shared__ double s_old[4][NB - 4];
+    __shared__ double s_turn[NW][16][17];
+    // panel K + 1's columns with panel K applied, 16 rows at a time on the
+    // matrix cores (as the tiles below), turned through LDS to a row per thread
+    constexpr int RB = RPT * NT <= 1536 ? RPT : 1;  // rows loaded together, as registers allow
+    double P[RPT][NB], bk[NB / 4];
+    bool used[RPT];
 #pragma unroll
-  for (int r = 0; r < RPT; r++) {
-    const int i = tid + 512 * r;
+    for (int k = 0; k < NB / 4; k++) {
+      const int t = 4 * k + lq;
+      bk[k] = t < nb ? D[(size_t)piv[t] * n + kb2 + l16] : 0.0;
+    }
+    unsigned long long zero[RPT];  // rows that start from zero: the pivot rows of panel K
 #pragma unroll
-    for (int j = 0; j < NB; j++) P[r][j] = (i < n && j < nb) ? D[(size_t)i * n + kb0 + j] : 0.0;
-  }
+    for (int r = 0; r < RPT; r++) {
+      const int i = NT * r + tid, at = i < n && kb2 > 0 ? stepof[i] : -1;
+      used[r] = i >= n || at >= 0;
+      zero[r] = __ballot(i >= n || (nb > 0 && at >= kb && at < kb + nb));
+    }
 #pragma unroll
-  for (int kk = 0; kk < NB; kk++) {
-    if (kk < nb) {
-      const int k = kb0 + kk, q = kk & 1;
-      double best = -1.0;
-      int bi = n;
+    for (int r0 = 0; r0 < RPT; r0 += RB) {
+      d4 C[RB][4];
+      double f[RB][4][NB / 4];
 #pragma unroll
-      for (int r = 0; r < RPT; r++) {
-        const int i = tid + 512 * r;
-        const double v = fabs(P[r][kk]);
-        if (i >= k && i < n && v > best) {
-          best = v;
-          bi = i;
+      for (int r = 0; r < RB; r++) {
+        const int ib = NT * (r0 + r) + 64 * w;
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int row = 16 * m + lq + 4 * e;
+            // past the last column: another row's, or the margin; unused
+            C[r][m][e] = (zero[r0 + r] >> row) & 1 ? 0.0 : D[(size_t)(ib + row) * n + kb2 + l16];
+          }
+#pragma unroll
+          for (int k = 0; k < NB / 4; k++) {
+            const int t = 4 * k + lq;
+            f[r][m][k] = t < nb && ib + 16 * m + l16 < n ? pan[(size_t)t * n + ib + 16 * m + l16] : 0.0;
+          }
         }
       }
-      pivot_combine<8>(best, bi);
-      pivot_combine<4>(best, bi);
-      pivot_combine<2>(best, bi);
-      pivot_combine<1>(best, bi);
-      // lanes 0, 16, 32, 48 hold their rows' candidates
+      if (nb > 0)
 #pragma unroll
-      for (int g = 1; g < 4; g++) {
-        const unsigned long long bb = __builtin_bit_cast(unsigned long long, best);
-        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)bb, 16 * g);
-        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(bb >> 32), 16 * g);
-        const double ov = __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-        const int oi = __builtin_amdgcn_readlane(bi, 16 * g);
-        if (lane == 0 && (ov > best || (ov == best && oi < bi))) {
-          best = ov;
-          bi = oi;
+        for (int k = 0; k < NB / 4; k++)
+#pragma unroll
+          for (int r = 0; r < RB; r++)
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+              C[r][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[r][m][k], bk[k], C[r][m], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < RB; r++)
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+          for (int e = 0; e < 4; e++) s_turn[w][lq + 4 * e][l16] = C[r][m][e];
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          if (lq == m)
+#pragma unroll
+            for (int j = 0; j < NB; j++) P[r0 + r][j] = s_turn[w][l16][j];
+        }
+    }
+    int step[RPT];
+#pragma unroll
+    for (int r = 0; r < RPT; r++) step[r] = -1;
+    __syncthreads();
+    // Four columns at a time, the others brought up to date after the four: a
+    // step then waits for four values of its pivot row, not for sixteen.  The
+    // columns move up four registers a round, so that the round's are always
+    // the first and the loop stays in the instruction cache.
+#pragma unroll 1
+    for (int c0 = 0; c0 < nb2; c0 += 4) {
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) {
+        if (c0 + kk >= nb2) continue;
+        const int q = kk & 1;
+        // candidate: 0 for a used row, 1 for a zero (or NaN), else the high word + 2
+        unsigned best = 0;
+        int br = 0;
+        double cand[4] = {P[0][0], P[0][1], P[0][2], P[0][3]};
+#pragma unroll
+        for (int r = 0; r < RPT; r++) {
+          const double v = fabs(P[r][kk]);
+          const unsigned hi = (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32);
+          const unsigned key = used[r] ? 0u : v > 0.0 ? hi + 2u : 1u;
+          if (r == 0 || key > best) {
+            best = key;
+            br = r;
+#pragma unroll
+            for (int j = 0; j < 4; j++) cand[j] = P[r][j];
+          }
+        }
+        double ci = reciprocal(cand[kk]);  // every lane's, beside the chain of the maximum
+        asm volatile("" : "+v"(ci));
+        const unsigned m = row_max16(best);
+        const unsigned long long at = __ballot(best == m);
+        if (lane == 16 * lq + __ffs((unsigned)(at >> (16 * lq)) & 0xffffu) - 1) {  // the first of its 16 lanes
+          Cand &c = s_cand[q][4 * w + lq];
+          s_key[q][4 * w + lq] = m;
+          c.row = tid + NT * br;
+          c.inv = ci;
+#pragma unroll
+          for (int j = 0; j < 4; j++) c.v[j] = cand[j];
+        }
+        __syncthreads();
+        unsigned wk[NK], wm = 0;
+#pragma unroll
+        for (int c = 0; c < NK; c++) {
+          wk[c] = s_key[q][NK * l16 + c];
+          wm = max(wm, wk[c]);
+        }
+        wm = row_max16(wm);
+        int g = 0;  // a group that has the maximum, the same in every wave
+#pragma unroll
+        for (int c = NK - 1; c >= 0; c--) {
+          const unsigned long long has = __ballot(wk[c] == wm);
+          g = has ? NK * (__ffsll(has) - 1) + c : g;
+        }
+        const Cand &c = s_cand[q][__builtin_amdgcn_readfirstlane(g)];
+        const double inv = c.inv, R[4] = {c.v[0], c.v[1], c.v[2], c.v[3]};
+        const int p = __builtin_amdgcn_readfirstlane(c.row);
+        if (tid == 0) {
+          piv2[c0 + kk] = p;
+          if (wm == 1u) flag[3] = 1;  // singular coarse matrix
+        }
+#pragma unroll
+        for (int r = 0; r < RPT; r++) {
+          const bool is = p == tid + NT * r;  // the pivot row: R inv, and inv itself
+          const double f = is ? -inv : P[r][kk] * inv;
+          used[r] = used[r] || is;
+          step[r] = is ? kb2 + c0 + kk : step[r];
+#pragma unroll
+          for (int j = 0; j < 4; j++) P[r][j] = j == kk ? -f : fma(R[j], -f, is ? 0.0 : P[r][j]);
         }
       }
-      if (lane == 0) {
-        sv[q][w] = best;
-        si[q][w] = bi;
-      }
+      // the other columns: zero in the four pivot rows, plus the four columns
+      // times those rows' old values
+#pragma unroll
+      for (int r = 0; r < RPT; r++)
+        if (step[r] >= kb2 + c0) {
+          double *old = s_old[step[r] - kb2 - c0];
+#pragma unroll
+          for (int j = 4; j < NB; j++) {
+            old[j - 4] = P[r][j];
+            P[r][j] = 0.0;
+          }
+        }
       __syncthreads();
-      double bv = sv[q][0];
-      int p = si[q][0];
+      double mine[4];
 #pragma unroll
-      for (int g = 1; g < 8; g++) {
-        const double ov = sv[q][g];
-        const int oi = si[q][g];
-        if (ov > bv || (ov == bv && oi < p)) {
-          bv = ov;
-          p = oi;
-        }
+      for (int kk = 0; kk < 4; kk++) mine[kk] = s_old[kk][l16 < NB - 4 ? l16 : 0];
+      double Q[RPT][NB];
+#pragma unroll
+      for (int r = 0; r < RPT; r++)
+#pragma unroll
+        for (int j = 4; j < NB; j++) Q[r][j - 4] = P[r][j];
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) {
+        if (c0 + kk >= nb2) continue;
+        double R[NB - 4];
+#pragma unroll
+        for (int j = 0; j < NB - 4; j++) R[j] = row_bcast(mine[kk], j);
+        __builtin_amdgcn_sched_barrier(0);  // the moves together, not each waited for by its products
+#pragma unroll
+        for (int j = 0; j < NB - 4; j++)
+#pragma unroll
+          for (int r = 0; r < RPT; r++) Q[r][j] = fma(R[j], P[r][kk], Q[r][j]);
       }
-      if (p >= n) p = k;
-      if (tid == 0) {
-        if (!(bv > 0.0)) flag[3] = 1;  // singular coarse matrix
-        perm[k] = p;
-      }
-      // rows k and p to LDS (row p is the new pivot row), then interchanged
 #pragma unroll
       for (int r = 0; r < RPT; r++) {
-        const int i = tid + 512 * r;
-        if (i == p)
 #pragma unroll
-          for (int j = 0; j < NB; j++) s_rp[q][j] = P[r][j];
-        if (i == k && p != k)
+        for (int j = 0; j < 4; j++) Q[r][NB - 4 + j] = P[r][j];
 #pragma unroll
-          for (int j = 0; j < NB; j++) s_rk[q][j] = P[r][j];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int r = 0; r < RPT; r++) {
-        const int i = tid + 512 * r;
-        if (p != k && i == k)
-#pragma unroll
-          for (int j = 0; j < NB; j++) P[r][j] = s_rp[q][j];
-        if (p != k && i == p)
-#pragma unroll
-          for (int j = 0; j < NB; j++) P[r][j] = s_rk[q][j];
-      }
-      const double piv = s_rp[q][kk];
-      const double inv = piv != 0.0 ? 1.0 / piv : 0.0;
-#pragma unroll
-      for (int r = 0; r < RPT; r++) {
-        const int i = tid + 512 * r;
-        const double f = P[r][kk];
-        if (i == k) {
-#pragma unroll
-          for (int j = 0; j < NB; j++) P[r][j] = j == kk ? inv : s_rp[q][j] * inv;
-        } else {
-          const double g = f * inv;
-#pragma unroll
-          for (int j = 0; j < NB; j++) P[r][j] = j == kk ? -g : P[r][j] - g * s_rp[q][j];
-        }
+        for (int j = 0; j < NB; j++) P[r][j] = Q[r][j];
       }
     }
-  }
+    const int moved = (nb2 + 3) & ~3;
 #pragma unroll
-  for (int r = 0; r < RPT; r++) {
-    const int i = tid + 512 * r;
-    if (i < n)
+    for (int r = 0; r < RPT; r++) {
+      const int i = tid + NT * r;
+      if (i >= n) continue;
+      if (step[r] >= 0 || kb2 == 0) stepof[i] = step[r];
 #pragma unroll
-      for (int j = 0; j < NB; j++)
-        if (j < nb) D[(size_t)i * n + kb0 + j] = P[r][j];
-  }
-}
-
-__global__ __launch_bounds__(256) void k_gjb_swap(int n, int kb0, int nb, double *__restrict__ D,
-                                                  const int *__restrict__ perm,
-                                                  double *__restrict__ BK) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n || (j >= kb0 && j < kb0 + nb)) return;
-  for (int kk = 0; kk < nb; kk++) {
-    const int k = kb0 + kk, p = perm[k];
-    if (p != k) {
-      const double t = D[(size_t)k * n + j];
-      D[(size_t)k * n + j] = D[(size_t)p * n + j];
-      D[(size_t)p * n + j] = t;
+      for (int j = 0; j < NB; j++) {
+        const int c = (j + moved) & (NB - 1);  // the column here by now
+        if (c < nb2) pan2[(size_t)c * n + i] = P[r][j];
+      }
     }
+    return;
   }
-  for (int kk = 0; kk < nb; kk++) BK[(size_t)kk * n + j] = D[(size_t)(kb0 + kk) * n + j];
-}
-
-// 64 x 64 output tile per workgroup, 4 x 4 per thread; columns of the panel
-// are left alone
-__global__ __launch_bounds__(256) void k_gjb_update(int n, int kb0, int nb, double *__restrict__ D,
-                                                    const double *__restrict__ BK) {
-  __shared__ double sP[64][GJ_NB + 1];
-  __shared__ double sB[GJ_NB][64];
-  const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64, tid = threadIdx.x;
-  for (int idx = tid; idx < 64 * GJ_NB; idx += 256) {
-    const int r = idx / GJ_NB, t = idx - r * GJ_NB, i = i0 + r;
-    sP[r][t] = (i < n && t < nb) ? D[(size_t)i * n + kb0 + t] : 0.0;
-  }
-  for (int idx = tid; idx < GJ_NB * 64; idx += 256) {
-    const int t = idx >> 6, c = idx & 63, j = j0 + c;
-    sB[t][c] = (t < nb && j < n) ? BK[(size_t)t * n + j] : 0.0;
-  }
-  __syncthreads();
-  const int tr = tid >> 4, tc = tid & 15;
-  double acc[4][4];
+  // 16 x 64 tiles, one per wave, on the matrix cores: lane l supplies
+  // A[l%16][l/16] and B[l/16][l%16] and holds D[l/16 + 4r][l%16]
+  const int tx = (n + 63) / 64, task = ((int)blockIdx.x - 1) * NW + w;
+  const int i0 = task / tx * 16, j0 = (task - task / tx * tx) * 64;
+  if (i0 >= n) return;
+  d4 C[4];
 #pragma unroll
-  for (int a = 0; a < 4; a++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) acc[a][c] = 0.0;
-  for (int t = 0; t < nb; t++) {
-    double pa[4], pb[4];
-#pragma unroll
-    for (int a = 0; a < 4; a++) pa[a] = sP[tr + 16 * a][t];
-#pragma unroll
-    for (int c = 0; c < 4; c++) pb[c] = sB[t][tc + 16 * c];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-      for (int c = 0; c < 4; c++) acc[a][c] += pa[a] * pb[c];
-  }
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const int i = i0 + tr + 16 * a;
-    if (i >= n) continue;
-    const bool krow = i >= kb0 && i < kb0 + nb;
+  for (int r = 0; r < 4; r++) {
+    const int i = i0 + lq + 4 * r;
+    const int at = i < n ? stepof[i] : -1;
+    const bool zero = i >= n || (at >= kb && at < kb + nb);
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      const int j = j0 + tc + 16 * c;
-      if (j >= n || (j >= kb0 && j < kb0 + nb)) continue;
-      const size_t at = (size_t)i * n + j;
-      D[at] = (krow ? 0.0 : D[at]) + acc[a][c];
+      const int j = j0 + 16 * c + l16;
+      C[c][r] = zero || j >= n ? 0.0 : D[(size_t)i * n + j];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NB; k += 4) {
+    const int t = k + lq;
+    const double a = t < nb && i0 + l16 < n ? pan[(size_t)t * n + i0 + l16] : 0.0;
+    const double *row = D + (size_t)(t < nb ? piv[t] : 0) * n;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int j = j0 + 16 * c + l16;
+      const double d = t < nb && j < n ? row[j] : 0.0;
+      C[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, d, C[c], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int i = i0 + lq + 4 * r;
+    if (i >= n) continue;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int j = j0 + 16 * c + l16;
+      if (j >= n || (j >= kb2 && j < kb2 + nb2)) continue;  // the next launch writes panel K + 1
+      O[(size_t)i * n + j] = j >= kb && j < kb + nb ? pan[(size_t)(j - kb) * n + i] : C[c][r];
     }
   }
 }
 
-__global__ void k_gj_unpermute(int n, const int *__restrict__ perm, double *__restrict__ D) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double *r = D + (size_t)i * n;
-  for (int k = n - 1; k >= 0; k--) {
-    const int p = perm[k];
-    if (p != k) {
-      const double t = r[k];
-      r[k] = r[p];
-      r[p] = t;
-    }
-  }
+// inverse[k][c] = D[pivot of k][step of c]
+__global__ __launch_bounds__(256) void k_gj_permute(int n, const int *__restrict__ piv, const int *__restrict__ stepof,
+                                                    const double *__restrict__ D, double *__restrict__ G) {
+  const int k = blockIdx.x;
+  const double *row = D + (size_t)piv[k] * n;
+  for (int c = threadIdx.x; c < n; c += 256) G[(size_t)k * n + c] = row[stepof[c]];
 }
 
 // x = D b, one wave per row
@@ -1319,42 +1420,51 @@ static int coarse_inverse(gm_ctx *c, MgLevel &L, int prec, hipStream_t s) {
     return GM_ERR_ARG;
   }
   if (L.dense_n != n) {
-    for (void *p : {(void *)L.d_dense, (void *)L.d_pcol, (void *)L.d_perm})
+    for (void *p : {(void *)L.d_dense, (void *)L.d_dense2, (void *)L.d_pcol, (void *)L.d_perm})
       if (p) (void)hipFree(p);
-    L.d_dense = L.d_pcol = nullptr;
+    L.d_dense = L.d_dense2 = L.d_pcol = nullptr;
     L.d_perm = nullptr;
     L.dense_n = 0;
-    GM_HIP(hipMalloc(&L.d_dense, (size_t)n * n * sizeof(double)));
-    GM_HIP(hipMalloc(&L.d_pcol, (size_t)GJ_NB * n * sizeof(double)));  // pivot rows B_K
-    GM_HIP(hipMalloc(&L.d_perm, (size_t)n * sizeof(int)));
+    const size_t cells = (size_t)n * n + GJ_NB;  // a margin: whole panels are read
+    GM_HIP(hipMalloc(&L.d_dense, cells * sizeof(double)));
+    GM_HIP(hipMalloc(&L.d_dense2, cells * sizeof(double)));
+    GM_HIP(hipMalloc(&L.d_pcol, (size_t)2 * GJ_NB * n * sizeof(double)));
+    GM_HIP(hipMalloc(&L.d_perm, (size_t)2 * n * sizeof(int)));
     L.dense_n = n;
   }
+  // panel width, rows per thread and threads: the panel in registers, up to 64 a thread
+  const int pw = n <= 1536 ? 16 : 8, np = (n + pw - 1) / pw;
+  const int nt = n <= 768 ? 256 : n <= 1536 ? 512 : 1024;
+  auto step = n <= 256    ? k_gjb_step<16, 1, 256>
+              : n <= 768  ? k_gjb_step<16, 3, 256>
+              : n <= 1536 ? k_gjb_step<16, 3, 512>
+                          : k_gjb_step<8, 4, 1024>;
+  static_assert(GM_MG_DIRECT_MAX <= 4096 && GJ_NB >= 16, "k_gjb_step's rows and columns");
+  // the last of the np launches that write the array writes d_dense2
+  double *from = np & 1 ? L.d_dense : L.d_dense2, *to = np & 1 ? L.d_dense2 : L.d_dense;
   const long long nn = (long long)n * n;
-  k_set<double><<<1024, 256, 0, s>>>(L.d_dense, nn, 0.0);
+  k_set<double><<<1024, 256, 0, s>>>(from, nn, 0.0);
   if (prec == GM_PREC_MIXED)
-    k_msr_to_dense<float><<<n, 64, 0, s>>>(n, (const float *)L.d_val, lc->d_bindx, L.d_dense);
+    k_msr_to_dense<float><<<n, 64, 0, s>>>(n, (const float *)L.d_val, lc->d_bindx, from);
   else
-    k_msr_to_dense<double><<<n, 64, 0, s>>>(n, (const double *)L.d_val, lc->d_bindx, L.d_dense);
+    k_msr_to_dense<double><<<n, 64, 0, s>>>(n, (const double *)L.d_val, lc->d_bindx, from);
   GM_HIP(hipMemsetAsync(c->d_flag + 3, 0, sizeof(int), s));
-  const int nt = (n + 63) / 64;
-  // panel width x rows per thread (512 threads; wider panels left the step
-  // loop partly rolled, the panel in scratch)
-  const int pw = n <= 1536 ? 16 : 8;  // 16-wide panels of more rows would spill
-  for (int kb0 = 0; kb0 < n; kb0 += pw) {
-    const int nb = std::min(pw, n - kb0);
-    // panel: read and written once; swap: the panel rows of the other columns
-    // read, written and copied; update: the matrix read and written
-    const double pb = 16.0 * n * nb, sb = 24.0 * n * nb, ub = 16.0 * (double)n * n;
-    auto panel = n <= 512 ? k_gjb_panel<16, 1> : n <= 1024 ? k_gjb_panel<16, 2>
-               : n <= 1536 ? k_gjb_panel<16, 3> : k_gjb_panel<8, 8>;
-    gm_launch(c, GM_K_COARSE_INV, pb, panel, dim3(1), dim3(512), 0, s, n, kb0, nb, L.d_dense,
-              L.d_perm, c->d_flag);
-    gm_launch(c, GM_K_COARSE_INV, sb, k_gjb_swap, dim3((n + 255) / 256), dim3(256), 0, s, n, kb0,
-              nb, L.d_dense, (const int *)L.d_perm, L.d_pcol);
-    gm_launch(c, GM_K_COARSE_INV, ub, k_gjb_update, dim3(nt, nt), dim3(256), 0, s, n, kb0, nb,
-              L.d_dense, (const double *)L.d_pcol);
+  const int tiles = ((n + 15) / 16) * ((n + 63) / 64);
+  const int blocks = (tiles + nt / 64 - 1) / (nt / 64);
+  int *piv = L.d_perm, *stepof = L.d_perm + n;
+  for (int k = -1; k < np; k++) {
+    // panel k applied to the array, panel k + 1 factored
+    const int kb = std::max(k, 0) * pw, nb = k < 0 ? 0 : std::min(pw, n - kb);
+    const int kb2 = (k + 1) * pw, nb2 = k + 1 < np ? std::min(pw, n - kb2) : 0;
+    double *p0 = L.d_pcol + (size_t)(k & 1) * GJ_NB * n, *p1 = L.d_pcol + (size_t)((k + 1) & 1) * GJ_NB * n;
+    // the array read and written, the next panel's columns
+    const double bytes = (k < 0 ? 0.0 : 16.0 * (double)nn) + 8.0 * n * nb2;
+    gm_launch(c, GM_K_COARSE_INV, bytes, step, dim3(1 + (k < 0 ? 0 : blocks)), dim3(nt), 0, s, n, kb, nb,
+              std::min(kb2, n), nb2, (const double *)from, to, (const double *)p0, p1, (const int *)(piv + kb),
+              piv + std::min(kb2, n), stepof, c->d_flag);
+    if (k >= 0) std::swap(from, to);
   }
-  k_gj_unpermute<<<(n + 255) / 256, 256, 0, s>>>(n, L.d_perm, L.d_dense);
+  k_gj_permute<<<n, 256, 0, s>>>(n, piv, stepof, L.d_dense2, L.d_dense);
   GM_HIP(hipGetLastError());
   return GM_OK;
 }
@@ -1740,7 +1850,7 @@ void gm_mg_free(gm_ctx *c) {
     void *p[] = {L.d_Prow, L.d_Pcol, L.d_Pval, L.d_Rrow, L.d_Rcol, L.d_Rval, L.d_inject,
                  L.d_state, L.d_rdummy, L.d_x, L.d_b, L.d_r, L.d_val_p[0], L.d_val_p[1],
                  L.d_ainv_p[0], L.d_ainv_p[1],
-                 L.d_dense, L.d_pcol, L.d_perm, L.d_child, L.d_Wp, L.d_Wi, L.d_Wv, L.d_Q};
+                 L.d_dense, L.d_dense2, L.d_pcol, L.d_perm, L.d_child, L.d_Wp, L.d_Wi, L.d_Wv, L.d_Q};
     for (void *q : p)
       if (q) (void)hipFree(q);
   };

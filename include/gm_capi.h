@@ -396,7 +396,7 @@ int gm_mg_copy_coarse_inverse(const gm_ctx *ctx, double *out);
 #define GM_K_BAND_SOLVE 18 /* k_band_step: 128 unknowns of one direction of the banded solve */
 #define GM_K_VANKA_GATHER 19 /* k_vanka_gather: additive smoother, element corrections summed per unknown */
 #define GM_K_ROW_SCALE 20 /* k_row_sum_scale: row sums and scaling of the Jacobian and residual */
-#define GM_K_COARSE_INV 21 /* k_gjb_panel / k_gjb_swap / k_gjb_update: one panel of the coarsest level's dense inverse */
+#define GM_K_COARSE_INV 21 /* k_gjb_step: one panel of the coarsest level's dense inverse */
 #define GM_K_COUNT 22
 /* on = 0: off; 1: time every launch; k > 1: time a pseudo-random one launch
  * in k of each kernel (lower overhead), durations scaled to all launches by

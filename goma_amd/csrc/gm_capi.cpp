@@ -109,7 +109,7 @@ static void free_ctx(gm_ctx *c) {
                   c->d_resid, c->d_dx,    c->d_scale, c->d_val32,    c->d_red,   c->d_xwork,
                   c->d_xsave, c->d_rtrial, c->d_w, c->d_mg_rows, c->d_mg_wmul, c->d_kel,
                   c->d_mg_gptr, c->d_mg_gent, c->d_mg_corr, c->d_stab, c->d_qs_ptr,
-                  c->d_qs_side, c->d_qs_q, c->d_nn_ptr, c->d_nn_list, c->d_pair,
+                  c->d_qs_side, c->d_qs_q, c->d_nn_ptr, c->d_nn_list, c->d_nn_cols, c->d_pair,
                   c->d_rank_t, c->d_src, c->d_re, c->d_ct};
   for (void *p : ptrs)
     if (p) hipFree(p);
@@ -201,12 +201,17 @@ static int create_impl(const gm_mesh *m, const gm_physics *ph, const gm_bc *bc, 
   if ((rc = upload(&c->d_dbc_val, c->dbc_val.data(), c->dbc_val.size()))) return rc;
   if ((rc = upload(&c->d_bindx, c->bindx.data(), c->bindx.size()))) return rc;
   c->nn_cap = 0;
+  std::vector<int> cols(c->nn_list.size());
   for (int n = 0; n < c->num_nodes; n++) {
     int len = 0;
-    for (int q = c->nn_ptr[n]; q < c->nn_ptr[n + 1]; q++)
-      len += c->first_unknown[c->nn_list[q] + 1] - c->first_unknown[c->nn_list[q]];
+    for (int q = c->nn_ptr[n]; q < c->nn_ptr[n + 1]; q++) {
+      const int f = c->first_unknown[c->nn_list[q]], l = c->first_unknown[c->nn_list[q] + 1] - f;
+      cols[q] = (int)((unsigned)f << 1 | (l > c->nv ? 1u : 0u));  // (N is far below 2^30: 32-bit row pointers)
+      len += l;
+    }
     c->nn_cap = std::max(c->nn_cap, len);
   }
+  if ((rc = upload(&c->d_nn_cols, cols.data(), cols.size()))) return rc;
   if ((rc = upload(&c->d_nn_ptr, c->nn_ptr.data(), c->nn_ptr.size()))) return rc;
   if ((rc = upload(&c->d_nn_list, c->nn_list.data(), c->nn_list.size()))) return rc;
   if ((rc = upload(&c->d_ecol_elems, c->ecol_elems.data(), c->ecol_elems.size()))) return rc;

@@ -174,6 +174,7 @@ struct gm_ctx {
   double *d_dbc_val = nullptr;
   int *d_bindx = nullptr;
   int *d_nn_ptr = nullptr, *d_nn_list = nullptr;  // node-node graph (the row kernels' runs)
+  int *d_nn_cols = nullptr;  // per neighbour: twice its first unknown, plus 1 with P unknowns
   int nn_cap = 0;  // longest column pattern of a node (sum of its neighbours' unknowns)
   int *d_ecol_elems = nullptr;
   int *d_e2nz = nullptr;        // [num_elems * lay.total]

@@ -56,113 +56,169 @@ __device__ inline double row_ror_f(double v) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
+// inclusive prefix sum over the wave (DPP row shifts, then the row totals)
+__device__ inline int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, true);   // row_bcast:15
+  return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, true);  // row_bcast:31
+}
+
 // The rows of the MSR matrix one node at a time, without reading a column
 // index per nonzero.  Row u of node n holds, for every neighbour node m of n
 // in ascending order (n itself included), the unknowns of m in ascending
 // order, minus the P columns in an energy row (the interaction mask) and
 // minus u itself (the diagonal, stored apart): the order
 // find_MSR_problem_graph builds (src/mm_fill_util.c:3229-3445).  One wave per
-// node writes the node's column pattern to LDS from its neighbour list (one
-// lane per neighbour, offsets by a wave prefix sum of the neighbours'
-// unknown counts): PA for rows that take every column, PT for the energy
-// row.  It then takes the node's rows four at a time, 16 lanes (one DPP row)
-// per row, with coalesced value loads (two entries per lane and step) and a
-// reduction by DPP row rotations; entry e of row r is pattern position e, or
-// e + 1 from the diagonal's position on.  The node graph costs 4 bytes per
-// neighbour for all the node's rows instead of 4 bytes per nonzero.
-// Measured at 48^3 HEX27: 2.05 ms per product (4.05 TB/s algorithmic), the
-// multigrid residual 0.596 ms averaged over the levels (4.0 TB/s).  Slower
-// variants: the node's rows in turn with 64 lanes each (2.49 ms: one row's
-// loads in flight at a time), 64 lanes per row with the column list (2.85),
-// four accumulators per lane (2.10), a workgroup per node with wave 0
-// building the pattern and a row per wave (3.39), the node's rows walked as
-// one block with per-entry row selection (3.55).  `cap` is the longest
-// pattern of the mesh (LDS: 2 cap ints per wave).  RESID: y = b - A x;
-// otherwise y = A x.
+// node copies the vector's entries at the node's columns to LDS from its
+// neighbour list (one lane per neighbour, offsets by a wave prefix sum of the
+// neighbours' unknown counts), with the energy row's places among them.  It
+// then takes the node's rows four at a time, 16 lanes (one DPP row) per row,
+// two neighbouring entries per lane and load, and a reduction by DPP row
+// rotations; entry e of row r is place e, or e + 1 from the diagonal's place
+// on.  The node graph costs 4 bytes per neighbour for all the node's rows
+// instead of 4 bytes per nonzero, and a vector entry is gathered once per node.
+// Bound by the values' bytes, and for small rows by the chain of loads that ends
+// in them: the first values leave before the neighbour list is read, up to
+// four loads of 16 bytes (FP32: 8) per lane stay in flight, and the list holds
+// the neighbours' first columns, so nothing is looked up per neighbour.  19^3
+// with energy, FP64: 116 us (4.3 TB/s of 5.1 a copy reaches) against 140 with
+// column places in LDS, one gather per nonzero and two 8-byte loads in flight;
+// 24^3, FP32 values: 169 against 197.  16-byte loads of FP32 values are slower
+// (209: the rows' ragged ends).  Slower at 48^3 in the older form: the node's
+// rows in turn with 64 lanes each (one row's loads in flight at a time), 64
+// lanes per row with the column list, a workgroup per node with a row per
+// wave, the node's rows walked as one block with per-entry row selection.
+// `cap` is the longest pattern of the mesh (LDS: cap + 1 entries and places
+// per wave).  RESID: y = b - A x; otherwise y = A x.
 template <typename AT, typename VT, typename XT, typename YT, bool RESID>
 __global__ __launch_bounds__(256) void k_msr_nodes(int num_nodes, int dim, int nvn, int cap,
                                                    const int *__restrict__ fu,
                                                    const int *__restrict__ nn_ptr,
-                                                   const int *__restrict__ nn_list,
+                                                   const int *__restrict__ nn_cols,
                                                    const int *__restrict__ bindx,
                                                    const VT *__restrict__ a,
                                                    const XT *__restrict__ x,
                                                    const XT *__restrict__ b, YT *__restrict__ y) {
-  extern __shared__ int s_pat[];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n = xcd_block() * (blockDim.x >> 6) + w;
+  constexpr int U = 4, MAXU = 8;  // loads in flight; unknowns of a node (HEX27: 4 nodal, 4 of P)
+  typedef VT Two __attribute__((ext_vector_type(2), aligned(sizeof(VT))));
+  extern __shared__ double s_pat[];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  const int n = xcd_block() * nw + w;
   const bool valid = n < num_nodes;
-  int *PA = s_pat + (size_t)w * 2 * cap, *PT = PA + cap;
-  int f0 = 0, nu = 0, selfA = 0, selfT = 0;
+  AT *X = (AT *)s_pat + (size_t)w * (cap + 1);
+  unsigned short *PT = (unsigned short *)((AT *)s_pat + (size_t)nw * (cap + 1)) + (size_t)w * (cap + 1);
+  const int g = lane >> 4, l = lane & 15;
+  int f0 = 0, nu = 0, selfA = 0, selfT = 0, endA = 0, endT = 0, k0 = 0, len = 0;
+  Two v[U];
+  // entries 2 l + 32 i, + 1 of this lane's row, from entry e0 on
+  auto fetch = [&](int e0) {
+#pragma unroll
+    for (int i = 0; i < U; i++) {
+      const int e = e0 + 32 * i + 2 * l;
+      v[i] = Two{0, 0};
+      if (e + 1 < len) v[i] = *(const Two *)(a + k0 + e);
+      else if (e < len) v[i][0] = a[k0 + e];
+    }
+  };
+  auto open = [&](int r) {  // the row's place in the matrix, its first loads
+    k0 = len = 0;
+    if (r < nu) {
+      k0 = bindx[f0 + r];
+      len = bindx[f0 + r + 1] - k0;
+    }
+    fetch(0);
+  };
   if (valid) {
     f0 = fu[n];
     nu = fu[n + 1] - f0;
     const int j0 = nn_ptr[n], nb = nn_ptr[n + 1] - j0;
-    int carryA = 0, carryT = 0;
+    int first = lane < nb ? nn_cols[j0 + lane] : -2;
+    open(g);
+    int carry = 0;  // places so far: of all columns, and in the high half of the energy row's
     for (int c0 = 0; c0 < nb; c0 += 64) {
-      const int jj = c0 + lane;
-      int m = -1, fm = 0, lm = 0;
-      if (jj < nb) {
-        m = nn_list[j0 + jj];
-        fm = fu[m];
-        lm = fu[m + 1] - fm;
-      }
-      const int lenT = lm < nvn ? lm : nvn;
-      int incA = lm, incT = lenT;
+      // first column of the neighbour, twice, plus 1 when it has P columns
+      if (c0) first = c0 + lane < nb ? nn_cols[j0 + c0 + lane] : -2;
+      const int fm = first >> 1, lenT = first >= 0 ? nvn : 0, lm = lenT + (first > 0 ? (first & 1) * (dim + 1) : 0);
+      const int own = lm | lenT << 16;
+      XT xm[MAXU];
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int tA = __shfl_up(incA, o), tT = __shfl_up(incT, o);
-        if (lane >= o) {
-          incA += tA;
-          incT += tT;
-        }
+      for (int q = 0; q < MAXU; q++) xm[q] = q < lm ? x[fm + q] : (XT)0;
+      const int inc = wave_scan(own), off = carry + inc - own, offA = off & 0xffff, offT = off >> 16;
+#pragma unroll
+      for (int q = 0; q < MAXU; q++) {
+        if (q < lm) X[offA + q] = (AT)xm[q];
+        if (q < lenT) PT[offT + q] = (unsigned short)(offA + q);
       }
-      const int offA = carryA + incA - lm, offT = carryT + incT - lenT;
-      for (int q = 0; q < lm; q++) PA[offA + q] = fm + q;
-      for (int q = 0; q < lenT; q++) PT[offT + q] = fm + q;
-      const unsigned long long sb = __ballot(m == n);
+      const unsigned long long sb = __ballot(fm == f0);
       if (sb) {
-        const int sl = __builtin_ctzll(sb);
-        selfA = __shfl(offA, sl);
-        selfT = __shfl(offT, sl);
+        const int so = __shfl(off, __builtin_ctzll(sb));
+        selfA = so & 0xffff;
+        selfT = so >> 16;
       }
-      carryA += __shfl(incA, 63);
-      carryT += __shfl(incT, 63);
+      carry += __shfl(inc, 63);
+    }
+    // a zero past the end, for the last loads' missing entries
+    endA = carry & 0xffff;
+    endT = carry >> 16;
+    if (lane == 0) {
+      X[endA] = 0;
+      PT[endT] = (unsigned short)endA;
     }
   }
-  __syncthreads();
   if (!valid) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own LDS
   const bool energy = nvn > dim;
-  // four rows at a time, 16 lanes (one DPP row) per row
-  const int g = lane >> 4, l = lane & 15;
   for (int r0 = 0; r0 < nu; r0 += 4) {
     const int r = r0 + g;
+    if (r0) open(r);
+    const bool tr = energy && r == dim;
+    const int hole = (tr ? selfT : selfA) + r, end = tr ? endT : endA;
     AT s0 = 0, s1 = 0;
-    int u = 0;
-    if (r < nu) {
-      u = f0 + r;
-      const int k0 = bindx[u], len = bindx[u + 1] - k0;
-      const bool tr = energy && r == dim;
-      const int *P = tr ? PT : PA;
-      const int hole = (tr ? selfT : selfA) + r;
-      int e = l;
-      for (; e + 16 < len; e += 32) {
-        const int e1 = e + 16;
-        s0 += (AT)a[k0 + e] * (AT)x[P[e + (e >= hole ? 1 : 0)]];
-        s1 += (AT)a[k0 + e1] * (AT)x[P[e1 + (e1 >= hole ? 1 : 0)]];
+    // the longest of the four rows, for all of them
+    int last = len;
+    last = max(last, __shfl_xor(last, 16));
+    last = max(last, __shfl_xor(last, 32));
+    for (int e0 = 0; e0 < last; e0 += 32 * U) {
+      Two c[U];
+#pragma unroll
+      for (int i = 0; i < U; i++) c[i] = v[i];
+      if (e0 + 32 * U < last) fetch(e0 + 32 * U);
+#pragma unroll
+      for (int i = 0; i < U; i++) {
+        const int e = e0 + 32 * i + 2 * l;
+        if (e0 + 32 * i >= last) break;
+        int p0 = min(e + (e >= hole ? 1 : 0), end), p1 = min(e + 1 + (e + 1 >= hole ? 1 : 0), end);
+        if (tr) {
+          p0 = PT[p0];
+          p1 = PT[p1];
+        }
+        s0 += (AT)c[i][0] * X[p0];
+        s1 += (AT)c[i][1] * X[p1];
       }
-      if (e < len) s0 += (AT)a[k0 + e] * (AT)x[P[e + (e >= hole ? 1 : 0)]];
     }
-    AT v = s0 + s1;
-    v += row_ror_f<8>(v);
-    v += row_ror_f<4>(v);
-    v += row_ror_f<2>(v);
-    v += row_ror_f<1>(v);
+    AT t = s0 + s1;
+    t += row_ror_f<8>(t);
+    t += row_ror_f<4>(t);
+    t += row_ror_f<2>(t);
+    t += row_ror_f<1>(t);
     if (l == 0 && r < nu) {
-      const AT d = (AT)a[u] * (AT)x[u];
-      y[u] = RESID ? (YT)((AT)b[u] - v - d) : (YT)(v + d);
+      const int u = f0 + r;
+      const AT d = (AT)a[u] * X[selfA + r];
+      y[u] = RESID ? (YT)((AT)b[u] - t - d) : (YT)(t + d);
     }
   }
+}
+
+// Waves per workgroup and LDS bytes of k_msr_nodes
+template <typename AT>
+static inline int gm_msr_nodes_shape(int cap, size_t *shm) {
+  const size_t wave = (size_t)(cap + 1) * (sizeof(AT) + 2);
+  const int nw = 4 * wave <= 64 * 1024 ? 4 : 2;
+  *shm = nw * wave;
+  return nw;
 }
 
 template <typename... P, typename... A>

@@ -268,9 +268,11 @@ static void spmv(gm_ctx *c, const VT *a, const XT *x, YT *y) {
     // pointers (QUAD9 rows, ~60 entries, are faster per row: 0.156 vs 0.345 ms)
     const double bytes = (double)(c->nval - 1) * sizeof(VT) +
                          4.0 * (2.0 * (c->num_nodes + 1) + c->N + c->nn_list.size()) + vec;
-    gm_launch(c, GM_K_SPMV, bytes, k_msr_nodes<AT, VT, XT, YT, false>, dim3((c->num_nodes + 3) / 4),
-              dim3(256), (size_t)4 * 2 * c->nn_cap * sizeof(int), c->stream, c->num_nodes, c->dim,
-              c->nv, c->nn_cap, c->d_fu, c->d_nn_ptr, c->d_nn_list, c->d_bindx, a, x,
+    size_t shm;
+    const int nw = gm_msr_nodes_shape<AT>(c->nn_cap, &shm);
+    gm_launch(c, GM_K_SPMV, bytes, k_msr_nodes<AT, VT, XT, YT, false>, dim3((c->num_nodes + nw - 1) / nw),
+              dim3(64 * nw), shm, c->stream, c->num_nodes, c->dim, c->nv, c->nn_cap, c->d_fu, c->d_nn_ptr, c->d_nn_cols,
+              c->d_bindx, a, x,
               (const XT *)nullptr, y);
     return;
   }

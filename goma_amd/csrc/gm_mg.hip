@@ -1666,10 +1666,11 @@ static void resid(gm_ctx *lc, hipStream_t s, const VT *a, const BT *x, const BT 
   const double bytes = (double)(lc->nval - 1) * sizeof(VT) +
                        4.0 * (2.0 * (lc->num_nodes + 1) + lc->N + lc->nn_list.size()) +
                        3.0 * lc->N * sizeof(BT);
+  size_t shm;
+  const int nw = gm_msr_nodes_shape<AT>(lc->nn_cap, &shm);
   gm_launch(g_prof_ctx, GM_K_MG_RESID, bytes, k_msr_nodes<AT, VT, BT, BT, true>,
-            dim3((lc->num_nodes + 3) / 4), dim3(256), (size_t)4 * 2 * lc->nn_cap * sizeof(int), s,
-            lc->num_nodes, lc->dim, lc->nv, lc->nn_cap, lc->d_fu, lc->d_nn_ptr, lc->d_nn_list,
-            lc->d_bindx, a, x, b, r);
+            dim3((lc->num_nodes + nw - 1) / nw), dim3(64 * nw), shm, s, lc->num_nodes, lc->dim, lc->nv,
+            lc->nn_cap, lc->d_fu, lc->d_nn_ptr, lc->d_nn_cols, lc->d_bindx, a, x, b, r);
 }
 
 template <typename VT, typename BT, int G>

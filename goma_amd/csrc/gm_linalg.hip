@@ -1104,52 +1104,127 @@ static int ilu_apply(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
                      : ilu_apply_ce<VT, RT, ZT, 4>(c, ywork, r, z);
 }
 
-// ---------------------------------------------------------------- Krylov kernels
-// partial dots: part[k*nb + blk] = sum_i V[k][i] w[i]  for k < nk; the last row
-// (k = nk) holds w.w.
-template <typename BT>
-__global__ __launch_bounds__(RED_THREADS) void k_mdot(int N, int nk, const BT *__restrict__ V,
-                                                      const BT *__restrict__ w,
-                                                      double *__restrict__ part) {
-  __shared__ double sh[RED_THREADS / 64];
-  const int nb = gridDim.x;
-  for (int k = 0; k <= nk; k++) {
-    const BT *vk = k < nk ? V + (size_t)k * N : w;
-    double s = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x)
-      s += (double)vk[i] * (double)w[i];
-    double t = block_sum(s, sh);
-    if (threadIdx.x == 0) part[(size_t)k * nb + blockIdx.x] = t;
-  }
+// The orthogonalisation of w against V[0 .. nk): three launches without the
+// host in between, each of the last two finishing the sums that the one before
+// left per block, so that nothing is copied and the host waits once an
+// iteration.  With four copies, two waits and sums over the blocks on the host
+// an iteration of 11,500 unknowns cost 85 us more; k_mdot took 20 us there with
+// one vector after the other, 5.4 with eight at a time.
+
+constexpr int DOT_T = 8;  // vectors per block of k_mdot
+
+constexpr int DOT_PARTS = 4096;  // most partial sums, tiles DOT_T chunks
+
+// chunks of the vectors for nk of them: a few hundred blocks, and not so many
+// partial sums that it takes the blocks of k_orth_update long to add them up
+static inline int mdot_chunks(int N, int nk) {
+  const int tiles = (nk + 1 + DOT_T - 1) / DOT_T;
+  return std::max(1, std::min((N + 1023) / 1024, DOT_PARTS / DOT_T / tiles));
 }
 
-// w -= sum_k h[k] V[k]; part[blk] = partial of w.w after the update
+// part[k * gridDim.x + chunk] = partial V[k].w (k < nk) and w.w (k = nk): w is
+// read once for DOT_T vectors, whose loads are in flight together
 template <typename BT>
-__global__ __launch_bounds__(RED_THREADS) void k_orth_update(int N, int nk,
-                                                             const BT *__restrict__ V,
-                                                             const double *__restrict__ h,
-                                                             BT *__restrict__ w,
-                                                             double *__restrict__ part) {
-  __shared__ double sh[RED_THREADS / 64];
-  __shared__ double s_h[128];
-  for (int k = threadIdx.x; k < nk; k += blockDim.x) s_h[k] = h[k];
+__global__ __launch_bounds__(256) void k_mdot(int N, int nk, const BT *__restrict__ V, const BT *__restrict__ w,
+                                              double *__restrict__ part) {
+  __shared__ double sh[DOT_T][4];
+  const int k0 = blockIdx.y * DOT_T, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const BT *v[DOT_T];
+  double acc[DOT_T];
+#pragma unroll
+  for (int q = 0; q < DOT_T; q++) {
+    v[q] = k0 + q < nk ? V + (size_t)(k0 + q) * N : w;
+    acc[q] = 0.0;
+  }
+#pragma unroll 2
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) {
+    const double x = (double)w[i];
+#pragma unroll
+    for (int q = 0; q < DOT_T; q++) acc[q] += (double)v[q][i] * x;
+  }
+#pragma unroll
+  for (int q = 0; q < DOT_T; q++) {
+    const double t = wave_sum(acc[q]);
+    if (lane == 0) sh[q][wv] = t;
+  }
   __syncthreads();
+  const int q = threadIdx.x;
+  if (q < DOT_T && k0 + q <= nk)
+    part[(size_t)(k0 + q) * gridDim.x + blockIdx.x] = (sh[q][0] + sh[q][1]) + (sh[q][2] + sh[q][3]);
+}
+
+// w -= sum_k h[k] V[k], h from k_mdot's partial sums (nc chunks); out (host
+// memory) = h and w.w before; wpart[block] = partial w.w after
+template <typename BT>
+__global__ __launch_bounds__(256) void k_orth_update(int N, int nk, int nc, const BT *__restrict__ V,
+                                                     const double *__restrict__ part, BT *__restrict__ w,
+                                                     double *__restrict__ wpart, double *__restrict__ out) {
+  __shared__ double sh[4], s_h[128];
+  {
+    // G neighbouring threads a sum: a power of two, as many as there are for
+    // nk + 1 >= 2 sums
+    int G = 128;
+    while (256 / G < nk + 1) G >>= 1;
+    const int k = threadIdx.x / G, l = threadIdx.x & (G - 1);
+    double s = 0.0;
+    if (k <= nk)
+      for (int c = l; c < nc; c += G) s += part[(size_t)k * nc + c];
+    if (G == 128) {  // two waves each
+      s = wave_sum(s);
+      if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+      __syncthreads();
+      if (threadIdx.x < 2) s_h[threadIdx.x] = sh[2 * threadIdx.x] + sh[2 * threadIdx.x + 1];
+      __syncthreads();
+    } else {
+      for (int o = G >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (l == 0 && k <= nk) s_h[k] = s;
+      __syncthreads();
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x <= nk) out[threadIdx.x] = s_h[threadIdx.x];
   double s = 0.0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) {
     double acc = (double)w[i];
-    for (int k = 0; k < nk; k++) acc -= s_h[k] * (double)V[(size_t)k * N + i];
+    int k = 0;
+    for (; k + DOT_T <= nk; k += DOT_T) {
+      BT t[DOT_T];
+#pragma unroll
+      for (int q = 0; q < DOT_T; q++) t[q] = V[(size_t)(k + q) * N + i];
+#pragma unroll
+      for (int q = 0; q < DOT_T; q++) acc -= s_h[k + q] * (double)t[q];
+    }
+    for (; k < nk; k++) acc -= s_h[k] * (double)V[(size_t)k * N + i];
     const BT wn = (BT)acc;
     w[i] = wn;
     s += (double)wn * (double)wn;
   }
-  double t = block_sum(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = t;
+  const double t = block_sum(s, sh);
+  if (threadIdx.x == 0) wpart[blockIdx.x] = t;
 }
 
 template <typename BT>
 __global__ void k_scale_into(int N, const BT *__restrict__ w, double inv, BT *__restrict__ v) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x)
     v[i] = (BT)((double)w[i] * inv);
+}
+
+// v = w / |w| (v untouched when w = 0), w.w from k_orth_update's nb partial
+// sums; out (host memory) = w.w
+template <typename BT>
+__global__ __launch_bounds__(256) void k_normalise(int N, int nb, const BT *__restrict__ w,
+                                                   const double *__restrict__ wpart, BT *__restrict__ v,
+                                                   double *__restrict__ out) {
+  __shared__ double sh[4], s_ww;
+  const double t = block_sum((int)threadIdx.x < nb ? wpart[threadIdx.x] : 0.0, sh);
+  if (threadIdx.x == 0) {
+    s_ww = t;
+    if (blockIdx.x == 0) *out = t;
+  }
+  __syncthreads();
+  const double hn = sqrt(s_ww);
+  if (hn == 0.0) return;
+  const double inv = 1.0 / hn;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) v[i] = (BT)((double)w[i] * inv);
 }
 
 // u = sum_k y[k] V[k]
@@ -1201,7 +1276,7 @@ static int sum_parts(gm_ctx *c, const double *d_part, int rows, int nb, double *
   return GM_OK;
 }
 
-static constexpr int KB = 256;  // blocks of the Krylov reductions
+static constexpr int KB = 256;  // blocks of the Krylov reductions (k_normalise: a thread each)
 
 static int ensure_krylov(gm_ctx *c, int m, int prec) {
   KrylovWork &K = c->kry;
@@ -1225,7 +1300,7 @@ static int ensure_krylov(gm_ctx *c, int m, int prec) {
   }
   GM_HIP(hipMalloc(&K.d_w, N * sizeof(double)));
   GM_HIP(hipMalloc(&K.d_z, 2 * N * sizeof(double)));
-  GM_HIP(hipMalloc(&K.d_part, (size_t)(m + 2) * KB * sizeof(double)));
+  GM_HIP(hipMalloc(&K.d_part, (DOT_PARTS + KB) * sizeof(double)));  // of the projections, of the norms
   GM_HIP(hipMalloc(&K.d_h, (m + 2) * sizeof(double)));
   K.m = m;
   K.prec = prec;
@@ -1248,7 +1323,7 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
   double *ax = K.d_w;  // FP64 scratch for A x (FP64 mode reuses w after use)
   double *ax2 = K.d_z + N;
   const bool pc = o->precond != GM_PC_NONE;
-  std::vector<double> H((size_t)(m + 1) * m, 0.0), g(m + 1), cs(m), sn(m), y(m), h(m + 2), h2(m + 2);
+  std::vector<double> H((size_t)(m + 1) * m, 0.0), g(m + 1), cs(m), sn(m), y(m), h(m + 2);
   const int grid = 2048;
 
   auto precond = [&](const BT *in, BT *out) {
@@ -1262,6 +1337,22 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
     } else {
       k_scale_into<BT><<<grid, 256, 0, c->stream>>>(N, in, 1.0, out);
     }
+  };
+
+  // w against V[0 .. j], the normalised rest in vn; the projections and w.w
+  // before it in h_red, w.w after it in ww
+  auto orthogonalise = [&](int j, BT *vn, double *ww) -> int {
+    const int nk = j + 1, nc = mdot_chunks(N, nk), nb = std::min(KB, (N + 255) / 256);
+    double *wpart = K.d_part + DOT_PARTS, *out = c->h_red;
+    gm_launch(c, GM_K_MDOT, (double)(nk + 1) * N * sizeof(BT), k_mdot<BT>, dim3(nc, (nk + DOT_T) / DOT_T), dim3(256), 0,
+              c->stream, N, nk, (const BT *)V, (const BT *)w, K.d_part);
+    gm_launch(c, GM_K_ORTH, (double)(nk + 2) * N * sizeof(BT), k_orth_update<BT>, dim3(nb), dim3(256), 0, c->stream, N,
+              nk, nc, (const BT *)V, (const double *)K.d_part, w, wpart, out);
+    k_normalise<BT><<<nb, 256, 0, c->stream>>>(N, nb, w, wpart, vn, out + nk + 1);
+    GM_HIP(hipGetLastError());
+    GM_HIP(hipStreamSynchronize(c->stream));
+    *ww = out[nk + 1];
+    return GM_OK;
   };
 
   // r0 = b - A x
@@ -1291,30 +1382,17 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
       BT *vj = V + (size_t)j * N, *vn = V + (size_t)(j + 1) * N;
       precond(vj, z);
       spmv<VT, BT, BT>(c, a, z, w);
-      gm_launch(c, GM_K_MDOT, (double)(j + 2) * N * sizeof(BT), k_mdot<BT>, dim3(KB),
-                dim3(RED_THREADS), 0, c->stream, N, j + 1, (const BT *)V, (const BT *)w, K.d_part);
-      GM_HIP(hipGetLastError());
-      if ((rc = sum_parts(c, K.d_part, j + 2, KB, h.data()))) return rc;
-      const double ww0 = h[j + 1];
-      GM_HIP(hipMemcpyAsync(K.d_h, h.data(), (j + 1) * sizeof(double), hipMemcpyHostToDevice, c->stream));
-      gm_launch(c, GM_K_ORTH, (double)(j + 3) * N * sizeof(BT), k_orth_update<BT>, dim3(KB),
-                dim3(RED_THREADS), 0, c->stream, N, j + 1, (const BT *)V, (const double *)K.d_h, w,
-                K.d_part);
       double ww;
-      if ((rc = sum_parts(c, K.d_part, 1, KB, &ww))) return rc;
-      if (ww < eta2 * ww0) {
-        k_mdot<BT><<<KB, RED_THREADS, 0, c->stream>>>(N, j + 1, V, w, K.d_part);
-        if ((rc = sum_parts(c, K.d_part, j + 2, KB, h2.data()))) return rc;
-        GM_HIP(hipMemcpyAsync(K.d_h, h2.data(), (j + 1) * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        k_orth_update<BT><<<KB, RED_THREADS, 0, c->stream>>>(N, j + 1, V, K.d_h, w, K.d_part);
-        if ((rc = sum_parts(c, K.d_part, 1, KB, &ww))) return rc;
-        for (int k = 0; k <= j; k++) h[k] += h2[k];
+      if ((rc = orthogonalise(j, vn, &ww))) return rc;
+      std::copy(c->h_red, c->h_red + j + 1, h.begin());
+      if (ww < eta2 * c->h_red[j + 1]) {
+        if ((rc = orthogonalise(j, vn, &ww))) return rc;
+        for (int k = 0; k <= j; k++) h[k] += c->h_red[k];
       }
       const double hn = std::sqrt(ww);
       double *hj = H.data() + (size_t)j * (m + 1);
       for (int k = 0; k <= j; k++) hj[k] = h[k];
       hj[j + 1] = hn;
-      if (hn != 0.0) k_scale_into<BT><<<grid, 256, 0, c->stream>>>(N, w, 1.0 / hn, vn);
       for (int k = 0; k < j; k++) {
         const double t0 = cs[k] * hj[k] + sn[k] * hj[k + 1];
         hj[k + 1] = -sn[k] * hj[k] + cs[k] * hj[k + 1];

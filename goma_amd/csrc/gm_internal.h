@@ -70,6 +70,7 @@ struct IluPlan {
   float *d_y32 = nullptr;
   int *d_node_first = nullptr, *d_node_last = nullptr;  // [N] node row range of each row
   int levels = 0;             // total forward levels over all patches
+  int maxrow = 0;             // longest row
   std::vector<long long> col_rows, col_nnzL, col_nnzU;  // per patch colour
   // per-patch level schedule of the factorisation
   int *d_lv_ptr = nullptr, *d_lv_nstart = nullptr, *d_lv_node = nullptr, *d_lv_rstart = nullptr;

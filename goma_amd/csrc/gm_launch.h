@@ -56,6 +56,45 @@ __device__ inline double row_ror_f(double v) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
+// maximum over the 16 lanes of a DPP row, in every lane
+__device__ inline unsigned row_max16(unsigned v) {
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));  // row_ror:8
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));
+  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false));
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
+}
+
+// the value of lane j of each DPP row of 16, in all of its lanes (row_newbcast)
+template <int j>
+__device__ inline double row_bcast_c(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  return __builtin_bit_cast(double, (unsigned long long)__builtin_amdgcn_update_dpp(0ull, b, 0x150 + j, 0xf, 0xf, true));
+}
+template <int j>
+__device__ inline float row_bcast_c(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + j, 0xf, 0xf, true));
+}
+template <typename T>
+__device__ __forceinline__ T row_bcast(T v, int j) {
+  switch (j) {
+#define GM_B(k) case k: return row_bcast_c<k>(v);
+    GM_B(0) GM_B(1) GM_B(2) GM_B(3) GM_B(4) GM_B(5) GM_B(6) GM_B(7)
+    GM_B(8) GM_B(9) GM_B(10) GM_B(11) GM_B(12) GM_B(13) GM_B(14)
+#undef GM_B
+    default: return row_bcast_c<15>(v);
+  }
+}
+
+// 1 / v to the last bit but one, 0 for 0: the hardware's estimate and two Newton
+// steps, half the chain of the correctly rounded division
+__device__ inline double reciprocal(double v) {
+  double y = __builtin_amdgcn_rcp(v);
+  y = fma(fma(-v, y, 1.0), y, y);
+  y = fma(fma(-v, y, 1.0), y, y);
+  return v != 0.0 ? y : 0.0;
+}
+__device__ inline float reciprocal(float v) { return v != 0.0f ? 1.0f / v : 0.0f; }
+
 // inclusive prefix sum over the wave (DPP row shifts, then the row totals)
 __device__ inline int wave_scan(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1

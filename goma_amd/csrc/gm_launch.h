@@ -123,17 +123,17 @@ __device__ inline int wave_scan(int v) {
 // in them: the first values leave before the neighbour list is read, up to
 // four loads of 16 bytes (FP32: 8) per lane stay in flight, and the list holds
 // the neighbours' first columns, so nothing is looked up per neighbour.  19^3
-// with energy, FP64: 116 us (4.3 TB/s of 5.1 a copy reaches) against 140 with
+// with energy, FP64: 114 us (4.3 TB/s of 5.1 a copy reaches) against 140 with
 // column places in LDS, one gather per nonzero and two 8-byte loads in flight;
-// 24^3, FP32 values: 169 against 197.  16-byte loads of FP32 values are slower
-// (209: the rows' ragged ends).  Slower at 48^3 in the older form: the node's
+// 24^3, FP32 values: 155 against 197.  Six waves per SIMD: with 86 VGPRs, five,
+// 121 us.  16-byte loads of FP32 values are slower (the rows' ragged ends).  Slower at 48^3 in the older form: the node's
 // rows in turn with 64 lanes each (one row's loads in flight at a time), 64
 // lanes per row with the column list, a workgroup per node with a row per
 // wave, the node's rows walked as one block with per-entry row selection.
 // `cap` is the longest pattern of the mesh (LDS: cap + 1 entries and places
 // per wave).  RESID: y = b - A x; otherwise y = A x.
 template <typename AT, typename VT, typename XT, typename YT, bool RESID>
-__global__ __launch_bounds__(256) void k_msr_nodes(int num_nodes, int dim, int nvn, int cap,
+__global__ __launch_bounds__(256, 6) void k_msr_nodes(int num_nodes, int dim, int nvn, int cap,
                                                    const int *__restrict__ fu,
                                                    const int *__restrict__ nn_ptr,
                                                    const int *__restrict__ nn_cols,
@@ -143,6 +143,7 @@ __global__ __launch_bounds__(256) void k_msr_nodes(int num_nodes, int dim, int n
                                                    const XT *__restrict__ b, YT *__restrict__ y) {
   constexpr int U = 4, MAXU = 8;  // loads in flight; unknowns of a node (HEX27: 4 nodal, 4 of P)
   typedef VT Two __attribute__((ext_vector_type(2), aligned(sizeof(VT))));
+  typedef XT XTwo __attribute__((ext_vector_type(2), aligned(sizeof(XT))));
   extern __shared__ double s_pat[];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
   const int n = xcd_block() * nw + w;
@@ -184,7 +185,16 @@ __global__ __launch_bounds__(256) void k_msr_nodes(int num_nodes, int dim, int n
       const int own = lm | lenT << 16;
       XT xm[MAXU];
 #pragma unroll
-      for (int q = 0; q < MAXU; q++) xm[q] = q < lm ? x[fm + q] : (XT)0;
+      for (int q = 0; q < MAXU; q += 2) {
+        xm[q] = xm[q + 1] = (XT)0;
+        if (q + 1 < lm) {
+          const XTwo t = *(const XTwo *)(x + fm + q);
+          xm[q] = t[0];
+          xm[q + 1] = t[1];
+        } else if (q < lm) {
+          xm[q] = x[fm + q];
+        }
+      }
       const int inc = wave_scan(own), off = carry + inc - own, offA = off & 0xffff, offT = off >> 16;
 #pragma unroll
       for (int q = 0; q < MAXU; q++) {
@@ -225,17 +235,21 @@ __global__ __launch_bounds__(256) void k_msr_nodes(int num_nodes, int dim, int n
 #pragma unroll
       for (int i = 0; i < U; i++) c[i] = v[i];
       if (e0 + 32 * U < last) fetch(e0 + 32 * U);
+      int p[2 * U];  // places: of all of them, then the energy row's own, then the products
 #pragma unroll
       for (int i = 0; i < U; i++) {
         const int e = e0 + 32 * i + 2 * l;
-        if (e0 + 32 * i >= last) break;
-        int p0 = min(e + (e >= hole ? 1 : 0), end), p1 = min(e + 1 + (e + 1 >= hole ? 1 : 0), end);
-        if (tr) {
-          p0 = PT[p0];
-          p1 = PT[p1];
-        }
-        s0 += (AT)c[i][0] * X[p0];
-        s1 += (AT)c[i][1] * X[p1];
+        p[2 * i] = min(e + (e >= hole ? 1 : 0), end);
+        p[2 * i + 1] = min(e + 1 + (e + 1 >= hole ? 1 : 0), end);
+      }
+      if (tr) {
+#pragma unroll
+        for (int i = 0; i < 2 * U; i++) p[i] = PT[p[i]];
+      }
+#pragma unroll
+      for (int i = 0; i < U; i++) {
+        s0 += (AT)c[i][0] * X[p[2 * i]];
+        s1 += (AT)c[i][1] * X[p[2 * i + 1]];
       }
     }
     AT t = s0 + s1;

@@ -106,90 +106,153 @@ __device__ inline void each(int m0, int n0, const d4v (&acc)[2][2], F f) {
       for (int r = 0; r < 4; r++) f(m0 + 16 * u + (lane >> 4) + 4 * r, n0 + 16 * v + (lane & 15), acc[u][v][r]);
 }
 
-// LU (no pivoting) of the 64 x 64 block s (LDS) by all 256 threads, as the
-// inverse triangles L^-1 (column-major, tri) and U^-1 (row-major, tri + 64 x
-// 64), each as its panel product reads it.  The
-// block is in registers (thread (tr, tc) of a 16 x 16 grid: rows tr + 16 a,
-// columns tc + 16 b) and both inverses grow in place: step k subtracts the
-// pivot row's multiples from the rows below it (their columns left of k hold
-// L^-1) and, right of k, from the rows above it (U^-1).  One barrier a step:
-// the pivot row and column pass through LDS, buffers alternating.
-__device__ __forceinline__ void block_triangles(const double (*s)[LDT], double *__restrict__ tri, int *flag) {
-  __shared__ double s_c[2][NB], s_r[2][NB];
-  const int tid = threadIdx.x, tr = tid & 15, tc = tid >> 4;
-  double A[4][4];
+// LU (no pivoting) of the 64 x 64 block s (LDS, overwritten) by all 256
+// threads, as the inverse triangles L^-1 (column-major, tri) and U^-1
+// (row-major, tri + 64 x 64), each as its panel product reads it.  Both
+// inverses grow in place, by blocks of 16: step K inverts the triangles of its
+// diagonal block, L_KK^-1 and U_KK^-1; multiplies its block row by the one
+// (left of K: L^-1; right: U) and its block column by the other (above: U^-1;
+// below: L); then the products of the two are subtracted below K and, right of
+// K, above it, and the row's and the column's other halves start as
+// -U_KK^-1 U_Kj and -L_iK L_KK^-1.  The block products run on the matrix cores.
+// A diagonal block is a row per lane of one wave, its 16 steps a chain of DPP
+// broadcasts without LDS or barriers: 0.11 us a step, 16 us for the block, where
+// steps through LDS with a barrier each took 0.41 (a panel's launch 33.6 us,
+// 28.8 now).
+__device__ __forceinline__ void block_triangles(double (*s)[LDT], double *__restrict__ tri, int *flag) {
+  constexpr int B = 16, LB = B + 1;
+  // block column and row of step K, the diagonal block's inverse triangles
+  __shared__ double s_f[4][B][LB], s_g[4][B][LB], s_tl[B][LB], s_tu[B][LB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  // two block products at a time: D[lq + 4 r][l16] = sum_k a[l16][k] b[k][l16]
+  auto products = [&](const double *a0, int la0, const double *b0, int lb0, const double *a1, int la1, const double *b1,
+                      int lb1, d4v &D0, d4v &D1) {
+    double x[2][4], y[2][4];
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+    for (int q = 0; q < 4; q++) {
+      const int k = 4 * q + lq;
+      x[0][q] = a0[l16 * la0 + k];
+      y[0][q] = b0[k * lb0 + l16];
+      x[1][q] = a1[l16 * la1 + k];
+      y[1][q] = b1[k * lb1 + l16];
+    }
+    D0 = D1 = d4v{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int b = 0; b < 4; b++) A[a][b] = s[tr + 16 * a][tc + 16 * b];
-  bool zero = false;
-#pragma unroll
-  for (int K = 0; K < 4; K++) {
+    for (int q = 0; q < 4; q++) {
+      D0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x[0][q], y[0][q], D0, 0, 0, 0);
+      D1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x[1][q], y[1][q], D1, 0, 0, 0);
+    }
+  };
 #pragma unroll 1
-    for (int r = 0; r < 16; r++) {
-      const int q = r & 1;
-      if (tc == r) {
+  for (int K = 0; K < 4; K++) {
+    const int k0 = B * K;
+    if (wave == 0) {
+      // every DPP row holds the block, a row per lane; a row's right part waits
+      // for its scale until the end
+      double P[B], scale = 0.0;
+      bool zero = false;
 #pragma unroll
-        for (int a = 0; a < 4; a++) s_c[q][tr + 16 * a] = A[a][K];
+      for (int j = 0; j < B; j++) P[j] = s[k0 + l16][k0 + j];
+#pragma unroll
+      for (int k = 0; k < B; k++) {
+        double piv = row_bcast(P[k], k);
+        if (piv == 0.0) {
+          zero = true;
+          piv = 1.0;
+        }
+        const double d = reciprocal(piv);
+        const bool is = l16 == k, below = l16 > k;
+        const double f = is ? 0.0 : P[k] * d, g = below ? f : 0.0;
+        scale = is ? -d : scale;
+#pragma unroll
+        for (int j = k + 1; j < B; j++) P[j] = fma(row_bcast(P[j], k), -f, P[j]);
+#pragma unroll
+        for (int j = 0; j < k; j++) P[j] = fma(row_bcast(P[j], k), -g, P[j]);
+        P[k] = is ? -1.0 : below ? -f : f;
       }
-      if (tr == r) {
+      // a DPP row stores a quarter of the columns
 #pragma unroll
-        for (int b = 0; b < 4; b++) s_r[q][tc + 16 * b] = A[K][b];
+      for (int c = 0; c < 4; c++) {
+        const int j = 4 * lq + c;
+        const double w = lq < 2 ? (lq == 0 ? P[c] : P[4 + c]) : (lq == 2 ? P[8 + c] : P[12 + c]);
+        s_tl[l16][j] = j < l16 ? w : j == l16 ? 1.0 : 0.0;
+        s_tu[l16][j] = j >= l16 ? w * scale : 0.0;
       }
-      __syncthreads();
-      double piv = s_r[q][16 * K + r];
-      if (piv == 0.0) {
-        zero = true;
-        piv = 1.0;
-      }
-      const double d = 1.0 / piv;
-      double c[4], rb[4];
+      if (zero && lane == 0) atomicOr(flag, 1);
+    }
+    __syncthreads();
+    if (wave < 3) {  // the block row and column
+      const int m = wave < K ? wave : wave + 1, m0 = B * m;
+      d4v G, F;
+      products(&s_tl[0][0], LB, &s[k0][m0], LDT, &s[m0][k0], LDT, &s_tu[0][0], LB, G, F);
 #pragma unroll
-      for (int a = 0; a < 4; a++) {
-        c[a] = s_c[q][tr + 16 * a];
-        rb[a] = s_r[q][tc + 16 * a] * d;
-      }
-      const double row = rb[K];  // the pivot row's scaled entry in column block K
-      const double lo = tc == r ? d : row, hi = tc < r ? 0.0 : lo;
-      const double own = A[K][K];
-      if (tc == r) {
-#pragma unroll
-        for (int a = 0; a < 4; a++) A[a][K] = 0.0;
-      }
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        if (a < K) {
-          A[a][K] -= c[a] * hi;
-#pragma unroll
-          for (int b = K + 1; b < 4; b++) A[a][b] -= c[a] * rb[b];
-        } else if (a > K) {
-#pragma unroll
-          for (int b = 0; b < 4; b++) A[a][b] -= c[a] * (b == K ? lo : rb[b]);
-        } else {
-          const double cl = tr > r ? c[a] : 0.0, ch = tr == r ? 0.0 : c[a];
-#pragma unroll
-          for (int b = 0; b < K; b++) A[a][b] -= cl * rb[b];
-          A[a][K] -= (tc < r ? cl : ch) * lo;
-#pragma unroll
-          for (int b = K + 1; b < 4; b++) A[a][b] -= ch * rb[b];
+      for (int r = 0; r < 4; r++) {
+        const int i = lq + 4 * r;
+        s_g[m][i][l16] = G[r];
+        s_f[m][i][l16] = F[r];
+        if (m < K) {  // final
+          s[k0 + i][m0 + l16] = G[r];
+          s[m0 + i][k0 + l16] = F[r];
         }
       }
-      if (tr == r) {
+    } else {
 #pragma unroll
-        for (int b = K + 1; b < 4; b++) A[K][b] = rb[b];
-        A[K][K] = tc < r ? own : lo;
+      for (int r = 0; r < 4; r++) {
+        const int i = lq + 4 * r;
+        s[k0 + i][k0 + l16] = i > l16 ? s_tl[i][l16] : s_tu[i][l16];
       }
     }
-  }
-  if (zero && tid == 0) atomicOr(flag, 1);
+    __syncthreads();
+    // the blocks below K and, right of K, above it; then the two halves of row
+    // and column K
+    const int nb = 3 - K, nu = 3 * nb + K * nb, nt = nu + 2 * nb;
+    auto task = [&](int t, const double *&a, const double *&b, double *&out, bool &sub) {
+      sub = t < nu;
+      int i = K, j = K;
+      if (t < 3 * nb) {
+        i = K + 1 + t / 3;
+        j = t % 3 < K ? t % 3 : t % 3 + 1;
+      } else if (t < nu) {
+        i = (t - 3 * nb) / nb;
+        j = K + 1 + (t - 3 * nb) % nb;
+      } else if (t < nu + nb) {
+        i = K + 1 + t - nu;
+      } else {
+        j = K + 1 + t - nu - nb;
+      }
+      a = i == K ? &s_tu[0][0] : &s_f[i][0][0];
+      b = j == K ? &s_tl[0][0] : &s_g[j][0][0];
+      out = &s[B * i][B * j];
+    };
+    for (int t = wave; t < nt; t += 8) {
+      const double *a[2], *b[2];
+      double *out[2];
+      bool sub[2];
+      const bool two = t + 4 < nt;
+      task(t, a[0], b[0], out[0], sub[0]);
+      task(two ? t + 4 : t, a[1], b[1], out[1], sub[1]);
+      d4v D[2];
+      products(a[0], LB, b[0], LB, a[1], LB, b[1], LB, D[0], D[1]);
 #pragma unroll
-  for (int a = 0; a < 4; a++)
+      for (int h = 0; h < 2; h++) {
+        if (h && !two) break;
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-      const int i = tr + 16 * a, j = tc + 16 * b;
-      tri[j * NB + i] = i > j ? A[a][b] : (i == j ? 1.0 : 0.0);
-      tri[NB * NB + i * NB + j] = i <= j ? A[a][b] : 0.0;
+        for (int r = 0; r < 4; r++) {
+          double *o = out[h] + (lq + 4 * r) * LDT + l16;
+          *o = (sub[h] ? *o : 0.0) - D[h][r];
+        }
+      }
     }
+    __syncthreads();
+  }
+#pragma unroll 4
+  for (int t = tid; t < NB * NB; t += 256) {
+    const int j = t >> 6, i = t & 63;
+    const double l = s[i][j], u = s[j][i];
+    tri[t] = i > j ? l : i == j ? 1.0 : 0.0;
+    tri[NB * NB + t] = j <= i ? u : 0.0;
+  }
 }
 
 // Inverse triangles of the panel at j0 (kb columns, padded with the identity).
@@ -249,7 +312,7 @@ __global__ __launch_bounds__(256) void k_band_panel(int j0, int re, int ce, int 
 // that the band's columns are read and written along their rows.  With next >
 // 0, workgroup (0, 0), whose tile holds the next panel's diagonal block, now
 // final, takes the inverse triangles of its next x next corner into
-// tri_next.  Measured at bandwidth 620 (FP64): 44 us a panel (this
+// tri_next.  Measured at bandwidth 620 (FP64): 38 us a panel (this
 // launch and k_band_panel) against 118 with an LU in LDS, two barriers a
 // column, and a thread's triangular solve per row and column.
 template <typename T>

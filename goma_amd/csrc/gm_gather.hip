@@ -100,14 +100,19 @@ __device__ inline void put_row(JT *val, int row, long long base, int fm, const d
 // nodes, eight dependent sources long, are waited for (11^3 elements with
 // energy, FP32: 70 us against 86; 16 x 16 QUAD9: 5.9 against 8.0).  The row's
 // columns of a pair stand together in the element matrices, two 16-byte reads
-// instead of a line for each: 16^3 with energy, FP64, 246 us against 300 (3.2
-// TB/s), 11^3 FP32 60 against 70.
+// instead of a line for each: 16^3 with energy, FP64, 246 us against 300, 11^3
+// FP32 60 against 70.  Pairs in ranges per XCD: two workgroups that share a
+// row's lines share an L2 (453 MB read there, 403 of them element matrices);
+// most pairs have one source, so the loop is left rolled: 230 and 52 us (3.4
+// TB/s).  Two or four pairs a thread (254, 334 us) and half a pair (273) are
+// slower.
 template <int DIM, int EN, typename JT>
 __global__ __launch_bounds__(64 * (DIM + EN)) void k_gather(GatherArgs A, JT *__restrict__ val) {
   constexpr int NVE = DIM == 2 ? 9 : 27, NP = DIM + 1, NV = DIM + EN, NVE2 = NVE * NVE, NT = 64 * NV;
   constexpr int CL = DIM == 2 ? 8 : 20;
-  if ((int)blockIdx.x >= A.nb_pairs) {
-    const int u = ((int)blockIdx.x - A.nb_pairs) * NT + threadIdx.x;
+  const int blk = xcd_block();
+  if (blk >= A.nb_pairs) {
+    const int u = (blk - A.nb_pairs) * NT + threadIdx.x;
     if (u >= A.N) return;
     const int k0 = A.gptr[u], k1 = A.gptr[u + 1];
     double s = 0.0;
@@ -117,7 +122,7 @@ __global__ __launch_bounds__(64 * (DIM + EN)) void k_gather(GatherArgs A, JT *__
     A.resid[u] += s;
     return;
   }
-  const int a = threadIdx.x >> 6, p = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int a = threadIdx.x >> 6, p = blk * 64 + (threadIdx.x & 63);
   if (p == 0 && a == 0 && A.assign) val[A.N] = (JT)0;  // the unused entry between diagonal and rows
   if (p >= A.npairs) return;
   const int4 P = A.pair[p];
@@ -132,7 +137,7 @@ __global__ __launch_bounds__(64 * (DIM + EN)) void k_gather(GatherArgs A, JT *__
 #pragma unroll
     for (int b = 0; b < NV + NP; b++) acc[b] = 0.0;
     if (!dir)
-#pragma unroll 2
+#pragma unroll 1
       for (int s = s0; s < s1; s++) {
         const int sv = A.src[s], e = sv / NVE2, t = sv - e * NVE2;
         const double *__restrict__ K = A.kel + (size_t)e * A.E, *__restrict__ B = K + (a * NVE2 + t) * NV;

@@ -1162,6 +1162,13 @@ constexpr int DOT_T = 8;  // vectors per block of k_mdot
 
 constexpr int DOT_PARTS = 4096;  // most partial sums, tiles DOT_T chunks
 
+// most blocks of k_orth_update and k_normalise, which each add up the sums
+// before them: four per CU keep enough loads in flight (4.1 million unknowns:
+// 50 and 12.8 us a call, 5.3 TB/s; 91 and 21.6 with one per CU, 60 and 14.7 with
+// two, 49 and 13.3 with eight; 986,000: 18.8 and 5.4, 29 and 6.5, 21.5 and 5.4,
+// 18.5 and 6.8)
+constexpr int ORTH_B = 1024;
+
 // chunks of the vectors for nk of them: a few hundred blocks, and not so many
 // partial sums that it takes the blocks of k_orth_update long to add them up
 static inline int mdot_chunks(int N, int nk) {
@@ -1262,7 +1269,9 @@ __global__ __launch_bounds__(256) void k_normalise(int N, int nb, const BT *__re
                                                    const double *__restrict__ wpart, BT *__restrict__ v,
                                                    double *__restrict__ out) {
   __shared__ double sh[4], s_ww;
-  const double t = block_sum((int)threadIdx.x < nb ? wpart[threadIdx.x] : 0.0, sh);
+  double p = 0.0;
+  for (int c = threadIdx.x; c < nb; c += 256) p += wpart[c];
+  const double t = block_sum(p, sh);
   if (threadIdx.x == 0) {
     s_ww = t;
     if (blockIdx.x == 0) *out = t;
@@ -1323,7 +1332,7 @@ static int sum_parts(gm_ctx *c, const double *d_part, int rows, int nb, double *
   return GM_OK;
 }
 
-static constexpr int KB = 256;  // blocks of the Krylov reductions (k_normalise: a thread each)
+static constexpr int KB = 256;  // blocks of the Krylov reductions
 
 static int ensure_krylov(gm_ctx *c, int m, int prec) {
   KrylovWork &K = c->kry;
@@ -1347,7 +1356,7 @@ static int ensure_krylov(gm_ctx *c, int m, int prec) {
   }
   GM_HIP(hipMalloc(&K.d_w, N * sizeof(double)));
   GM_HIP(hipMalloc(&K.d_z, 2 * N * sizeof(double)));
-  GM_HIP(hipMalloc(&K.d_part, (DOT_PARTS + KB) * sizeof(double)));  // of the projections, of the norms
+  GM_HIP(hipMalloc(&K.d_part, (DOT_PARTS + ORTH_B) * sizeof(double)));  // of the projections, of the norms
   GM_HIP(hipMalloc(&K.d_h, (m + 2) * sizeof(double)));
   K.m = m;
   K.prec = prec;
@@ -1389,7 +1398,7 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
   // w against V[0 .. j], the normalised rest in vn; the projections and w.w
   // before it in h_red, w.w after it in ww
   auto orthogonalise = [&](int j, BT *vn, double *ww) -> int {
-    const int nk = j + 1, nc = mdot_chunks(N, nk), nb = std::min(KB, (N + 255) / 256);
+    const int nk = j + 1, nc = mdot_chunks(N, nk), nb = std::min(ORTH_B, (N + 255) / 256);
     double *wpart = K.d_part + DOT_PARTS, *out = c->h_red;
     gm_launch(c, GM_K_MDOT, (double)(nk + 1) * N * sizeof(BT), k_mdot<BT>, dim3(nc, (nk + DOT_T) / DOT_T), dim3(256), 0,
               c->stream, N, nk, (const BT *)V, (const BT *)w, K.d_part);

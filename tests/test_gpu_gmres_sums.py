@@ -53,3 +53,10 @@ def test_residual_is_the_minimum(n, ks, oracle_mod):
         own = np.linalg.norm(b - A @ xd.cpu().numpy()) / np.linalg.norm(b)
         assert abs(rel - want) <= 1e-9 * want and abs(own - want) <= 1e-9 * want
     ctx.close()
+
+
+# more blocks of the update than threads that add up its norms (433), and the
+# most blocks there are (1024 for 282,882 unknowns)
+@pytest.mark.parametrize("n", [100, 160])
+def test_many_blocks(n, oracle_mod):
+    test_residual_is_the_minimum(n, (2, 9), oracle_mod)

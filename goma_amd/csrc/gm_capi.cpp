@@ -586,8 +586,8 @@ static int solve_impl(gm_ctx *c, double *x, const gm_solver_opts *o, gm_newton_r
   *stalled = false;
   std::memset(rep, 0, sizeof(*rep));
   const int prec = o->precision;
-  int rc = ensure_newton_buffers(c, prec);
-  if (rc) return rc;
+  int rc = gm_kspace_check(o);
+  if (rc || (rc = ensure_newton_buffers(c, prec))) return rc;
   const double t0 = now_s();
   int converged = 0, inewton = 0;
   bool have_pc = false, last_ok = true;  // preconditioner reuse state

@@ -10,6 +10,7 @@
 #include "../../include/gm_capi.h"
 
 #define GM_QS_MAX 5 /* QSIDE / QCONV side entries per element */
+#define GM_KSPACE_MAX 4094 /* longest GMRES restart cycle (sums of k_orth_update in LDS) */
 #define GM_MAXROW 1024 /* longest Jacobian row (HEX27 vertex row: 125 nodes x 4 + 8 x 4 P = 532) */
 
 void gm_set_error(const char *fmt, ...);
@@ -275,6 +276,7 @@ int gm_lin3(gm_ctx *c, double *out, double w0, const double *v0, double w1, cons
 int gm_dot(gm_ctx *c, const double *a, const double *b, double *out);
 int gm_ilu_plan(gm_ctx *c, int bins);
 int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec);
+int gm_kspace_check(const gm_solver_opts *o);  // GM_ERR_ARG for a restart length out of range
 int gm_gmres_run(gm_ctx *c, const double *val, const float *val32, const double *b, double *x,
                  const gm_solver_opts *o, int *its, double *relres);
 int gm_gmres_run_nofactor(gm_ctx *c, const double *val, const float *val32, const double *b,

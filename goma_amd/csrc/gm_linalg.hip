@@ -1161,6 +1161,7 @@ static int ilu_apply(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
 constexpr int DOT_T = 8;  // vectors per block of k_mdot
 
 constexpr int DOT_PARTS = 4096;  // most partial sums, tiles DOT_T chunks
+static_assert(GM_KSPACE_MAX + 1 <= DOT_PARTS, "a partial sum for every vector and for w.w");
 
 // most blocks of k_orth_update and k_normalise, which each add up the sums
 // before them: four per CU keep enough loads in flight (4.1 million unknowns:
@@ -1208,17 +1209,19 @@ __global__ __launch_bounds__(256) void k_mdot(int N, int nk, const BT *__restric
 }
 
 // w -= sum_k h[k] V[k], h from k_mdot's partial sums (nc chunks); out (host
-// memory) = h and w.w before; wpart[block] = partial w.w after
+// memory) = h and w.w before; wpart[block] = partial w.w after.  LDS: nk + 1
+// sums (any nk up to GM_KSPACE_MAX, 32 KB).
 template <typename BT>
 __global__ __launch_bounds__(256) void k_orth_update(int N, int nk, int nc, const BT *__restrict__ V,
                                                      const double *__restrict__ part, BT *__restrict__ w,
                                                      double *__restrict__ wpart, double *__restrict__ out) {
-  __shared__ double sh[4], s_h[128];
+  __shared__ double sh[4];
+  extern __shared__ double s_h[];
   {
     // G neighbouring threads a sum: a power of two, as many as there are for
-    // nk + 1 >= 2 sums
+    // nk + 1 >= 2 sums, one from 129 sums on, which then go round by 256
     int G = 128;
-    while (256 / G < nk + 1) G >>= 1;
+    while (G > 1 && 256 / G < nk + 1) G >>= 1;
     const int k = threadIdx.x / G, l = threadIdx.x & (G - 1);
     double s = 0.0;
     if (k <= nk)
@@ -1232,10 +1235,16 @@ __global__ __launch_bounds__(256) void k_orth_update(int N, int nk, int nc, cons
     } else {
       for (int o = G >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
       if (l == 0 && k <= nk) s_h[k] = s;
+      for (int q = 256 + threadIdx.x; q <= nk; q += 256) {
+        s = 0.0;
+        for (int c = 0; c < nc; c++) s += part[(size_t)q * nc + c];
+        s_h[q] = s;
+      }
       __syncthreads();
     }
   }
-  if (blockIdx.x == 0 && threadIdx.x <= nk) out[threadIdx.x] = s_h[threadIdx.x];
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k <= nk; k += 256) out[k] = s_h[k];
   double s = 0.0;
   for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) {
     double acc = (double)w[i];
@@ -1283,16 +1292,16 @@ __global__ __launch_bounds__(256) void k_normalise(int N, int nb, const BT *__re
   for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) v[i] = (BT)((double)w[i] * inv);
 }
 
-// u = sum_k y[k] V[k]
+// u = sum_k y[k] V[k]; LDS: nk coefficients
 template <typename BT>
 __global__ void k_combine(int N, int nk, const BT *__restrict__ V, const double *__restrict__ y,
                           BT *__restrict__ u) {
-  __shared__ double s_y[128];
-  for (int k = threadIdx.x; k < nk; k += blockDim.x) s_y[k] = y[k];
+  extern __shared__ double s_h[];
+  for (int k = threadIdx.x; k < nk; k += blockDim.x) s_h[k] = y[k];
   __syncthreads();
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
     double acc = 0.0;
-    for (int k = 0; k < nk; k++) acc += s_y[k] * (double)V[(size_t)k * N + i];
+    for (int k = 0; k < nk; k++) acc += s_h[k] * (double)V[(size_t)k * N + i];
     u[i] = (BT)acc;
   }
 }
@@ -1370,7 +1379,7 @@ static int ensure_krylov(gm_ctx *c, int m, int prec) {
 template <typename BT, typename VT>
 static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x,
                    const gm_solver_opts *o, int *its_out, double *relres) {
-  const int N = c->N, m = o->kspace;
+  const int N = c->N, m = std::max(1, std::min(o->kspace, o->max_its));  // longest cycle
   KrylovWork &K = c->kry;
   BT *V = sizeof(BT) == 8 ? (BT *)K.d_V : (BT *)K.d_V32;
   BT *w = sizeof(BT) == 8 ? (BT *)K.d_w : (BT *)K.d_w32;
@@ -1402,8 +1411,8 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
     double *wpart = K.d_part + DOT_PARTS, *out = c->h_red;
     gm_launch(c, GM_K_MDOT, (double)(nk + 1) * N * sizeof(BT), k_mdot<BT>, dim3(nc, (nk + DOT_T) / DOT_T), dim3(256), 0,
               c->stream, N, nk, (const BT *)V, (const BT *)w, K.d_part);
-    gm_launch(c, GM_K_ORTH, (double)(nk + 2) * N * sizeof(BT), k_orth_update<BT>, dim3(nb), dim3(256), 0, c->stream, N,
-              nk, nc, (const BT *)V, (const double *)K.d_part, w, wpart, out);
+    gm_launch(c, GM_K_ORTH, (double)(nk + 2) * N * sizeof(BT), k_orth_update<BT>, dim3(nb), dim3(256),
+              (nk + 1) * sizeof(double), c->stream, N, nk, nc, (const BT *)V, (const double *)K.d_part, w, wpart, out);
     k_normalise<BT><<<nb, 256, 0, c->stream>>>(N, nb, w, wpart, vn, out + nk + 1);
     GM_HIP(hipGetLastError());
     GM_HIP(hipStreamSynchronize(c->stream));
@@ -1473,7 +1482,7 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
       y[k] = t / H[(size_t)k * (m + 1) + k];
     }
     GM_HIP(hipMemcpyAsync(K.d_h, y.data(), j * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    k_combine<BT><<<grid, 256, 0, c->stream>>>(N, j, V, K.d_h, u);
+    k_combine<BT><<<grid, 256, j * sizeof(double), c->stream>>>(N, j, V, K.d_h, u);
     precond(u, z);
     k_add<BT><<<grid, 256, 0, c->stream>>>(N, x, z);
     spmv<VT, double, double>(c, a, x, axp);
@@ -1486,6 +1495,14 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
   *its_out = its;
   *relres = rn / r0;
   return GM_OK;
+}
+
+// A restart cycle keeps min(kspace, max_its) vectors; a length below 1 would
+// never advance.
+int gm_kspace_check(const gm_solver_opts *o) {
+  if (o->kspace >= 1 && std::min(o->kspace, o->max_its) <= GM_KSPACE_MAX) return GM_OK;
+  gm_set_error("GMRES restart length %d outside [1, %d]", o->kspace, GM_KSPACE_MAX);
+  return GM_ERR_ARG;
 }
 
 int gm_gmres_run(gm_ctx *c, const double *val, const float *val32, const double *b, double *x,
@@ -1514,8 +1531,8 @@ int gm_gmres_run(gm_ctx *c, const double *val, const float *val32, const double 
 int gm_gmres_run_nofactor(gm_ctx *c, const double *val, const float *val32, const double *b,
                           double *x, const gm_solver_opts *o, int *its, double *relres) {
   const int prec = o->precision;
-  int rc = ensure_krylov(c, o->kspace, GM_PREC_FP64);
-  if (rc) return rc;
+  int rc = gm_kspace_check(o);
+  if (rc || (rc = ensure_krylov(c, o->kspace, GM_PREC_FP64))) return rc;
   if (prec == GM_PREC_MIXED) {
     if (!val32) {
       gm_set_error("mixed precision needs FP32 Jacobian values");

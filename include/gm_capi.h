@@ -102,7 +102,8 @@ typedef struct gm_solver_opts {
   double eps_resid;    /* Normalized Residual Tolerance (Epsilon[0]) */
   double eps_corr;     /* Normalized Correction Tolerance (Epsilon[2]); >1 disables */
   double damp;         /* full-step damping factor */
-  int kspace;          /* GMRES restart length */
+  int kspace;          /* GMRES restart length: 1 to 120 in gm_gmres_dev; in Newton the
+                          longer cycle that kspace and max_its allow is at most 4094 */
   int max_its;         /* GMRES iteration limit per Newton step */
   double lin_tol;      /* ||r||/||r0|| tolerance */
   int precond;         /* GM_PC_NONE | GM_PC_ILU0 | GM_PC_MG | GM_PC_BAND */

@@ -32,6 +32,7 @@
 // (GM_ERR_PIVOT), never divided by.
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 #include "gm_launch.h"
 
@@ -476,9 +477,10 @@ __global__ __launch_bounds__(256) void k_band_copy(int n, const double *__restri
 
 }  // namespace
 
-static int band_plan(gm_ctx *c) {
+// The bandwidths of the graph.
+static void band_plan(gm_ctx *c) {
   BandLU &B = c->band;
-  if (B.kl >= 0) return GM_OK;
+  if (B.kl >= 0) return;
   int kl = 0, ku = 0;
   for (int i = 0; i < c->N; i++)
     for (int k = c->bindx[i]; k < c->bindx[i + 1]; k++) {
@@ -489,12 +491,40 @@ static int band_plan(gm_ctx *c) {
   B.kl = kl;
   B.ku = ku;
   B.ld = (long long)kl + ku + 1 + 2 * MG;
-  GM_HIP(hipMalloc(&B.d_w1, (size_t)c->N * sizeof(double)));
-  GM_HIP(hipMalloc(&B.d_w2, (size_t)c->N * sizeof(double)));
-  const size_t np = (c->N + NB - 1) / NB;
-  // (one panel beyond the last, so that an update's successor is always inside)
-  GM_HIP(hipMalloc(&B.d_tri, (np + 1) * TRI * sizeof(double)));
-  GM_HIP(hipMalloc(&B.d_ops, (np + 1) / 2 * OPS * sizeof(double)));
+}
+
+// The buffers that a factorisation in precision pi still needs, all of them or,
+// when one does not fit, none.
+static int band_buffers(gm_ctx *c, int pi) {
+  BandLU &B = c->band;
+  const size_t N = c->N, np = (N + NB - 1) / NB;
+  struct {
+    void **p;
+    size_t bytes;
+  } need[] = {{&B.d_ab[pi], N * B.ld * (pi ? sizeof(float) : sizeof(double))},
+              {(void **)&B.d_w1, N * sizeof(double)},
+              {(void **)&B.d_w2, N * sizeof(double)},
+              // (one panel beyond the last, so that an update's successor is always inside)
+              {(void **)&B.d_tri, (np + 1) * TRI * sizeof(double)},
+              {(void **)&B.d_ops, (np + 1) / 2 * OPS * sizeof(double)}};
+  std::vector<void **> made;
+  for (auto &q : need) {
+    if (*q.p) continue;
+    if (hipMalloc(q.p, q.bytes) == hipSuccess) {
+      made.push_back(q.p);
+      continue;
+    }
+    (void)hipGetLastError();
+    *q.p = nullptr;
+    for (void **m : made) {
+      (void)hipFree(*m);
+      *m = nullptr;
+    }
+    double total = 0.0;
+    for (auto &r : need) total += *r.p ? 0.0 : (double)r.bytes;
+    gm_set_error("banded LU needs %.1f GB (N %d, bandwidths %d / %d)", total / 1e9, c->N, B.kl, B.ku);
+    return GM_ERR_ARG;
+  }
   return GM_OK;
 }
 
@@ -543,21 +573,11 @@ static int band_factor_t(gm_ctx *c, const VT *val, T *ab) {
 }
 
 int gm_band_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
-  int rc = band_plan(c);
-  if (rc) return rc;
+  band_plan(c);
   BandLU &B = c->band;
   const int pi = prec == GM_PREC_MIXED ? 1 : 0;
-  const size_t es = pi ? sizeof(float) : sizeof(double);
-  if (!B.d_ab[pi]) {
-    const hipError_t e = hipMalloc(&B.d_ab[pi], (size_t)c->N * B.ld * es);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      B.d_ab[pi] = nullptr;
-      gm_set_error("banded LU needs %.1f GB (N %d, bandwidths %d / %d)",
-                   (double)c->N * B.ld * es / 1e9, c->N, B.kl, B.ku);
-      return GM_ERR_ARG;
-    }
-  }
+  const int rc = band_buffers(c, pi);
+  if (rc) return rc;
   B.prec = pi;
   if (pi) {
     if (!val32) {

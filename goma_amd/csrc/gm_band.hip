@@ -22,14 +22,19 @@
 //   k_band_panel   L21 = A21 U11^-1 and U12 = L11^-1 A12, a 64 x 64 tile each;
 //   k_band_update  A22 -= L21 U12 by 64 x 64 tiles.
 // The chain of panels bounds it for bandwidths of a few thousand, and in it
-// the diagonal block.  (The inverse of the whole block in place of its
-// triangles saves the panel launch, but costs a digit and a half: relative
-// residual 5.9e-10 against 7e-11 on a shear-thinning 8 x 8 case, 1.7e-11 with
-// scalar triangular solves.)
+// the diagonal block.
 // Solve: forward and backward by pairs of panels (SB = 128 unknowns), whose
 // operators k_band_ops forms for all pairs at once after the factorisation;
 // one launch per pair and direction.  Zero pivots are reported
 // (GM_ERR_PIVOT), never divided by.
+// Where a diagonal block's triangles are ill-conditioned (saddle points),
+// products with their inverses leave more than triangular substitution does, so
+// an FP64 solve is refined once against the matrix.  Relative residual of one
+// solve, geometric means of six states, substitution / inverses / inverses
+// refined: 8 x 8 shear-thinning 5.6e-12 / 2.5e-11 / 4.2e-14, 3^3 cavity
+// 1.4e-12 / 1.6e-11 (one state 1000 times the substitution's) / 1.9e-15, 32 x 32
+// shear-thinning 6.7e-13 / 6.2e-13 / 5.1e-14.  Newton on the 40 x 40
+// shear-thinning case: 690 / 204 / 250 ms.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -475,6 +480,11 @@ __global__ __launch_bounds__(256) void k_band_copy(int n, const double *__restri
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) b[i] = a[i];
 }
 
+// r = a + f b
+__global__ __launch_bounds__(256) void k_band_sum(int n, const double *a, double f, const double *b, double *r) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) r[i] = a[i] + f * b[i];
+}
+
 }  // namespace
 
 // The bandwidths of the graph.
@@ -504,6 +514,7 @@ static int band_buffers(gm_ctx *c, int pi) {
   } need[] = {{&B.d_ab[pi], N * B.ld * (pi ? sizeof(float) : sizeof(double))},
               {(void **)&B.d_w1, N * sizeof(double)},
               {(void **)&B.d_w2, N * sizeof(double)},
+              {(void **)&B.d_ax, N * sizeof(double)},
               // (one panel beyond the last, so that an update's successor is always inside)
               {(void **)&B.d_tri, (np + 1) * TRI * sizeof(double)},
               {(void **)&B.d_ops, (np + 1) / 2 * OPS * sizeof(double)}};
@@ -579,6 +590,7 @@ int gm_band_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
   const int rc = band_buffers(c, pi);
   if (rc) return rc;
   B.prec = pi;
+  B.fresh = true;
   if (pi) {
     if (!val32) {
       gm_set_error("mixed precision needs FP32 Jacobian values");
@@ -589,13 +601,13 @@ int gm_band_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
   return band_factor_t<double, double>(c, val, (double *)B.d_ab[0]);
 }
 
+// out = (L U)^-1 w1, through w2; w1 is overwritten
 template <typename T>
-static void band_apply_t(gm_ctx *c, const T *ab, const double *in, double *out) {
+static void band_solve(gm_ctx *c, const T *ab, double *out) {
   BandLU &B = c->band;
   const int N = c->N, kl = B.kl, ku = B.ku;
   const long long off = MG + ku, lda = B.ld - 1;
   hipStream_t s = c->stream;
-  k_band_copy<<<1024, 256, 0, s>>>(N, in, B.d_w1);
   const int ns = (N + SB - 1) / SB;
   for (int b = 0; b < ns; b++) {
     const int s0 = b * SB, R = std::max(0, std::min(kl, N - s0 - SB));
@@ -611,21 +623,39 @@ static void band_apply_t(gm_ctx *c, const T *ab, const double *in, double *out) 
   }
 }
 
-int gm_band_apply(gm_ctx *c, const double *in, double *out) {
+// out = M^-1 in.  val: the FP64 matrix that was factored, or null.  With it the
+// solve is refined once: the inverse triangles leave 1.2 to 12 times the
+// residual of triangular substitution, a step of refinement the rounding of
+// A x itself.  FP32 factors are not refined: their rounding outweighs the
+// inverses', which are FP64.
+int gm_band_apply(gm_ctx *c, const double *val, const double *in, double *out) {
   BandLU &B = c->band;
   if (B.prec < 0 || !B.d_ab[B.prec]) {
     gm_set_error("banded LU not factored");
     return GM_ERR_ARG;
   }
-  if (B.prec == 1) band_apply_t<float>(c, (const float *)B.d_ab[1], in, out);
-  else band_apply_t<double>(c, (const double *)B.d_ab[0], in, out);
+  hipStream_t s = c->stream;
+  k_band_copy<<<1024, 256, 0, s>>>(c->N, in, B.d_w1);
+  if (B.prec == 1) {
+    band_solve<float>(c, (const float *)B.d_ab[1], out);
+  } else {
+    const double *ab = (const double *)B.d_ab[0];
+    band_solve<double>(c, ab, out);
+    if (val && B.fresh) {
+      const int rc = gm_spmv_launch(c, val, out, B.d_ax);
+      if (rc) return rc;
+      k_band_sum<<<1024, 256, 0, s>>>(c->N, in, -1.0, B.d_ax, B.d_w1);
+      band_solve<double>(c, ab, B.d_ax);
+      k_band_sum<<<1024, 256, 0, s>>>(c->N, out, 1.0, B.d_ax, out);
+    }
+  }
   GM_HIP(hipGetLastError());
   return GM_OK;
 }
 
 void gm_band_free(gm_ctx *c) {
   BandLU &B = c->band;
-  void *p[] = {B.d_ab[0], B.d_ab[1], B.d_w1, B.d_w2, B.d_tri, B.d_ops};
+  void *p[] = {B.d_ab[0], B.d_ab[1], B.d_w1, B.d_w2, B.d_ax, B.d_tri, B.d_ops};
   for (void *q : p)
     if (q) (void)hipFree(q);
   c->band = BandLU();

@@ -662,6 +662,7 @@ static int solve_impl(gm_ctx *c, double *x, const gm_solver_opts *o, gm_newton_r
       L2_prev = L2;
       const bool rebuild = !have_pc || o->pc_reuse == 0 ||
                            (o->pc_reuse == 2 && (!last_ok || last_its > 1.5 * its_ref + 2));
+      if (!rebuild) c->band.fresh = false;
       // preconditioner set-up timed separately, then GMRES
       if (rebuild && o->precond == GM_PC_ILU0) {
         const int bins = o->patch_bins > 0 ? o->patch_bins : gm_default_bins(c);

@@ -97,7 +97,8 @@ struct BandLU {
   long long ld = 0;           // entries per stored column
   int prec = -1;              // precision of the last factorisation (0 FP64, 1 FP32)
   void *d_ab[2] = {nullptr, nullptr};  // [N][ld] per precision
-  double *d_w1 = nullptr, *d_w2 = nullptr;  // solve work vectors
+  bool fresh = false;         // the factors are those of the current matrix
+  double *d_w1 = nullptr, *d_w2 = nullptr, *d_ax = nullptr;  // solve work vectors
   double *d_tri = nullptr;   // [panels][2][64][64] inverse triangles of the diagonal blocks
   double *d_ops = nullptr;   // per pair of panels: the solve's operators (k_band_ops)
 };
@@ -293,7 +294,7 @@ void gm_mg_free(gm_ctx *c);
 
 // banded LU (gm_band.hip)
 int gm_band_factor(gm_ctx *c, const double *val, const float *val32, int prec);
-int gm_band_apply(gm_ctx *c, const double *in, double *out);
+int gm_band_apply(gm_ctx *c, const double *val, const double *in, double *out);
 void gm_band_free(gm_ctx *c);
 
 // timing helper (used through gm_launch in gm_launch.h): adds `bytes` to the

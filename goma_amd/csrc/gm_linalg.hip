@@ -1396,7 +1396,7 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
       if constexpr (sizeof(VT) == 8) gm_mg_apply_d(c, (const double *)a, (const double *)in, (double *)out, o);
       else gm_mg_apply_f(c, (const float *)a, (const double *)in, (double *)out, o);
     } else if (o->precond == GM_PC_BAND) {
-      gm_band_apply(c, (const double *)in, (double *)out);
+      gm_band_apply(c, sizeof(VT) == 8 ? (const double *)a : nullptr, (const double *)in, (double *)out);
     } else if (pc) {
       (void)ilu_apply<VT, BT, BT>(c, ywork, in, out);
     } else {

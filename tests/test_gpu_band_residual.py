@@ -1,0 +1,46 @@
+"""The banded solve's residual is that of rounding A x.
+
+One GMRES iteration preconditioned by the FP64 banded LU, on Jacobians whose
+diagonal blocks' triangles are ill-conditioned (saddle points: shear-thinning
+flow, 3D cavities) and well.  A solve refined once in working precision leaves
+at most (n + 1) eps |A||x| a row, n the row's entries; the bar is twice that,
+in the 2-norm.  Inverse triangles alone leave up to 1000 times as much.
+"""
+import numpy as np
+import pytest
+
+from goma_amd import problems
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+CASES = [("carreau2d", s, lambda s: problems.natural_convection(n=8, Ra=1e4, carreau=True, jitter=0.15, seed=s))
+         for s in range(4)]
+CASES += [("natconv2d", 0, lambda s: problems.natural_convection(n=16, Ra=1e5))]
+CASES += [("cavity3d", s, lambda s: problems.lid_cavity(n=3, Re=400.0, dim=3, energy=True, Ra=1e4)) for s in range(6)]
+
+
+@pytest.mark.parametrize("name,seed,make", CASES, ids=[f"{c[0]}-{c[1]}" for c in CASES])
+def test_residual_is_rounding(name, seed, make, oracle_mod):
+    from goma_amd import capi
+
+    prob = make(seed)
+    print(f"[case] band residual {name} seed={seed}", flush=True)
+    ctx = capi.Context(prob)
+    orc = oracle_mod.Oracle(prob)
+    x = np.random.default_rng(seed).standard_normal(orc.N) * 0.3
+    rc, r, v = orc.fill(x)
+    s = np.zeros(orc.N)
+    oracle_mod.lib().om_row_sum_scale(orc.N, v, orc.ija, r, s)
+    vd, bd = torch.from_numpy(v).cuda(), torch.from_numpy(r).cuda()
+    zd = torch.zeros(ctx.N, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    its, _ = ctx.gmres_dev(vd.data_ptr(), bd.data_ptr(), zd.data_ptr(), kspace=4, max_its=1, lin_tol=1e-30, precond=3)
+    ctx.close()
+    A = oracle_mod.msr_to_scipy(orc.ija, v, orc.N).tocsr()
+    z = zd.cpu().numpy()
+    assert its == 1
+    n = np.diff(A.indptr)
+    bar = 2 * np.finfo(float).eps * np.linalg.norm((n + 1) * (abs(A) @ abs(z) + abs(r)))
+    assert np.linalg.norm(r - A @ z) <= bar

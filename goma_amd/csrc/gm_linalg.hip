@@ -724,8 +724,7 @@ static int ilu_factor_colour(gm_ctx *c, VT *lu, int p0, int cnt) {
   // 16 waves where their rows fit (2D, HEX27), 8 beyond
   const int nw = 16 * wave <= (size_t)ILU_LDS ? 16 : 8;
   if (nw * wave > 64 * 1024)
-    GM_HIP(hipFuncSetAttribute((const void *)k_ilu_factor<VT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)(nw * wave)));
+    GM_HIP(hipFuncSetAttribute((const void *)k_ilu_factor<VT>, hipFuncAttributeMaxDynamicSharedMemorySize, ILU_LDS));
   gm_launch(c, GM_K_ILU_FACT, 0.0, k_ilu_factor<VT>, dim3(cnt), dim3(64 * nw), nw * wave, c->stream, lv_args(P), lu, p0,
             P.maxrow, c->d_flag);
   return GM_OK;
@@ -1075,6 +1074,27 @@ static void ilu_streams(gm_ctx *c, const VT *lu, int pi) {
   }
 }
 
+// the kernel of sweep u
+template <typename VT, typename RT, typename ZT, int CE>
+static auto ilu_kernel(const IluStream &T, int u) {
+  return T.halo_lds ? (u ? k_ilu_sweep<VT, RT, ZT, CE, true, true> : k_ilu_sweep<VT, RT, ZT, CE, false, true>)
+                    : (u ? k_ilu_sweep<VT, RT, ZT, CE, true, false> : k_ilu_sweep<VT, RT, ZT, CE, false, false>);
+}
+
+// Allows the sweeps the LDS they take, before the factorisation that they apply:
+// the application itself has no call that fails.  (A kernel's limit is the
+// process's: every context sets the same.)
+template <typename VT>
+static int ilu_sweep_lds(gm_ctx *c) {
+  for (int u = 0; u < 2; u++) {
+    const IluStream &T = c->ilu.sweep[u];
+    if ((size_t)T.lds_rows * sizeof(VT) <= 64 * 1024) continue;
+    auto kern = c->dim == 2 ? ilu_kernel<VT, double, double, 3>(T, u) : ilu_kernel<VT, double, double, 4>(T, u);
+    GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, ILU_LDS));
+  }
+  return GM_OK;
+}
+
 // factorise the (scaled) Jacobian; prec 0: FP64 values, 1: FP32 values
 int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
   IluPlan &P = c->ilu;
@@ -1089,6 +1109,8 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
       GM_HIP(hipMalloc(&T.d_inv[pi], (size_t)T.chunks * 64 * es));
       GM_HIP(hipMalloc(&T.d_val[pi], (size_t)T.entries * es));
     }
+  int rc = pi ? ilu_sweep_lds<float>(c) : ilu_sweep_lds<double>(c);
+  if (rc) return rc;
   GM_HIP(hipMemsetAsync(c->d_flag + 2, 0, sizeof(int), c->stream));
   if (prec == GM_PREC_MIXED) {
     if (val32) k_gather<float, float><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val32, P.d_lu32);
@@ -1099,7 +1121,7 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
   for (int col = 0; col < P.ncol; col++) {
     const int p0 = P.colour_ptr[col], cnt = P.colour_ptr[col + 1] - p0;
     if (!cnt) continue;
-    const int rc = pi ? ilu_factor_colour(c, P.d_lu32, p0, cnt) : ilu_factor_colour(c, P.d_lu, p0, cnt);
+    rc = pi ? ilu_factor_colour(c, P.d_lu32, p0, cnt) : ilu_factor_colour(c, P.d_lu, p0, cnt);
     if (rc) return rc;
   }
   if (prec == GM_PREC_MIXED) ilu_streams<float>(c, P.d_lu32, 1);
@@ -1117,16 +1139,13 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
 
 // z = M^-1 r  (r, z unpermuted)
 template <typename VT, typename RT, typename ZT, int CE>
-static int ilu_apply_ce(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
+static void ilu_apply_ce(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
   IluPlan &P = c->ilu;
   constexpr int pi = sizeof(VT) == 8 ? 0 : 1;
   for (int u = 0; u < 2; u++) {
     const IluStream &T = P.sweep[u];
-    auto kern = T.halo_lds ? (u ? k_ilu_sweep<VT, RT, ZT, CE, true, true> : k_ilu_sweep<VT, RT, ZT, CE, false, true>)
-                           : (u ? k_ilu_sweep<VT, RT, ZT, CE, true, false> : k_ilu_sweep<VT, RT, ZT, CE, false, false>);
+    auto kern = ilu_kernel<VT, RT, ZT, CE>(T, u);
     const size_t lds = (size_t)T.lds_rows * sizeof(VT);
-    if (lds > 64 * 1024)
-      GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const IluSw S{P.d_patch_row, T.d_sp, T.d_pre, T.d_idx, T.d_hptr, T.d_halo, T.d_ctl};
     for (int k = 0; k < P.ncol; k++) {
       const int col = u ? P.ncol - 1 - k : k;
@@ -1142,13 +1161,12 @@ static int ilu_apply_ce(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
                 (const int *)P.d_perm, r, ywork, z);
     }
   }
-  return GM_OK;
 }
 
 template <typename VT, typename RT, typename ZT>
-static int ilu_apply(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
-  return c->dim == 2 ? ilu_apply_ce<VT, RT, ZT, 3>(c, ywork, r, z)
-                     : ilu_apply_ce<VT, RT, ZT, 4>(c, ywork, r, z);
+static void ilu_apply(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
+  if (c->dim == 2) ilu_apply_ce<VT, RT, ZT, 3>(c, ywork, r, z);
+  else ilu_apply_ce<VT, RT, ZT, 4>(c, ywork, r, z);
 }
 
 // The orthogonalisation of w against V[0 .. nk): three launches without the
@@ -1391,17 +1409,16 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
   std::vector<double> H((size_t)(m + 1) * m, 0.0), g(m + 1), cs(m), sn(m), y(m), h(m + 2);
   const int grid = 2048;
 
-  auto precond = [&](const BT *in, BT *out) {
+  auto precond = [&](const BT *in, BT *out) -> int {
     if (o->precond == GM_PC_MG) {
-      if constexpr (sizeof(VT) == 8) gm_mg_apply_d(c, (const double *)a, (const double *)in, (double *)out, o);
-      else gm_mg_apply_f(c, (const float *)a, (const double *)in, (double *)out, o);
-    } else if (o->precond == GM_PC_BAND) {
-      gm_band_apply(c, sizeof(VT) == 8 ? (const double *)a : nullptr, (const double *)in, (double *)out);
-    } else if (pc) {
-      (void)ilu_apply<VT, BT, BT>(c, ywork, in, out);
-    } else {
-      k_scale_into<BT><<<grid, 256, 0, c->stream>>>(N, in, 1.0, out);
+      if constexpr (sizeof(VT) == 8) return gm_mg_apply_d(c, (const double *)a, (const double *)in, (double *)out, o);
+      else return gm_mg_apply_f(c, (const float *)a, (const double *)in, (double *)out, o);
     }
+    if (o->precond == GM_PC_BAND)
+      return gm_band_apply(c, sizeof(VT) == 8 ? (const double *)a : nullptr, (const double *)in, (double *)out);
+    if (pc) ilu_apply<VT, BT, BT>(c, ywork, in, out);
+    else k_scale_into<BT><<<grid, 256, 0, c->stream>>>(N, in, 1.0, out);
+    return GM_OK;
   };
 
   // w against V[0 .. j], the normalised rest in vn; the projections and w.w
@@ -1445,7 +1462,7 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
     int j;
     for (j = 0; j < m && its < o->max_its; j++) {
       BT *vj = V + (size_t)j * N, *vn = V + (size_t)(j + 1) * N;
-      precond(vj, z);
+      if ((rc = precond(vj, z))) return rc;
       spmv<VT, BT, BT>(c, a, z, w);
       double ww;
       if ((rc = orthogonalise(j, vn, &ww))) return rc;
@@ -1483,7 +1500,7 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
     }
     GM_HIP(hipMemcpyAsync(K.d_h, y.data(), j * sizeof(double), hipMemcpyHostToDevice, c->stream));
     k_combine<BT><<<grid, 256, j * sizeof(double), c->stream>>>(N, j, V, K.d_h, u);
-    precond(u, z);
+    if ((rc = precond(u, z))) return rc;
     k_add<BT><<<grid, 256, 0, c->stream>>>(N, x, z);
     spmv<VT, double, double>(c, a, x, axp);
     k_resid<BT><<<KB, RED_THREADS, 0, c->stream>>>(N, b, axp, w, K.d_part);

@@ -45,8 +45,8 @@ struct IluStream {
   int *d_src = nullptr;    // [chunks * 64 * CE] position in the factors, -1: padding
   int2 *d_node = nullptr;  // [nodes] (first row, last chunk) of each node
   int *d_hptr = nullptr, *d_halo = nullptr;  // [npatch + 1], rows outside the patch it reads
-  void *d_val[2] = {nullptr, nullptr};       // per precision: the entries, in stream order
-  void *d_inv[2] = {nullptr, nullptr};       // per precision: [chunks][8][8] inverse triangles, at last chunks
+  double *d_val = nullptr;   // the entries, in stream order
+  double *d_tri = nullptr;   // [chunks][64] the nodes' triangles, at their last chunks
   long long chunks = 0, entries = 0;
   int nodes = 0, lds_rows = 0;
   bool halo_lds = true;    // every patch's rows and halo fit in LDS
@@ -68,7 +68,6 @@ struct IluPlan {
   double *d_lu = nullptr;     // [nnz]
   float *d_lu32 = nullptr;    // [nnz] (mixed precision)
   double *d_y = nullptr;      // [N] work (permuted numbering)
-  float *d_y32 = nullptr;
   int *d_node_first = nullptr, *d_node_last = nullptr;  // [N] node row range of each row
   int levels = 0;             // total forward levels over all patches
   int maxrow = 0;             // longest row

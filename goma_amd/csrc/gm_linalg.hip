@@ -416,8 +416,96 @@ __device__ inline T sum8(T v) {
   return v;
 }
 
+// v of lane i (the same i in every lane)
+__device__ inline int lane_of(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
+__device__ inline float lane_of(float v, int i) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+}
+__device__ inline double lane_of(double v, int i) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, i);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), i);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// The place among a node's 64 values (8 or 16 lanes a row, n unknowns) where
+// its upper triangle keeps the reciprocal of diagonal k: the triangle leaves
+// them free.
+__host__ __device__ constexpr int ilu_recip_lane(int lsh, int n, int k) {
+  return lsh == 4 ? (k << 4) + 8 + k : k < n - 1 ? ((n - 1) << 3) + k : (n - 2) << 3;
+}
+
+// x of T x = t, a node's triangle: t_i, then x_i, in all of the 1 << LSH lanes
+// of row i; entry (i, k) of T in lane k of row i, unit diagonal unless UPPER.
+// In the order of the sequential algorithm: x_k leaves its row through scalar
+// registers, and every row takes its part of it (a finished row's is not read).
+// Divisions by the reciprocal and one correction, rounded as a division; the
+// reciprocals are 0 where one would leave the normal range.
+template <int LSH, bool UPPER>
+__device__ __forceinline__ double ilu_node_solve(double t, double T, int n) {
+  const int lane = threadIdx.x & 63, i = lane >> LSH;
+  double x = t;
+  if (UPPER && lane_of(T, ilu_recip_lane(LSH, n, 0)) == 0.0) {
+    for (int k = n - 1; k >= 0; k--) {
+      const double q = __shfl(t, k << LSH) / __shfl(T, (k << LSH) + k);
+      x = i == k ? q : x;
+      t -= __shfl(T, (i << LSH) + k) * q;
+    }
+    return x;
+  }
+  auto step = [&](int k) {
+    double q = lane_of(t, k << LSH);
+    if constexpr (UPPER) {
+      const double d = lane_of(T, (k << LSH) + k), r = lane_of(T, ilu_recip_lane(LSH, n, k)), q0 = q;
+      q = q0 * r;
+      q = fma(fma(-d, q, q0), r, q);
+    }
+    x = i == k ? q : x;
+    double c = row_bcast(T, k);
+    if constexpr (LSH == 3) c = (lane & 8) ? row_bcast(T, k + 8) : c;
+    t = fma(-c, q, t);
+  };
+  if constexpr (UPPER) {
+    if constexpr (LSH == 3) {  // five to eight unknowns
+      if (n > 6) {
+        if (n > 7) step(7);
+        step(6);
+      }
+      if (n > 5) step(5);
+      step(4);
+      step(3);
+      step(2);
+      step(1);
+    } else {
+      if (n > 3) step(3);
+      if (n > 2) step(2);
+      if (n > 1) step(1);
+    }
+    step(0);
+    return x;
+  } else {
+    if constexpr (LSH == 3) {
+      step(0);
+      step(1);
+      step(2);
+      step(3);
+      if (n > 5) step(4);
+      if (n > 6) {
+        step(5);
+        if (n > 7) step(6);
+      }
+    } else {
+      if (n > 1) step(0);
+      if (n > 2) step(1);
+      if (n > 3) step(2);
+    }
+    return i == n - 1 ? t : x;
+  }
+}
+
 // One triangular sweep over the patches of one colour: y = L^-1 (P b) (UPPER
 // false, L unit lower) or y = U^-1 y with the unpermuted copy in out (UPPER).
+// FP64 for the factors of either precision.
 //
 // The sweep is a chain of levels (about 65 for an 8 x 8 QUAD9 patch, 105 for
 // a 4 x 4 x 4 HEX27 one) with only a few nodes each, so it is bound by the
@@ -425,27 +513,28 @@ __device__ inline T sum8(T v) {
 // may therefore sit on that chain: the entries come from streams laid out in
 // the order they are used, one per wave, and are loaded ILU_D chunks ahead
 // into registers; the patch's rows and the rows of other patches it reads (its
-// halo) are in LDS; and a node's small triangle T is applied as its inverse,
-// already multiplied into the node's entries, T^-1 (b - B y) = T^-1 b -
-// (T^-1 B) y, where T^-1 b needs nothing of the level before.  A level is then
-// LDS reads of y, a few FMAs, one row reduction, an LDS write and a barrier.
+// halo) are in LDS; and a node's small triangle is solved in registers
+// (ilu_node_solve).  A level is then LDS reads of y, a few FMAs, one row
+// reduction, two to four dependent steps of the triangle, an LDS write and a
+// barrier.
 // A chunk is CE entries per lane of one node: four rows of 16 lanes, or eight
 // rows of 8 lanes (nodes of more than four unknowns).  LDSH: every patch's
 // halo is in LDS; otherwise a load of y may stand in the chain, and the wait
 // for it takes the loads in flight along.  A wave without a node in a level
 // only takes its barrier (ctl.z).
-// Measured on the 32 x 32 QUAD9 cavity (four patches a colour, 62 levels): 29
-// us a launch, 0.46 us a level; with the entries read through the CSR factors
-// level by level, two barriers a level and the triangle solved row after row
-// it took 226 (upper) and 190 us (lower).
-template <typename VT, typename BT, typename OT, int CE, bool UPPER, bool LDSH>
-__global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__restrict__ val,
-                                                           const VT *__restrict__ inv, int patch0,
+// Measured on the 32 x 32 QUAD9 cavity (four patches a colour, 62 levels): 35
+// us a launch forward (0.57 us a level) and 43 backward (0.70); with the entries
+// read through the CSR factors level by level, two barriers a level and the
+// triangle solved row after row through LDS it took 190 and 226.  With the
+// node's inverse triangle multiplied into its entries, 29 us; but on saddle
+// points its residual was up to 100,000 times the substitution's.
+template <typename BT, typename OT, int CE, bool UPPER, bool LDSH>
+__global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const double *__restrict__ val,
+                                                           const double *__restrict__ tri, int patch0,
                                                            const int *__restrict__ perm,
-                                                           const BT *__restrict__ b, VT *y,
+                                                           const BT *__restrict__ b, double *y,
                                                            OT *__restrict__ out) {
-  extern __shared__ __align__(16) unsigned char s_raw[];
-  VT *s_y = (VT *)s_raw;
+  extern __shared__ double s_y[];
   const int P = patch0 + blockIdx.x;
   const int r0 = S.patch_row[P], nr = S.patch_row[P + 1] - r0;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -453,7 +542,7 @@ __global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__
   const int c0 = S.sp[P * ILU_NW + w], c1 = S.sp[P * ILU_NW + w + 1];
   const int npre = S.pre[P * ILU_NW + w];
 
-  VT rv[ILU_D][CE], ri[ILU_D];
+  double rv[ILU_D][CE], rt[ILU_D];
   int rx[ILU_D][CE];
   int4 rc[ILU_D];
   // The control words go through vector registers (vz is 0, but not known to
@@ -467,12 +556,12 @@ __global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__
       rv[d][e] = val[at + 64 * e];
       rx[d][e] = S.idx[at + 64 * e];
     }
-    ri[d] = inv[(size_t)c * 64 + lane];
+    rt[d] = tri[(size_t)c * 64 + lane];
   };
 #pragma unroll
   for (int d = 0; d < ILU_D; d++) fetch(d, c0 + d);  // the streams end in ILU_D spare chunks
 
-  for (int i = tid; i < nr; i += ILU_NW * 64) s_y[i] = UPPER ? y[r0 + i] : (VT)b[perm[r0 + i]];
+  for (int i = tid; i < nr; i += ILU_NW * 64) s_y[i] = UPPER ? y[r0 + i] : (double)b[perm[r0 + i]];
   const int h0 = S.hptr[P], nh = S.hptr[P + 1] - h0;
   for (int i = tid; i < nh; i += ILU_NW * 64) s_y[nr + i] = y[S.halo[h0 + i]];
   auto level_end = [&]() {  // the solution in LDS, nothing of the loads in flight
@@ -483,7 +572,7 @@ __global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__
   level_end();
   for (int k = 0; k < npre; k++) level_end();
 
-  VT acc = 0;
+  double acc = 0;
   for (int c = c0; c < c1; c += ILU_D) {
 #pragma unroll
     for (int d = 0; d < ILU_D; d++) {
@@ -491,8 +580,10 @@ __global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__
       const int bars = __builtin_amdgcn_readfirstlane(rc[d].z);
       const int lsh = (flags & ILU_R8) ? 3 : 4;  // log2 of the lanes of a row
       const int row = flags & (ILU_FIRST - 1), k = lane & ((1 << lsh) - 1);
-      VT s = acc;
-      if (flags & ILU_FIRST) s = k < n ? ri[d] * s_y[row + k] : (VT)0;
+      const int i = lane >> lsh;
+      const double T = rt[d];
+      double s = acc;
+      if (flags & ILU_FIRST) s = k == 0 && i < n ? s_y[row + i] : 0.0;
 #pragma unroll
       for (int e = 0; e < CE; e++) {
         const int j = rx[d][e];
@@ -502,8 +593,12 @@ __global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__
       fetch(d, c + d + ILU_D);
       if (flags & ILU_LAST) {
         s = sum8(s);
-        if (lsh == 4) s += dpp_mov<0x140>(s);  // row_mirror: the other half of the 16 lanes
-        const int i = lane >> lsh;
+        if (lsh == 4) {
+          s += dpp_mov<0x140>(s);  // row_mirror: the other half of the 16 lanes
+          s = ilu_node_solve<4, UPPER>(s, T, n);
+        } else {
+          s = ilu_node_solve<3, UPPER>(s, T, n);
+        }
         if (k == 0 && i < n) s_y[row + i] = s;
       }
       for (int q = 0; q < bars; q++) level_end();
@@ -511,86 +606,56 @@ __global__ __launch_bounds__(ILU_NW * 64) void k_ilu_sweep(IluSw S, const VT *__
   }
   level_end();
   for (int i = tid; i < nr; i += ILU_NW * 64) {
-    const VT v = s_y[i];
+    const double v = s_y[i];
     y[r0 + i] = v;
     if (UPPER) out[perm[r0 + i]] = (OT)v;
   }
 }
 
-// Inverse of each node's triangle of the factors (at most 8 x 8): entry (i, k)
-// at lane k of the lanes that row i has in the node's chunks, zero outside the
-// node's rows; at its first chunk's place.  A wave per node, in FP64.
+// Each node's triangle of the factors (at most 8 x 8) as ilu_node_solve takes
+// it, at the place of the node's last chunk; a wave per node.
 template <typename VT, bool UPPER>
-__global__ __launch_bounds__(256) void k_ilu_node_inv(int nodes, const int2 *__restrict__ node,
+__global__ __launch_bounds__(256) void k_ilu_node_tri(int nodes, const int2 *__restrict__ node,
                                                       const int *__restrict__ node_last,
                                                       const int *__restrict__ rowptr,
                                                       const int *__restrict__ col,
                                                       const int *__restrict__ diag,
-                                                      const VT *__restrict__ lu, VT *__restrict__ inv) {
-  __shared__ double sm[4][8][9], sx[4][8][9];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + w, i = lane >> 3, k = lane & 7;
-  int n = 0;
-  if (t < nodes) {
-    const int nf = node[t].x;
-    n = node_last[nf] - nf + 1;
-    double v = 0.0;
-    if (i < n && k < n) {
-      const int r = nf + i, cc = nf + k, d = diag[r];
-      if (!UPPER) {
-        for (int p = d - 1; p >= rowptr[r] && col[p] >= cc; p--)
-          if (col[p] == cc) v = (double)lu[p];
-        if (i == k) v = 1.0;
-      } else {
-        for (int p = d; p < rowptr[r + 1] && col[p] <= cc; p++)
-          if (col[p] == cc) v = (double)lu[p];
-      }
-    }
-    sm[w][i][k] = v;
-    sx[w][i][k] = 0.0;
-  }
-  __syncthreads();
-  if (t < nodes && lane < n) {
-    const int c = lane;  // column c of the inverse
-    for (int a = 0; a < n; a++) {
-      const int r = UPPER ? n - 1 - a : a;
-      double s = r == c ? 1.0 : 0.0;
-      if (UPPER)
-        for (int j = r + 1; j < n; j++) s -= sm[w][r][j] * sx[w][j][c];
-      else
-        for (int j = 0; j < r; j++) s -= sm[w][r][j] * sx[w][j][c];
-      sx[w][r][c] = s / sm[w][r][r];
+                                                      const VT *__restrict__ lu, double *__restrict__ tri) {
+  const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= nodes) return;
+  const int nf = node[t].x, n = node_last[nf] - nf + 1, lsh = n > 4 ? 3 : 4;
+  const int i = lane >> lsh, k = lane & ((1 << lsh) - 1);
+  double v = 0.0;
+  if (i < n && k < n) {
+    const int r = nf + i, cc = nf + k, d = diag[r];
+    if (!UPPER) {
+      for (int p = d - 1; p >= rowptr[r] && col[p] >= cc; p--)
+        if (col[p] == cc) v = (double)lu[p];
+    } else {
+      for (int p = d; p < rowptr[r + 1] && col[p] <= cc; p++)
+        if (col[p] == cc) v = (double)lu[p];
     }
   }
-  __syncthreads();
-  if (t < nodes) {
-    const int lsh = n > 4 ? 3 : 4, row = lane >> lsh, q = lane & ((1 << lsh) - 1);
-    inv[(size_t)node[t].y * 64 + lane] = (VT)(row < 8 && q < 8 ? sx[w][row][q] : 0.0);
+  if (UPPER) {
+    bool normal = true;
+    for (int q = 0; q < n; q++) {
+      const double r = 1.0 / (double)lu[diag[nf + q]];
+      normal = normal && fabs(r) >= 0x1p-1021 && fabs(r) <= 0x1p1021;
+      if (lane == ilu_recip_lane(lsh, n, q)) v = r;
+    }
+    if (!normal)
+      for (int q = 0; q < n; q++)
+        if (lane == ilu_recip_lane(lsh, n, q)) v = 0.0;
   }
+  tri[(size_t)node[t].y * 64 + lane] = v;
 }
 
-// The factors' off-node entries in stream order, each node's rows multiplied by
-// the inverse of its triangle (zero where a chunk is padded); a wave per chunk.
-template <typename VT, int CE>
-__global__ __launch_bounds__(256) void k_ilu_pack(int chunks, const int4 *__restrict__ ctl,
-                                                  const int *__restrict__ src,
-                                                  const VT *__restrict__ lu,
-                                                  const VT *__restrict__ inv, VT *__restrict__ val) {
-  const int lane = threadIdx.x & 63;
-  for (int c = blockIdx.x * 4 + (threadIdx.x >> 6); c < chunks; c += gridDim.x * 4) {
-    const int4 ct = ctl[c];
-    const size_t at = (size_t)c * (64 * CE) + lane;
-    const int lsh = (ct.x & ILU_R8) ? 3 : 4, row = lane >> lsh, l = lane & ((1 << lsh) - 1);
-    const double iv = ct.y ? (double)inv[(size_t)ct.w * 64 + lane] : 0.0;
-#pragma unroll
-    for (int e = 0; e < CE; e++) {
-      const int k = src[at + 64 * e];
-      const double v = k >= 0 ? (double)lu[k] : 0.0;
-      double s = 0.0;
-      for (int q = 0; q < ct.y; q++) s += __shfl(iv, (row << lsh) + q) * __shfl(v, (q << lsh) + l);
-      val[at + 64 * e] = (VT)s;
-    }
-  }
+// The factors' off-node entries in stream order, zero where a chunk is padded.
+template <typename VT>
+__global__ __launch_bounds__(256) void k_ilu_pack(long long n, const int *__restrict__ src,
+                                                  const VT *__restrict__ lu, double *__restrict__ val) {
+  for (long long i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL)
+    val[i] = src[i] >= 0 ? (double)lu[src[i]] : 0.0;
 }
 
 static IluLv lv_args(const IluPlan &P) {
@@ -607,18 +672,6 @@ static IluLv lv_args(const IluPlan &P) {
   S.lv_rstart = P.d_lv_rstart;
   S.lv_row = P.d_lv_row;
   return S;
-}
-
-// v of lane i (the same i in every lane)
-__device__ inline int lane_of(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
-__device__ inline float lane_of(float v, int i) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
-}
-__device__ inline double lane_of(double v, int i) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, i);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), i);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
 // IKJ elimination of row r by the pivot rows whose column lies in [kb, ke),
@@ -741,13 +794,13 @@ __global__ void k_gather(long long n, const int *__restrict__ src, const VT *__r
 
 static void free_plan(IluPlan &P) {
   void *ptrs[] = {P.d_perm, P.d_rowptr, P.d_col, P.d_diag, P.d_src, P.d_patch_row, P.d_lu,
-                  P.d_lu32, P.d_y, P.d_y32, P.d_node_first, P.d_node_last,
+                  P.d_lu32, P.d_y, P.d_node_first, P.d_node_last,
                   P.d_lv_ptr, P.d_lv_nstart, P.d_lv_node, P.d_lv_rstart, P.d_lv_row};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (const IluStream &T : P.sweep) {
     void *q[] = {T.d_sp, T.d_pre, T.d_ctl, T.d_idx, T.d_src, T.d_node, T.d_hptr, T.d_halo,
-                 T.d_val[0], T.d_val[1], T.d_inv[0], T.d_inv[1]};
+                 T.d_val, T.d_tri};
     for (void *p : q)
       if (p) (void)hipFree(p);
   }
@@ -876,11 +929,10 @@ static int build_stream(IluPlan &P, const IluHost &H, bool upper, int CE,
           ct.x = (nf - r0) | (ch == 0 ? ILU_FIRST : 0) | (ch == nchunk[k] - 1 ? ILU_LAST : 0) |
                  (n > 4 ? ILU_R8 : 0);
           ct.y = n;
-          ct.w = at[w];
         }
         at[w] += nchunk[k];
         last[w] = at[w] - 1;
-        node[k] = make_int2(nf, last[w] + 1 - nchunk[k]);
+        node[k] = make_int2(nf, last[w]);
       }
       for (int w = 0; w < ILU_NW; w++) {
         if (last[w] < 0) pre[(size_t)p * ILU_NW + w]++;
@@ -1059,37 +1111,35 @@ int gm_ilu_plan(gm_ctx *c, int bins) {
   return GM_OK;
 }
 
-// the sweeps' streams from the factors: entries and inverse triangles
+// the sweeps' streams from the factors: entries and triangles
 template <typename VT>
-static void ilu_streams(gm_ctx *c, const VT *lu, int pi) {
+static void ilu_streams(gm_ctx *c, const VT *lu) {
   IluPlan &P = c->ilu;
   for (int u = 0; u < 2; u++) {
     IluStream &T = P.sweep[u];
-    auto kern = u ? k_ilu_node_inv<VT, true> : k_ilu_node_inv<VT, false>;
+    auto kern = u ? k_ilu_node_tri<VT, true> : k_ilu_node_tri<VT, false>;
     kern<<<(T.nodes + 3) / 4, 256, 0, c->stream>>>(T.nodes, T.d_node, P.d_node_last, P.d_rowptr,
-                                                   P.d_col, P.d_diag, lu, (VT *)T.d_inv[pi]);
-    auto pack = c->dim == 2 ? k_ilu_pack<VT, 3> : k_ilu_pack<VT, 4>;
-    pack<<<(int)std::min<long long>((T.chunks + 3) / 4, 16384), 256, 0, c->stream>>>(
-        (int)T.chunks, T.d_ctl, T.d_src, lu, (const VT *)T.d_inv[pi], (VT *)T.d_val[pi]);
+                                                   P.d_col, P.d_diag, lu, T.d_tri);
+    k_ilu_pack<VT><<<(int)std::min<long long>((T.entries + 255) / 256, 16384), 256, 0, c->stream>>>(
+        T.entries, T.d_src, lu, T.d_val);
   }
 }
 
 // the kernel of sweep u
-template <typename VT, typename RT, typename ZT, int CE>
+template <typename RT, typename ZT, int CE>
 static auto ilu_kernel(const IluStream &T, int u) {
-  return T.halo_lds ? (u ? k_ilu_sweep<VT, RT, ZT, CE, true, true> : k_ilu_sweep<VT, RT, ZT, CE, false, true>)
-                    : (u ? k_ilu_sweep<VT, RT, ZT, CE, true, false> : k_ilu_sweep<VT, RT, ZT, CE, false, false>);
+  return T.halo_lds ? (u ? k_ilu_sweep<RT, ZT, CE, true, true> : k_ilu_sweep<RT, ZT, CE, false, true>)
+                    : (u ? k_ilu_sweep<RT, ZT, CE, true, false> : k_ilu_sweep<RT, ZT, CE, false, false>);
 }
 
 // Allows the sweeps the LDS they take, before the factorisation that they apply:
 // the application itself has no call that fails.  (A kernel's limit is the
 // process's: every context sets the same.)
-template <typename VT>
 static int ilu_sweep_lds(gm_ctx *c) {
   for (int u = 0; u < 2; u++) {
     const IluStream &T = c->ilu.sweep[u];
-    if ((size_t)T.lds_rows * sizeof(VT) <= 64 * 1024) continue;
-    auto kern = c->dim == 2 ? ilu_kernel<VT, double, double, 3>(T, u) : ilu_kernel<VT, double, double, 4>(T, u);
+    if ((size_t)T.lds_rows * sizeof(double) <= 64 * 1024) continue;
+    auto kern = c->dim == 2 ? ilu_kernel<double, double, 3>(T, u) : ilu_kernel<double, double, 4>(T, u);
     GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, ILU_LDS));
   }
   return GM_OK;
@@ -1098,18 +1148,13 @@ static int ilu_sweep_lds(gm_ctx *c) {
 // factorise the (scaled) Jacobian; prec 0: FP64 values, 1: FP32 values
 int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
   IluPlan &P = c->ilu;
-  if (prec == GM_PREC_MIXED && !P.d_lu32) {
-    GM_HIP(hipMalloc(&P.d_lu32, P.nnz * sizeof(float)));
-    GM_HIP(hipMalloc(&P.d_y32, c->N * sizeof(float)));
-  }
+  if (prec == GM_PREC_MIXED && !P.d_lu32) GM_HIP(hipMalloc(&P.d_lu32, P.nnz * sizeof(float)));
   const int pi = prec == GM_PREC_MIXED ? 1 : 0;
-  const size_t es = pi ? sizeof(float) : sizeof(double);
-  for (IluStream &T : P.sweep)
-    if (!T.d_val[pi]) {
-      GM_HIP(hipMalloc(&T.d_inv[pi], (size_t)T.chunks * 64 * es));
-      GM_HIP(hipMalloc(&T.d_val[pi], (size_t)T.entries * es));
-    }
-  int rc = pi ? ilu_sweep_lds<float>(c) : ilu_sweep_lds<double>(c);
+  for (IluStream &T : P.sweep) {
+    if (!T.d_tri) GM_HIP(hipMalloc(&T.d_tri, (size_t)T.chunks * 64 * sizeof(double)));
+    if (!T.d_val) GM_HIP(hipMalloc(&T.d_val, (size_t)T.entries * sizeof(double)));
+  }
+  int rc = ilu_sweep_lds(c);
   if (rc) return rc;
   GM_HIP(hipMemsetAsync(c->d_flag + 2, 0, sizeof(int), c->stream));
   if (prec == GM_PREC_MIXED) {
@@ -1124,8 +1169,8 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
     rc = pi ? ilu_factor_colour(c, P.d_lu32, p0, cnt) : ilu_factor_colour(c, P.d_lu, p0, cnt);
     if (rc) return rc;
   }
-  if (prec == GM_PREC_MIXED) ilu_streams<float>(c, P.d_lu32, 1);
-  else ilu_streams<double>(c, P.d_lu, 0);
+  if (prec == GM_PREC_MIXED) ilu_streams<float>(c, P.d_lu32);
+  else ilu_streams<double>(c, P.d_lu);
   GM_HIP(hipGetLastError());
   int flag = 0;
   GM_HIP(hipMemcpyAsync(&flag, c->d_flag + 2, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -1138,14 +1183,13 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
 }
 
 // z = M^-1 r  (r, z unpermuted)
-template <typename VT, typename RT, typename ZT, int CE>
-static void ilu_apply_ce(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
+template <typename RT, typename ZT, int CE>
+static void ilu_apply_ce(gm_ctx *c, const RT *r, ZT *z) {
   IluPlan &P = c->ilu;
-  constexpr int pi = sizeof(VT) == 8 ? 0 : 1;
   for (int u = 0; u < 2; u++) {
     const IluStream &T = P.sweep[u];
-    auto kern = ilu_kernel<VT, RT, ZT, CE>(T, u);
-    const size_t lds = (size_t)T.lds_rows * sizeof(VT);
+    auto kern = ilu_kernel<RT, ZT, CE>(T, u);
+    const size_t lds = (size_t)T.lds_rows * sizeof(double);
     const IluSw S{P.d_patch_row, T.d_sp, T.d_pre, T.d_idx, T.d_hptr, T.d_halo, T.d_ctl};
     for (int k = 0; k < P.ncol; k++) {
       const int col = u ? P.ncol - 1 - k : k;
@@ -1153,20 +1197,18 @@ static void ilu_apply_ce(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
       if (!cnt) continue;
       // values + columns of the triangle, the permutation, the input (gathered)
       // and output vectors
-      const double bytes = (double)(u ? P.col_nnzU[col] : P.col_nnzL[col]) * (sizeof(VT) + 4) +
-                           (double)P.col_rows[col] * (4 + (u ? 2 * sizeof(VT) + sizeof(ZT)
-                                                             : sizeof(RT) + sizeof(VT)));
+      const double bytes = (double)(u ? P.col_nnzU[col] : P.col_nnzL[col]) * 12.0 +
+                           (double)P.col_rows[col] * (4 + (u ? 16 + sizeof(ZT) : 8 + sizeof(RT)));
       gm_launch(c, u ? GM_K_ILU_UPPER : GM_K_ILU_LOWER, bytes, kern, dim3(cnt), dim3(ILU_NW * 64), lds,
-                c->stream, S, (const VT *)T.d_val[pi], (const VT *)T.d_inv[pi], p0,
-                (const int *)P.d_perm, r, ywork, z);
+                c->stream, S, (const double *)T.d_val, (const double *)T.d_tri, p0, (const int *)P.d_perm, r, P.d_y, z);
     }
   }
 }
 
-template <typename VT, typename RT, typename ZT>
-static void ilu_apply(gm_ctx *c, VT *ywork, const RT *r, ZT *z) {
-  if (c->dim == 2) ilu_apply_ce<VT, RT, ZT, 3>(c, ywork, r, z);
-  else ilu_apply_ce<VT, RT, ZT, 4>(c, ywork, r, z);
+template <typename RT, typename ZT>
+static void ilu_apply(gm_ctx *c, const RT *r, ZT *z) {
+  if (c->dim == 2) ilu_apply_ce<RT, ZT, 3>(c, r, z);
+  else ilu_apply_ce<RT, ZT, 4>(c, r, z);
 }
 
 // The orthogonalisation of w against V[0 .. nk): three launches without the
@@ -1395,7 +1437,7 @@ static int ensure_krylov(gm_ctx *c, int m, int prec) {
 // convergence ||b - A x|| / ||b - A x0|| < tol (Goma's AztecOO defaults
 // AZ_gmres / AZ_classic / AZ_r0, src/sl_util.c:392-960).
 template <typename BT, typename VT>
-static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x,
+static int gmres_t(gm_ctx *c, const VT *a, const double *b, double *x,
                    const gm_solver_opts *o, int *its_out, double *relres) {
   const int N = c->N, m = std::max(1, std::min(o->kspace, o->max_its));  // longest cycle
   KrylovWork &K = c->kry;
@@ -1416,7 +1458,7 @@ static int gmres_t(gm_ctx *c, const VT *a, VT *ywork, const double *b, double *x
     }
     if (o->precond == GM_PC_BAND)
       return gm_band_apply(c, sizeof(VT) == 8 ? (const double *)a : nullptr, (const double *)in, (double *)out);
-    if (pc) ilu_apply<VT, BT, BT>(c, ywork, in, out);
+    if (pc) ilu_apply<BT, BT>(c, in, out);
     else k_scale_into<BT><<<grid, 256, 0, c->stream>>>(N, in, 1.0, out);
     return GM_OK;
   };
@@ -1557,9 +1599,9 @@ int gm_gmres_run_nofactor(gm_ctx *c, const double *val, const float *val32, cons
     }
     // FP32 Jacobian values and preconditioner; Krylov basis, dot products
     // and the update in FP64
-    return gmres_t<double, float>(c, val32, c->ilu.d_y32, b, x, o, its, relres);
+    return gmres_t<double, float>(c, val32, b, x, o, its, relres);
   }
-  return gmres_t<double, double>(c, val, c->ilu.d_y, b, x, o, its, relres);
+  return gmres_t<double, double>(c, val, b, x, o, its, relres);
 }
 
 void gm_free_linalg(gm_ctx *c) {

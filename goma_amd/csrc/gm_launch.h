@@ -85,14 +85,8 @@ __device__ __forceinline__ T row_bcast(T v, int j) {
   }
 }
 
-// 1 / v to the last bit but one, 0 for 0: the hardware's estimate and two Newton
-// steps, half the chain of the correctly rounded division
-__device__ inline double reciprocal(double v) {
-  double y = __builtin_amdgcn_rcp(v);
-  y = fma(fma(-v, y, 1.0), y, y);
-  y = fma(fma(-v, y, 1.0), y, y);
-  return v != 0.0 ? y : 0.0;
-}
+// 1 / v, rounded, for every v (subnormal and infinite ones too), 0 for 0
+__device__ inline double reciprocal(double v) { return v != 0.0 ? 1.0 / v : 0.0; }
 __device__ inline float reciprocal(float v) { return v != 0.0f ? 1.0f / v : 0.0f; }
 
 // inclusive prefix sum over the wave (DPP row shifts, then the row totals)

@@ -64,6 +64,12 @@ __device__ inline unsigned row_max16(unsigned v) {
   return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
 }
 
+// of 64 bits: of the high words, then of their low words
+__device__ inline unsigned long long row_max16(unsigned long long v) {
+  const unsigned hi = (unsigned)(v >> 32), m = row_max16(hi);
+  return (unsigned long long)m << 32 | row_max16(hi == m ? (unsigned)v : 0u);
+}
+
 // the value of lane j of each DPP row of 16, in all of its lanes (row_newbcast)
 template <int j>
 __device__ inline double row_bcast_c(double v) {

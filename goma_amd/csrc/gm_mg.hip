@@ -67,8 +67,13 @@ __device__ inline long long local_pos(const LevelDev &L, int li, int lj) {
   return L.off_cp + (long long)k * NP + (lj - NN);
 }
 
-// The pivot's rank of |v|: 0 for a used row, 1 for a zero or a NaN, else the
-// leading bits, which order as the values do
+// The pivot's rank of |v|, all of its bits: 0 for a used row, 1 for a zero or a
+// NaN, else the bits + 2, which order as the values do
+__device__ inline unsigned long long pivot_rank(double v, bool used) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v) & ~(1ull << 63);
+  return used ? 0ull : fabs(v) > 0.0 ? b + 2ull : 1ull;
+}
+// its leading bits
 __device__ inline unsigned pivot_key(double v, bool used) {
   const unsigned hi = (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32) & 0x7fffffffu;
   return used ? 0u : fabs(v) > 0.0 ? hi + 2u : 1u;
@@ -381,8 +386,8 @@ __global__ void k_msr_to_dense(int n, const VT *__restrict__ a, const int *__res
 
 // Dense Gauss-Jordan inverse of the coarsest level with partial pivoting,
 // blocked in panels of NB columns.  Rows stay where they are: step k takes as
-// pivot the unused row with the largest entry of column k (to 20 bits; the
-// first on ties), and the finished array holds inverse row k in the row that
+// pivot the unused row with the largest entry of column k (the first on ties),
+// and the finished array holds inverse row k in the row that
 // was step k's pivot, its columns in pivot order too (k_gj_permute).
 //
 // One launch per panel, from one copy D of the array into the other, O:
@@ -394,7 +399,7 @@ __global__ void k_msr_to_dense(int n, const VT *__restrict__ a, const int *__res
 // The panel workgroup is a chain of dependent steps that the tiles hide behind
 // (for 1480 unknowns they take 17 us of the launch): thread t owns rows
 // t + NT r of the panel.  Per step each group of 16 lanes finds its candidate
-// with a 32-bit maximum (DPP rotations); the lane that holds it puts its key,
+// with two 32-bit maxima (DPP rotations); the lane that holds it puts its key,
 // its reciprocal and its row into LDS, and after the step's only barrier every
 // wave picks the winner.  The buffers alternate by step parity, so no second
 // barrier guards their reuse.  Few waves with several rows a thread: the step
@@ -422,7 +427,7 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
       int row;
     };
     __shared__ Cand s_cand[2][NG];
-    __shared__ unsigned s_key[2][NG];
+    __shared__ unsigned long long s_key[2][NG];
     __shared__ double s_old[4][NB - 4];
     __shared__ double s_turn[NW][16][17];
     // panel K + 1's columns with panel K applied, 16 rows at a time on the
@@ -499,15 +504,12 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
       for (int kk = 0; kk < 4; kk++) {
         if (c0 + kk >= nb2) continue;
         const int q = kk & 1;
-        // candidate: 0 for a used row, 1 for a zero (or NaN), else the high word + 2
-        unsigned best = 0;
+        unsigned long long best = 0;  // pivot_rank of the thread's candidate
         int br = 0;
         double cand[4] = {P[0][0], P[0][1], P[0][2], P[0][3]};
 #pragma unroll
         for (int r = 0; r < RPT; r++) {
-          const double v = fabs(P[r][kk]);
-          const unsigned hi = (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32);
-          const unsigned key = used[r] ? 0u : v > 0.0 ? hi + 2u : 1u;
+          const unsigned long long key = pivot_rank(P[r][kk], used[r]);
           if (r == 0 || key > best) {
             best = key;
             br = r;
@@ -517,8 +519,7 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
         }
         double ci = reciprocal(cand[kk]);  // every lane's, beside the chain of the maximum
         asm volatile("" : "+v"(ci));
-        const unsigned m = row_max16(best);
-        const unsigned long long at = __ballot(best == m);
+        const unsigned long long m = row_max16(best), at = __ballot(best == m);
         if (lane == 16 * lq + __ffs((unsigned)(at >> (16 * lq)) & 0xffffu) - 1) {  // the first of its 16 lanes
           Cand &c = s_cand[q][4 * w + lq];
           s_key[q][4 * w + lq] = m;
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
           for (int j = 0; j < 4; j++) c.v[j] = cand[j];
         }
         __syncthreads();
-        unsigned wk[NK], wm = 0;
+        unsigned long long wk[NK], wm = 0;
 #pragma unroll
         for (int c = 0; c < NK; c++) {
           wk[c] = s_key[q][NK * l16 + c];
@@ -546,7 +547,7 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
         const int p = __builtin_amdgcn_readfirstlane(c.row);
         if (tid == 0) {
           piv2[c0 + kk] = p;
-          if (wm == 1u) flag[3] = 1;  // singular coarse matrix
+          if (wm == 1) flag[3] = 1;  // singular coarse matrix
         }
 #pragma unroll
         for (int r = 0; r < RPT; r++) {

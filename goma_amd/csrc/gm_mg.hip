@@ -73,13 +73,13 @@ __device__ inline unsigned long long pivot_rank(double v, bool used) {
   const unsigned long long b = __builtin_bit_cast(unsigned long long, v) & ~(1ull << 63);
   return used ? 0ull : fabs(v) > 0.0 ? b + 2ull : 1ull;
 }
-// its leading bits
-__device__ inline unsigned pivot_key(double v, bool used) {
-  const unsigned hi = (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32) & 0x7fffffffu;
-  return used ? 0u : fabs(v) > 0.0 ? hi + 2u : 1u;
-}
-__device__ inline unsigned pivot_key(float v, bool used) {
+__device__ inline unsigned pivot_rank(float v, bool used) {
   return used ? 0u : fabsf(v) > 0.0f ? (__builtin_bit_cast(unsigned, v) & 0x7fffffffu) + 2u : 1u;
+}
+// v of lane i (the same i in every lane)
+__device__ inline unsigned rank_of(unsigned v, int i) { return (unsigned)__builtin_amdgcn_readlane((int)v, i); }
+__device__ inline unsigned long long rank_of(unsigned long long v, int i) {
+  return (unsigned long long)rank_of((unsigned)(v >> 32), i) << 32 | rank_of((unsigned)v, i);
 }
 
 // local matrix -> inverse (stored transposed: ainv[e][j][i] = (A_e^-1)[i][j])
@@ -87,10 +87,11 @@ __device__ inline unsigned pivot_key(float v, bool used) {
 // pivoting in compute type CT (FP64, or FP32 for the mixed precision), two
 // blocks per wave: lane i of a half holds row i in registers.  Rows stay
 // where they are; step k takes the unused row with the largest entry of
-// column k (FP64: to 20 bits; the first on ties), which passes through LDS
-// within the wave: two reads a lane, then DPP broadcasts.  The pivot row waits
-// for its scale until it is stored.  No workgroup barrier.  A structurally empty column (a local pressure mode with no
-// velocity coupling inside the element) leaves that unknown untouched.
+// column k (the first on ties), which passes through LDS within the wave: two
+// reads a lane, then DPP broadcasts.  The pivot row waits for its scale until it
+// is stored.  No workgroup barrier.  A structurally empty column (a local
+// pressure mode with no velocity coupling inside the element) leaves that
+// unknown untouched.
 // Measured (16384 blocks of 30 unknowns, FP64): 141 us against 450 with a
 // workgroup per block in LDS and three barriers a step.
 template <int DIM, int EN, typename VT, typename AT, typename CT>
@@ -130,9 +131,8 @@ __global__ __launch_bounds__(256) void k_vanka_invert(LevelDev L, int nelem, con
   // the columns move up one register a step, so that the step's is the first
 #pragma unroll 1
   for (int k = 0; k < n; k++) {
-    const unsigned key = pivot_key(P[0], used), m = row_max16(key);
-    const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)m, 0), b = (unsigned)__builtin_amdgcn_readlane((int)m, 16);
-    const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)m, 32), d = (unsigned)__builtin_amdgcn_readlane((int)m, 48);
+    const auto key = pivot_rank(P[0], used), m = row_max16(key);
+    const auto a = rank_of(m, 0), b = rank_of(m, 16), c = rank_of(m, 32), d = rank_of(m, 48);
     const unsigned long long at = __ballot(key == (lane < 32 ? max(a, b) : max(c, d)));
     const int p = __ffs(lane < 32 ? (unsigned)at : (unsigned)(at >> 32)) - 1;
     const bool is = i == p;

@@ -1392,26 +1392,35 @@ int gm_fill_setup_device(gm_ctx *c) {
   std::vector<double> stab = make_side_tables(c->dim);
   GM_HIP(hipMalloc(&c->d_stab, stab.size() * sizeof(double)));
   GM_HIP(hipMemcpy(c->d_stab, stab.data(), stab.size() * sizeof(double), hipMemcpyHostToDevice));
-  const size_t ne = (size_t)c->num_elems;
-  GM_HIP(hipMalloc(&c->d_e2nz, ne * L.total * sizeof(int)));
-  GM_HIP(hipMemsetAsync(c->d_flag, 0, 4 * sizeof(int), c->stream));
-  if (c->dim == 2)
-    k_build_e2nz<2><<<c->num_elems, 256, 0, c->stream>>>(c->d_conn, c->d_fu, c->d_centroid, c->d_bindx,
-                                                        c->energy, L.total, L.off_mp, L.off_cv,
-                                                        L.off_cp, c->d_e2nz, c->d_flag);
-  else
-    k_build_e2nz<3><<<c->num_elems, 256, 0, c->stream>>>(c->d_conn, c->d_fu, c->d_centroid, c->d_bindx,
-                                                        c->energy, L.total, L.off_mp, L.off_cv,
-                                                        L.off_cp, c->d_e2nz, c->d_flag);
-  GM_HIP(hipGetLastError());
-  int flag[4];
-  GM_HIP(hipMemcpyAsync(flag, c->d_flag, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  GM_HIP(hipStreamSynchronize(c->stream));
-  if (flag[1]) {
-    gm_set_error("element-to-nonzero map: entry missing from the MSR graph");
-    return GM_ERR_ARG;
-  }
   return gm_gather_setup(c);
+}
+
+// The element-to-nonzero map, which the multigrid's element-block inversions
+// read: built when a context becomes a level of a hierarchy.
+int gm_e2nz_setup(gm_ctx *c) {
+  if (c->d_e2nz) return GM_OK;
+  const ElemLayout &L = c->lay;
+  int *map = nullptr;
+  auto build = [&]() -> int {
+    GM_HIP(hipMalloc(&map, (size_t)c->num_elems * L.total * sizeof(int)));
+    GM_HIP(hipMemsetAsync(c->d_flag, 0, 4 * sizeof(int), c->stream));
+    auto kern = c->dim == 2 ? k_build_e2nz<2> : k_build_e2nz<3>;
+    kern<<<c->num_elems, 256, 0, c->stream>>>(c->d_conn, c->d_fu, c->d_centroid, c->d_bindx, c->energy, L.total,
+                                              L.off_mp, L.off_cv, L.off_cp, map, c->d_flag);
+    GM_HIP(hipGetLastError());
+    int flag[4];
+    GM_HIP(hipMemcpyAsync(flag, c->d_flag, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    GM_HIP(hipStreamSynchronize(c->stream));
+    if (flag[1]) {
+      gm_set_error("element-to-nonzero map: entry missing from the MSR graph");
+      return GM_ERR_ARG;
+    }
+    return GM_OK;
+  };
+  const int rc = build();
+  if (rc) (void)hipFree(map);
+  else c->d_e2nz = map;
+  return rc;
 }
 
 static int elem_buffers(gm_ctx *c) {

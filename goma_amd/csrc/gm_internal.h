@@ -179,7 +179,7 @@ struct gm_ctx {
   int *d_nn_cols = nullptr;  // per neighbour: twice its first unknown, plus 1 with P unknowns
   int nn_cap = 0;  // longest column pattern of a node (sum of its neighbours' unknowns)
   int *d_ecol_elems = nullptr;
-  int *d_e2nz = nullptr;        // [num_elems * lay.total]
+  int *d_e2nz = nullptr;        // [num_elems * lay.total], levels of a multigrid hierarchy only
   int *d_flag = nullptr;        // device error flags
   int *h_flag = nullptr;        // pinned: set by the assembly kernels on a bad element
   // node pairs of the graph with the elements that hold them (k_gather)
@@ -248,6 +248,8 @@ int gm_fill_launch(gm_ctx *c, const double *x, double *resid, double *val, float
 void gm_q2_basis(int dim, const double *xi, double *phi);  // host: Q2 basis at one reference point
 int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, float *val32,
                       int resid_only);
+
+int gm_e2nz_setup(gm_ctx *c);
 
 // element matrices to MSR rows (gm_gather.hip)
 int gm_gather_setup(gm_ctx *c);

@@ -1253,6 +1253,8 @@ extern "C" int gm_mg_add_level(gm_ctx *fine, gm_ctx *coarse, const int *P_rowptr
       gm_set_error("injection map entry outside the finer level");
       return GM_ERR_ARG;
     }
+  int rc;
+  if ((rc = gm_e2nz_setup(fine)) || (rc = gm_e2nz_setup(coarse))) return rc;
   // R = P^T
   std::vector<int> rrow(Nc + 1, 0), rcol(nnz);
   std::vector<double> rval(nnz);
@@ -1265,7 +1267,6 @@ extern "C" int gm_mg_add_level(gm_ctx *fine, gm_ctx *coarse, const int *P_rowptr
       rcol[q] = i;
       rval[q] = P_val[k];
     }
-  int rc;
   if ((rc = upv(&L.d_Prow, P_rowptr, Nf + 1)) || (rc = upv(&L.d_Pcol, P_col, nnz)) ||
       (rc = upv(&L.d_Pval, P_val, nnz)) || (rc = upv(&L.d_Rrow, rrow.data(), Nc + 1)) ||
       (rc = upv(&L.d_Rcol, rcol.data(), nnz)) || (rc = upv(&L.d_Rval, rval.data(), nnz)) ||

@@ -1,0 +1,39 @@
+"""Device memory of a context that only assembles.
+
+The element-to-nonzero map (4 bytes an entry of every element matrix) is read
+by the multigrid's block inversions alone: a context holds it once it is a
+level of a hierarchy.  Bars: what a context holds otherwise, computed from the
+mesh (MSR columns 4 bytes a nonzero; 28 bytes a coupled node pair, of which
+each has at least 9 nonzeros; 4 bytes an element's node pair; 64 bytes an
+unknown), plus half of the map.
+"""
+import pytest
+
+from goma_amd import problems
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def _free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def test_no_map_without_a_hierarchy():
+    from goma_amd import capi
+
+    capi.Context(problems.lid_cavity(n=2, dim=3)).close()  # the library's own first allocations
+    free = _free()
+    ctx = capi.Context(problems.lid_cavity(n=12, Re=100.0, dim=3, energy=True, Ra=1e3))
+    held = free - _free()
+    elems = 12 ** 3
+    entries = 16 * 27 * 27 + 2 * 3 * 27 * 4 + 16
+    print(f"[case] context memory {held / 1e6:.1f} MB, map {4e-6 * elems * entries:.1f} MB", flush=True)
+    rest = 4 * ctx.nval + 28 * ctx.nval // 9 + 4 * 27 * 27 * elems + 64 * ctx.N
+    assert held <= rest + 2 * elems * entries
+    free = _free()
+    ctx.attach_multigrid(3)
+    assert free - _free() >= 4 * elems * entries
+    ctx.close()

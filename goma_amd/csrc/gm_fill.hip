@@ -1423,9 +1423,10 @@ int gm_e2nz_setup(gm_ctx *c) {
   return rc;
 }
 
-static int elem_buffers(gm_ctx *c) {
+// ct: the continuity x temperature entries are assembled too
+static int elem_buffers(gm_ctx *c, bool ct) {
   if (!c->d_re) GM_HIP(hipMalloc(&c->d_re, (size_t)c->num_elems * (c->nv * c->nve + c->np) * sizeof(double)));
-  if (!c->d_ct) GM_HIP(hipMalloc(&c->d_ct, (size_t)c->num_elems * c->np * c->nve * sizeof(double)));
+  if (ct && !c->d_ct) GM_HIP(hipMalloc(&c->d_ct, (size_t)c->num_elems * c->np * c->nve * sizeof(double)));
   return GM_OK;
 }
 
@@ -1493,7 +1494,7 @@ int gm_fill_launch_ex(gm_ctx *c, const double *x, double *resid, double *val, fl
   *c->h_flag = 0;  // nothing that could set it is in flight: every call waits for its kernels
   a.flag = c->h_flag;
   int rc = resid_only ? GM_OK : gm_mg_kel_alloc(c);
-  if (rc || (rc = elem_buffers(c))) return rc;
+  if (rc || (rc = elem_buffers(c, !resid_only && c->energy && a.tau_pspg != 0.0))) return rc;
   a.kel = c->d_kel;
   a.re = c->d_re;
   a.ct = c->d_ct;

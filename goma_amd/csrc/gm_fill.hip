@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
     if constexpr (VISC == 1) {
       // calc_shearrate + carreau_viscosity (src/mm_fill_util.c:4564,
       // src/mm_viscosity.c:1065-1116); the derivative's powers are the
-      // viscosity's own over one factor each
+      // viscosity's own over one factor each (1 where the first overflows)
       double gd = 0.0;
 #pragma unroll
       for (int a = 0; a < DIM; a++)
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
       const double val2 = nz ? pow(A.lam * gd, A.aexp) : 0.0;
       const double pm = pow(1.0 + val2, (A.nexp - 1.0) / A.aexp);
       mu = A.muinf + (A.mu0 - A.muinf) * pm;
-      if (nz) dmu = (A.mu0 - A.muinf) * (A.nexp - 1.0) * (val2 / gd) * (pm / (1.0 + val2)) / gd;
+      if (nz) dmu = (A.mu0 - A.muinf) * (A.nexp - 1.0) * pm * (val2 > 1.0e300 ? 1.0 : val2 / (1.0 + val2)) / gd / gd;
     }
     S.P[q] = P;
     S.mu[q] = mu;
@@ -906,8 +906,9 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
         const double val2 = nz ? pow(A.lam * gd, A.aexp) : 0.0;
         const double pm = pow(1.0 + val2, (A.nexp - 1.0) / A.aexp);
         mu = A.muinf + (A.mu0 - A.muinf) * pm;
-        // d mu / d gammadot / gammadot; lam^a gd^(a-1) = val2 / gd
-        if (nz) dmu = (A.mu0 - A.muinf) * (A.nexp - 1.0) * (val2 / gd) * (pm / (1.0 + val2)) / gd;
+        // d mu / d gammadot / gammadot; lam^a gd^(a-1) = val2 / gd, and
+        // val2 / (1 + val2) is 1 where val2 overflows
+        if (nz) dmu = (A.mu0 - A.muinf) * (A.nexp - 1.0) * pm * (val2 > 1.0e300 ? 1.0 : val2 / (1.0 + val2)) / gd / gd;
       }
       double P = 0.0;
 #pragma unroll

@@ -328,7 +328,7 @@ __global__ void k_mlp_copy_out(int M, int n_out, const float *__restrict__ y, fl
 // its own rows of the weights (from L2) and nothing is staged.  Sums run over
 // the same 32-feature steps as the layer-by-layer kernels: the same bits.
 static constexpr int NET_W = 256, NET_L = 16;
-static constexpr int NET_LDS = 160 * 1024;
+static constexpr int NET_LDS = 160 * 1024, NET_STATIC = 1024;  // of a CU; most of it that is static
 
 struct NetArgs {
   int L, n_in, n_out, M, Mpad;
@@ -1004,7 +1004,7 @@ static size_t net_lds(int width, int hidden, int pts, bool train) {
 // the whole-network kernels take this network (others go layer by layer)
 static bool net_fits(const gm_mlp *m, bool train) {
   return m->s.width <= NET_W && m->L <= NET_L &&
-         (!train || net_lds(m->s.width, m->s.hidden, 32, true) <= (size_t)NET_LDS - 1024);
+         (!train || net_lds(m->s.width, m->s.hidden, 32, true) <= (size_t)NET_LDS - NET_STATIC);
 }
 
 template <bool LARGE, bool TRAIN>
@@ -1022,8 +1022,9 @@ static int net_launch(gm_mlp *m, const NetArgs &A, long long points) {
          : w == 192 ? k_mlp_net<12, 1, TM, TRAIN> : k_mlp_net<8, 2, TM, TRAIN>;
     nw = w == 64 ? 4 : w == 192 ? 12 : 8;
   }
+  // (a kernel's limit is the process's: every network sets the same)
   if (lds > 64 * 1024)
-    GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    GM_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, NET_LDS - NET_STATIC));
   kern<<<(unsigned)((points + 16 * TM - 1) / (16 * TM)), 64 * nw, lds, m->stream>>>(A);
   return GM_OK;
 }

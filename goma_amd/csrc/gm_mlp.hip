@@ -582,7 +582,7 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad_all(WgradArgs A) {
       for (int mb = mbeg; mb < mend; mb += 128) {
         u4v v[16];
 #pragma unroll
-        for (int u = 0; u < 16; u++) v[u] = *(const u4v *)(d + (mb / 32 + u / 4) * 512 + (u & 3) * 128);
+        for (int u = 0; u < 16; u++) v[u] = *(const u4v *)(d + (size_t)(mb / 32 + u / 4) * 512 + (u & 3) * 128);
 #pragma unroll
         for (int u = 0; u < 16; u++)
 #pragma unroll
@@ -618,10 +618,10 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad_all(WgradArgs A) {
     bf8 a[4][2], b[4][2];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      a[u][0] = load8(pd + (mb / 32 + u) * 512);
-      a[u][1] = load8(pd + d1 + (mb / 32 + u) * 512);
-      b[u][0] = load8(px + (mb / 32 + u) * 512);
-      b[u][1] = load8(px + x1 + (mb / 32 + u) * 512);
+      a[u][0] = load8(pd + (size_t)(mb / 32 + u) * 512);
+      a[u][1] = load8(pd + d1 + (size_t)(mb / 32 + u) * 512);
+      b[u][0] = load8(px + (size_t)(mb / 32 + u) * 512);
+      b[u][1] = load8(px + x1 + (size_t)(mb / 32 + u) * 512);
     }
 #pragma unroll
     for (int u = 0; u < 4; u++)

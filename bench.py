@@ -241,7 +241,7 @@ def kernel_roofline(name, k, prob, prec, workload):
         tr = recorded_traffic(workload, name) if prec == 0 else None
         return dict(kernel=name, bound="mfma", achieved=round(tf, 2), peak=peak, unit="TFLOP/s",
                     frac=round(tf / peak, 4), traffic=round(tr) if tr else None,
-                    flops_per_assembly=round(flops),
+                    flops_per_launch=round(flops),
                     avg_launch_ms=round(k["avg_ms"], 5),
                     precision="fp64" if prec == 0 else "fp32")
     a = k["GBps"] or 0.0

@@ -252,6 +252,36 @@ def kernel_roofline(name, k, prob, prec, workload):
                 avg_launch_ms=round(k["avg_ms"], 5))
 
 
+def assembly_roofline(k, nasm, call_bytes, prob, workload):
+    """Roofline entry of a Jacobian + residual assembly: the bytes that the call
+    cannot do without over its kernels' time.  One launch of the element kernel
+    and one of the gather make an assembly; what they write and read between
+    them (the element matrices) is in kernel_bytes_per_assembly, not in the
+    roofline."""
+    s = k["total_ms"] * 1e-3 / nasm
+    a, own = call_bytes / s / 1e9, (k["bytes_per_launch"] or 0) * k["launches"] / nasm
+    tr = recorded_traffic(workload, "k_fill")
+    out = dict(kernel="k_fill", bound="hbm", achieved=round(a, 1), peak=HBM_PEAK_GBS, unit="GB/s",
+               frac=round(a / HBM_PEAK_GBS, 4), bytes_per_assembly=round(call_bytes),
+               kernel_bytes_per_assembly=round(own), kernel_GBps=round(own / s / 1e9, 1),
+               traffic=round(tr * k["launches"] / nasm) if tr else None, per_assembly_s=round(s, 6))
+    if prob.mesh.dim == 3:
+        # HEX27 node-pair blocks on the FP64 matrix cores (k_elem3): per
+        # element and wave, 7 k-steps of 5 shared products (3 more with
+        # Carreau), 6 per momentum block row and 3 for the energy row, and
+        # 14 for the state at the points; four waves; 2 * 16 * 16 * 4 flop
+        # per v_mfma_f64_16x16x4f64
+        en, vm = int(prob.phys.energy), int(prob.phys.visc_model)
+        per_wave = 7 * ((5 + 3 * vm) + 3 * (6 + 3 * vm) + 3 * en) + 14
+        flops = 4 * per_wave * 2048.0 * prob.mesh.num_elems
+        tf = flops / s / 1e12
+        out["mfma"] = dict(bound="mfma", achieved=round(tf, 2), peak=FP64_PEAK_TFS, unit="TFLOP/s",
+                           frac=round(tf / FP64_PEAK_TFS, 4), flops_per_assembly=round(flops),
+                           note="padded 32 x 32 x 28 products over the time of the assembly (element "
+                                "matrices and gather)")
+    return out
+
+
 def learned_variants(args, torch, ctx, prob, target, x_ref, t_plain, fp64, mixed, log):
     """Previous-step and learned guesses at a Rayleigh number held out of a
     continuation sweep, in FP64 and mixed precision.
@@ -408,30 +438,11 @@ def headline(args, torch, capi):
 
     dom = max(kern, key=lambda k: kern[k]["total_ms"])
     roof = kernel_roofline(dom, kern[dom], prob, 0, prob.name)
-    # assembly: a Jacobian + residual assembly is one launch of the element
-    # kernel and one of the gather per Newton pass, both counted as k_fill
-    nasm = prep.newton_its
+    nasm = max(prep.newton_its, 1)
     k_fill = kern.get("k_fill")
-    asm_s = k_fill["total_ms"] * 1e-3 / max(nasm, 1) if k_fill else None
-    byt = algorithmic_bytes(ctx, prob, 0)
-    asm_roof = kernel_roofline("k_fill", k_fill, prob, 0, prob.name) if k_fill else None
-    if asm_roof:
-        asm_roof["per_assembly_s"] = round(asm_s, 6)
-        if prob.mesh.dim == 3:
-            # HEX27 node-pair blocks on the FP64 matrix cores (k_elem3): per
-            # element and wave, 7 k-steps of 5 shared products (3 more with
-            # Carreau), 6 per momentum block row and 3 for the energy row, and
-            # 14 for the state at the points; four waves; 2 * 16 * 16 * 4 flop
-            # per v_mfma_f64_16x16x4f64
-            en, vm = int(prob.phys.energy), int(prob.phys.visc_model)
-            per_wave = 7 * ((5 + 3 * vm) + 3 * (6 + 3 * vm) + 3 * en) + 14
-            flops = 4 * per_wave * 2048.0 * prob.mesh.num_elems
-            tf = flops / asm_s / 1e12
-            asm_roof["mfma"] = dict(bound="mfma", achieved=round(tf, 2), peak=FP64_PEAK_TFS,
-                                    unit="TFLOP/s", frac=round(tf / FP64_PEAK_TFS, 4),
-                                    flops_per_assembly=round(flops),
-                                    note="padded 32 x 32 x 28 products over the time of the assembly (element "
-                                         "matrices and gather)")
+    asm_s = k_fill["total_ms"] * 1e-3 / nasm if k_fill else None
+    asm_roof = assembly_roofline(k_fill, nasm, algorithmic_bytes(ctx, prob, 0)["asm"], prob,
+                                 prob.name) if k_fill else None
     out = {
         "metric": METRIC,
         "value": round(t_plain, 4),
@@ -462,7 +473,7 @@ def headline(args, torch, capi):
         "roofline": roof,
         "assembly": dict(asm_roof or {}, element_assemblies_per_s=(
             round(prob.mesh.num_elems / asm_s, 1) if asm_s else None),
-            GBps=round(byt["asm"] / asm_s / 1e9, 1) if asm_s else None),
+            GBps=asm_roof["achieved"] if asm_roof else None),
         "kernels": {k: {kk: (round(vv, 4) if isinstance(vv, float) else vv) for kk, vv in v.items()}
                     for k, v in kern.items()},
         "kernel_timing": ("HIP events stamped by each launch's own dispatch, on the library "

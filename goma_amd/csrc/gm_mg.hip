@@ -396,6 +396,8 @@ __global__ void k_msr_to_dense(int n, const VT *__restrict__ a, const int *__res
 //     rows zeroed; panel K's own columns become Pan;
 //   the first workgroup meanwhile brings panel K + 1 up to date in registers
 //     and runs its column steps.
+// A panel's terms of an entry are added up from zero and to the entry once:
+// added one by one they left 1.6 times the residual (1059 unknowns).
 // The panel workgroup is a chain of dependent steps that the tiles hide behind
 // (for 1480 unknowns they take 17 us of the launch): thread t owns rows
 // t + NT r of the panel.  Per step each group of 16 lanes finds its candidate
@@ -432,7 +434,8 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
     __shared__ double s_turn[NW][16][17];
     // panel K + 1's columns with panel K applied, 16 rows at a time on the
     // matrix cores (as the tiles below), turned through LDS to a row per thread
-    constexpr int RB = RPT * NT <= 1536 ? RPT : 1;  // rows loaded together, as registers allow
+    // rows loaded together and sets of 16 lanes of them, as registers allow
+    constexpr int RB = NT == 256 ? RPT : 1, MB = NT == 1024 ? 2 : 4;
     double P[RPT][NB], bk[NB / 4];
     bool used[RPT];
 #pragma unroll
@@ -448,48 +451,51 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
       zero[r] = __ballot(i >= n || (nb > 0 && at >= kb && at < kb + nb));
     }
 #pragma unroll
-    for (int r0 = 0; r0 < RPT; r0 += RB) {
-      d4 C[RB][4];
-      double f[RB][4][NB / 4];
+    for (int r0 = 0; r0 < RPT; r0 += RB)
 #pragma unroll
-      for (int r = 0; r < RB; r++) {
-        const int ib = NT * (r0 + r) + 64 * w;
+      for (int m0 = 0; m0 < 4; m0 += MB) {
+        d4 B[RB][MB], C[RB][MB];  // the columns before, what panel K adds
+        double f[RB][MB][NB / 4];
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
+        for (int r = 0; r < RB; r++) {
+          const int ib = NT * (r0 + r) + 64 * w + 16 * m0;
 #pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const int row = 16 * m + lq + 4 * e;
-            // past the last column: another row's, or the margin; unused
-            C[r][m][e] = (zero[r0 + r] >> row) & 1 ? 0.0 : D[(size_t)(ib + row) * n + kb2 + l16];
-          }
+          for (int m = 0; m < MB; m++) {
 #pragma unroll
-          for (int k = 0; k < NB / 4; k++) {
-            const int t = 4 * k + lq;
-            f[r][m][k] = t < nb && ib + 16 * m + l16 < n ? pan[(size_t)t * n + ib + 16 * m + l16] : 0.0;
+            for (int e = 0; e < 4; e++) {
+              const int row = 16 * m + lq + 4 * e;
+              // past the last column: another row's, or the margin; unused
+              B[r][m][e] = (zero[r0 + r] >> (16 * m0 + row)) & 1 ? 0.0 : D[(size_t)(ib + row) * n + kb2 + l16];
+            }
+            C[r][m] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k = 0; k < NB / 4; k++) {
+              const int t = 4 * k + lq;
+              f[r][m][k] = t < nb && ib + 16 * m + l16 < n ? pan[(size_t)t * n + ib + 16 * m + l16] : 0.0;
+            }
           }
         }
+        if (nb > 0)
+#pragma unroll
+          for (int k = 0; k < NB / 4; k++)
+#pragma unroll
+            for (int r = 0; r < RB; r++)
+#pragma unroll
+              for (int m = 0; m < MB; m++)
+                C[r][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[r][m][k], bk[k], C[r][m], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+          for (int m = 0; m < MB; m++) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int e = 0; e < 4; e++) s_turn[w][lq + 4 * e][l16] = B[r][m][e] + C[r][m][e];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (lq == m0 + m)
+#pragma unroll
+              for (int j = 0; j < NB; j++) P[r0 + r][j] = s_turn[w][l16][j];
+          }
       }
-      if (nb > 0)
-#pragma unroll
-        for (int k = 0; k < NB / 4; k++)
-#pragma unroll
-          for (int r = 0; r < RB; r++)
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-              C[r][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[r][m][k], bk[k], C[r][m], 0, 0, 0);
-#pragma unroll
-      for (int r = 0; r < RB; r++)
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-          for (int e = 0; e < 4; e++) s_turn[w][lq + 4 * e][l16] = C[r][m][e];
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          if (lq == m)
-#pragma unroll
-            for (int j = 0; j < NB; j++) P[r0 + r][j] = s_turn[w][l16][j];
-        }
-    }
     int step[RPT];
 #pragma unroll
     for (int r = 0; r < RPT; r++) step[r] = -1;
@@ -619,7 +625,7 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
   const int tx = (n + 63) / 64, task = ((int)blockIdx.x - 1) * NW + w;
   const int i0 = task / tx * 16, j0 = (task - task / tx * tx) * 64;
   if (i0 >= n) return;
-  d4 C[4];
+  d4 B[4], C[4];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int i = i0 + lq + 4 * r;
@@ -628,7 +634,8 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       const int j = j0 + 16 * c + l16;
-      C[c][r] = zero || j >= n ? 0.0 : D[(size_t)i * n + j];
+      B[c][r] = zero || j >= n ? 0.0 : D[(size_t)i * n + j];
+      C[c][r] = 0.0;
     }
   }
 #pragma unroll
@@ -651,7 +658,7 @@ __global__ __launch_bounds__(NT) void k_gjb_step(int n, int kb, int nb, int kb2,
     for (int c = 0; c < 4; c++) {
       const int j = j0 + 16 * c + l16;
       if (j >= n || (j >= kb2 && j < kb2 + nb2)) continue;  // the next launch writes panel K + 1
-      O[(size_t)i * n + j] = j >= kb && j < kb + nb ? pan[(size_t)(j - kb) * n + i] : C[c][r];
+      O[(size_t)i * n + j] = j >= kb && j < kb + nb ? pan[(size_t)(j - kb) * n + i] : B[c][r] + C[c][r];
     }
   }
 }

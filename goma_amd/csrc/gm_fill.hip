@@ -956,7 +956,7 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
   const bool node = j < NVE;
   double *__restrict__ re = A.re + (size_t)e * NL;
   double *__restrict__ K = A.kel + (size_t)e * A.E;
-  d4v A1 = z, L1 = z, Dadv = z, Lmu = z;
+  d4v A1 = z, Lp[DIM] = {z, z, z}, Dadv = z, Lmu = z;
   if (!A.resid_only) {
 #pragma unroll 1
     for (int q = kk; q < KP; q += 4) {
@@ -969,7 +969,7 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
 #pragma unroll
       for (int p = 0; p < DIM; p++) {
         const double gA = s_G[p][q][ii] * dAq, gB = s_G[p][q][j];
-        L1 = GM_MFMA64(gA, gB, L1);
+        Lp[p] = GM_MFMA64(gA, gB, Lp[p]);
         if constexpr (VISC == 1) Lmu = GM_MFMA64(gA * s_mu[q], gB, Lmu);
       }
     }
@@ -979,9 +979,10 @@ __global__ __launch_bounds__(256, 4) void k_elem3(FillArgs A) {
       const double dAq = s_dA[q];
       A1 = GM_MFMA64(s_Phi[q][ii] * dAq, s_Phi[q][j], A1);
 #pragma unroll
-      for (int p = 0; p < DIM; p++) L1 = GM_MFMA64(s_G[p][q][ii] * dAq, s_G[p][q][j], L1);
+      for (int p = 0; p < DIM; p++) Lp[p] = GM_MFMA64(s_G[p][q][ii] * dAq, s_G[p][q][j], Lp[p]);
     }
   }
+  const d4v L1 = Lp[0] + Lp[1] + Lp[2];
   if (j >= NVE && j < NVE + NV) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {

@@ -166,10 +166,10 @@ __device__ inline void supg_params(double s, const XA &x, const double *vc, doub
 // them into the MSR rows.  All elements are one launch.
 // Bound by the element matrices' traffic for large meshes and by the chain of
 // phases (about 10 us) for small ones.  Measured (assembly of 128 x 128
-// shear-thinning elements with energy, FP64): 209 us with k_gather
-// against 408 with four coloured launches of a workgroup per element, a
+// shear-thinning elements with energy, FP64): 206 us with k_gather
+// against 406 with four coloured launches of a workgroup per element, a
 // thread per node pair and += through the element-to-nonzero map; 16 x 16
-// cavity 59 us against 98.
+// cavity 60 us against 100.
 typedef double d4v __attribute__((ext_vector_type(4)));
 
 // entry r of n tiles to n neighbouring places, 16 bytes at a time
@@ -669,9 +669,9 @@ __global__ __launch_bounds__(256, EN && VISC ? 4 : 5) void k_elem2(FillArgs A, i
 // (ct); k_gather sums them into the MSR rows.
 // Bound by the element matrices' bytes (98 KB an element with energy) and the
 // 182 products a wave (64 cycles each).  Measured, with k_gather (16^3
-// elements with energy, FP64): 449 us against 743 with eight coloured
+// elements with energy, FP64): 430 us against 742 with eight coloured
 // launches that staged the state by threads and added into the rows through a
-// rank map; 11^3 shear-thinning, FP32 matrix: 198 against 629.
+// rank map; 11^3 shear-thinning, FP32 matrix: 194 against 625.
 
 struct NodeCols {  // coordinates as x[a][i] from rows of 16 doubles a node
   const double *p;

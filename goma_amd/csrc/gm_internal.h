@@ -259,7 +259,6 @@ int gm_gather(gm_ctx *prof, int id, gm_ctx *c, hipStream_t s, const double *kel,
 
 // linear algebra (gm_linalg.hip)
 int gm_zero(gm_ctx *c, double *p, long long n);
-int gm_zero32(gm_ctx *c, float *p, long long n);
 int gm_scale_launch(gm_ctx *c, double *val, float *val32, double *b, double *scale);
 int gm_norms(gm_ctx *c, const double *v, long long n, double *l2, double *loo);
 // PSPG: mean square of the velocity unknowns of x (device), the mesh's mean

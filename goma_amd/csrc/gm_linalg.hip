@@ -1,8 +1,9 @@
 // Linear algebra on the MSR Jacobian: row-sum scaling, norms, SpMV,
 // ILU(0) in patch order, restarted right-preconditioned GMRES.
 //
-// All reductions are two-stage (per-block partials, then a fixed-order sum on
-// the host), so results are bitwise reproducible run to run.
+// All reductions are two-stage (per-block partials, then a fixed-order sum: on
+// the host, or for GMRES's projections and norms in the kernel that uses them),
+// so results are bitwise reproducible run to run.
 #include <algorithm>
 #include <type_traits>
 #include <cmath>
@@ -44,11 +45,6 @@ __global__ void k_fill_value(T *p, long long n, T v) {
 
 int gm_zero(gm_ctx *c, double *p, long long n) {
   k_fill_value<double><<<2048, 256, 0, c->stream>>>(p, n, 0.0);
-  GM_HIP(hipGetLastError());
-  return GM_OK;
-}
-int gm_zero32(gm_ctx *c, float *p, long long n) {
-  k_fill_value<float><<<2048, 256, 0, c->stream>>>(p, n, 0.0f);
   GM_HIP(hipGetLastError());
   return GM_OK;
 }
@@ -785,7 +781,7 @@ static int ilu_factor_colour(gm_ctx *c, VT *lu, int p0, int cnt) {
 
 // gather MSR values into the permuted CSR
 template <typename VT, typename DT>
-__global__ void k_gather(long long n, const int *__restrict__ src, const VT *__restrict__ a,
+__global__ void k_ilu_gather(long long n, const int *__restrict__ src, const VT *__restrict__ a,
                          DT *__restrict__ lu) {
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x)
@@ -1158,10 +1154,10 @@ int gm_ilu_factor(gm_ctx *c, const double *val, const float *val32, int prec) {
   if (rc) return rc;
   GM_HIP(hipMemsetAsync(c->d_flag + 2, 0, sizeof(int), c->stream));
   if (prec == GM_PREC_MIXED) {
-    if (val32) k_gather<float, float><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val32, P.d_lu32);
-    else k_gather<double, float><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val, P.d_lu32);
+    if (val32) k_ilu_gather<float, float><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val32, P.d_lu32);
+    else k_ilu_gather<double, float><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val, P.d_lu32);
   } else {
-    k_gather<double, double><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val, P.d_lu);
+    k_ilu_gather<double, double><<<4096, 256, 0, c->stream>>>(P.nnz, P.d_src, val, P.d_lu);
   }
   for (int col = 0; col < P.ncol; col++) {
     const int p0 = P.colour_ptr[col], cnt = P.colour_ptr[col + 1] - p0;

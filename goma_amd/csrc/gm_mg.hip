@@ -13,7 +13,7 @@
 // the colour's updates, so the sweep is deterministic (block Gauss-Seidel
 // across colours, block Jacobi within a colour).  The local inverses are
 // formed once per Newton step by Gauss-Jordan elimination with partial
-// pivoting in LDS.
+// pivoting in registers.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -92,7 +92,7 @@ __device__ inline unsigned long long rank_of(unsigned long long v, int i) {
 // is stored.  No workgroup barrier.  A structurally empty column (a local
 // pressure mode with no velocity coupling inside the element) leaves that
 // unknown untouched.
-// Measured (16384 blocks of 30 unknowns, FP64): 141 us against 450 with a
+// Measured (16384 blocks of 30 unknowns, FP64): 186 us against 450 with a
 // workgroup per block in LDS and three barriers a step.
 template <int DIM, int EN, typename VT, typename AT, typename CT>
 __global__ __launch_bounds__(256) void k_vanka_invert(LevelDev L, int nelem, const VT *__restrict__ val,
@@ -406,7 +406,7 @@ __global__ void k_msr_to_dense(int n, const VT *__restrict__ a, const int *__res
 // wave picks the winner.  The buffers alternate by step parity, so no second
 // barrier guards their reuse.  Few waves with several rows a thread: the step
 // is latency, not work.
-// Measured: 32 us a panel of 16 for 1480 unknowns, 22 for 532, 14 for 87,
+// Measured: 33 us a panel of 16 for 1480 unknowns, 22 for 532, 14 for 87,
 // against 80, 59 and 46 with row interchanges, two barriers a step and launches
 // of their own for the panel, the interchanges and the update; the rows'
 // final order costs 9 us instead of 295.
@@ -930,18 +930,6 @@ static std::string build_galerkin_maps(const gm_ctx *f, const gm_ctx *c, const i
   return "";
 }
 
-// Coarse element matrices P_e^T K_e P_e summed over the children of each coarse
-// element, in the element matrices' layout: nodal block rows a as [i][j][b],
-// then momentum x P, continuity x velocity, P x P.
-//
-// A workgroup takes RW block rows of one coarse element (HEX27: one, QUAD9:
-// all), another its pressure couplings: the blocks are independent, and with
-// one workgroup for all of them the levels of up to a few hundred elements
-// leave most of the chip idle behind 128 rounds of three barriers (64 coarse
-// elements with energy, FP64: 57 us against 580).  Per child: K_e's rows from
-// memory a child ahead, T = K W over them in LDS, W^T T summed in registers.
-// Larger levels are bound by reading the finer element matrices once (1728
-// coarse elements with energy, FP32 products: 353 us for 1.4 GB).
 // One weight of a child's nodal interpolation and the finer node it is for
 template <typename CT>
 struct alignas(2 * sizeof(CT)) GalW {
@@ -967,6 +955,18 @@ __device__ inline void load_cols(const CT *p, CT *v) {
   }
 }
 
+// Coarse element matrices P_e^T K_e P_e summed over the children of each coarse
+// element, in the element matrices' layout: nodal block rows a as [i][j][b],
+// then momentum x P, continuity x velocity, P x P.
+//
+// A workgroup takes RW block rows of one coarse element (HEX27: one, QUAD9:
+// all), another its pressure couplings: the blocks are independent, and with
+// one workgroup for all of them the levels of up to a few hundred elements
+// leave most of the chip idle behind 128 rounds of three barriers (64 coarse
+// elements with energy, FP64: 57 us against 580).  Per child: K_e's rows from
+// memory a child ahead, T = K W over them in LDS, W^T T summed in registers.
+// Larger levels are bound by reading the finer element matrices once (1728
+// coarse elements with energy, FP32 products: 353 us for 1.4 GB).
 template <int DIM, int EN, typename CT>
 __global__ __launch_bounds__(256) void k_galerkin(const double *__restrict__ kf,
                                                   const int *__restrict__ child,

@@ -54,7 +54,7 @@ extern "C" {
 #define GM_VAR_P 9
 
 #define GM_PREC_FP64 0   /* Jacobian, ILU and Krylov in FP64 */
-#define GM_PREC_MIXED 1  /* Jacobian values, ILU and inner Krylov FP32; R, dots, update FP64 */
+#define GM_PREC_MIXED 1  /* Jacobian values and preconditioner FP32 (ILU sweeps FP64); R, dots, update FP64 */
 
 #define GM_PC_NONE 0
 #define GM_PC_ILU0 1     /* ILU(0) in patch order (see gm_solver_opts.patch_bins) */
@@ -374,7 +374,8 @@ int gm_mg_copy_coarse_inverse(const gm_ctx *ctx, double *out);
  * events that their own dispatch stamps (hipExtLaunchKernel), so a duration
  * is the kernel's execution alone; gm_prof_get returns the launch count, the
  * summed duration and the summed algorithmic HBM bytes (compulsory traffic,
- * each array counted once per launch) of those launches. */
+ * each array counted once per launch, scratch between launches such as the
+ * assembly's element matrices included) of those launches. */
 #define GM_K_FILL 0       /* assembly: k_elem2 / k_elem3, the element matrices, and k_gather, the rows */
 #define GM_K_SPMV 1       /* k_spmv_msr: MSR matvec */
 #define GM_K_ILU_LOWER 2  /* k_ilu_sweep: forward sweep of one patch colour */
@@ -463,11 +464,11 @@ int gm_mlp_predict_dev(gm_mlp *m, long long npts, const float *in_dev, float *ou
 int gm_mlp_predict(gm_mlp *m, long long npts, const float *in, float *out);
 /* Allocation-free gm_mlp_predict_dev: no counterpart in the reference; for
  * callers that cannot allocate device memory (code under HIP graph capture,
- * tight serving loops, harnesses that forbid hipMalloc).  Activations and
- * outputs pass through a scratch array the library keeps on each GPU for the
- * life of the process (two 2048-point x 512-feature BF16 buffers and
- * 2048 x 64 FP32 outputs, 4.5 MiB), 2048 points at a time, so any npts is
- * accepted; a network with a layer wider than 512 features is refused with
+ * tight serving loops, harnesses that forbid hipMalloc).  Networks up to 256 wide keep their activations in LDS; those of
+ * wider ones, and their outputs, pass through a scratch array the library keeps
+ * on each GPU for the life of the process (two 2048-point x 512-feature BF16
+ * buffers and 2048 x 64 FP32 outputs, 4.5 MiB), 2048 points at a time.  Any
+ * npts is accepted; a network with a layer wider than 512 features is refused with
  * GM_ERR_ARG.  Calls on one GPU share its scratch: calls that overlap on one
  * GPU race.  Makes no hipMalloc or hipFree call.  Same outputs as
  * gm_mlp_predict_dev, bit for bit. */

@@ -44,3 +44,24 @@ def test_residual_is_rounding(name, seed, make, oracle_mod):
     n = np.diff(A.indptr)
     bar = 2 * np.finfo(float).eps * np.linalg.norm((n + 1) * (abs(A) @ abs(z) + abs(r)))
     assert np.linalg.norm(r - A @ z) <= bar
+
+
+@pytest.mark.parametrize("reuse", [1, 2])
+def test_reused_factors_are_not_refined_with_another_matrix(reuse):
+    """Factors kept from the first pass (or while they serve) precondition the
+    later matrices as they are; Newton ends where fresh factors take it."""
+    from goma_amd import capi
+
+    prob = problems.natural_convection(n=8, Ra=1e3, carreau=True, jitter=0.15)
+    ctx = capi.Context(prob)
+    sol = []
+    for r in (0, reuse):
+        print(f"[case] newton band pc_reuse={r}", flush=True)
+        xd = torch.zeros(ctx.N, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        _, rep = ctx.solve_dev(xd.data_ptr(), kspace=40, max_its=200, precond=3, line_search=1, pc_reuse=r)
+        assert rep.converged
+        assert rep.pc_builds < rep.newton_its if r else rep.pc_builds >= rep.newton_its - 1
+        sol.append(xd.cpu().numpy())
+    ctx.close()
+    assert np.abs(sol[1] - sol[0]).max() <= 1e-9 * np.abs(sol[0]).max()
